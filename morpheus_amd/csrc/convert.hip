@@ -107,21 +107,47 @@ __global__ __launch_bounds__(kT) void row_hist_kernel(const int32_t* __restrict_
   lds_histogram(nnz, cnt, [&](int64_t i) { return ri[i]; });
 }
 
-__global__ void max_kernel(const int32_t* __restrict__ a, int64_t n,
-                           int32_t* __restrict__ out) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) atomicMax(out, a[i]);
+// Reductions to one word: a workgroup strides over the array, reduces in
+// registers and LDS, and adds its result with one atomic.  An atomic per
+// element on one address was served one at a time: the maxima of 14.6M COO
+// indices took 2.6 ms, now about 15 us (the 58 MB read at the stream rate).
+constexpr int64_t kReduceBlocks = 2048;
+inline unsigned reduce_blocks(int64_t n) {
+  return (unsigned)std::min<int64_t>(blocks_for(n, 4 * kT), kReduceBlocks);
 }
 
-// sum over rows of min(cnt[r], K) -> out (int64 via two int32 atomics is
-// avoided: per-thread values fit, totals use unsigned long long atomics)
-__global__ void clipped_sum_kernel(const int32_t* __restrict__ cnt, int64_t n,
-                                   int32_t K, unsigned long long* out) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) {
-    const int32_t c = cnt[i];
-    atomicAdd(out, (unsigned long long)(c < K ? c : K));
-  }
+template <typename T, typename Op>
+__device__ __forceinline__ T block_reduce(T v, Op op) {
+  __shared__ T part[kT / kWave];
+  for (int d = kWave / 2; d > 0; d >>= 1) v = op(v, shfl_xor(v, d));
+  __syncthreads();  // (the previous reduction's partials are read)
+  if (threadIdx.x % kWave == 0) part[threadIdx.x / kWave] = v;
+  __syncthreads();
+  v = part[0];
+  for (int w = 1; w < kT / kWave; w++) v = op(v, part[w]);
+  return v;
+}
+
+// the largest of a[0, n) and 0
+__global__ __launch_bounds__(kT) void max_kernel(const int32_t* __restrict__ a, int64_t n,
+                                                 int32_t* __restrict__ out) {
+  const int64_t step = (int64_t)gridDim.x * kT;
+  int32_t m = 0;
+  for (int64_t i = (int64_t)blockIdx.x * kT + threadIdx.x; i < n; i += step) m = max(m, a[i]);
+  m = block_reduce(m, [](int32_t u, int32_t v) { return max(u, v); });
+  if (threadIdx.x == 0 && m > 0) atomicMax(out, m);
+}
+
+// sum over rows of min(cnt[r], K)
+__global__ __launch_bounds__(kT) void clipped_sum_kernel(const int32_t* __restrict__ cnt,
+                                                         int64_t n, int32_t K,
+                                                         unsigned long long* out) {
+  const int64_t step = (int64_t)gridDim.x * kT;
+  unsigned long long t = 0;
+  for (int64_t i = (int64_t)blockIdx.x * kT + threadIdx.x; i < n; i += step)
+    t += (unsigned long long)min(cnt[i], K);
+  t = block_reduce(t, [](unsigned long long u, unsigned long long v) { return u + v; });
+  if (threadIdx.x == 0 && t > 0) atomicAdd(out, t);
 }
 
 __global__ void unsorted_kernel(const int32_t* __restrict__ ri,
@@ -368,8 +394,8 @@ int sort_coo(int64_t nnz, int64_t nrows, int64_t ncols, int32_t* ri, int32_t* ci
   int32_t* mx;
   MPH_CHECK_STATUS(t.alloc(&mx, 2));
   MPH_CHECK_STATUS(fill_i32(mx, 2, 0, s));
-  hipLaunchKernelGGL(max_kernel, dim3(blocks_for(nnz)), dim3(kT), 0, s, ri, nnz, mx);
-  hipLaunchKernelGGL(max_kernel, dim3(blocks_for(nnz)), dim3(kT), 0, s, ci, nnz, mx + 1);
+  hipLaunchKernelGGL(max_kernel, dim3(reduce_blocks(nnz)), dim3(kT), 0, s, ri, nnz, mx);
+  hipLaunchKernelGGL(max_kernel, dim3(reduce_blocks(nnz)), dim3(kT), 0, s, ci, nnz, mx + 1);
   int32_t hm[2];
   MPH_HIP_CHECK(hipMemcpyAsync(hm, mx, sizeof(hm), hipMemcpyDeviceToHost, s));
   MPH_HIP_CHECK(hipStreamSynchronize(s));
@@ -657,16 +683,28 @@ __global__ void compact_offsets_kernel(const int32_t* __restrict__ flag,
 }
 
 // HDC sizes: selected diagonals (cnt >= thr), their entries, the rest
-__global__ void hdc_sizes_kernel(const int32_t* __restrict__ cnt, int64_t n, int32_t thr,
-                                 unsigned long long* out /* ndiag, dia_nnz, csr_nnz */) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const int32_t c = cnt[i];
-  if (c >= thr) {
-    atomicAdd(&out[0], 1ull);
-    atomicAdd(&out[1], (unsigned long long)c);
-  } else if (c != 0) {
-    atomicAdd(&out[2], (unsigned long long)c);
+__global__ __launch_bounds__(kT) void hdc_sizes_kernel(
+    const int32_t* __restrict__ cnt, int64_t n, int32_t thr,
+    unsigned long long* out /* ndiag, dia_nnz, csr_nnz */) {
+  const int64_t step = (int64_t)gridDim.x * kT;
+  unsigned long long nd = 0, in = 0, rest = 0;
+  for (int64_t i = (int64_t)blockIdx.x * kT + threadIdx.x; i < n; i += step) {
+    const int32_t c = cnt[i];
+    if (c >= thr) {
+      nd++;
+      in += c;
+    } else {
+      rest += c;
+    }
+  }
+  auto add = [](unsigned long long u, unsigned long long v) { return u + v; };
+  nd = block_reduce(nd, add);
+  in = block_reduce(in, add);
+  rest = block_reduce(rest, add);
+  if (threadIdx.x == 0) {
+    if (nd) atomicAdd(&out[0], nd);
+    if (in) atomicAdd(&out[1], in);
+    if (rest) atomicAdd(&out[2], rest);
   }
 }
 
@@ -926,7 +964,7 @@ int mph_convert_coo_to_ell_size(int64_t nrows, int64_t nnz, const int32_t* ri, i
   MPH_CHECK_STATUS(t.alloc(&mx, 1));
   MPH_CHECK_STATUS(fill_i32(mx, 1, 0, s));
   if (nrows > 0)
-    hipLaunchKernelGGL(max_kernel, dim3(blocks_for(nrows)), dim3(kT), 0, s, cnt, nrows, mx);
+    hipLaunchKernelGGL(max_kernel, dim3(reduce_blocks(nrows)), dim3(kT), 0, s, cnt, nrows, mx);
   MPH_HIP_CHECK(hipGetLastError());
   int32_t h = 0;
   MPH_CHECK_STATUS(sync_read_i32(mx, &h, s));
@@ -1015,7 +1053,7 @@ int mph_convert_coo_to_hyb_size(int64_t nrows, int64_t nnz, const int32_t* ri, i
   MPH_CHECK_STATUS(row_counts(ri, nnz, nrows, t, &cnt, s));
   MPH_CHECK_STATUS(t.alloc(&acc, 1));
   MPH_CHECK_STATUS(fill_zero(acc, sizeof(unsigned long long), s));
-  hipLaunchKernelGGL(clipped_sum_kernel, dim3(blocks_for(nrows)), dim3(kT), 0, s, cnt, nrows,
+  hipLaunchKernelGGL(clipped_sum_kernel, dim3(reduce_blocks(nrows)), dim3(kT), 0, s, cnt, nrows,
                      (int32_t)std::min<int64_t>(k, INT32_MAX), acc);
   MPH_HIP_CHECK(hipGetLastError());
   unsigned long long h = 0;
@@ -1141,7 +1179,7 @@ int mph_convert_coo_to_hdc_size(int64_t nrows, int64_t ncols, int64_t nnz, const
   if (nnz > 0)
     hipLaunchKernelGGL(diag_hist_kernel, dim3(hist_blocks(nnz)), dim3(kT), 0, s, ri, ci, nnz,
                        nrows, cnt);
-  hipLaunchKernelGGL(hdc_sizes_kernel, dim3(blocks_for(nb)), dim3(kT), 0, s, cnt, nb, thr, acc);
+  hipLaunchKernelGGL(hdc_sizes_kernel, dim3(reduce_blocks(nb)), dim3(kT), 0, s, cnt, nb, thr, acc);
   MPH_HIP_CHECK(hipGetLastError());
   unsigned long long h[3];
   MPH_HIP_CHECK(hipMemcpyAsync(h, acc, sizeof(h), hipMemcpyDeviceToHost, s));
