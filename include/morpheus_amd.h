@@ -78,7 +78,8 @@ const char* mph_last_error(void);
  * the reference re-queries them on every launch
  * (core/src/impl/Morpheus_HIPUtils.hpp:77-90). */
 int mph_initialize(int device);
-/* Morpheus::finalize (core/src/impl/Morpheus_Core.cpp:215-222). */
+/* Morpheus::finalize (core/src/impl/Morpheus_Core.cpp:215-222): gives back
+ * the memory that the library keeps for temporaries. */
 int mph_finalize(void);
 
 /* ------------------------------------------------------------ matrices */
@@ -286,9 +287,14 @@ int mph_ell_multiply(int64_t nrows, int64_t ncols, int64_t nnz,
  * (core/src/impl/<Fmt>/Serial/Morpheus_Convert_Impl.hpp).  The reference
  * HIP converters throw NotImplementedException
  * (core/src/impl/Csr/HIP/Morpheus_Convert_Impl.hpp:39-76); these succeed.
- * Size queries synchronise `stream`; fills are asynchronous but use
- * stream-ordered temporary allocations.  Output arrays are caller-owned and
- * sized from the size queries. */
+ * Size queries synchronise `stream`; fills may be asynchronous, and use
+ * temporary arrays of the library's own, which keeps up to 2 GiB of them
+ * until mph_finalize; a call whose temporaries the device still reads waits
+ * for `stream` before it returns.  Output arrays are caller-owned and sized
+ * from the size queries; every entry is written.
+ * Between CSR and COO, ci_out and v_out may be the input's ci and v: the
+ * entries then stay where they are (or, COO rows not sorted, are sorted in
+ * place). */
 
 /* core/src/impl/Csr/Serial/Morpheus_Convert_Impl.hpp:66-97 */
 int mph_convert_csr_to_coo(int64_t nrows, int64_t nnz,

@@ -5,6 +5,8 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <utility>
+#include <vector>
 
 #include "mph_internal.hpp"
 
@@ -15,9 +17,100 @@ thread_local std::string g_last_error;
 std::mutex g_dev_mutex;
 int g_cu_count = 0;
 int g_cu_device = -1;
+
+// free blocks of temporaries, per device (-1: pinned host memory)
+struct TmpCache {
+  std::mutex m;
+  std::vector<std::pair<int, TmpBlock>> blocks;
+  size_t bytes = 0;
+};
+TmpCache& tmp_cache() {
+  static TmpCache* c = new TmpCache;  // lives as long as the process
+  return *c;
+}
+int tmp_device(bool host) {
+  int dev = 0;
+  if (host || hipGetDevice(&dev) != hipSuccess) return -1;
+  return dev;
+}
+void tmp_release(const TmpBlock& b) {
+  if (b.host)
+    (void)hipHostFree(b.p);
+  else
+    (void)hipFree(b.p);
+}
 }  // namespace
 
 void set_error(const std::string& msg) { g_last_error = msg; }
+
+int tmp_take(TmpBlock* b, size_t bytes, bool host) {
+  // sizes in steps of an eighth of their power of two, at least 4 KiB, so
+  // that calls of like size share blocks
+  size_t step = 4096;
+  while (step * 16 <= bytes) step <<= 1;
+  bytes = (bytes + step - 1) / step * step;
+  const int dev = tmp_device(host);
+  TmpCache& c = tmp_cache();
+  {
+    std::lock_guard<std::mutex> lk(c.m);
+    size_t best = c.blocks.size();
+    for (size_t i = 0; i < c.blocks.size(); i++) {
+      const TmpBlock& f = c.blocks[i].second;
+      if (c.blocks[i].first == dev && f.host == host && f.bytes >= bytes &&
+          f.bytes <= std::max<size_t>(4 * bytes, 1 << 16) &&
+          (best == c.blocks.size() || f.bytes < c.blocks[best].second.bytes))
+        best = i;
+    }
+    if (best < c.blocks.size()) {
+      *b = c.blocks[best].second;
+      c.bytes -= b->bytes;
+      c.blocks.erase(c.blocks.begin() + best);
+      return MPH_OK;
+    }
+  }
+  b->bytes = bytes;
+  b->host = host;
+  auto get = [&]() {
+    return host ? hipHostMalloc(&b->p, bytes, hipHostMallocDefault) : hipMalloc(&b->p, bytes);
+  };
+  hipError_t e = get();
+  if (e == hipErrorOutOfMemory) {
+    (void)hipGetLastError();
+    tmp_trim();
+    e = get();
+  }
+  if (e != hipSuccess) {
+    b->p = nullptr;
+    set_error(std::string("temporary: ") + hipGetErrorString(e));
+    return e == hipErrorOutOfMemory ? MPH_ERR_OUT_OF_MEMORY : MPH_ERR_HIP;
+  }
+  return MPH_OK;
+}
+
+void tmp_give(const TmpBlock& b) {
+  const int dev = tmp_device(b.host);
+  TmpCache& c = tmp_cache();
+  {
+    std::lock_guard<std::mutex> lk(c.m);
+    if (c.bytes + b.bytes <= kTmpKeepBytes && c.blocks.size() < kTmpKeepBlocks) {
+      c.blocks.emplace_back(dev, b);
+      c.bytes += b.bytes;
+      return;
+    }
+  }
+  tmp_release(b);
+}
+
+void tmp_trim() {
+  TmpCache& c = tmp_cache();
+  std::vector<std::pair<int, TmpBlock>> out;
+  {
+    std::lock_guard<std::mutex> lk(c.m);
+    out.swap(c.blocks);
+    c.bytes = 0;
+  }
+  for (auto& f : out) tmp_release(f.second);
+}
 
 int device_cu_count() {
   int dev = 0;
@@ -357,7 +450,10 @@ int mph_initialize(int device) {
   return noalloc_scratch(&scratch);
 }
 
-int mph_finalize(void) { return MPH_OK; }
+int mph_finalize(void) {
+  tmp_trim();
+  return MPH_OK;
+}
 
 int mph_matrix_create_coo(mph_matrix_t* out, int64_t nrows, int64_t ncols,
                           int64_t nnz, const int32_t* ri, const int32_t* ci,

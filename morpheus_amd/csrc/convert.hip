@@ -265,34 +265,6 @@ int bits_for(int64_t maxv) {
   return b;
 }
 
-// RAII bag of stream-ordered temporaries
-struct Tmp {
-  hipStream_t s;
-  std::vector<void*> ptrs;
-  explicit Tmp(hipStream_t st) : s(st) {}
-  ~Tmp() {
-    for (void* p : ptrs) (void)hipFreeAsync(p, s);
-  }
-  template <typename T>
-  int alloc(T** p, int64_t n) {
-    *p = nullptr;
-    hipError_t e = hipMallocAsync(reinterpret_cast<void**>(p),
-                                  sizeof(T) * (size_t)std::max<int64_t>(n, 1), s);
-    if (e != hipSuccess) {
-      set_error(std::string("convert temporary: ") + hipGetErrorString(e));
-      return e == hipErrorOutOfMemory ? MPH_ERR_OUT_OF_MEMORY : MPH_ERR_HIP;
-    }
-    ptrs.push_back(*p);
-    return MPH_OK;
-  }
-};
-
-int sync_read_i32(const int32_t* d, int32_t* h, hipStream_t s) {
-  MPH_HIP_CHECK(hipMemcpyAsync(h, d, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-  MPH_HIP_CHECK(hipStreamSynchronize(s));
-  return MPH_OK;
-}
-
 int fill_i32(int32_t* p, int64_t n, int32_t v, hipStream_t s) {
   if (n <= 0) return MPH_OK;
   hipLaunchKernelGGL(fill_i32_kernel, dim3(blocks_for(n)), dim3(kT), 0, s, p, n, v);
@@ -379,7 +351,7 @@ int is_sorted_dev(const int32_t* ri, const int32_t* ci, int64_t nnz, hipStream_t
   MPH_CHECK_STATUS(fill_i32(flag, 1, 0, s));
   hipLaunchKernelGGL(unsorted_kernel, dim3(blocks_for(nnz)), dim3(kT), 0, s, ri, ci, nnz, flag);
   int32_t h = 0;
-  MPH_CHECK_STATUS(sync_read_i32(flag, &h, s));
+  MPH_CHECK_STATUS(t.read(flag, &h));
   *sorted = !h;
   return MPH_OK;
 }
@@ -397,8 +369,7 @@ int sort_coo(int64_t nnz, int64_t nrows, int64_t ncols, int32_t* ri, int32_t* ci
   hipLaunchKernelGGL(max_kernel, dim3(reduce_blocks(nnz)), dim3(kT), 0, s, ri, nnz, mx);
   hipLaunchKernelGGL(max_kernel, dim3(reduce_blocks(nnz)), dim3(kT), 0, s, ci, nnz, mx + 1);
   int32_t hm[2];
-  MPH_HIP_CHECK(hipMemcpyAsync(hm, mx, sizeof(hm), hipMemcpyDeviceToHost, s));
-  MPH_HIP_CHECK(hipStreamSynchronize(s));
+  MPH_CHECK_STATUS(t.read(mx, hm, 2));
   // counting-sort bins run to the largest key (Sort_Impl.hpp:137-142)
   nrows = std::min<int64_t>(nrows, (int64_t)hm[0] + 1);
   ncols = std::min<int64_t>(ncols, (int64_t)hm[1] + 1);
@@ -785,7 +756,7 @@ int emit_dia_part(int64_t nrows, int64_t ncols, int64_t ndiag, int64_t pitch,
   MPH_HIP_CHECK(hipGetLastError());
   MPH_CHECK_STATUS(exclusive_scan_i32(flag, pos, T, tmp, s));
   int32_t tot = 0;
-  MPH_CHECK_STATUS(sync_read_i32(pos + T, &tot, s));
+  MPH_CHECK_STATUS(t.read(pos + T, &tot));
   if (tot > cap) return invalid("DIA holds more non-zeros than its nnz");
   if (tot > 0) {
     MPH_LAUNCH_W(dia_emit_kernel, vsize, dim3(blocks_for(T)), s, nrows, ndiag, pitch, off,
@@ -826,8 +797,8 @@ int mph_convert_csr_to_coo(int64_t nrows, int64_t nnz, const int32_t* ro, const 
   hipLaunchKernelGGL(expand_rows_kernel, dim3(blocks_for(nnz)), dim3(kT), 0, s, ro, nrows, nnz,
                      (int64_t)0, ri_out);
   MPH_HIP_CHECK(hipGetLastError());
-  MPH_CHECK_STATUS(copy_dev(ci_out, ci, sizeof(int32_t) * nnz, s));
-  MPH_CHECK_STATUS(copy_dev(v_out, v, value_size(vt) * nnz, s));
+  if (ci_out != ci) MPH_CHECK_STATUS(copy_dev(ci_out, ci, sizeof(int32_t) * nnz, s));
+  if (v_out != v) MPH_CHECK_STATUS(copy_dev(v_out, v, value_size(vt) * nnz, s));
   return MPH_OK;
 }
 
@@ -849,8 +820,8 @@ int mph_convert_coo_to_csr(int64_t nrows, int64_t nnz, const int32_t* ri, const 
   int sorted_rows = 1;
   MPH_CHECK_STATUS(rows_sorted(ri, nnz, nrows, s, &sorted_rows));
   if (sorted_rows) {
-    MPH_CHECK_STATUS(copy_dev(ci_out, ci, sizeof(int32_t) * nnz, s));
-    MPH_CHECK_STATUS(copy_dev(v_out, v, (size_t)vs * nnz, s));
+    if (ci_out != ci) MPH_CHECK_STATUS(copy_dev(ci_out, ci, sizeof(int32_t) * nnz, s));
+    if (v_out != v) MPH_CHECK_STATUS(copy_dev(v_out, v, (size_t)vs * nnz, s));
     return MPH_OK;
   }
   MPH_CHECK_STATUS(t.alloc(&r2, nnz));
@@ -860,6 +831,12 @@ int mph_convert_coo_to_csr(int64_t nrows, int64_t nnz, const int32_t* ri, const 
   MPH_CHECK_STATUS(copy_dev(c2, ci, sizeof(int32_t) * nnz, s));
   MPH_CHECK_STATUS(radix_sort_pairs(r2, c2, nnz, nrows, 0, false, perm, s));
   MPH_CHECK_STATUS(copy_dev(ci_out, c2, sizeof(int32_t) * nnz, s));
+  if (v_out == v) {  // in place: gathered from a copy
+    uint8_t* vtmp;
+    MPH_CHECK_STATUS(t.alloc(&vtmp, nnz * vs));
+    MPH_CHECK_STATUS(copy_dev(vtmp, v, (size_t)nnz * vs, s));
+    v = vtmp;
+  }
   MPH_CHECK_STATUS(gather_values(v, perm, nnz, v_out, vs, s));
   MPH_HIP_CHECK(hipStreamSynchronize(s));
   return MPH_OK;
@@ -887,7 +864,7 @@ int mph_convert_coo_to_dia_size(int64_t nrows, int64_t ncols, int64_t nnz, const
   MPH_HIP_CHECK(hipGetLastError());
   MPH_CHECK_STATUS(exclusive_scan_i32(flag, pos, nb, tmp, s));
   int32_t nd = 0;
-  MPH_CHECK_STATUS(sync_read_i32(pos + nb, &nd, s));
+  MPH_CHECK_STATUS(t.read(pos + nb, &nd));
   *ndiag = nd;
   if (mph_exceeds_tolerance(nrows, nnz, nd)) {
     set_error("DiaMatrix fill-in would exceed maximum tolerance");
@@ -967,7 +944,7 @@ int mph_convert_coo_to_ell_size(int64_t nrows, int64_t nnz, const int32_t* ri, i
     hipLaunchKernelGGL(max_kernel, dim3(reduce_blocks(nrows)), dim3(kT), 0, s, cnt, nrows, mx);
   MPH_HIP_CHECK(hipGetLastError());
   int32_t h = 0;
-  MPH_CHECK_STATUS(sync_read_i32(mx, &h, s));
+  MPH_CHECK_STATUS(t.read(mx, &h));
   *K = h;
   if (mph_exceeds_tolerance(nrows, nnz, h)) {
     set_error("EllMatrix fill-in would exceed maximum tolerance");
@@ -1027,7 +1004,7 @@ int mph_convert_ell_to_coo(int64_t nrows, int64_t nnz, int64_t width, int64_t pi
       hipLaunchKernelGGL(ell_flag_kernel, dim3(blocks_for(T)), dim3(kT), 0, s, nrows, width, pitch,
                          eci, flag);
     MPH_CHECK_STATUS(exclusive_scan_i32(flag, pos, T, tmp, s));
-    MPH_CHECK_STATUS(sync_read_i32(pos + T, &tot, s));
+    MPH_CHECK_STATUS(t.read(pos + T, &tot));
     if (tot > nnz) return invalid("ELL holds more entries than its nnz");
     if (tot > 0)
       MPH_LAUNCH_W(ell_emit_kernel, vs, dim3(blocks_for(T)), s, nrows, width, pitch, eci,
@@ -1057,8 +1034,7 @@ int mph_convert_coo_to_hyb_size(int64_t nrows, int64_t nnz, const int32_t* ri, i
                      (int32_t)std::min<int64_t>(k, INT32_MAX), acc);
   MPH_HIP_CHECK(hipGetLastError());
   unsigned long long h = 0;
-  MPH_HIP_CHECK(hipMemcpyAsync(&h, acc, sizeof(h), hipMemcpyDeviceToHost, s));
-  MPH_HIP_CHECK(hipStreamSynchronize(s));
+  MPH_CHECK_STATUS(t.read(acc, &h));
   *K = k;
   *ell_nnz = (int64_t)h;
   *coo_nnz = nnz - (int64_t)h;
@@ -1101,7 +1077,7 @@ int mph_convert_coo_to_hyb(int64_t nrows, int64_t nnz, const int32_t* ri, const 
                R.runpos, win, eci, ev);
   MPH_CHECK_STATUS(exclusive_scan_i32(over, opos, nnz, tmp, s));
   int32_t tail = 0;
-  MPH_CHECK_STATUS(sync_read_i32(opos + nnz, &tail, s));
+  MPH_CHECK_STATUS(t.read(opos + nnz, &tail));
   if (tail > cn) return invalid("COO entries are not grouped by row (HYB tail overflow)");
   if (tail < cn) MPH_CHECK_STATUS(zero_tail(tail, cn, cri, cci, cv, vs, s));
   if (tail > 0)
@@ -1136,7 +1112,7 @@ int mph_convert_hyb_to_coo(int64_t nrows, int64_t nnz, int64_t width, int64_t pi
       hipLaunchKernelGGL(first_descent_kernel, dim3(blocks_for(coo_nnz)), dim3(kT), 0, s, cri,
                          coo_nnz, P);
     int32_t hP = 0;
-    MPH_CHECK_STATUS(sync_read_i32(P, &hP, s));
+    MPH_CHECK_STATUS(t.read(P, &hP));
     MPH_CHECK_STATUS(t.alloc(&tro, nrows + 1));
     hipLaunchKernelGGL(sorted_offsets_kernel, dim3(blocks_for((int64_t)hP + 1)), dim3(kT), 0, s,
                        cri, (int64_t)hP, nrows, tro);
@@ -1146,7 +1122,7 @@ int mph_convert_hyb_to_coo(int64_t nrows, int64_t nnz, int64_t width, int64_t pi
     hipLaunchKernelGGL(hyb_rowcount_kernel, dim3(blocks_for(nrows)), dim3(kT), 0, s, nrows, width,
                        pitch, eci, tro, cnt);
     MPH_CHECK_STATUS(exclusive_scan_i32(cnt, rowpos, nrows, tmp, s));
-    MPH_CHECK_STATUS(sync_read_i32(rowpos + nrows, &total, s));
+    MPH_CHECK_STATUS(t.read(rowpos + nrows, &total));
     if (total > nnz) return invalid("HYB holds more entries than its nnz");
     const int wpb = kT / kWave;
     MPH_LAUNCH_W(hyb_emit_kernel, vs, dim3(blocks_for(nrows, wpb)), s, nrows, width, pitch, eci,
@@ -1182,8 +1158,7 @@ int mph_convert_coo_to_hdc_size(int64_t nrows, int64_t ncols, int64_t nnz, const
   hipLaunchKernelGGL(hdc_sizes_kernel, dim3(reduce_blocks(nb)), dim3(kT), 0, s, cnt, nb, thr, acc);
   MPH_HIP_CHECK(hipGetLastError());
   unsigned long long h[3];
-  MPH_HIP_CHECK(hipMemcpyAsync(h, acc, sizeof(h), hipMemcpyDeviceToHost, s));
-  MPH_HIP_CHECK(hipStreamSynchronize(s));
+  MPH_CHECK_STATUS(t.read(acc, h, 3));
   *ndiag = (int64_t)h[0];
   *dia_nnz = (int64_t)h[1];
   *csr_nnz = (int64_t)h[2];
@@ -1231,7 +1206,7 @@ int mph_convert_coo_to_hdc(int64_t nrows, int64_t ncols, int64_t nnz, const int3
   const int64_t mid = nb / 2;
   if (nrows != ncols && ndiag > 0) {
     int32_t sel = 0;
-    MPH_CHECK_STATUS(sync_read_i32(flag + mid, &sel, s));
+    MPH_CHECK_STATUS(t.read(flag + mid, &sel));
     if (sel) {
       std::vector<int32_t> h(ndiag);
       MPH_HIP_CHECK(hipMemcpyAsync(h.data(), off_out, sizeof(int32_t) * ndiag,
@@ -1262,7 +1237,7 @@ int mph_convert_coo_to_hdc(int64_t nrows, int64_t ncols, int64_t nnz, const int3
   }
   MPH_CHECK_STATUS(exclusive_scan_i32(rest, rpos, nnz, tmp, s));
   int32_t nrest = 0;
-  MPH_CHECK_STATUS(sync_read_i32(rpos + nnz, &nrest, s));
+  MPH_CHECK_STATUS(t.read(rpos + nnz, &nrest));
   if (nrest > cn) return invalid("HDC CSR part overflow (non-square midpoint diagonal)");
   // CSR part: per-row counts of the rest, exclusive scan, row_offsets[n] = cn
   MPH_CHECK_STATUS(t.alloc(&rows_rest, std::max<int64_t>(cn, 1)));

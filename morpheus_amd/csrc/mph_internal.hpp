@@ -2,6 +2,7 @@
 // entry points shared between the kernel translation units and the C-ABI.
 #pragma once
 
+#include <algorithm>
 #include <cstdint>
 #include <vector>
 
@@ -257,6 +258,58 @@ int exclusive_scan_i32(const int32_t* in, int32_t* out, int64_t n,
 int fill_zero(void* p, size_t bytes, hipStream_t s);
 
 int device_cu_count();
+
+// Temporaries of one call, from blocks the library keeps per device.  The
+// runtime's stream-ordered pools mapped and unmapped memory at the
+// conversions' synchronisations whatever their release threshold: 25-60 us an
+// allocation and up to 1.1 ms a release, 3 ms of a 5.4 ms CSR -> HYB -> CSR
+// round trip of 16M entries.  A block goes back to the cache only after its
+// stream has been synchronised, so any thread and stream may take it next;
+// the cache holds at most kTmpKeepBytes in kTmpKeepBlocks blocks a device,
+// and mph_finalize, or an allocation that fails, gives them back.
+constexpr size_t kTmpKeepBytes = (size_t)2 << 30;
+constexpr size_t kTmpKeepBlocks = 48;
+struct TmpBlock {
+  void* p = nullptr;
+  size_t bytes = 0;
+  bool host = false;  // pinned host memory
+};
+int tmp_take(TmpBlock* b, size_t bytes, bool host);
+void tmp_give(const TmpBlock& b);
+void tmp_trim();
+
+struct Tmp {
+  hipStream_t s;
+  bool idle = false;  // the stream was synchronised after the last launch
+  std::vector<TmpBlock> blocks;
+  explicit Tmp(hipStream_t st) : s(st) {}
+  Tmp(const Tmp&) = delete;
+  Tmp& operator=(const Tmp&) = delete;
+  ~Tmp() {
+    if (!blocks.empty() && !idle) (void)hipStreamSynchronize(s);
+    for (const TmpBlock& b : blocks) tmp_give(b);
+  }
+  template <typename T>
+  int alloc(T** p, int64_t n, bool host = false) {
+    *p = nullptr;
+    TmpBlock b;
+    const int st = tmp_take(&b, sizeof(T) * (size_t)std::max<int64_t>(n, 1), host);
+    if (st != MPH_OK) return st;
+    blocks.push_back(b);
+    *p = static_cast<T*>(b.p);
+    return MPH_OK;
+  }
+  // n words of device memory to the host, and the stream synchronised
+  template <typename T>
+  int read(const T* d, T* h, int64_t n = 1) {
+    T* pin = nullptr;
+    MPH_CHECK_STATUS(alloc(&pin, n, true));
+    MPH_HIP_CHECK(hipMemcpyAsync(pin, d, sizeof(T) * (size_t)n, hipMemcpyDeviceToHost, s));
+    MPH_HIP_CHECK(hipStreamSynchronize(s));
+    std::copy(pin, pin + n, h);
+    return MPH_OK;
+  }
+};
 
 // validate.hip
 int check_index_range(const int32_t* idx, int64_t n, int64_t hi, bool allow_m1,

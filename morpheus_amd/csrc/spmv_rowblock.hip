@@ -1654,54 +1654,39 @@ int default_chunk(int vt) {
   return vt == MPH_F64 ? kDefaultChunkF64 : kDefaultChunkF32;
 }
 
-namespace {
-
-int read_flag(int32_t* dflag, hipStream_t s, int* out) {
-  int32_t h = 0;
-  MPH_HIP_CHECK(hipMemcpyAsync(&h, dflag, sizeof(int32_t),
-                               hipMemcpyDeviceToHost, s));
-  MPH_HIP_CHECK(hipStreamSynchronize(s));
-  *out = h;
-  return MPH_OK;
-}
-
-}  // namespace
-
 int ell_padding_only(const int32_t* ci, int64_t pitch, int64_t nrows, int64_t K,
                      int64_t width, hipStream_t s, int* padding_only) {
   *padding_only = 1;
   if (width <= K || nrows == 0) return MPH_OK;
+  Tmp t(s);
   int32_t* flag = nullptr;
-  MPH_HIP_CHECK(hipMalloc(&flag, sizeof(int32_t)));
-  int st = fill_zero(flag, sizeof(int32_t), s);
-  if (st == MPH_OK) {
-    const int64_t total = nrows * (width - K);
-    hipLaunchKernelGGL(ell_tail_check_kernel, dim3((unsigned)ceil_div(total, 256)),
-                       dim3(256), 0, s, ci, pitch, nrows, K, width, flag);
-    int f = 0;
-    st = read_flag(flag, s, &f);
-    *padding_only = !f;
-  }
-  dfree(flag);
-  return st;
+  MPH_CHECK_STATUS(t.alloc(&flag, 1));
+  MPH_CHECK_STATUS(fill_zero(flag, sizeof(int32_t), s));
+  const int64_t total = nrows * (width - K);
+  hipLaunchKernelGGL(ell_tail_check_kernel, dim3((unsigned)ceil_div(total, 256)), dim3(256), 0, s,
+                     ci, pitch, nrows, K, width, flag);
+  int32_t f = 0;
+  MPH_CHECK_STATUS(t.read(flag, &f));
+  t.idle = true;
+  *padding_only = !f;
+  return MPH_OK;
 }
 
 int rows_sorted(const int32_t* ri, int64_t nnz, int64_t nrows, hipStream_t s,
                 int* sorted) {
   *sorted = 1;
   if (nnz == 0) return MPH_OK;
+  Tmp t(s);
   int32_t* flag = nullptr;
-  MPH_HIP_CHECK(hipMalloc(&flag, sizeof(int32_t)));
-  int st = fill_zero(flag, sizeof(int32_t), s);
-  if (st == MPH_OK) {
-    hipLaunchKernelGGL(rows_unsorted_kernel, dim3((unsigned)ceil_div(nnz, 256)),
-                       dim3(256), 0, s, ri, nnz, nrows, flag);
-    int f = 0;
-    st = read_flag(flag, s, &f);
-    *sorted = !f;
-  }
-  dfree(flag);
-  return st;
+  MPH_CHECK_STATUS(t.alloc(&flag, 1));
+  MPH_CHECK_STATUS(fill_zero(flag, sizeof(int32_t), s));
+  hipLaunchKernelGGL(rows_unsorted_kernel, dim3((unsigned)ceil_div(nnz, 256)), dim3(256), 0, s, ri,
+                     nnz, nrows, flag);
+  int32_t f = 0;
+  MPH_CHECK_STATUS(t.read(flag, &f));
+  t.idle = true;
+  *sorted = !f;
+  return MPH_OK;
 }
 
 namespace {

@@ -41,23 +41,15 @@ __global__ void row_offsets_kernel(const int32_t* __restrict__ ro,
 
 int run_flag_check(hipStream_t s, int* bad,
                    const std::function<void(int32_t*)>& launch) {
+  Tmp t(s);
   int32_t* flag = nullptr;
-  MPH_HIP_CHECK(hipMalloc(&flag, sizeof(int32_t)));
-  int st = fill_zero(flag, sizeof(int32_t), s);
-  int32_t h = 0;
-  if (st == MPH_OK) {
-    launch(flag);
-    hipError_t e = hipGetLastError();
-    if (e == hipSuccess) e = hipMemcpyAsync(&h, flag, sizeof(int32_t), hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-    if (e != hipSuccess) {
-      set_error(std::string("index check: ") + hipGetErrorString(e));
-      st = MPH_ERR_HIP;
-    }
-  }
-  dfree(flag);
-  *bad = h;
-  return st;
+  MPH_CHECK_STATUS(t.alloc(&flag, 1));
+  MPH_CHECK_STATUS(fill_zero(flag, sizeof(int32_t), s));
+  launch(flag);
+  MPH_HIP_CHECK(hipGetLastError());
+  MPH_CHECK_STATUS(t.read(flag, bad));
+  t.idle = true;
+  return MPH_OK;
 }
 
 }  // namespace

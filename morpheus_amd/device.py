@@ -262,20 +262,20 @@ def _empty_i(n):
     return torch.empty(max(int(n), 0), dtype=torch.int32, device="cuda")
 
 
-def _zeros_i(n):
-    return torch.zeros(max(int(n), 0), dtype=torch.int32, device="cuda")
+def _empty_v(n, dtype):
+    return torch.empty(max(int(n), 0), dtype=DTYPES[dtype][0], device="cuda")
 
 
-def _zeros_v(n, dtype):
-    return torch.zeros(max(int(n), 0), dtype=DTYPES[dtype][0], device="cuda")
-
-
-def to_coo(A: DeviceMatrix, stream=None) -> DeviceMatrix:
-    """Any format -> COO on the GPU (the reference Serial semantics)."""
+def to_coo(A: DeviceMatrix, stream=None, share: bool = False) -> DeviceMatrix:
+    """Any format -> COO on the GPU (the reference Serial semantics).  share:
+    from CSR, the result uses A's column and value arrays instead of copies
+    (the temporary of a conversion)."""
     s = stream_handle(stream)
     a, m, vt = A.arrays, A.meta, A.vt
     n, nnz = A.nrows, A.nnz
-    ri, ci, v = _zeros_i(nnz), _zeros_i(nnz), _zeros_v(nnz, A.dtype)
+    share = share and A.format == CSR_FORMAT
+    ri = _empty_i(nnz)
+    ci, v = (a["ci"], a["v"]) if share else (_empty_i(nnz), _empty_v(nnz, A.dtype))
     if A.format == COO_FORMAT:
         ri.copy_(a["ri"])
         ci.copy_(a["ci"])
@@ -300,8 +300,9 @@ def to_coo(A: DeviceMatrix, stream=None) -> DeviceMatrix:
     return DeviceMatrix(COO_FORMAT, n, A.ncols, nnz, A.dtype, dict(ri=ri, ci=ci, v=v), {})
 
 
-def from_coo(A: DeviceMatrix, fmt: int, stream=None) -> DeviceMatrix:
-    """COO -> any format on the GPU (the reference Serial semantics)."""
+def from_coo(A: DeviceMatrix, fmt: int, stream=None, reuse: bool = False) -> DeviceMatrix:
+    """COO -> any format on the GPU (the reference Serial semantics).  reuse:
+    A is a temporary, whose column and value arrays become the CSR's."""
     assert A.format == COO_FORMAT
     s = stream_handle(stream)
     a, vt, dt = A.arrays, A.vt, A.dtype
@@ -309,7 +310,8 @@ def from_coo(A: DeviceMatrix, fmt: int, stream=None) -> DeviceMatrix:
     if fmt == COO_FORMAT:
         return to_coo(A, stream)
     if fmt == CSR_FORMAT:
-        ro, ci, v = _zeros_i(n + 1), _zeros_i(nnz), _zeros_v(nnz, dt)
+        ro = _empty_i(n + 1)
+        ci, v = (a["ci"], a["v"]) if reuse else (_empty_i(nnz), _empty_v(nnz, dt))
         capi.call("mph_convert_coo_to_csr", n, nnz, _p(a["ri"]), _p(a["ci"]), _p(a["v"]), vt,
                   _p(ro), _p(ci), _p(v), s)
         return DeviceMatrix(CSR_FORMAT, n, nc, nnz, dt, dict(ro=ro, ci=ci, v=v), {})
@@ -318,7 +320,7 @@ def from_coo(A: DeviceMatrix, fmt: int, stream=None) -> DeviceMatrix:
         capi.call("mph_convert_coo_to_dia_size", n, nc, nnz, _p(a["ri"]), _p(a["ci"]),
                   C.byref(nd), s)
         pitch = pad_size(n, ALIGNMENT)
-        off, v = _zeros_i(nd.value), _zeros_v(pitch * nd.value, dt)
+        off, v = _empty_i(nd.value), _empty_v(pitch * nd.value, dt)
         capi.call("mph_convert_coo_to_dia", n, nc, nnz, _p(a["ri"]), _p(a["ci"]), _p(a["v"]),
                   vt, nd.value, pitch, _p(off), _p(v), s)
         return DeviceMatrix(DIA_FORMAT, n, nc, nnz, dt, dict(off=off, v=v),
@@ -327,7 +329,7 @@ def from_coo(A: DeviceMatrix, fmt: int, stream=None) -> DeviceMatrix:
         K = C.c_int64()
         capi.call("mph_convert_coo_to_ell_size", n, nnz, _p(a["ri"]), C.byref(K), s)
         width, pitch = pad_size(K.value, ALIGNMENT), n
-        ci, v = _zeros_i(width * pitch), _zeros_v(width * pitch, dt)
+        ci, v = _empty_i(width * pitch), _empty_v(width * pitch, dt)
         capi.call("mph_convert_coo_to_ell", n, nnz, _p(a["ri"]), _p(a["ci"]), _p(a["v"]), vt,
                   K.value, width, pitch, _p(ci), _p(v), s)
         return DeviceMatrix(ELL_FORMAT, n, nc, nnz, dt, dict(ci=ci, v=v),
@@ -337,8 +339,8 @@ def from_coo(A: DeviceMatrix, fmt: int, stream=None) -> DeviceMatrix:
         capi.call("mph_convert_coo_to_hyb_size", n, nnz, _p(a["ri"]), C.byref(K), C.byref(en),
                   C.byref(cn), s)
         width, pitch = pad_size(K.value, ALIGNMENT), n
-        eci, ev = _zeros_i(width * pitch), _zeros_v(width * pitch, dt)
-        cri, cci, cv = _zeros_i(cn.value), _zeros_i(cn.value), _zeros_v(cn.value, dt)
+        eci, ev = _empty_i(width * pitch), _empty_v(width * pitch, dt)
+        cri, cci, cv = _empty_i(cn.value), _empty_i(cn.value), _empty_v(cn.value, dt)
         capi.call("mph_convert_coo_to_hyb", n, nnz, _p(a["ri"]), _p(a["ci"]), _p(a["v"]), vt,
                   K.value, width, pitch, _p(eci), _p(ev), _p(cri), _p(cci), _p(cv), s)
         return DeviceMatrix(HYB_FORMAT, n, nc, nnz, dt,
@@ -350,8 +352,8 @@ def from_coo(A: DeviceMatrix, fmt: int, stream=None) -> DeviceMatrix:
         capi.call("mph_convert_coo_to_hdc_size", n, nc, nnz, _p(a["ri"]), _p(a["ci"]),
                   C.byref(nd), C.byref(dn), C.byref(cn), s)
         pitch = pad_size(n, ALIGNMENT)
-        off, dv = _zeros_i(nd.value), _zeros_v(pitch * nd.value, dt)
-        ro, ci, cv = _zeros_i(n + 1), _zeros_i(cn.value), _zeros_v(cn.value, dt)
+        off, dv = _empty_i(nd.value), _empty_v(pitch * nd.value, dt)
+        ro, ci, cv = _empty_i(n + 1), _empty_i(cn.value), _empty_v(cn.value, dt)
         capi.call("mph_convert_coo_to_hdc", n, nc, nnz, _p(a["ri"]), _p(a["ci"]), _p(a["v"]),
                   vt, nd.value, pitch, _p(off), _p(dv), _p(ro), _p(ci), _p(cv), s)
         return DeviceMatrix(HDC_FORMAT, n, nc, nnz, dt, dict(off=off, dv=dv, ro=ro, ci=ci, cv=cv),
@@ -500,10 +502,13 @@ def convert(A: DeviceMatrix, fmt: int, stream=None) -> DeviceMatrix:
                             {k: t.clone() for k, t in A.arrays.items()}, dict(A.meta))
     if A.format == COO_FORMAT:
         return from_coo(A, fmt, stream)
-    coo = to_coo(A, stream)
     if fmt == COO_FORMAT:
-        return coo
-    return from_coo(coo, fmt, stream)
+        return to_coo(A, stream)
+    coo = to_coo(A, stream, share=True)
+    if stream is not None:  # the temporary is released while its last kernels may run
+        for t in coo.arrays.values():
+            t.record_stream(stream)
+    return from_coo(coo, fmt, stream, reuse=A.format != CSR_FORMAT)
 
 
 # ------------------------------------------------------------------ batched
