@@ -166,22 +166,222 @@ __global__ void first_descent_kernel(const int32_t* __restrict__ ri, int64_t n,
   if (i >= 1 && i < n && ri[i] < ri[i - 1]) atomicMin(out, (int32_t)i);
 }
 
-// row of entry j of a CSR: the last r with ro[r] <= j (ro non-decreasing)
-__device__ __forceinline__ int32_t row_of(const int32_t* ro, int64_t nrows, int64_t j) {
-  int64_t lo = 0, hi = nrows;  // invariant: ro[lo] <= j < ro[hi]
-  while (hi - lo > 1) {
-    const int64_t mid = (lo + hi) >> 1;
-    if (ro[mid] <= j) lo = mid; else hi = mid;
+// One pass over the entries of a COO list: index ranges, the order of the
+// entries, and (rows not decreasing) the row offsets, whose slots ro[prev + 1
+// .. r] entry i fills when its row r differs from the entry before it.  Reads
+// 8 B an entry once, where the range checks, the sortedness test and a row
+// histogram (an LDS hash table: 6 ps an entry) each were a pass.  With
+// indices out of range, or rows that decrease, ro is incomplete; every write
+// stays inside it.
+constexpr int32_t kBadRow = 1, kBadCol = 2, kRowsDown = 4, kUnsorted = 8, kRepeated = 16;
+constexpr int kScanPer = 8;  // entries per thread
+constexpr int kScanTile = kT * kScanPer;
+
+// rows (lo, hi] start at entry i; long gaps are filled by the whole wave
+__device__ __forceinline__ void fill_offsets(int32_t* __restrict__ ro, int64_t lo, int64_t hi,
+                                             int32_t i) {
+  constexpr int64_t kLongGap = 32;
+  const int lane = threadIdx.x % kWave;
+  const bool lng = hi - lo > kLongGap;
+  if (!lng)
+    for (int64_t r = lo + 1; r <= hi; r++) ro[r] = i;
+  uint64_t m = __ballot(lng);
+  while (m) {
+    const int src = __ffsll((unsigned long long)m) - 1;
+    m &= m - 1;
+    const int64_t l = shfl((int32_t)lo, src), h = shfl((int32_t)hi, src);
+    const int32_t at = shfl(i, src);
+    for (int64_t r = l + 1 + lane; r <= h; r += kWave) ro[r] = at;
   }
-  return (int32_t)lo;
 }
 
-__global__ void expand_rows_kernel(const int32_t* __restrict__ ro, int64_t nrows,
-                                   int64_t nnz, int64_t shift,
-                                   int32_t* __restrict__ ri_out) {
-  const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (j < nnz) ri_out[j + shift] = row_of(ro, nrows, j);
+// sets the bits of `bad` any lane of the wave has; a word that already holds
+// them is not written again (unsorted entries would all hit one address)
+__device__ __forceinline__ void raise_flags(int32_t* __restrict__ flags, int32_t bad) {
+  for (int d = kWave / 2; d > 0; d >>= 1) bad |= shfl_xor(bad, d);
+  if (bad && threadIdx.x % kWave == 0 &&
+      (__hip_atomic_load(flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & bad) != bad)
+    atomicOr(flags, bad);
 }
+
+// Marks the bits of keys in a bitmap (lanes with `need` set; every lane of
+// the wave calls it).  A workgroup gathers its keys in an LDS table (linear
+// probing, kSeenProbe steps), equal keys of a wave entered once; keys that
+// find no slot mark their bit at once.  mark_bits_flush then sets the
+// table's bits that are not yet set: a stencil's few diagonals would
+// otherwise queue up on a few words (about 11 ns for each wave's atomic on
+// one address; 117 us for 14.6M entries when each wave read and set its bits
+// itself, 52 us so).
+constexpr int kSeen = 2 * kT;
+constexpr int kSeenProbe = 4;
+__device__ __forceinline__ uint32_t seen_slot(int32_t key) {
+  return ((uint32_t)key * 2654435761u) >> 23;  // 9 bits
+}
+
+__device__ __forceinline__ void mark_bits(uint32_t* __restrict__ bits, int32_t* seen, int32_t key,
+                                          bool need) {
+  const int lane = threadIdx.x % kWave;
+  const uint32_t slot = seen_slot(key);
+#pragma unroll
+  for (int p = 0; p < kSeenProbe; p++) need = need && seen[(slot + p) & (kSeen - 1)] != key;
+  uint64_t m = __ballot(need);
+  for (int round = 0; m && round < 12; round++) {
+    const int src = __ffsll((unsigned long long)m) - 1;
+    const int32_t k = shfl(key, src);
+    if (lane == src) {
+      int p = 0;
+      for (; p < kSeenProbe; p++) {
+        const int32_t old = atomicCAS(&seen[(slot + p) & (kSeen - 1)], -1, k);
+        if (old == -1 || old == k) break;
+      }
+      if (p == kSeenProbe) atomicOr(&bits[k >> 5], 1u << (k & 31));
+    }
+    if (key == k) need = false;
+    m = __ballot(need);
+  }
+  if (need) atomicOr(&bits[key >> 5], 1u << (key & 31));
+}
+
+__device__ __forceinline__ void mark_bits_flush(uint32_t* __restrict__ bits, const int32_t* seen) {
+  __syncthreads();
+  for (int q = threadIdx.x; q < kSeen; q += kT) {
+    const int32_t k = seen[q];
+    if (k < 0) continue;
+    const uint32_t bit = 1u << (k & 31);
+    if (!(__hip_atomic_load(&bits[k >> 5], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & bit))
+      atomicOr(&bits[k >> 5], bit);
+  }
+}
+
+template <bool COLS, bool OFFSETS, bool DIAGS>
+__global__ __launch_bounds__(kT) void coo_scan_kernel(
+    const int32_t* __restrict__ ri, const int32_t* __restrict__ ci, int64_t nnz, int64_t nrows,
+    int64_t ncols, int32_t* __restrict__ ro, uint32_t* __restrict__ diags,
+    int32_t* __restrict__ flags) {
+  __shared__ int32_t seen[kSeen];
+  if (DIAGS) {
+    for (int q = threadIdx.x; q < kSeen; q += kT) seen[q] = -1;
+    __syncthreads();
+  }
+  const int64_t base = (int64_t)blockIdx.x * kScanTile + threadIdx.x;
+  const int lane = threadIdx.x % kWave;
+  int32_t r[kScanPer], c[kScanPer], bad = 0;
+  int64_t last = -2;  // the last entry's row, in the lane that holds it
+#pragma unroll
+  for (int k = 0; k < kScanPer; k++) {
+    const int64_t i = base + (int64_t)k * kT;
+    r[k] = i < nnz ? ri[i] : 0;
+    c[k] = COLS && i < nnz ? ci[i] : 0;
+  }
+#pragma unroll
+  for (int k = 0; k < kScanPer; k++) {
+    const int64_t i = base + (int64_t)k * kT;
+    int32_t pr = shfl_up(r[k], 1), pc = COLS ? shfl_up(c[k], 1) : 0;
+    if (lane == 0 && i > 0 && i < nnz) {
+      pr = ri[i - 1];
+      if (COLS) pc = ci[i - 1];
+    }
+    const bool in = i < nnz;
+    const bool row_ok = r[k] >= 0 && r[k] < nrows, col_ok = !COLS || (c[k] >= 0 && c[k] < ncols);
+    if (in) {
+      if (!row_ok) bad |= kBadRow;
+      if (!col_ok) bad |= kBadCol;
+      if (i > 0) {
+        if (pr > r[k]) bad |= kRowsDown | kUnsorted | kRepeated;
+        if (COLS && pr == r[k] && pc > c[k]) bad |= kUnsorted | kRepeated;
+        if (COLS && pr == r[k] && pc == c[k]) bad |= kRepeated;
+      }
+    }
+    if (OFFSETS) {
+      const int64_t hi = in && row_ok ? r[k] : 0;
+      const int64_t lo = in && row_ok ? (i == 0 ? -1 : min((int64_t)max(pr, -1), hi)) : 0;
+      fill_offsets(ro, lo, hi, (int32_t)i);
+      if (in && i == nnz - 1 && row_ok) last = r[k];
+    }
+    if (DIAGS)
+      mark_bits(diags, seen, (int32_t)((int64_t)c[k] - r[k] + nrows - 1), in && row_ok && col_ok);
+  }
+  if (OFFSETS && blockIdx.x == gridDim.x - 1)  // the rows after the last entry's
+    fill_offsets(ro, last >= -1 ? last : 0, last >= -1 ? nrows : 0, (int32_t)nnz);
+  raise_flags(flags, bad);
+  if (DIAGS) mark_bits_flush(diags, seen);
+}
+
+// rows of a CSR's entries, a workgroup per kScanTile of them: each row that
+// starts in the tile marks its first entry in LDS (of rows without entries
+// the last mark stays), a maximum scan spreads the marks, and the rows are
+// written in order.  A binary search of the offsets per entry took 205 us for
+// 14.6M entries (0.28 TB/s).  A tile that spans more rows than the marks are
+// worth (long runs of empty rows) searches the offsets instead.
+__global__ __launch_bounds__(kT) void expand_rows_kernel(const int32_t* __restrict__ ro,
+                                                         int64_t nrows, int64_t nnz, int64_t shift,
+                                                         int32_t* __restrict__ ri_out) {
+  __shared__ int32_t mark[kScanTile];
+  __shared__ int32_t wtop[kT / kWave];
+  __shared__ int32_t ends[2];
+  const int64_t base = (int64_t)blockIdx.x * kScanTile;
+  const int n = (int)min((int64_t)kScanTile, nnz - base);
+  if (threadIdx.x < 2 * kWave) {
+    // the row of the tile's first / last entry, the last r with ro[r] <= j:
+    // one wave each, 64 probes a round
+    const int lane = threadIdx.x % kWave;
+    const int64_t j = threadIdx.x < kWave ? base : base + n - 1;
+    int64_t lo = 0, hi = nrows;  // ro[lo] <= j < ro[hi]
+    while (hi - lo > 1) {
+      const int64_t step = (hi - lo + kWave - 1) / kWave;
+      const int64_t at = lo + step * lane;
+      const uint64_t le = __ballot(at < hi && ro[at] <= j);
+      const int top = 63 - __clzll((unsigned long long)le);
+      lo += step * top;
+      hi = min(hi, lo + step);
+    }
+    if (lane == 0) ends[threadIdx.x / kWave] = (int32_t)lo;
+  }
+  for (int q = threadIdx.x; q < kScanTile; q += kT) mark[q] = 0;
+  __syncthreads();
+  const int64_t r0 = ends[0], r1 = ends[1];
+  if (r1 - r0 > 16 * kScanTile) {
+    for (int q = threadIdx.x; q < n; q += kT) {
+      const int64_t j = base + q;
+      int64_t lo = r0, hi = r1 + 1;
+      while (hi - lo > 1) {
+        const int64_t mid = (lo + hi) >> 1;
+        if (ro[mid] <= j) lo = mid; else hi = mid;
+      }
+      ri_out[j + shift] = (int32_t)lo;
+    }
+    return;
+  }
+  for (int64_t r = r0 + 1 + threadIdx.x; r <= r1; r += kT) {
+    const int64_t at = ro[r] - base;
+    if (at >= 0 && at < kScanTile) atomicMax(&mark[at], (int32_t)(r - r0));
+  }
+  __syncthreads();
+  // thread t scans entries [8 t, 8 t + 8)
+  int32_t m[kScanPer], top = 0;
+#pragma unroll
+  for (int k = 0; k < kScanPer; k++) {
+    top = max(top, mark[threadIdx.x * kScanPer + k]);
+    m[k] = top;
+  }
+  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+  int32_t inc = top;
+  for (int d = 1; d < kWave; d <<= 1) {
+    const int32_t o = shfl_up(inc, d);
+    if (lane >= d) inc = max(inc, o);
+  }
+  if (lane == kWave - 1) wtop[wave] = inc;
+  int32_t before = shfl_up(inc, 1);
+  if (lane == 0) before = 0;
+  __syncthreads();
+  for (int w = 0; w < wave; w++) before = max(before, wtop[w]);
+#pragma unroll
+  for (int k = 0; k < kScanPer; k++) mark[threadIdx.x * kScanPer + k] = max(before, m[k]);
+  __syncthreads();
+  for (int q = threadIdx.x; q < n; q += kT) ri_out[base + q + shift] = (int32_t)(r0 + mark[q]);
+}
+
+inline unsigned scan_blocks(int64_t n) { return blocks_for(n, kScanTile); }
 
 template <typename W>
 __global__ void gather_kernel(const W* __restrict__ src, const int32_t* __restrict__ perm,
@@ -392,40 +592,155 @@ int finish_coo(int64_t nnz, int64_t nrows, int64_t ncols, int32_t* ri, int32_t* 
 }
 
 // ------------------------------------------------------------- emitters
-// DIA part: flags over (diagonal d, row r) in diagonal-major order.
-// (row r, diagonal d) lies on the stored diagonal iff its column is inside
-// [0, ncols): rows i_start + n, n < N of :97-101
-// (full_mask: integer values, where every bit counts; floating-point values
-// drop the sign bit, so that -0.0 is a zero too)
+// Entries of a DIA part in (row, column) order.  The Serial converter walks
+// the diagonals and sorts the entries afterwards; walking the rows, with the
+// diagonals in ascending order of their offsets (equal offsets in storage
+// order, as the stable sort leaves them), gives that order at once: a count
+// per row, a scan over the rows, and the entries written to their places.
+// (row r, diagonal d) is stored iff its column is inside [0, ncols) (rows
+// i_start + n, n < N of :97-101) and its value is not a zero (full_mask:
+// integer values, where every bit counts; floating-point values drop the sign
+// bit, so that -0.0 is a zero too).
 template <typename W>
-__global__ void dia_flag_kernel(int64_t nrows, int64_t ncols, int64_t ndiag, int64_t pitch,
-                                const int32_t* __restrict__ off, const void* __restrict__ val_,
-                                int32_t* __restrict__ flag, int full_mask) {
-  const W* val = static_cast<const W*>(val_);
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= nrows * ndiag) return;
-  const int64_t d = t / nrows, r = t % nrows;
-  const int64_t c = r + off[d];
-  const bool in = c >= 0 && c < ncols;
-  const W mag = full_mask ? (W)~(W)0 : RawT<sizeof(W)>::mag;
-  flag[t] = (in && (val[r + pitch * d] & mag) != 0) ? 1 : 0;
-}
+struct DiaSlots {
+  const W* val;
+  const int32_t* off;  // by slot
+  const int32_t* ord;  // slot -> stored diagonal (null: the same)
+  int64_t pitch, ncols;
+  W mask;
+  __device__ __forceinline__ void load(int64_t r, int s, int32_t& c, W& v, bool& ok) const {
+    const int64_t col = r + off[s];
+    v = val[r + pitch * (ord ? ord[s] : s)];
+    ok = col >= 0 && col < ncols;
+    c = (int32_t)col;
+  }
+  __device__ __forceinline__ void finish(int64_t, int, int32_t, W& v, bool& ok) const {
+    ok = ok && (v & mask) != 0;
+  }
+};
+
+// Entries of an ELL part, slots that hold a column, in slot order.
+template <typename W>
+struct EllSlots {
+  const int32_t* eci;
+  const W* ev;
+  int64_t pitch;
+  __device__ __forceinline__ void load(int64_t r, int s, int32_t& c, W&, bool& ok) const {
+    c = eci[r + pitch * s];
+    ok = c != -1;
+  }
+  __device__ __forceinline__ void finish(int64_t r, int s, int32_t, W& v, bool& ok) const {
+    if (ok) v = ev[r + pitch * s];
+  }
+};
 
 template <typename W>
-__global__ void dia_emit_kernel(int64_t nrows, int64_t ndiag, int64_t pitch,
-                                const int32_t* __restrict__ off, const void* __restrict__ val_,
-                                const int32_t* __restrict__ flag, const int32_t* __restrict__ pos,
-                                int32_t* __restrict__ ri, int32_t* __restrict__ ci,
-                                void* __restrict__ vo_) {
-  const W* val = static_cast<const W*>(val_);
-  W* vo = static_cast<W*>(vo_);
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= nrows * ndiag || !flag[t]) return;
-  const int64_t d = t / nrows, r = t % nrows;
-  const int64_t p = pos[t];
-  ri[p] = (int32_t)r;
-  ci[p] = (int32_t)(r + off[d]);
-  vo[p] = val[r + pitch * d];
+__global__ __launch_bounds__(kT) void dia_row_count_kernel(DiaSlots<W> src, int64_t nrows,
+                                                           int32_t ns,
+                                                           int32_t* __restrict__ cnt) {
+  const int64_t r = (int64_t)blockIdx.x * kT + threadIdx.x;
+  if (r >= nrows) return;
+  int32_t n = 0;
+  for (int s0 = 0; s0 < ns; s0 += kScanPer) {
+    W v[kScanPer];
+    bool ok[kScanPer];
+    int32_t c;
+#pragma unroll
+    for (int k = 0; k < kScanPer; k++) {
+      ok[k] = false;
+      if (s0 + k < ns) src.load(r, s0 + k, c, v[k], ok[k]);
+    }
+#pragma unroll
+    for (int k = 0; k < kScanPer; k++) {
+      if (ok[k]) src.finish(r, s0 + k, c, v[k], ok[k]);
+      n += ok[k] ? 1 : 0;
+    }
+  }
+  cnt[r] = n;
+}
+
+// The entries of 64 rows a workgroup: lane = row, each wave a quarter of the
+// slots, batches of 32 slots.  The entries are staged in LDS in output order
+// and written coalesced (written from the row walk, each store of a wave
+// spreads over 64 rows' entries); row r's go to rowpos[r], rowpos[r] + 1, ...
+// (a row's range may be longer: HYB's COO entries follow).  Reads the slots
+// once, coalesced, writes 8 + W bytes an entry once.
+constexpr int kEmitRows = kWave;
+constexpr int kEmitWaves = kT / kWave;
+constexpr int kEmitPer = 8;  // slots per lane and batch
+constexpr int kEmitBatch = kEmitWaves * kEmitPer;
+
+template <typename W, typename Src>
+__global__ __launch_bounds__(kT) void emit_rows_kernel(Src src, int64_t nrows, int32_t ns,
+                                                       const int32_t* __restrict__ rowpos,
+                                                       int32_t* __restrict__ ri,
+                                                       int32_t* __restrict__ ci,
+                                                       W* __restrict__ vo) {
+  __shared__ W sv[kEmitRows * kEmitBatch];
+  __shared__ int32_t sc[kEmitRows * kEmitBatch];
+  __shared__ uint8_t sr[kEmitRows * kEmitBatch];
+  __shared__ int32_t cnt[kEmitWaves][kEmitRows];
+  __shared__ int32_t dst[kEmitRows];  // output position of the row's first entry, less its LDS place
+  __shared__ int32_t total;
+  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+  const int64_t r0 = (int64_t)blockIdx.x * kEmitRows, r = r0 + lane;
+  int32_t pos = r < nrows ? rowpos[r] : 0;
+  for (int s0 = 0; s0 < ns; s0 += kEmitBatch) {
+    // the batch's slots in order over the waves
+    const int per = (min(kEmitBatch, ns - s0) + kEmitWaves - 1) / kEmitWaves;
+    const int sb = s0 + wave * per, se = min(min(sb + per, s0 + kEmitBatch), (int)ns);
+    W v[kEmitPer];
+    int32_t c[kEmitPer];
+    bool ok[kEmitPer];
+#pragma unroll
+    for (int k = 0; k < kEmitPer; k++) {
+      ok[k] = false;
+      if (sb + k < se && r < nrows) src.load(r, sb + k, c[k], v[k], ok[k]);
+    }
+    int32_t n = 0;
+#pragma unroll
+    for (int k = 0; k < kEmitPer; k++) {
+      if (ok[k]) src.finish(r, sb + k, c[k], v[k], ok[k]);
+      n += ok[k] ? 1 : 0;
+    }
+    cnt[wave][lane] = n;
+    __syncthreads();
+    int32_t before = 0, row_n = 0;
+    for (int w = 0; w < kEmitWaves; w++) {
+      const int32_t q = cnt[w][lane];
+      before += w < wave ? q : 0;
+      row_n += q;
+    }
+    int32_t inc = row_n;  // (the same in every wave)
+    for (int d = 1; d < kWave; d <<= 1) {
+      const int32_t o = shfl_up(inc, d);
+      if (lane >= d) inc += o;
+    }
+    const int32_t first = inc - row_n;
+    if (wave == 0) {
+      dst[lane] = pos - first;
+      if (lane == kWave - 1) total = inc;
+    }
+    int32_t at = first + before;
+#pragma unroll
+    for (int k = 0; k < kEmitPer; k++)
+      if (ok[k]) {
+        sv[at] = v[k];
+        sc[at] = c[k];
+        sr[at] = (uint8_t)lane;
+        at++;
+      }
+    __syncthreads();
+    for (int j = threadIdx.x; j < total; j += kT) {
+      const int q = sr[j];
+      const int64_t o = (int64_t)dst[q] + j;
+      ri[o] = (int32_t)(r0 + q);
+      ci[o] = sc[j];
+      vo[o] = sv[j];
+    }
+    pos += row_n;
+    __syncthreads();
+  }
 }
 
 // zero the COO slots [from, nnz) left unfilled
@@ -634,6 +949,62 @@ __global__ void dia_place_kernel(const int32_t* __restrict__ ri, const int32_t* 
   if (winner[slot] == (int32_t)i) dv[slot] = v[i];
 }
 
+// DIA / HDC placement of entries in strictly ascending (row, column) order:
+// no slot is written twice, so the values go straight to their slots.
+// Consecutive entries of a diagonal are consecutive in memory; a workgroup's
+// kScanTile entries write runs of hundreds of rows.  (With repeated or
+// unsorted entries, the latest entry claims each slot first, below.)
+constexpr int kPlaceOffsets = 1024;  // offsets kept in LDS
+template <typename W>
+__global__ __launch_bounds__(kT) void dia_place_once_kernel(
+    const int32_t* __restrict__ ri, const int32_t* __restrict__ ci, const void* __restrict__ v_,
+    int64_t nnz, const int32_t* __restrict__ off, int64_t ndiag, int64_t pitch,
+    void* __restrict__ dv_) {
+  __shared__ int32_t soff[kPlaceOffsets];
+  const W* v = static_cast<const W*>(v_);
+  W* dv = static_cast<W*>(dv_);
+  const bool lds = ndiag <= kPlaceOffsets;
+  if (lds) {
+    for (int q = threadIdx.x; q < ndiag; q += kT) soff[q] = off[q];
+    __syncthreads();
+  }
+  const int64_t base = (int64_t)blockIdx.x * kScanTile + threadIdx.x;
+  int32_t r[kScanPer], c[kScanPer];
+  W x[kScanPer];
+#pragma unroll
+  for (int k = 0; k < kScanPer; k++) {
+    const int64_t i = base + (int64_t)k * kT;
+    if (i < nnz) {
+      r[k] = ri[i];
+      c[k] = ci[i];
+      x[k] = v[i];
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < kScanPer; k++) {
+    if (base + (int64_t)k * kT >= nnz) break;
+    const int64_t d = find_first(lds ? soff : off, ndiag, c[k] - r[k]);
+    if (d >= 0) dv[r[k] + pitch * d] = x[k];
+  }
+}
+
+// The bitmap of used diagonals (bit col - row + nrows - 1) to ascending offsets.
+__global__ void bit_count_kernel(const uint32_t* __restrict__ bits, int64_t words,
+                                 int32_t* __restrict__ cnt) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < words) cnt[i] = __popc(bits[i]);
+}
+
+__global__ void bit_offsets_kernel(const uint32_t* __restrict__ bits,
+                                   const int32_t* __restrict__ pos, int64_t words, int64_t nrows,
+                                   int32_t* __restrict__ off) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= words) return;
+  int64_t p = pos[i];
+  for (uint32_t w = bits[i]; w; w &= w - 1)
+    off[p++] = (int32_t)(i * 32 + __ffs(w) - 1 - nrows + 1);
+}
+
 __global__ __launch_bounds__(kT) void diag_hist_kernel(const int32_t* __restrict__ ri,
                                                        const int32_t* __restrict__ ci, int64_t nnz,
                                                        int64_t nrows, int32_t* __restrict__ cnt) {
@@ -737,36 +1108,143 @@ int row_counts(const int32_t* ri, int64_t nnz, int64_t nrows, Tmp& t, int32_t** 
   return MPH_OK;
 }
 
-// DIA-part emission shared by DIA -> COO and HDC -> COO; returns the count
+// What coo_scan_kernel finds, as check_coo_in reports it.
+int scan_status(int32_t flags) {
+  if (flags & kBadRow) return invalid("COO row_indices: index out of range");
+  if (flags & kBadCol) return invalid("COO column_indices: index out of range");
+  return MPH_OK;
+}
+
+int check_coo_args(int64_t nrows, int64_t ncols, int64_t nnz, const int32_t* ri,
+                   const int32_t* ci, bool cols) {
+  if (nrows < 0 || ncols < 0 || nnz < 0) return invalid("negative size");
+  if (nnz > 0 && !ri) return invalid("null COO row indices");
+  if (nnz > 0 && cols && !ci) return invalid("null COO column indices");
+  return MPH_OK;
+}
+
+// The diagonals a COO list uses, and how its entries are ordered.
+struct DiaScan {
+  uint32_t* bits = nullptr;
+  int32_t* pos = nullptr;
+  int64_t words = 0, ndiag = 0;
+  int32_t flags = 0;
+};
+
+int dia_scan(int64_t nrows, int64_t ncols, int64_t nnz, const int32_t* ri, const int32_t* ci,
+             Tmp& t, DiaScan& D, hipStream_t s) {
+  D.words = ceil_div(nrows + ncols - 1, 32);
+  int32_t *flags, *cnt, *hf, *hn;
+  int64_t* tmp;
+  MPH_CHECK_STATUS(t.alloc(&D.bits, D.words + 1));
+  MPH_CHECK_STATUS(t.alloc(&cnt, D.words));
+  MPH_CHECK_STATUS(t.alloc(&D.pos, D.words + 1));
+  MPH_CHECK_STATUS(t.alloc(&tmp, scan_tmp_elems(D.words)));
+  MPH_CHECK_STATUS(fill_zero(D.bits, sizeof(uint32_t) * (size_t)(D.words + 1), s));
+  flags = reinterpret_cast<int32_t*>(D.bits + D.words);
+  hipLaunchKernelGGL((coo_scan_kernel<true, false, true>), dim3(scan_blocks(nnz)), dim3(kT), 0, s,
+                     ri, ci, nnz, nrows, ncols, (int32_t*)nullptr, D.bits, flags);
+  hipLaunchKernelGGL(bit_count_kernel, dim3(blocks_for(D.words)), dim3(kT), 0, s, D.bits, D.words,
+                     cnt);
+  MPH_HIP_CHECK(hipGetLastError());
+  MPH_CHECK_STATUS(exclusive_scan_i32(cnt, D.pos, D.words, tmp, s));
+  MPH_CHECK_STATUS(t.fetch(flags, &hf));
+  MPH_CHECK_STATUS(t.fetch(D.pos + D.words, &hn));
+  MPH_CHECK_STATUS(t.wait());
+  D.flags = *hf;
+  D.ndiag = *hn;
+  return scan_status(D.flags);
+}
+
+// The values of a COO list on the diagonals of `off` (ascending); values of
+// slots without an entry are 0.  `flags` as coo_scan_kernel leaves them.
+// rest, if given, is set where an entry's diagonal is not among them.
+int dia_place(int64_t nnz, const int32_t* ri, const int32_t* ci, const void* v, int vs,
+              const int32_t* off, int64_t ndiag, int64_t pitch, int32_t flags, void* dv,
+              int32_t* rest, Tmp& t, hipStream_t s) {
+  MPH_CHECK_STATUS(fill_zero(dv, (size_t)vs * pitch * ndiag, s));
+  if (nnz == 0) return MPH_OK;
+  if (!(flags & kRepeated) && !rest) {
+    MPH_LAUNCH_W(dia_place_once_kernel, vs, dim3(scan_blocks(nnz)), s, ri, ci, v, nnz, off, ndiag,
+                 pitch, dv);
+  } else {
+    int32_t* win;
+    MPH_CHECK_STATUS(t.alloc(&win, std::max<int64_t>(pitch * ndiag, 1)));
+    MPH_CHECK_STATUS(fill_i32(win, pitch * ndiag, -1, s));
+    hipLaunchKernelGGL(dia_claim_kernel, dim3(blocks_for(nnz)), dim3(kT), 0, s, ri, ci, nnz, off,
+                       ndiag, pitch, win, rest);
+    MPH_LAUNCH_W(dia_place_kernel, vs, dim3(blocks_for(nnz)), s, ri, ci, v, nnz, off, ndiag, pitch,
+                 win, dv);
+  }
+  MPH_HIP_CHECK(hipGetLastError());
+  return MPH_OK;
+}
+
+// The entries of a DIA part in (row, column) order, shared by DIA -> COO and
+// HDC -> COO; returns their count.
+template <typename W>
+int emit_dia_part_w(int64_t nrows, int64_t ncols, int64_t ndiag, int64_t pitch,
+                    const int32_t* off, const void* val, int vt, int64_t cap, int32_t* ri,
+                    int32_t* ci, void* v, int64_t* count, hipStream_t s) {
+  *count = 0;
+  if (nrows == 0 || ndiag == 0) return MPH_OK;
+  Tmp t(s);
+  int32_t *cnt, *rowpos, *htot, *hoff;
+  int64_t* tmp;
+  MPH_CHECK_STATUS(t.alloc(&cnt, nrows));
+  MPH_CHECK_STATUS(t.alloc(&rowpos, nrows + 1));
+  MPH_CHECK_STATUS(t.alloc(&tmp, scan_tmp_elems(nrows)));
+  DiaSlots<W> src{static_cast<const W*>(val), off, nullptr, pitch, ncols,
+                  vt == MPH_I32 ? (W)~(W)0 : RawT<sizeof(W)>::mag};
+  hipLaunchKernelGGL(dia_row_count_kernel<W>, dim3(blocks_for(nrows)), dim3(kT), 0, s, src, nrows,
+                     (int32_t)ndiag, cnt);
+  MPH_HIP_CHECK(hipGetLastError());
+  MPH_CHECK_STATUS(exclusive_scan_i32(cnt, rowpos, nrows, tmp, s));
+  MPH_CHECK_STATUS(t.fetch(rowpos + nrows, &htot));
+  MPH_CHECK_STATUS(t.fetch(off, &hoff, ndiag));
+  MPH_CHECK_STATUS(t.wait());
+  const int64_t tot = *htot;
+  if (tot > cap) return invalid("DIA holds more non-zeros than its nnz");
+  if (!std::is_sorted(hoff, hoff + ndiag)) {
+    // slots in ascending order of the offsets, equal ones in storage order
+    std::vector<int32_t> ord(ndiag);
+    for (int64_t d = 0; d < ndiag; d++) ord[d] = (int32_t)d;
+    std::stable_sort(ord.begin(), ord.end(), [&](int32_t a, int32_t b) { return hoff[a] < hoff[b]; });
+    int32_t *d_ord, *d_off, *h;
+    MPH_CHECK_STATUS(t.alloc(&h, 2 * ndiag, true));
+    MPH_CHECK_STATUS(t.alloc(&d_ord, 2 * ndiag));
+    d_off = d_ord + ndiag;
+    for (int64_t d = 0; d < ndiag; d++) {
+      h[d] = ord[d];
+      h[ndiag + d] = hoff[ord[d]];
+    }
+    MPH_HIP_CHECK(hipMemcpyAsync(d_ord, h, sizeof(int32_t) * 2 * (size_t)ndiag,
+                                 hipMemcpyHostToDevice, s));
+    src.ord = d_ord;
+    src.off = d_off;
+  }
+  if (tot > 0) {
+    hipLaunchKernelGGL((emit_rows_kernel<W, DiaSlots<W>>), dim3(blocks_for(nrows, kEmitRows)),
+                       dim3(kT), 0, s, src, nrows, (int32_t)ndiag, rowpos, ri, ci,
+                       static_cast<W*>(v));
+    MPH_HIP_CHECK(hipGetLastError());
+  }
+  *count = tot;
+  return MPH_OK;  // (t waits for the stream)
+}
+
 int emit_dia_part(int64_t nrows, int64_t ncols, int64_t ndiag, int64_t pitch,
                   const int32_t* off, const void* val, int vt, int64_t cap, int32_t* ri,
                   int32_t* ci, void* v, int64_t* count, hipStream_t s) {
-  const int vsize = (int)value_size(vt);
-  *count = 0;
-  const int64_t T = nrows * ndiag;
-  if (T == 0) return MPH_OK;
-  Tmp t(s);
-  int32_t *flag, *pos;
-  int64_t* tmp;
-  MPH_CHECK_STATUS(t.alloc(&flag, T));
-  MPH_CHECK_STATUS(t.alloc(&pos, T + 1));
-  MPH_CHECK_STATUS(t.alloc(&tmp, scan_tmp_elems(T)));
-  MPH_LAUNCH_W(dia_flag_kernel, vsize, dim3(blocks_for(T)), s, nrows, ncols, ndiag, pitch, off,
-               val, flag, vt == MPH_I32 ? 1 : 0);
-  MPH_HIP_CHECK(hipGetLastError());
-  MPH_CHECK_STATUS(exclusive_scan_i32(flag, pos, T, tmp, s));
-  int32_t tot = 0;
-  MPH_CHECK_STATUS(t.read(pos + T, &tot));
-  if (tot > cap) return invalid("DIA holds more non-zeros than its nnz");
-  if (tot > 0) {
-    MPH_LAUNCH_W(dia_emit_kernel, vsize, dim3(blocks_for(T)), s, nrows, ndiag, pitch, off,
-                 val, flag, pos, ri, ci,
-                 v);
-    MPH_HIP_CHECK(hipGetLastError());
+  auto go = [&](auto tag) {
+    return emit_dia_part_w<decltype(tag)>(nrows, ncols, ndiag, pitch, off, val, vt, cap, ri, ci, v,
+                                          count, s);
+  };
+  switch (value_size(vt)) {
+    case 8: return go(uint64_t{});
+    case 4: return go(uint32_t{});
+    default: return go(uint16_t{});
   }
-  MPH_HIP_CHECK(hipStreamSynchronize(s));
-  *count = tot;
-  return MPH_OK;
 }
 
 int zero_tail(int64_t from, int64_t nnz, int32_t* ri, int32_t* ci, void* v, int vsize,
@@ -794,7 +1272,7 @@ int mph_convert_csr_to_coo(int64_t nrows, int64_t nnz, const int32_t* ro, const 
   if (nrows < 0 || nnz < 0) return invalid("negative size");
   MPH_CHECK_STATUS(check_row_offsets(ro, nrows, nnz, s, "CSR row_offsets"));
   if (nnz == 0) return MPH_OK;
-  hipLaunchKernelGGL(expand_rows_kernel, dim3(blocks_for(nnz)), dim3(kT), 0, s, ro, nrows, nnz,
+  hipLaunchKernelGGL(expand_rows_kernel, dim3(scan_blocks(nnz)), dim3(kT), 0, s, ro, nrows, nnz,
                      (int64_t)0, ri_out);
   MPH_HIP_CHECK(hipGetLastError());
   if (ci_out != ci) MPH_CHECK_STATUS(copy_dev(ci_out, ci, sizeof(int32_t) * nnz, s));
@@ -807,23 +1285,31 @@ int mph_convert_coo_to_csr(int64_t nrows, int64_t nnz, const int32_t* ri, const 
                            void* v_out, mph_stream_t stream) {
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   MPH_CHECK_STATUS(check_vt(vt));
-  MPH_CHECK_STATUS(check_coo_in(nrows, INT32_MAX, nnz, ri, nullptr, s));
+  MPH_CHECK_STATUS(check_coo_args(nrows, INT32_MAX, nnz, ri, nullptr, false));
+  if (nnz == 0) return fill_zero(ro_out, sizeof(int32_t) * (size_t)(nrows + 1), s);
   const int vs = (int)value_size(vt);
   Tmp t(s);
+  int32_t* flags;
+  int32_t h = 0;
+  MPH_CHECK_STATUS(t.alloc(&flags, 1));
+  MPH_CHECK_STATUS(fill_zero(flags, sizeof(int32_t), s));
+  hipLaunchKernelGGL((coo_scan_kernel<false, true, false>), dim3(scan_blocks(nnz)), dim3(kT), 0, s,
+                     ri, ci, nnz, nrows, (int64_t)INT32_MAX, ro_out, (uint32_t*)nullptr, flags);
+  MPH_HIP_CHECK(hipGetLastError());
+  MPH_CHECK_STATUS(t.read(flags, &h));
+  MPH_CHECK_STATUS(scan_status(h));
+  if (!(h & kRowsDown)) {
+    t.idle = true;
+    if (ci_out != ci) MPH_CHECK_STATUS(copy_dev(ci_out, ci, sizeof(int32_t) * nnz, s));
+    if (v_out != v) MPH_CHECK_STATUS(copy_dev(v_out, v, (size_t)vs * nnz, s));
+    return MPH_OK;
+  }
+  // stable scatter by row in input order == stable sort by row
   int32_t *cnt, *r2, *c2, *perm;
   int64_t* tmp;
   MPH_CHECK_STATUS(row_counts(ri, nnz, nrows, t, &cnt, s));
   MPH_CHECK_STATUS(t.alloc(&tmp, scan_tmp_elems(nrows)));
   MPH_CHECK_STATUS(exclusive_scan_i32(cnt, ro_out, nrows, tmp, s));
-  if (nnz == 0) return MPH_OK;
-  // stable scatter by row in input order == stable sort by row
-  int sorted_rows = 1;
-  MPH_CHECK_STATUS(rows_sorted(ri, nnz, nrows, s, &sorted_rows));
-  if (sorted_rows) {
-    if (ci_out != ci) MPH_CHECK_STATUS(copy_dev(ci_out, ci, sizeof(int32_t) * nnz, s));
-    if (v_out != v) MPH_CHECK_STATUS(copy_dev(v_out, v, (size_t)vs * nnz, s));
-    return MPH_OK;
-  }
   MPH_CHECK_STATUS(t.alloc(&r2, nnz));
   MPH_CHECK_STATUS(t.alloc(&c2, nnz));
   MPH_CHECK_STATUS(t.alloc(&perm, nnz));
@@ -837,9 +1323,7 @@ int mph_convert_coo_to_csr(int64_t nrows, int64_t nnz, const int32_t* ri, const 
     MPH_CHECK_STATUS(copy_dev(vtmp, v, (size_t)nnz * vs, s));
     v = vtmp;
   }
-  MPH_CHECK_STATUS(gather_values(v, perm, nnz, v_out, vs, s));
-  MPH_HIP_CHECK(hipStreamSynchronize(s));
-  return MPH_OK;
+  return gather_values(v, perm, nnz, v_out, vs, s);
 }
 
 int mph_convert_coo_to_dia_size(int64_t nrows, int64_t ncols, int64_t nnz, const int32_t* ri,
@@ -847,26 +1331,14 @@ int mph_convert_coo_to_dia_size(int64_t nrows, int64_t ncols, int64_t nnz, const
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   if (!ndiag) return invalid("null ndiag");
   *ndiag = 0;
-  MPH_CHECK_STATUS(check_coo_in(nrows, ncols, nnz, ri, ci, s));
+  MPH_CHECK_STATUS(check_coo_args(nrows, ncols, nnz, ri, ci, true));
   if (nnz == 0) return MPH_OK;
   Tmp t(s);
-  const int64_t nb = nrows + ncols - 1;
-  int32_t *cnt, *flag, *pos;
-  int64_t* tmp;
-  MPH_CHECK_STATUS(t.alloc(&cnt, nb));
-  MPH_CHECK_STATUS(t.alloc(&flag, nb));
-  MPH_CHECK_STATUS(t.alloc(&pos, nb + 1));
-  MPH_CHECK_STATUS(t.alloc(&tmp, scan_tmp_elems(nb)));
-  MPH_CHECK_STATUS(fill_i32(cnt, nb, 0, s));
-  hipLaunchKernelGGL(diag_hist_kernel, dim3(hist_blocks(nnz)), dim3(kT), 0, s, ri, ci, nnz, nrows,
-                     cnt);
-  hipLaunchKernelGGL(nonzero_flag_kernel, dim3(blocks_for(nb)), dim3(kT), 0, s, cnt, nb, 1, flag);
-  MPH_HIP_CHECK(hipGetLastError());
-  MPH_CHECK_STATUS(exclusive_scan_i32(flag, pos, nb, tmp, s));
-  int32_t nd = 0;
-  MPH_CHECK_STATUS(t.read(pos + nb, &nd));
-  *ndiag = nd;
-  if (mph_exceeds_tolerance(nrows, nnz, nd)) {
+  DiaScan D;
+  MPH_CHECK_STATUS(dia_scan(nrows, ncols, nnz, ri, ci, t, D, s));
+  t.idle = true;
+  *ndiag = D.ndiag;
+  if (mph_exceeds_tolerance(nrows, nnz, D.ndiag)) {
     set_error("DiaMatrix fill-in would exceed maximum tolerance");
     return MPH_ERR_FORMAT_CONVERSION;
   }
@@ -880,37 +1352,21 @@ int mph_convert_coo_to_dia(int64_t nrows, int64_t ncols, int64_t nnz, const int3
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   MPH_CHECK_STATUS(check_vt(vt));
   if (nnz == 0) return MPH_OK;
-  int64_t nd = 0;
-  MPH_CHECK_STATUS(mph_convert_coo_to_dia_size(nrows, ncols, nnz, ri, ci, &nd, stream));
-  if (nd != ndiag) return invalid("ndiag does not match the COO entries");
-  if (pitch < nrows) return invalid("pitch must be >= nrows");
-  const int vs = (int)value_size(vt);
+  MPH_CHECK_STATUS(check_coo_args(nrows, ncols, nnz, ri, ci, true));
   Tmp t(s);
-  const int64_t nb = nrows + ncols - 1;
-  int32_t *cnt, *flag, *pos, *win;
-  int64_t* tmp;
-  MPH_CHECK_STATUS(t.alloc(&cnt, nb));
-  MPH_CHECK_STATUS(t.alloc(&flag, nb));
-  MPH_CHECK_STATUS(t.alloc(&pos, nb + 1));
-  MPH_CHECK_STATUS(t.alloc(&tmp, scan_tmp_elems(nb)));
-  MPH_CHECK_STATUS(t.alloc(&win, pitch * ndiag));
-  MPH_CHECK_STATUS(fill_i32(cnt, nb, 0, s));
-  hipLaunchKernelGGL(diag_hist_kernel, dim3(hist_blocks(nnz)), dim3(kT), 0, s, ri, ci, nnz, nrows,
-                     cnt);
-  hipLaunchKernelGGL(nonzero_flag_kernel, dim3(blocks_for(nb)), dim3(kT), 0, s, cnt, nb, 1, flag);
-  MPH_CHECK_STATUS(exclusive_scan_i32(flag, pos, nb, tmp, s));
-  hipLaunchKernelGGL(compact_offsets_kernel, dim3(blocks_for(nb)), dim3(kT), 0, s, flag, pos, nb,
-                     nrows, off_out);
-  MPH_CHECK_STATUS(fill_i32(win, pitch * ndiag, -1, s));
-  hipLaunchKernelGGL(dia_claim_kernel, dim3(blocks_for(nnz)), dim3(kT), 0, s, ri, ci, nnz,
-                     off_out, ndiag, pitch, win, (int32_t*)nullptr);
-  MPH_CHECK_STATUS(fill_zero(val_out, (size_t)vs * pitch * ndiag, s));
-  MPH_LAUNCH_W(dia_place_kernel, vs, dim3(blocks_for(nnz)), s, ri, ci,
-               v, nnz, off_out, ndiag, pitch, win,
-               val_out);
+  DiaScan D;
+  MPH_CHECK_STATUS(dia_scan(nrows, ncols, nnz, ri, ci, t, D, s));
+  if (mph_exceeds_tolerance(nrows, nnz, D.ndiag)) {
+    set_error("DiaMatrix fill-in would exceed maximum tolerance");
+    return MPH_ERR_FORMAT_CONVERSION;
+  }
+  if (D.ndiag != ndiag) return invalid("ndiag does not match the COO entries");
+  if (pitch < nrows) return invalid("pitch must be >= nrows");
+  hipLaunchKernelGGL(bit_offsets_kernel, dim3(blocks_for(D.words)), dim3(kT), 0, s, D.bits, D.pos,
+                     D.words, nrows, off_out);
   MPH_HIP_CHECK(hipGetLastError());
-  MPH_HIP_CHECK(hipStreamSynchronize(s));
-  return MPH_OK;
+  return dia_place(nnz, ri, ci, v, (int)value_size(vt), off_out, ndiag, pitch, D.flags, val_out,
+                   nullptr, t, s);
 }
 
 int mph_convert_dia_to_coo(int64_t nrows, int64_t ncols, int64_t nnz, int64_t ndiag,
@@ -925,6 +1381,7 @@ int mph_convert_dia_to_coo(int64_t nrows, int64_t ncols, int64_t nnz, int64_t nd
   int64_t cnt = 0;
   MPH_CHECK_STATUS(emit_dia_part(nrows, ncols, ndiag, pitch, off, val, vt, nnz, ri_out, ci_out,
                                  v_out, &cnt, s));
+  if (cnt == nnz) return MPH_OK;  // in order
   MPH_CHECK_STATUS(zero_tail(cnt, nnz, ri_out, ci_out, v_out, vs, s));
   return finish_coo(nnz, nrows, ncols, ri_out, ci_out, v_out, vs, s);
 }
@@ -1280,7 +1737,7 @@ int mph_convert_hdc_to_coo(int64_t nrows, int64_t ncols, int64_t nnz, int64_t nd
                                  v_out, &nd, s));
   if (nd + csr_nnz > nnz) return invalid("HDC holds more entries than its nnz");
   if (csr_nnz > 0) {
-    hipLaunchKernelGGL(expand_rows_kernel, dim3(blocks_for(csr_nnz)), dim3(kT), 0, s, csr_ro,
+    hipLaunchKernelGGL(expand_rows_kernel, dim3(scan_blocks(csr_nnz)), dim3(kT), 0, s, csr_ro,
                        nrows, csr_nnz, nd, ri_out);
     MPH_HIP_CHECK(hipGetLastError());
     MPH_CHECK_STATUS(copy_dev(ci_out + nd, csr_ci, sizeof(int32_t) * csr_nnz, s));

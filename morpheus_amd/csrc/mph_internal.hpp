@@ -299,13 +299,24 @@ struct Tmp {
     *p = static_cast<T*>(b.p);
     return MPH_OK;
   }
+  // enqueues the copy of n words of device memory to pinned memory, there to
+  // be read once the stream has been synchronised
+  template <typename T>
+  int fetch(const T* d, T** pin, int64_t n = 1) {
+    MPH_CHECK_STATUS(alloc(pin, n, true));
+    MPH_HIP_CHECK(hipMemcpyAsync(*pin, d, sizeof(T) * (size_t)n, hipMemcpyDeviceToHost, s));
+    return MPH_OK;
+  }
+  int wait() {
+    MPH_HIP_CHECK(hipStreamSynchronize(s));
+    return MPH_OK;
+  }
   // n words of device memory to the host, and the stream synchronised
   template <typename T>
   int read(const T* d, T* h, int64_t n = 1) {
     T* pin = nullptr;
-    MPH_CHECK_STATUS(alloc(&pin, n, true));
-    MPH_HIP_CHECK(hipMemcpyAsync(pin, d, sizeof(T) * (size_t)n, hipMemcpyDeviceToHost, s));
-    MPH_HIP_CHECK(hipStreamSynchronize(s));
+    MPH_CHECK_STATUS(fetch(d, &pin, n));
+    MPH_CHECK_STATUS(wait());
     std::copy(pin, pin + n, h);
     return MPH_OK;
   }

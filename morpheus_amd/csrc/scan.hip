@@ -86,16 +86,11 @@ __global__ __launch_bounds__(kScanThreads) void tile_scan_kernel(
   if (blockIdx.x == 0 && threadIdx.x == 0) out[n] = (int32_t)sums[nt];
 }
 
-__global__ void fill_zero_kernel(uint32_t* __restrict__ p, int64_t nwords) {
+template <typename W>
+__global__ __launch_bounds__(256) void fill_zero_kernel(W* __restrict__ p, int64_t nwords) {
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nwords;
-       i += stride)
-    p[i] = 0u;
-}
-
-__global__ void fill_zero_bytes_kernel(uint8_t* __restrict__ p, int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = 0;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nwords; i += stride)
+    p[i] = W{};
 }
 
 }  // namespace
@@ -108,8 +103,7 @@ int exclusive_scan_i32(const int32_t* in, int32_t* out, int64_t n,
   const int64_t nt = ceil_div(n, kScanTile);
   if (nt == 0) {
     // out[0] = 0
-    hipLaunchKernelGGL(fill_zero_kernel, dim3(1), dim3(64), 0, s,
-                       reinterpret_cast<uint32_t*>(out), (int64_t)1);
+    hipLaunchKernelGGL(fill_zero_kernel<int32_t>, dim3(1), dim3(64), 0, s, out, (int64_t)1);
     MPH_HIP_CHECK(hipGetLastError());
     return MPH_OK;
   }
@@ -124,20 +118,23 @@ int exclusive_scan_i32(const int32_t* in, int32_t* out, int64_t n,
 }
 
 // Clears device memory with a kernel rather than hipMemsetAsync so that the
-// call stays safe inside captured hipGraphs.
+// call stays safe inside captured hipGraphs.  16-byte stores over the aligned
+// part, then the bytes left.
 int fill_zero(void* p, size_t bytes, hipStream_t s) {
   if (bytes == 0) return MPH_OK;
-  const int64_t words = (int64_t)(bytes / 4);
-  if (words > 0) {
-    const int64_t blocks = std::min<int64_t>(ceil_div(words, 256), 65536);
-    hipLaunchKernelGGL(fill_zero_kernel, dim3((unsigned)blocks), dim3(256), 0,
-                       s, reinterpret_cast<uint32_t*>(p), words);
-  }
-  const int64_t rem = (int64_t)(bytes % 4);
-  if (rem > 0) {
-    hipLaunchKernelGGL(fill_zero_bytes_kernel, dim3(1), dim3(64), 0, s,
-                       reinterpret_cast<uint8_t*>(p) + words * 4, rem);
-  }
+  const size_t wide = reinterpret_cast<uintptr_t>(p) % 16 == 0 ? bytes / 16
+                                                                : 0;
+  const size_t word = reinterpret_cast<uintptr_t>(p) % 4 == 0 ? (bytes - wide * 16) / 4 : 0;
+  auto launch = [&](auto tag, size_t at, size_t n) {
+    using W = decltype(tag);
+    if (n == 0) return;
+    const unsigned g = (unsigned)std::min<int64_t>(ceil_div((int64_t)n, 256), 16384);
+    hipLaunchKernelGGL(fill_zero_kernel<W>, dim3(g), dim3(256), 0, s,
+                       reinterpret_cast<W*>(static_cast<uint8_t*>(p) + at), (int64_t)n);
+  };
+  launch(uint4{}, 0, wide);
+  launch(uint32_t{}, wide * 16, word);
+  launch(uint8_t{}, wide * 16 + word * 4, bytes - wide * 16 - word * 4);
   MPH_HIP_CHECK(hipGetLastError());
   return MPH_OK;
 }

@@ -1,0 +1,112 @@
+"""Conversions at the edges of their kernels' tiles (64 rows, 256 threads, 2048
+entries, 32 slots a batch), bit-exact against the CPU oracle: entry counts and
+row counts around the tiles, long runs of empty rows, repeated and unsorted
+entries, diagonals in any order and repeated, sizes that leave phantom slots."""
+import numpy as np
+import pytest
+
+import oracle
+from morpheus_amd.formats import (COO_FORMAT, CSR_FORMAT, DIA_FORMAT, ELL_FORMAT, HDC_FORMAT,
+                                  HYB_FORMAT, Coo, Dia)
+from tests.helpers import same_container
+from tests.test_convert_gpu import gpu_convert, round_values
+
+pytestmark = pytest.mark.gpu
+
+COO_TARGETS = [CSR_FORMAT, DIA_FORMAT, ELL_FORMAT, HYB_FORMAT, HDC_FORMAT]
+
+
+def _check(A, fmt, dtype="f64"):
+    A = round_values(A, dtype)
+    try:
+        ref = oracle.from_coo(A, fmt) if isinstance(A, Coo) else oracle.convert(A, fmt)
+    except oracle.FormatConversion:
+        return
+    assert same_container(gpu_convert(A, fmt, dtype), ref), fmt
+
+
+def _entries(nrows, ncols, nnz, seed, band=None):
+    """nnz distinct entries in (row, column) order, values 1, 2, ..."""
+    rng = np.random.default_rng(seed)
+    if band is None:
+        key = np.sort(rng.choice(nrows * ncols, size=nnz, replace=False))
+    else:
+        r, o = rng.integers(0, nrows, 4 * nnz), rng.integers(-band, band + 1, 4 * nnz)
+        ok = (r + o >= 0) & (r + o < ncols)
+        key = np.unique(r[ok] * ncols + r[ok] + o[ok])[:nnz]
+    return Coo(nrows, ncols, key // ncols, key % ncols, 1.0 + np.arange(key.size))
+
+
+@pytest.mark.parametrize("nnz", [1, 2, 63, 64, 65, 255, 256, 257, 2047, 2048, 2049, 4097])
+@pytest.mark.parametrize("fmt", COO_TARGETS)
+def test_entry_counts(gpu, nnz, fmt):
+    _check(_entries(120, 120, nnz, nnz), fmt)
+    A = _entries(120, 120, nnz, nnz)
+    back = oracle.convert(oracle.from_coo(A, CSR_FORMAT), fmt)
+    assert same_container(gpu_convert(oracle.from_coo(A, CSR_FORMAT), fmt), back)
+    assert same_container(gpu_convert(back, CSR_FORMAT), oracle.convert(back, CSR_FORMAT))
+
+
+@pytest.mark.parametrize("nrows", [1, 63, 64, 65, 127, 129, 255, 257, 1000])
+@pytest.mark.parametrize("band", [1, 15, 16, 40])
+@pytest.mark.parametrize("dtype", ["f64", "f32", "bf16"])
+def test_row_counts_and_slots(gpu, nrows, band, dtype):
+    A = _entries(nrows, nrows, max(1, min(nrows * 3, nrows * nrows // 2)), nrows + band, band)
+    A.values = (A.values % 200) + 1.0  # exact in BF16
+    for fmt in COO_TARGETS:
+        _check(A, fmt, dtype)
+        try:
+            B = oracle.from_coo(A, fmt)
+        except oracle.FormatConversion:
+            continue
+        got = gpu_convert(B, COO_FORMAT, dtype)
+        assert same_container(got, oracle.to_coo(B)), fmt
+
+
+@pytest.mark.parametrize("where", ["first", "middle", "last", "spread"])
+def test_long_runs_of_empty_rows(gpu, where):
+    n = 90000
+    rows = {"first": np.arange(10), "last": n - 1 - np.arange(10)[::-1],
+            "middle": np.r_[0, 1, 2, n - 3, n - 2, n - 1],
+            "spread": np.arange(0, n, 2500)}[where]
+    rows = np.repeat(rows, 3)
+    cols = np.tile([0, 5, 9], rows.size // 3)
+    A = Coo(n, 12, rows, cols, 1.0 + np.arange(rows.size))
+    csr = oracle.from_coo(A, CSR_FORMAT)
+    _check(A, CSR_FORMAT)
+    assert same_container(gpu_convert(csr, COO_FORMAT), oracle.to_coo(csr))
+
+
+@pytest.mark.parametrize("order", ["repeated", "unsorted columns", "unsorted rows"])
+@pytest.mark.parametrize("fmt", COO_TARGETS)
+def test_repeated_and_unsorted_entries(gpu, order, fmt):
+    A = _entries(300, 300, 2100, 7, 4)
+    rng = np.random.default_rng(3)
+    at = np.arange(A.nnz)
+    if order == "repeated":
+        at = np.sort(np.r_[at, rng.integers(0, A.nnz, 200)])
+    elif order == "unsorted columns":
+        at = np.lexsort((rng.random(A.nnz), A.row_indices))
+    else:
+        at = rng.permutation(A.nnz)
+    B = Coo(300, 300, A.row_indices[at], A.column_indices[at], 1.0 + np.arange(at.size))
+    _check(B, fmt)
+
+
+@pytest.mark.parametrize("offsets", [[5, -3, 0, 2, -70], [0, 0, 1], [-1, 2, -1, 0, 2],
+                                     list(range(20, -21, -1))])
+@pytest.mark.parametrize("extra", [0, 3])
+def test_dia_in_any_order(gpu, offsets, extra):
+    """Diagonals unsorted or repeated; nnz above the stored non-zeros leaves
+    phantom entries."""
+    n, pitch = 130, 160
+    rng = np.random.default_rng(9)
+    v = rng.integers(-2, 3, size=(len(offsets), pitch)).astype(float)
+    v[:, ::7] = -0.0
+    v[:, n:] = 0.0
+    off = np.array(offsets, dtype=np.int32)
+    inside = (np.arange(pitch)[None, :] + off[:, None] >= 0) & \
+        (np.arange(pitch)[None, :] + off[:, None] < n)
+    nnz = int(np.count_nonzero(v * inside)) + extra
+    A = Dia(n, n, nnz, off, v.reshape(-1), pitch)
+    assert same_container(gpu_convert(A, COO_FORMAT), oracle.to_coo(A))
