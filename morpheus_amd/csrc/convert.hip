@@ -111,7 +111,7 @@ __global__ __launch_bounds__(kT) void row_hist_kernel(const int32_t* __restrict_
 // registers and LDS, and adds its result with one atomic.  An atomic per
 // element on one address was served one at a time: the maxima of 14.6M COO
 // indices took 2.6 ms, now about 15 us (the 58 MB read at the stream rate).
-constexpr int64_t kReduceBlocks = 2048;
+constexpr int64_t kReduceBlocks = 512;  // (2048 spent 20 us on the atomics)
 inline unsigned reduce_blocks(int64_t n) {
   return (unsigned)std::min<int64_t>(blocks_for(n, 4 * kT), kReduceBlocks);
 }
@@ -755,89 +755,62 @@ __global__ void zero_tail_kernel(int64_t from, int64_t nnz, int32_t* ri, int32_t
   }
 }
 
-// ELL part: flags over (row r, slot n) in row-major order.
-__global__ void ell_flag_kernel(int64_t nrows, int64_t width, int64_t pitch,
-                                const int32_t* __restrict__ eci, int32_t* __restrict__ flag) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= nrows * width) return;
-  const int64_t r = t / width, n = t % width;
-  flag[t] = eci[r + pitch * n] != -1 ? 1 : 0;
+// Per row, the ELL slots that hold a column plus the row's entries of the
+// row-sorted COO part (tro null: none); stats: [0] raised when some row's
+// columns are not in ascending order (its COO entries after its slots; the
+// order among the COO entries is checked by coo_scan_kernel), [1] 1 + the
+// last slot any row uses.
+__global__ __launch_bounds__(kT) void ell_row_count_kernel(
+    const int32_t* __restrict__ eci, int64_t nrows, int64_t width, int64_t pitch,
+    const int32_t* __restrict__ tro, const int32_t* __restrict__ tci, int32_t* __restrict__ cnt,
+    int32_t* __restrict__ stats) {
+  const int64_t r = (int64_t)blockIdx.x * kT + threadIdx.x;
+  int32_t n = 0, prev = INT32_MIN, bad = 0, top = 0;
+  if (r < nrows) {
+    for (int64_t s0 = 0; s0 < width; s0 += kScanPer) {
+      int32_t c[kScanPer];
+#pragma unroll
+      for (int k = 0; k < kScanPer; k++) c[k] = s0 + k < width ? eci[r + pitch * (s0 + k)] : -1;
+#pragma unroll
+      for (int k = 0; k < kScanPer; k++)
+        if (c[k] != -1) {
+          bad |= c[k] < prev ? 1 : 0;
+          prev = c[k];
+          n++;
+          top = (int32_t)(s0 + k) + 1;
+        }
+    }
+    if (tro) {
+      const int32_t ts = tro[r], te = tro[r + 1];
+      if (te > ts && n > 0 && tci[ts] < prev) bad = 1;
+      n += te - ts;
+    }
+    cnt[r] = n;
+  }
+  raise_flags(&stats[0], bad);
+  top = block_reduce(top, [](int32_t u, int32_t v) { return max(u, v); });
+  if (threadIdx.x == 0 && top > 0 &&
+      __hip_atomic_load(&stats[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < top)
+    atomicMax(&stats[1], top);
 }
 
+// HYB -> COO, the COO part: entry j of row r ends r's range
 template <typename W>
-__global__ void ell_emit_kernel(int64_t nrows, int64_t width, int64_t pitch,
-                                const int32_t* __restrict__ eci, const void* __restrict__ ev_,
-                                const int32_t* __restrict__ flag, const int32_t* __restrict__ pos,
-                                int32_t* __restrict__ ri, int32_t* __restrict__ ci,
-                                void* __restrict__ vo_) {
-  const W* ev = static_cast<const W*>(ev_);
-  W* vo = static_cast<W*>(vo_);
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= nrows * width || !flag[t]) return;
-  const int64_t r = t / width, n = t % width;
-  const int64_t p = pos[t];
-  ri[p] = (int32_t)r;
-  ci[p] = eci[r + pitch * n];
-  vo[p] = ev[r + pitch * n];
-}
-
-// HYB -> COO: row r's block starts at rowpos[r]; ELL slots first (compacted
-// in slot order), then the row's entries of the row-sorted COO part.
-template <typename W>
-__global__ void hyb_emit_kernel(int64_t nrows, int64_t width, int64_t pitch,
-                                const int32_t* __restrict__ eci, const void* __restrict__ ev_,
-                                const int32_t* __restrict__ tro, const int32_t* __restrict__ tci,
-                                const void* __restrict__ tv_, const int32_t* __restrict__ rowpos,
-                                int32_t* __restrict__ ri, int32_t* __restrict__ ci,
-                                void* __restrict__ vo_) {
-  const W* ev = static_cast<const W*>(ev_);
+__global__ void hyb_tail_emit_kernel(const int32_t* __restrict__ tri,
+                                     const int32_t* __restrict__ tci,
+                                     const void* __restrict__ tv_, int64_t n,
+                                     const int32_t* __restrict__ tro,
+                                     const int32_t* __restrict__ rowpos, int32_t* __restrict__ ri,
+                                     int32_t* __restrict__ ci, void* __restrict__ vo_) {
   const W* tv = static_cast<const W*>(tv_);
   W* vo = static_cast<W*>(vo_);
-  const int64_t r = (int64_t)blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave;
-  const int lane = threadIdx.x % kWave;
-  if (r >= nrows) return;
-  const uint64_t lt = (lane == 0) ? 0ull : ((~0ull) >> (64 - lane));
-  int64_t p = rowpos[r];
-  for (int64_t n0 = 0; n0 < width; n0 += kWave) {
-    const int64_t n = n0 + lane;
-    const int32_t c = n < width ? eci[r + pitch * n] : -1;
-    const uint64_t m = __ballot(c != -1);
-    if (c != -1) {
-      const int64_t q = p + __popcll(m & lt);
-      ri[q] = (int32_t)r;
-      ci[q] = c;
-      vo[q] = ev[r + pitch * n];
-    }
-    p += __popcll(m);
-  }
-  const int64_t ts = tro[r], te = tro[r + 1];
-  for (int64_t j = ts + lane; j < te; j += kWave) {
-    const int64_t q = p + (j - ts);
-    ri[q] = (int32_t)r;
-    ci[q] = tci[j];
-    vo[q] = tv[j];
-  }
-}
-
-__global__ void hyb_rowcount_kernel(int64_t nrows, int64_t width, int64_t pitch,
-                                    const int32_t* __restrict__ eci,
-                                    const int32_t* __restrict__ tro,
-                                    int32_t* __restrict__ cnt) {
-  const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= nrows) return;
-  int32_t c = tro[r + 1] - tro[r];
-  for (int64_t n = 0; n < width; n++) c += eci[r + pitch * n] != -1;
-  cnt[r] = c;
-}
-
-// offsets of a row-sorted COO prefix [0, P): rows in (ri[i-1], ri[i]] start at i
-__global__ void sorted_offsets_kernel(const int32_t* __restrict__ ri, int64_t P,
-                                      int64_t nrows, int32_t* __restrict__ ro) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i > P) return;
-  const int64_t prev = i == 0 ? -1 : ri[i - 1];
-  const int64_t cur = i == P ? nrows : ri[i];
-  for (int64_t r = prev + 1; r <= cur; r++) ro[r] = (int32_t)i;
+  const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (j >= n) return;
+  const int32_t r = tri[j];
+  const int64_t o = (int64_t)rowpos[r + 1] - tro[r + 1] + j;
+  ri[o] = r;
+  ci[o] = tci[j];
+  vo[o] = tv[j];
 }
 
 // ------------------------------------------------------------- COO -> X
@@ -910,6 +883,114 @@ __global__ void tail_place_kernel(const int32_t* __restrict__ ri, const int32_t*
   tri[p] = ri[i];
   tci[p] = ci[i];
   tv[p] = v[i];
+}
+
+// COO -> ELL / HYB when the rows do not decrease: row r's entries are
+// [ro[r], ro[r + 1]), its n-th in slot n, so every slot is written once, in
+// row order per slot (coalesced), padding (-1, 0) included.  64 rows a
+// workgroup, each wave every fourth slot; the rows' entries are read
+// coalesced into LDS when they fit, or directly.  (With rows that decrease,
+// a row may have several runs, and the latest entry claims each slot first,
+// above.)
+constexpr int kEllStage = 2048;
+template <typename W>
+__global__ __launch_bounds__(kT) void ell_fill_rows_kernel(
+    const int32_t* __restrict__ ro, const int32_t* __restrict__ ci, const void* __restrict__ v_,
+    int64_t nrows, int64_t K, int64_t width, int64_t pitch, int32_t* __restrict__ eci,
+    void* __restrict__ ev_) {
+  __shared__ int32_t sc[kEllStage];
+  __shared__ W sv[kEllStage];
+  const W* v = static_cast<const W*>(v_);
+  W* ev = static_cast<W*>(ev_);
+  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+  const int64_t r0 = (int64_t)blockIdx.x * kWave, r = r0 + lane;
+  const int64_t e0 = ro[min(r0, nrows)], e1 = ro[min(r0 + kWave, nrows)];
+  const bool staged = e1 - e0 <= kEllStage;
+  if (staged) {
+    for (int64_t q = threadIdx.x; q < e1 - e0; q += kT) {
+      sc[q] = ci[e0 + q];
+      sv[q] = v[e0 + q];
+    }
+    __syncthreads();
+  }
+  if (r >= pitch) return;
+  const int64_t b = r < nrows ? ro[r] : 0, len = r < nrows ? min((int64_t)ro[r + 1] - b, K) : 0;
+  for (int64_t n = wave; n < width; n += kT / kWave) {
+    int32_t c = -1;
+    W x = 0;
+    if (n < len) {
+      c = staged ? sc[b - e0 + n] : ci[b + n];
+      x = staged ? sv[b - e0 + n] : v[b + n];
+    }
+    eci[r + pitch * n] = c;
+    ev[r + pitch * n] = x;
+  }
+}
+
+// entries past a row's first K, per row
+__global__ void over_count_kernel(const int32_t* __restrict__ ro, int64_t nrows, int32_t K,
+                                  int32_t* __restrict__ cnt) {
+  const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (r < nrows) cnt[r] = max(0, ro[r + 1] - ro[r] - K);
+}
+
+// HYB's COO part: those entries, row r's at opos[r], opos[r] + 1, ...  A
+// thread's entries are loaded together, so the row lookups of all are in
+// flight at once: 101 us for 16M power-law FP32 entries, 13.4M of them past
+// their row's K (106 us with one entry a thread).
+template <typename W>
+__global__ __launch_bounds__(kT) void over_place_kernel(
+    const int32_t* __restrict__ ri, const int32_t* __restrict__ ci, const void* __restrict__ v_,
+    int64_t nnz, int64_t K, const int32_t* __restrict__ ro, const int32_t* __restrict__ opos,
+    int32_t* __restrict__ tri, int32_t* __restrict__ tci, void* __restrict__ tv_) {
+  const W* v = static_cast<const W*>(v_);
+  W* tv = static_cast<W*>(tv_);
+  const int64_t base = (int64_t)blockIdx.x * kScanTile + threadIdx.x;
+  int32_t r[kScanPer], c[kScanPer], b[kScanPer], o[kScanPer];
+  W x[kScanPer];
+#pragma unroll
+  for (int k = 0; k < kScanPer; k++) {
+    const int64_t i = min(base + (int64_t)k * kT, nnz - 1);
+    r[k] = ri[i];
+    c[k] = ci[i];
+    x[k] = v[i];
+  }
+#pragma unroll
+  for (int k = 0; k < kScanPer; k++) {
+    b[k] = ro[r[k]];
+    o[k] = opos[r[k]];
+  }
+#pragma unroll
+  for (int k = 0; k < kScanPer; k++) {
+    const int64_t i = base + (int64_t)k * kT, n = i - b[k] - K;
+    if (i >= nnz || n < 0) continue;
+    const int64_t at = o[k] + n;
+    tri[at] = r[k];
+    tci[at] = c[k];
+    tv[at] = x[k];
+  }
+}
+
+// of row offsets: the longest row, and the sum of min(length, K)
+__global__ __launch_bounds__(kT) void row_lengths_kernel(const int32_t* __restrict__ ro,
+                                                         int64_t nrows, int32_t K,
+                                                         unsigned long long* __restrict__ out) {
+  const int64_t step = (int64_t)gridDim.x * kT;
+  int32_t m = 0;
+  unsigned long long t = 0;
+  for (int64_t r = (int64_t)blockIdx.x * kT + threadIdx.x; r < nrows; r += step) {
+    const int32_t len = ro[r + 1] - ro[r];
+    m = max(m, len);
+    t += (unsigned long long)max(0, min(len, K));
+  }
+  m = block_reduce(m, [](int32_t u, int32_t v) { return max(u, v); });
+  t = block_reduce(t, [](unsigned long long u, unsigned long long v) { return u + v; });
+  if (threadIdx.x == 0) {
+    if (__hip_atomic_load(&out[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) <
+        (unsigned long long)m)
+      atomicMax(&out[0], (unsigned long long)m);
+    if (t > 0) atomicAdd(&out[1], t);
+  }
 }
 
 // DIA / HDC placement: the first offset equal to col - row (binary search of
@@ -1156,6 +1237,57 @@ int dia_scan(int64_t nrows, int64_t ncols, int64_t nnz, const int32_t* ri, const
   return scan_status(D.flags);
 }
 
+// The rows of a COO list: the longest, the sum of min(length, K), the order
+// of the entries and, rows not decreasing, their offsets.
+struct RowScan {
+  int32_t* ro = nullptr;
+  int32_t flags = 0;
+  int64_t longest = 0, clipped = 0;
+};
+
+int row_scan(int64_t nrows, int64_t nnz, const int32_t* ri, int64_t K, Tmp& t, RowScan& R,
+             hipStream_t s) {
+  unsigned long long *acc, *h;  // longest, clipped, flags
+  const int32_t k = (int32_t)std::min<int64_t>(K, INT32_MAX);
+  MPH_CHECK_STATUS(t.alloc(&R.ro, nrows + 1));
+  MPH_CHECK_STATUS(t.alloc(&acc, 3));
+  MPH_CHECK_STATUS(fill_zero(acc, 3 * sizeof(unsigned long long), s));
+  int32_t* flags = reinterpret_cast<int32_t*>(acc + 2);
+  if (nnz > 0)
+    hipLaunchKernelGGL((coo_scan_kernel<false, true, false>), dim3(scan_blocks(nnz)), dim3(kT), 0,
+                       s, ri, (const int32_t*)nullptr, nnz, nrows, (int64_t)INT32_MAX, R.ro,
+                       (uint32_t*)nullptr, flags);
+  else
+    MPH_CHECK_STATUS(fill_zero(R.ro, sizeof(int32_t) * (size_t)(nrows + 1), s));
+  // (offsets left incomplete by decreasing rows give numbers not used)
+  hipLaunchKernelGGL(row_lengths_kernel, dim3(reduce_blocks(nrows)), dim3(kT), 0, s, R.ro, nrows, k,
+                     acc);
+  MPH_HIP_CHECK(hipGetLastError());
+  MPH_CHECK_STATUS(t.fetch(acc, &h, 3));
+  MPH_CHECK_STATUS(t.wait());
+  R.flags = (int32_t)h[2];
+  MPH_CHECK_STATUS(scan_status(R.flags));
+  R.longest = (int64_t)h[0];
+  R.clipped = (int64_t)h[1];
+  if (R.flags & kRowsDown) {  // count the entries of each row
+    int32_t *cnt, *mx, *hm;
+    MPH_CHECK_STATUS(row_counts(ri, nnz, nrows, t, &cnt, s));
+    MPH_CHECK_STATUS(t.alloc(&mx, 1));
+    MPH_CHECK_STATUS(fill_zero(mx, sizeof(int32_t), s));
+    MPH_CHECK_STATUS(fill_zero(acc, sizeof(unsigned long long), s));
+    hipLaunchKernelGGL(max_kernel, dim3(reduce_blocks(nrows)), dim3(kT), 0, s, cnt, nrows, mx);
+    hipLaunchKernelGGL(clipped_sum_kernel, dim3(reduce_blocks(nrows)), dim3(kT), 0, s, cnt, nrows,
+                       k, acc);
+    MPH_HIP_CHECK(hipGetLastError());
+    MPH_CHECK_STATUS(t.fetch(mx, &hm));
+    MPH_CHECK_STATUS(t.fetch(acc, &h));
+    MPH_CHECK_STATUS(t.wait());
+    R.longest = *hm;
+    R.clipped = (int64_t)*h;
+  }
+  return MPH_OK;
+}
+
 // The values of a COO list on the diagonals of `off` (ascending); values of
 // slots without an entry are 0.  `flags` as coo_scan_kernel leaves them.
 // rest, if given, is set where an entry's diagonal is not among them.
@@ -1176,6 +1308,34 @@ int dia_place(int64_t nnz, const int32_t* ri, const int32_t* ci, const void* v, 
     MPH_LAUNCH_W(dia_place_kernel, vs, dim3(blocks_for(nnz)), s, ri, ci, v, nnz, off, ndiag, pitch,
                  win, dv);
   }
+  MPH_HIP_CHECK(hipGetLastError());
+  return MPH_OK;
+}
+
+// The ELL part of a COO list: each row's first K entries, slots without one
+// padded.  over, if given (nnz words, cleared), is set for the entries past
+// the K-th; it needs rows that decrease.
+int ell_place(int64_t nrows, int64_t nnz, const int32_t* ri, const int32_t* ci, const void* v,
+              int vs, int64_t K, int64_t width, int64_t pitch, const RowScan& S, int32_t* eci,
+              void* ev, int32_t* over, Tmp& t, hipStream_t s) {
+  if (width * pitch == 0) return MPH_OK;
+  if (!(S.flags & kRowsDown)) {
+    MPH_LAUNCH_W(ell_fill_rows_kernel, vs, dim3(blocks_for(pitch, kWave)), s, S.ro, ci, v, nrows, K,
+                 width, pitch, eci, ev);
+    MPH_HIP_CHECK(hipGetLastError());
+    return MPH_OK;
+  }
+  Runs R;
+  int32_t* win;
+  MPH_CHECK_STATUS(fill_i32(eci, width * pitch, -1, s));
+  MPH_CHECK_STATUS(fill_zero(ev, (size_t)vs * width * pitch, s));
+  MPH_CHECK_STATUS(build_runs(ri, nnz, t, R, s));
+  MPH_CHECK_STATUS(t.alloc(&win, width * pitch));
+  MPH_CHECK_STATUS(fill_i32(win, width * pitch, -1, s));
+  hipLaunchKernelGGL(ell_claim_kernel, dim3(blocks_for(nnz)), dim3(kT), 0, s, ri, nnz, K, pitch,
+                     R.head, R.hscan, R.runpos, win, over);
+  MPH_LAUNCH_W(ell_place_kernel, vs, dim3(blocks_for(nnz)), s, ri, ci, v, nnz, K, pitch, R.head,
+               R.hscan, R.runpos, win, eci, ev);
   MPH_HIP_CHECK(hipGetLastError());
   return MPH_OK;
 }
@@ -1254,6 +1414,57 @@ int zero_tail(int64_t from, int64_t nnz, int32_t* ri, int32_t* ci, void* v, int 
                v);
   MPH_HIP_CHECK(hipGetLastError());
   return MPH_OK;
+}
+
+// ELL (+ a COO part of tnnz entries with row offsets tro, tail_sorted when
+// each row's columns ascend) -> COO, rows in order: counts, a scan, the
+// slots, the COO part.  Sorted only if the stored order is not already.
+int ell_part_to_coo(int64_t nrows, int64_t nnz, int64_t width, int64_t pitch, const int32_t* eci,
+                    const void* ev, const int32_t* tro, int64_t tnnz, const int32_t* tri,
+                    const int32_t* tci, const void* tv, bool tail_unsorted, const char* too_many,
+                    int vt, int32_t* ri_out, int32_t* ci_out, void* v_out, hipStream_t s) {
+  const int vs = (int)value_size(vt);
+  int64_t tot = 0;
+  bool sorted = true;
+  if (nrows > 0) {
+    Tmp t(s);
+    int32_t *cnt, *rowpos, *stats, *ht, *hs;
+    int64_t* tmp;
+    MPH_CHECK_STATUS(t.alloc(&cnt, nrows));
+    MPH_CHECK_STATUS(t.alloc(&rowpos, nrows + 1));
+    MPH_CHECK_STATUS(t.alloc(&tmp, scan_tmp_elems(nrows)));
+    MPH_CHECK_STATUS(t.alloc(&stats, 2));
+    MPH_CHECK_STATUS(fill_zero(stats, 2 * sizeof(int32_t), s));
+    hipLaunchKernelGGL(ell_row_count_kernel, dim3(blocks_for(nrows)), dim3(kT), 0, s, eci, nrows,
+                       width, pitch, tro, tci, cnt, stats);
+    MPH_HIP_CHECK(hipGetLastError());
+    MPH_CHECK_STATUS(exclusive_scan_i32(cnt, rowpos, nrows, tmp, s));
+    MPH_CHECK_STATUS(t.fetch(rowpos + nrows, &ht));
+    MPH_CHECK_STATUS(t.fetch(stats, &hs, 2));
+    MPH_CHECK_STATUS(t.wait());
+    tot = *ht;
+    sorted = hs[0] == 0 && !tail_unsorted;
+    const int32_t slots = hs[1];
+    if (tot > nnz) return invalid(too_many);
+    if (slots > 0) {
+      auto emit = [&](auto tag) {
+        using W = decltype(tag);
+        hipLaunchKernelGGL((emit_rows_kernel<W, EllSlots<W>>), dim3(blocks_for(nrows, kEmitRows)),
+                           dim3(kT), 0, s, EllSlots<W>{eci, static_cast<const W*>(ev), pitch},
+                           nrows, slots, rowpos, ri_out, ci_out, static_cast<W*>(v_out));
+      };
+      if (vs == 8) emit(uint64_t{});
+      else if (vs == 4) emit(uint32_t{});
+      else emit(uint16_t{});
+    }
+    if (tnnz > 0)
+      MPH_LAUNCH_W(hyb_tail_emit_kernel, vs, dim3(blocks_for(tnnz)), s, tri, tci, tv, tnnz, tro,
+                   rowpos, ri_out, ci_out, v_out);
+    MPH_HIP_CHECK(hipGetLastError());
+  }
+  if (tot == nnz && sorted) return MPH_OK;
+  MPH_CHECK_STATUS(zero_tail(tot, nnz, ri_out, ci_out, v_out, vs, s));
+  return finish_coo(nnz, nrows, INT32_MAX, ri_out, ci_out, v_out, vs, s);
 }
 
 }  // namespace
@@ -1391,19 +1602,13 @@ int mph_convert_coo_to_ell_size(int64_t nrows, int64_t nnz, const int32_t* ri, i
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   if (!K) return invalid("null entries_per_row");
   *K = 0;
-  MPH_CHECK_STATUS(check_coo_in(nrows, INT32_MAX, nnz, ri, nullptr, s));
+  MPH_CHECK_STATUS(check_coo_args(nrows, INT32_MAX, nnz, ri, nullptr, false));
   Tmp t(s);
-  int32_t *cnt, *mx;
-  MPH_CHECK_STATUS(row_counts(ri, nnz, nrows, t, &cnt, s));
-  MPH_CHECK_STATUS(t.alloc(&mx, 1));
-  MPH_CHECK_STATUS(fill_i32(mx, 1, 0, s));
-  if (nrows > 0)
-    hipLaunchKernelGGL(max_kernel, dim3(reduce_blocks(nrows)), dim3(kT), 0, s, cnt, nrows, mx);
-  MPH_HIP_CHECK(hipGetLastError());
-  int32_t h = 0;
-  MPH_CHECK_STATUS(t.read(mx, &h));
-  *K = h;
-  if (mph_exceeds_tolerance(nrows, nnz, h)) {
+  RowScan R;
+  MPH_CHECK_STATUS(row_scan(nrows, nnz, ri, 0, t, R, s));
+  t.idle = true;
+  *K = R.longest;
+  if (mph_exceeds_tolerance(nrows, nnz, R.longest)) {
     set_error("EllMatrix fill-in would exceed maximum tolerance");
     return MPH_ERR_FORMAT_CONVERSION;
   }
@@ -1415,28 +1620,18 @@ int mph_convert_coo_to_ell(int64_t nrows, int64_t nnz, const int32_t* ri, const 
                            int32_t* ci_out, void* v_out, mph_stream_t stream) {
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   MPH_CHECK_STATUS(check_vt(vt));
-  int64_t k2 = 0;
-  MPH_CHECK_STATUS(mph_convert_coo_to_ell_size(nrows, nnz, ri, &k2, stream));
-  if (k2 != K) return invalid("entries_per_row does not match the COO entries");
-  if (width < K || pitch < nrows) return invalid("ELL width / pitch too small");
-  const int vs = (int)value_size(vt);
-  MPH_CHECK_STATUS(fill_i32(ci_out, width * pitch, -1, s));
-  MPH_CHECK_STATUS(fill_zero(v_out, (size_t)vs * width * pitch, s));
-  if (nnz == 0) return MPH_OK;
+  MPH_CHECK_STATUS(check_coo_args(nrows, INT32_MAX, nnz, ri, nullptr, false));
   Tmp t(s);
-  Runs R;
-  int32_t* win;
-  MPH_CHECK_STATUS(build_runs(ri, nnz, t, R, s));
-  MPH_CHECK_STATUS(t.alloc(&win, width * pitch));
-  MPH_CHECK_STATUS(fill_i32(win, width * pitch, -1, s));
-  hipLaunchKernelGGL(ell_claim_kernel, dim3(blocks_for(nnz)), dim3(kT), 0, s, ri, nnz, width,
-                     pitch, R.head, R.hscan, R.runpos, win, (int32_t*)nullptr);
-  MPH_LAUNCH_W(ell_place_kernel, vs, dim3(blocks_for(nnz)), s, ri, ci,
-               v, nnz, width, pitch, R.head, R.hscan,
-               R.runpos, win, ci_out, v_out);
-  MPH_HIP_CHECK(hipGetLastError());
-  MPH_HIP_CHECK(hipStreamSynchronize(s));
-  return MPH_OK;
+  RowScan R;
+  MPH_CHECK_STATUS(row_scan(nrows, nnz, ri, 0, t, R, s));
+  if (mph_exceeds_tolerance(nrows, nnz, R.longest)) {
+    set_error("EllMatrix fill-in would exceed maximum tolerance");
+    return MPH_ERR_FORMAT_CONVERSION;
+  }
+  if (R.longest != K) return invalid("entries_per_row does not match the COO entries");
+  if (width < K || pitch < nrows) return invalid("ELL width / pitch too small");
+  return ell_place(nrows, nnz, ri, ci, v, (int)value_size(vt), width, width, pitch, R, ci_out,
+                   v_out, nullptr, t, s);
 }
 
 int mph_convert_ell_to_coo(int64_t nrows, int64_t nnz, int64_t width, int64_t pitch,
@@ -1446,32 +1641,9 @@ int mph_convert_ell_to_coo(int64_t nrows, int64_t nnz, int64_t width, int64_t pi
   MPH_CHECK_STATUS(check_vt(vt));
   if (nnz == 0) return MPH_OK;
   if (width > 0 && pitch < nrows) return invalid("pitch must be >= nrows");
-  const int vs = (int)value_size(vt);
-  const int64_t T = nrows * width;
-  int32_t tot = 0;
-  int64_t ncols_bound = INT32_MAX;
-  {
-    Tmp t(s);
-    int32_t *flag, *pos;
-    int64_t* tmp;
-    MPH_CHECK_STATUS(t.alloc(&flag, T));
-    MPH_CHECK_STATUS(t.alloc(&pos, T + 1));
-    MPH_CHECK_STATUS(t.alloc(&tmp, scan_tmp_elems(T)));
-    if (T > 0)
-      hipLaunchKernelGGL(ell_flag_kernel, dim3(blocks_for(T)), dim3(kT), 0, s, nrows, width, pitch,
-                         eci, flag);
-    MPH_CHECK_STATUS(exclusive_scan_i32(flag, pos, T, tmp, s));
-    MPH_CHECK_STATUS(t.read(pos + T, &tot));
-    if (tot > nnz) return invalid("ELL holds more entries than its nnz");
-    if (tot > 0)
-      MPH_LAUNCH_W(ell_emit_kernel, vs, dim3(blocks_for(T)), s, nrows, width, pitch, eci,
-                   ev, flag, pos, ri_out, ci_out,
-                   v_out);
-    MPH_HIP_CHECK(hipGetLastError());
-    MPH_HIP_CHECK(hipStreamSynchronize(s));
-  }
-  MPH_CHECK_STATUS(zero_tail(tot, nnz, ri_out, ci_out, v_out, vs, s));
-  return finish_coo(nnz, nrows, ncols_bound, ri_out, ci_out, v_out, vs, s);
+  return ell_part_to_coo(nrows, nnz, width, pitch, eci, ev, nullptr, 0, nullptr, nullptr, nullptr,
+                         false, "ELL holds more entries than its nnz", vt, ri_out, ci_out, v_out,
+                         s);
 }
 
 int mph_convert_coo_to_hyb_size(int64_t nrows, int64_t nnz, const int32_t* ri, int64_t* K,
@@ -1479,23 +1651,15 @@ int mph_convert_coo_to_hyb_size(int64_t nrows, int64_t nnz, const int32_t* ri, i
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   if (!K || !ell_nnz || !coo_nnz) return invalid("null size outputs");
   if (nrows <= 0) return invalid("HYB needs at least one row");
-  MPH_CHECK_STATUS(check_coo_in(nrows, INT32_MAX, nnz, ri, nullptr, s));
-  const int64_t k = std::max<int64_t>(1, nnz / nrows);
+  MPH_CHECK_STATUS(check_coo_args(nrows, INT32_MAX, nnz, ri, nullptr, false));
   Tmp t(s);
-  int32_t* cnt;
-  unsigned long long* acc;
-  MPH_CHECK_STATUS(row_counts(ri, nnz, nrows, t, &cnt, s));
-  MPH_CHECK_STATUS(t.alloc(&acc, 1));
-  MPH_CHECK_STATUS(fill_zero(acc, sizeof(unsigned long long), s));
-  hipLaunchKernelGGL(clipped_sum_kernel, dim3(reduce_blocks(nrows)), dim3(kT), 0, s, cnt, nrows,
-                     (int32_t)std::min<int64_t>(k, INT32_MAX), acc);
-  MPH_HIP_CHECK(hipGetLastError());
-  unsigned long long h = 0;
-  MPH_CHECK_STATUS(t.read(acc, &h));
-  *K = k;
-  *ell_nnz = (int64_t)h;
-  *coo_nnz = nnz - (int64_t)h;
-  if (mph_exceeds_tolerance(nrows, (int64_t)h, k)) {
+  RowScan R;
+  *K = std::max<int64_t>(1, nnz / nrows);
+  MPH_CHECK_STATUS(row_scan(nrows, nnz, ri, *K, t, R, s));
+  t.idle = true;
+  *ell_nnz = R.clipped;
+  *coo_nnz = nnz - R.clipped;
+  if (mph_exceeds_tolerance(nrows, R.clipped, *K)) {
     set_error("EllMatrix fill-in would exceed maximum tolerance");
     return MPH_ERR_FORMAT_CONVERSION;
   }
@@ -1508,41 +1672,53 @@ int mph_convert_coo_to_hyb(int64_t nrows, int64_t nnz, const int32_t* ri, const 
                            mph_stream_t stream) {
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   MPH_CHECK_STATUS(check_vt(vt));
-  int64_t k2, en, cn;
-  MPH_CHECK_STATUS(mph_convert_coo_to_hyb_size(nrows, nnz, ri, &k2, &en, &cn, stream));
-  if (k2 != K) return invalid("entries_per_row does not match the COO entries");
+  if (nrows <= 0) return invalid("HYB needs at least one row");
+  MPH_CHECK_STATUS(check_coo_args(nrows, INT32_MAX, nnz, ri, nullptr, false));
+  Tmp t(s);
+  RowScan R;
+  const int64_t k = std::max<int64_t>(1, nnz / nrows);
+  MPH_CHECK_STATUS(row_scan(nrows, nnz, ri, k, t, R, s));
+  if (mph_exceeds_tolerance(nrows, R.clipped, k)) {
+    set_error("EllMatrix fill-in would exceed maximum tolerance");
+    return MPH_ERR_FORMAT_CONVERSION;
+  }
+  if (k != K) return invalid("entries_per_row does not match the COO entries");
   if (width < K || pitch < nrows) return invalid("ELL width / pitch too small");
   const int vs = (int)value_size(vt);
-  MPH_CHECK_STATUS(fill_i32(eci, width * pitch, -1, s));
-  MPH_CHECK_STATUS(fill_zero(ev, (size_t)vs * width * pitch, s));
-  if (nnz == 0) return MPH_OK;
-  Tmp t(s);
-  Runs R;
-  int32_t *win, *over, *opos;
+  const int64_t cn = nnz - R.clipped;
+  if (!(R.flags & kRowsDown)) {
+    // row r's entries past the K-th follow those of the rows before it
+    MPH_CHECK_STATUS(ell_place(nrows, nnz, ri, ci, v, vs, K, width, pitch, R, eci, ev, nullptr, t, s));
+    if (cn == 0) return MPH_OK;
+    int32_t *cnt, *opos;
+    int64_t* tmp;
+    MPH_CHECK_STATUS(t.alloc(&cnt, nrows));
+    MPH_CHECK_STATUS(t.alloc(&opos, nrows + 1));
+    MPH_CHECK_STATUS(t.alloc(&tmp, scan_tmp_elems(nrows)));
+    hipLaunchKernelGGL(over_count_kernel, dim3(blocks_for(nrows)), dim3(kT), 0, s, R.ro, nrows,
+                       (int32_t)K, cnt);
+    MPH_CHECK_STATUS(exclusive_scan_i32(cnt, opos, nrows, tmp, s));
+    MPH_LAUNCH_W(over_place_kernel, vs, dim3(scan_blocks(nnz)), s, ri, ci, v, nnz, K, R.ro, opos, cri,
+                 cci, cv);
+    MPH_HIP_CHECK(hipGetLastError());
+    return MPH_OK;
+  }
+  int32_t *over, *opos;
   int64_t* tmp;
-  MPH_CHECK_STATUS(build_runs(ri, nnz, t, R, s));
-  MPH_CHECK_STATUS(t.alloc(&win, width * pitch));
   MPH_CHECK_STATUS(t.alloc(&over, nnz));
   MPH_CHECK_STATUS(t.alloc(&opos, nnz + 1));
   MPH_CHECK_STATUS(t.alloc(&tmp, scan_tmp_elems(nnz)));
-  MPH_CHECK_STATUS(fill_i32(win, width * pitch, -1, s));
   MPH_CHECK_STATUS(fill_i32(over, nnz, 0, s));
-  hipLaunchKernelGGL(ell_claim_kernel, dim3(blocks_for(nnz)), dim3(kT), 0, s, ri, nnz, K, pitch,
-                     R.head, R.hscan, R.runpos, win, over);
-  MPH_LAUNCH_W(ell_place_kernel, vs, dim3(blocks_for(nnz)), s, ri, ci,
-               v, nnz, K, pitch, R.head, R.hscan,
-               R.runpos, win, eci, ev);
+  MPH_CHECK_STATUS(ell_place(nrows, nnz, ri, ci, v, vs, K, width, pitch, R, eci, ev, over, t, s));
   MPH_CHECK_STATUS(exclusive_scan_i32(over, opos, nnz, tmp, s));
   int32_t tail = 0;
   MPH_CHECK_STATUS(t.read(opos + nnz, &tail));
   if (tail > cn) return invalid("COO entries are not grouped by row (HYB tail overflow)");
   if (tail < cn) MPH_CHECK_STATUS(zero_tail(tail, cn, cri, cci, cv, vs, s));
   if (tail > 0)
-    MPH_LAUNCH_W(tail_place_kernel, vs, dim3(blocks_for(nnz)), s, ri, ci,
-                 v, nnz, over, opos, cri, cci,
-                 cv);
+    MPH_LAUNCH_W(tail_place_kernel, vs, dim3(blocks_for(nnz)), s, ri, ci, v, nnz, over, opos, cri,
+                 cci, cv);
   MPH_HIP_CHECK(hipGetLastError());
-  MPH_HIP_CHECK(hipStreamSynchronize(s));
   return MPH_OK;
 }
 
@@ -1555,42 +1731,39 @@ int mph_convert_hyb_to_coo(int64_t nrows, int64_t nnz, int64_t width, int64_t pi
   MPH_CHECK_STATUS(check_vt(vt));
   if (nnz == 0) return MPH_OK;
   if (width > 0 && pitch < nrows) return invalid("pitch must be >= nrows");
-  MPH_CHECK_STATUS(check_index_range(cri, coo_nnz, nrows, false, s, "HYB COO row_indices"));
-  const int vs = (int)value_size(vt);
-  int32_t total = 0;
-  {
-    Tmp t(s);
-    int32_t *P, *tro, *cnt, *rowpos;
-    int64_t* tmp;
-    // the reference's forward walk consumes the longest row-sorted prefix
-    MPH_CHECK_STATUS(t.alloc(&P, 1));
-    MPH_CHECK_STATUS(fill_i32(P, 1, (int32_t)coo_nnz, s));
-    if (coo_nnz > 1)
-      hipLaunchKernelGGL(first_descent_kernel, dim3(blocks_for(coo_nnz)), dim3(kT), 0, s, cri,
-                         coo_nnz, P);
-    int32_t hP = 0;
-    MPH_CHECK_STATUS(t.read(P, &hP));
-    MPH_CHECK_STATUS(t.alloc(&tro, nrows + 1));
-    hipLaunchKernelGGL(sorted_offsets_kernel, dim3(blocks_for((int64_t)hP + 1)), dim3(kT), 0, s,
-                       cri, (int64_t)hP, nrows, tro);
-    MPH_CHECK_STATUS(t.alloc(&cnt, nrows));
-    MPH_CHECK_STATUS(t.alloc(&rowpos, nrows + 1));
-    MPH_CHECK_STATUS(t.alloc(&tmp, scan_tmp_elems(nrows)));
-    hipLaunchKernelGGL(hyb_rowcount_kernel, dim3(blocks_for(nrows)), dim3(kT), 0, s, nrows, width,
-                       pitch, eci, tro, cnt);
-    MPH_CHECK_STATUS(exclusive_scan_i32(cnt, rowpos, nrows, tmp, s));
-    MPH_CHECK_STATUS(t.read(rowpos + nrows, &total));
-    if (total > nnz) return invalid("HYB holds more entries than its nnz");
-    const int wpb = kT / kWave;
-    MPH_LAUNCH_W(hyb_emit_kernel, vs, dim3(blocks_for(nrows, wpb)), s, nrows, width, pitch, eci,
-                 ev, tro, cci,
-                 cv, rowpos, ri_out, ci_out,
-                 v_out);
+  Tmp t(s);
+  int32_t *tro, *flags, h = 0;
+  int64_t P = std::max<int64_t>(coo_nnz, 0);
+  MPH_CHECK_STATUS(t.alloc(&tro, std::max<int64_t>(nrows, 0) + 1));
+  if (P > 0) {
+    MPH_CHECK_STATUS(t.alloc(&flags, 1));
+    MPH_CHECK_STATUS(fill_zero(flags, sizeof(int32_t), s));
+    hipLaunchKernelGGL((coo_scan_kernel<true, true, false>), dim3(scan_blocks(P)), dim3(kT), 0, s,
+                       cri, cci, P, nrows, (int64_t)INT32_MAX, tro, (uint32_t*)nullptr, flags);
     MPH_HIP_CHECK(hipGetLastError());
-    MPH_HIP_CHECK(hipStreamSynchronize(s));
+    MPH_CHECK_STATUS(t.read(flags, &h));
+    if (h & kBadRow) return invalid("HYB COO row_indices: index out of range");
+    if (h & kRowsDown) {
+      // the reference's forward walk consumes the longest row-sorted prefix
+      int32_t *d, first = 0;
+      MPH_CHECK_STATUS(t.alloc(&d, 1));
+      MPH_CHECK_STATUS(fill_i32(d, 1, (int32_t)P, s));
+      hipLaunchKernelGGL(first_descent_kernel, dim3(blocks_for(P)), dim3(kT), 0, s, cri, P, d);
+      MPH_HIP_CHECK(hipGetLastError());
+      MPH_CHECK_STATUS(t.read(d, &first));
+      P = first;
+      MPH_CHECK_STATUS(fill_zero(flags, sizeof(int32_t), s));
+      hipLaunchKernelGGL((coo_scan_kernel<true, true, false>), dim3(scan_blocks(P)), dim3(kT), 0, s,
+                         cri, cci, P, nrows, (int64_t)INT32_MAX, tro, (uint32_t*)nullptr, flags);
+      MPH_HIP_CHECK(hipGetLastError());
+      MPH_CHECK_STATUS(t.read(flags, &h));
+    }
+  } else {
+    MPH_CHECK_STATUS(fill_zero(tro, sizeof(int32_t) * (size_t)(std::max<int64_t>(nrows, 0) + 1), s));
   }
-  MPH_CHECK_STATUS(zero_tail(total, nnz, ri_out, ci_out, v_out, vs, s));
-  return finish_coo(nnz, nrows, INT32_MAX, ri_out, ci_out, v_out, vs, s);
+  return ell_part_to_coo(nrows, nnz, width, pitch, eci, ev, tro, P, cri, cci, cv,
+                         (h & kUnsorted) != 0, "HYB holds more entries than its nnz", vt, ri_out,
+                         ci_out, v_out, s);
 }
 
 int mph_convert_coo_to_hdc_size(int64_t nrows, int64_t ncols, int64_t nnz, const int32_t* ri,
