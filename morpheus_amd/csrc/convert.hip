@@ -206,16 +206,37 @@ __device__ __forceinline__ void raise_flags(int32_t* __restrict__ flags, int32_t
 
 // Marks the bits of keys in a bitmap (lanes with `need` set; every lane of
 // the wave calls it).  A workgroup gathers its keys in an LDS table (linear
-// probing, kSeenProbe steps), equal keys of a wave entered once; keys that
-// find no slot mark their bit at once.  mark_bits_flush then sets the
+// probing, kSeenProbe steps), equal keys of a wave entered once for its first
+// kMatchRounds distinct ones; keys that find no slot mark their bit at once.  mark_bits_flush then sets the
 // table's bits that are not yet set: a stencil's few diagonals would
 // otherwise queue up on a few words (about 11 ns for each wave's atomic on
 // one address; 117 us for 14.6M entries when each wave read and set its bits
 // itself, 52 us so).
 constexpr int kSeen = 2 * kT;
 constexpr int kSeenProbe = 4;
+constexpr int kMatchRounds = 8;
 __device__ __forceinline__ uint32_t seen_slot(int32_t key) {
   return ((uint32_t)key * 2654435761u) >> 23;  // 9 bits
+}
+
+__device__ __forceinline__ void set_bit(uint32_t* __restrict__ bits, int32_t key) {
+  const uint32_t bit = 1u << (key & 31);
+  if (!(__hip_atomic_load(&bits[key >> 5], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & bit))
+    atomicOr(&bits[key >> 5], bit);
+}
+
+__device__ __forceinline__ void enter_key(uint32_t* __restrict__ bits, int32_t* seen, int32_t key) {
+  const uint32_t slot = seen_slot(key);
+  for (int p = 0; p < kSeenProbe; p++) {
+    const uint32_t q = (slot + p) & (kSeen - 1);
+    int32_t cur = seen[q];
+    if (cur == -1) {
+      const int32_t old = atomicCAS(&seen[q], -1, key);
+      cur = old == -1 ? key : old;
+    }
+    if (cur == key) return;
+  }
+  set_bit(bits, key);
 }
 
 __device__ __forceinline__ void mark_bits(uint32_t* __restrict__ bits, int32_t* seen, int32_t key,
@@ -225,86 +246,131 @@ __device__ __forceinline__ void mark_bits(uint32_t* __restrict__ bits, int32_t* 
 #pragma unroll
   for (int p = 0; p < kSeenProbe; p++) need = need && seen[(slot + p) & (kSeen - 1)] != key;
   uint64_t m = __ballot(need);
-  for (int round = 0; m && round < 12; round++) {
+  for (int round = 0; m && round < kMatchRounds; round++) {
     const int src = __ffsll((unsigned long long)m) - 1;
     const int32_t k = shfl(key, src);
-    if (lane == src) {
-      int p = 0;
-      for (; p < kSeenProbe; p++) {
-        const int32_t old = atomicCAS(&seen[(slot + p) & (kSeen - 1)], -1, k);
-        if (old == -1 || old == k) break;
-      }
-      if (p == kSeenProbe) atomicOr(&bits[k >> 5], 1u << (k & 31));
-    }
+    if (lane == src) enter_key(bits, seen, k);
     if (key == k) need = false;
     m = __ballot(need);
   }
-  if (need) atomicOr(&bits[key >> 5], 1u << (key & 31));
+  if (need) enter_key(bits, seen, key);
 }
 
 __device__ __forceinline__ void mark_bits_flush(uint32_t* __restrict__ bits, const int32_t* seen) {
   __syncthreads();
-  for (int q = threadIdx.x; q < kSeen; q += kT) {
-    const int32_t k = seen[q];
-    if (k < 0) continue;
-    const uint32_t bit = 1u << (k & 31);
-    if (!(__hip_atomic_load(&bits[k >> 5], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & bit))
-      atomicOr(&bits[k >> 5], bit);
-  }
+  for (int q = threadIdx.x; q < kSeen; q += kT)
+    if (seen[q] >= 0) set_bit(bits, seen[q]);
 }
 
-template <bool COLS, bool OFFSETS, bool DIAGS>
+// Adds keys to counters cnt, the same way: counts gather in the workgroup's
+// table and reach memory once; equal keys of a wave are added together for
+// the first kMatchRounds distinct ones, the other lanes add themselves.  Few
+// workgroups take many tiles each (kCountBlocks), since every workgroup's
+// atomic on a stencil's counters waits its turn.
+constexpr int64_t kCountBlocks = 1024;
+__device__ __forceinline__ void add_key(int32_t* __restrict__ cnt, int32_t* hk, int32_t* hc,
+                                        int32_t key, int32_t n) {
+  const uint32_t slot = seen_slot(key);
+  for (int p = 0; p < kSeenProbe; p++) {
+    const uint32_t q = (slot + p) & (kSeen - 1);
+    int32_t cur = hk[q];
+    if (cur == -1) {
+      const int32_t old = atomicCAS(&hk[q], -1, key);
+      cur = old == -1 ? key : old;
+    }
+    if (cur == key) {
+      atomicAdd(&hc[q], n);
+      return;
+    }
+  }
+  atomicAdd(&cnt[key], n);
+}
+
+__device__ __forceinline__ void count_keys(int32_t* __restrict__ cnt, int32_t* hk, int32_t* hc,
+                                           int32_t key, bool need) {
+  const int lane = threadIdx.x % kWave;
+  uint64_t m = __ballot(need);
+  for (int round = 0; m && round < kMatchRounds; round++) {
+    const int src = __ffsll((unsigned long long)m) - 1;
+    const int32_t k = shfl(key, src);
+    const uint64_t same = __ballot(need && key == k);
+    if (lane == src) add_key(cnt, hk, hc, k, __popcll(same));
+    if (key == k) need = false;
+    m &= ~same;
+  }
+  if (need) add_key(cnt, hk, hc, key, 1);
+}
+
+enum DiagMode { kNoDiags, kDiagBits, kDiagCounts };
+
+template <bool COLS, bool OFFSETS, DiagMode DIAGS>
 __global__ __launch_bounds__(kT) void coo_scan_kernel(
     const int32_t* __restrict__ ri, const int32_t* __restrict__ ci, int64_t nnz, int64_t nrows,
     int64_t ncols, int32_t* __restrict__ ro, uint32_t* __restrict__ diags,
     int32_t* __restrict__ flags) {
   __shared__ int32_t seen[kSeen];
-  if (DIAGS) {
-    for (int q = threadIdx.x; q < kSeen; q += kT) seen[q] = -1;
+  __shared__ int32_t seen_n[DIAGS == kDiagCounts ? kSeen : 1];
+  if (DIAGS != kNoDiags) {
+    for (int q = threadIdx.x; q < kSeen; q += kT) {
+      seen[q] = -1;
+      if (DIAGS == kDiagCounts) seen_n[q] = 0;
+    }
     __syncthreads();
   }
-  const int64_t base = (int64_t)blockIdx.x * kScanTile + threadIdx.x;
   const int lane = threadIdx.x % kWave;
-  int32_t r[kScanPer], c[kScanPer], bad = 0;
+  int32_t bad = 0;
   int64_t last = -2;  // the last entry's row, in the lane that holds it
+  for (int64_t tile = (int64_t)blockIdx.x * kScanTile; tile < nnz;
+       tile += (int64_t)gridDim.x * kScanTile) {
+    const int64_t base = tile + threadIdx.x;
+    int32_t r[kScanPer], c[kScanPer];
 #pragma unroll
-  for (int k = 0; k < kScanPer; k++) {
-    const int64_t i = base + (int64_t)k * kT;
-    r[k] = i < nnz ? ri[i] : 0;
-    c[k] = COLS && i < nnz ? ci[i] : 0;
-  }
-#pragma unroll
-  for (int k = 0; k < kScanPer; k++) {
-    const int64_t i = base + (int64_t)k * kT;
-    int32_t pr = shfl_up(r[k], 1), pc = COLS ? shfl_up(c[k], 1) : 0;
-    if (lane == 0 && i > 0 && i < nnz) {
-      pr = ri[i - 1];
-      if (COLS) pc = ci[i - 1];
+    for (int k = 0; k < kScanPer; k++) {
+      const int64_t i = base + (int64_t)k * kT;
+      r[k] = i < nnz ? ri[i] : 0;
+      c[k] = COLS && i < nnz ? ci[i] : 0;
     }
-    const bool in = i < nnz;
-    const bool row_ok = r[k] >= 0 && r[k] < nrows, col_ok = !COLS || (c[k] >= 0 && c[k] < ncols);
-    if (in) {
-      if (!row_ok) bad |= kBadRow;
-      if (!col_ok) bad |= kBadCol;
-      if (i > 0) {
-        if (pr > r[k]) bad |= kRowsDown | kUnsorted | kRepeated;
-        if (COLS && pr == r[k] && pc > c[k]) bad |= kUnsorted | kRepeated;
-        if (COLS && pr == r[k] && pc == c[k]) bad |= kRepeated;
+#pragma unroll
+    for (int k = 0; k < kScanPer; k++) {
+      const int64_t i = base + (int64_t)k * kT;
+      int32_t pr = shfl_up(r[k], 1), pc = COLS ? shfl_up(c[k], 1) : 0;
+      if (lane == 0 && i > 0 && i < nnz) {
+        pr = ri[i - 1];
+        if (COLS) pc = ci[i - 1];
       }
+      const bool in = i < nnz;
+      const bool row_ok = r[k] >= 0 && r[k] < nrows;
+      const bool col_ok = !COLS || (c[k] >= 0 && c[k] < ncols);
+      if (in) {
+        if (!row_ok) bad |= kBadRow;
+        if (!col_ok) bad |= kBadCol;
+        if (i > 0) {
+          if (pr > r[k]) bad |= kRowsDown | kUnsorted | kRepeated;
+          if (COLS && pr == r[k] && pc > c[k]) bad |= kUnsorted | kRepeated;
+          if (COLS && pr == r[k] && pc == c[k]) bad |= kRepeated;
+        }
+      }
+      if (OFFSETS) {
+        const int64_t hi = in && row_ok ? r[k] : 0;
+        const int64_t lo = in && row_ok ? (i == 0 ? -1 : min((int64_t)max(pr, -1), hi)) : 0;
+        fill_offsets(ro, lo, hi, (int32_t)i);
+        if (in && i == nnz - 1 && row_ok) last = r[k];
+      }
+      const int32_t key = (int32_t)((int64_t)c[k] - r[k] + nrows - 1);
+      if (DIAGS == kDiagBits) mark_bits(diags, seen, key, in && row_ok && col_ok);
+      if (DIAGS == kDiagCounts)
+        count_keys(reinterpret_cast<int32_t*>(diags), seen, seen_n, key, in && row_ok && col_ok);
     }
-    if (OFFSETS) {
-      const int64_t hi = in && row_ok ? r[k] : 0;
-      const int64_t lo = in && row_ok ? (i == 0 ? -1 : min((int64_t)max(pr, -1), hi)) : 0;
-      fill_offsets(ro, lo, hi, (int32_t)i);
-      if (in && i == nnz - 1 && row_ok) last = r[k];
-    }
-    if (DIAGS)
-      mark_bits(diags, seen, (int32_t)((int64_t)c[k] - r[k] + nrows - 1), in && row_ok && col_ok);
   }
-  if (OFFSETS && blockIdx.x == gridDim.x - 1)  // the rows after the last entry's
+  if (OFFSETS)  // the rows after the last entry's
     fill_offsets(ro, last >= -1 ? last : 0, last >= -1 ? nrows : 0, (int32_t)nnz);
   raise_flags(flags, bad);
-  if (DIAGS) mark_bits_flush(diags, seen);
+  if (DIAGS == kDiagBits) mark_bits_flush(diags, seen);
+  if (DIAGS == kDiagCounts) {
+    __syncthreads();
+    for (int q = threadIdx.x; q < kSeen; q += kT)
+      if (seen_n[q] > 0) atomicAdd(reinterpret_cast<int32_t*>(diags) + seen[q], seen_n[q]);
+  }
 }
 
 // rows of a CSR's entries, a workgroup per kScanTile of them: each row that
@@ -1069,6 +1135,93 @@ __global__ __launch_bounds__(kT) void dia_place_once_kernel(
   }
 }
 
+// HDC from entries in strictly ascending order: entries whose diagonal is
+// not among the offsets are counted per tile; then, with the tiles' positions
+// known, the values go to their diagonals and the others, in order, to the
+// CSR part's arrays.
+template <bool PLACE, typename W>
+__global__ __launch_bounds__(kT) void hdc_split_kernel(
+    const int32_t* __restrict__ ri, const int32_t* __restrict__ ci, const void* __restrict__ v_,
+    int64_t nnz, const int32_t* __restrict__ off, int64_t ndiag, int64_t pitch,
+    void* __restrict__ dv_, int32_t* __restrict__ tile_n, const int32_t* __restrict__ tile_pos,
+    int32_t* __restrict__ rri, int32_t* __restrict__ rci, void* __restrict__ rv_) {
+  __shared__ int32_t soff[kPlaceOffsets];
+  __shared__ int32_t wn[kScanPer][kT / kWave];
+  const W* v = static_cast<const W*>(v_);
+  const bool lds = ndiag <= kPlaceOffsets;
+  if (lds)
+    for (int q = threadIdx.x; q < ndiag; q += kT) soff[q] = off[q];
+  __syncthreads();
+  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+  const uint64_t lt = (lane == 0) ? 0ull : ((~0ull) >> (64 - lane));
+  const int64_t base = (int64_t)blockIdx.x * kScanTile + threadIdx.x;
+  int32_t r[kScanPer], c[kScanPer], rank[kScanPer];
+  W x[kScanPer];
+#pragma unroll
+  for (int k = 0; k < kScanPer; k++) {
+    const int64_t i = base + (int64_t)k * kT;
+    r[k] = c[k] = 0;
+    if (i < nnz) {
+      r[k] = ri[i];
+      c[k] = ci[i];
+      if (PLACE) x[k] = v[i];
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < kScanPer; k++) {
+    const bool in = base + (int64_t)k * kT < nnz;
+    const int64_t d = in ? find_first(lds ? soff : off, ndiag, c[k] - r[k]) : 0;
+    const uint64_t m = __ballot(in && d < 0);
+    rank[k] = in && d < 0 ? __popcll(m & lt) : -1;
+    if (lane == 0) wn[k][wave] = __popcll(m);
+    if (PLACE && in && d >= 0) static_cast<W*>(dv_)[r[k] + pitch * d] = x[k];
+  }
+  __syncthreads();
+  if (!PLACE) {
+    if (threadIdx.x == 0) {
+      int32_t n = 0;
+      for (int q = 0; q < kScanPer * (kT / kWave); q++) n += wn[q / (kT / kWave)][q % (kT / kWave)];
+      tile_n[blockIdx.x] = n;
+    }
+    return;
+  }
+  int32_t before = tile_pos[blockIdx.x];
+#pragma unroll
+  for (int k = 0; k < kScanPer; k++) {
+    for (int w = 0; w < kT / kWave; w++) {
+      if (w == wave && rank[k] >= 0) {
+        const int64_t o = before + rank[k];
+        rri[o] = r[k];
+        rci[o] = c[k];
+        static_cast<W*>(rv_)[o] = x[k];
+      }
+      before += wn[k][w];
+    }
+  }
+}
+
+// Two lists in (row, column) order merged: entry e of list A lands after the
+// B entries before it.  LATER: A's entries follow equal ones of B.
+template <bool LATER, typename W>
+__global__ __launch_bounds__(kT) void merge_rows_kernel(
+    const int32_t* __restrict__ ri, const int32_t* __restrict__ ci, const void* __restrict__ v_,
+    int64_t n, const int32_t* __restrict__ bro, const int32_t* __restrict__ bci,
+    int32_t* __restrict__ ri_out, int32_t* __restrict__ ci_out, void* __restrict__ vo_) {
+  const int64_t e = (int64_t)blockIdx.x * kT + threadIdx.x;
+  if (e >= n) return;
+  const int32_t r = ri[e], c = ci[e];
+  const W x = static_cast<const W*>(v_)[e];
+  int64_t lo = bro[r], hi = bro[r + 1];  // B entries of the row before (r, c)
+  while (lo < hi) {
+    const int64_t mid = (lo + hi) >> 1;
+    if (LATER ? bci[mid] <= c : bci[mid] < c) lo = mid + 1; else hi = mid;
+  }
+  const int64_t o = e + lo;
+  ri_out[o] = r;
+  ci_out[o] = c;
+  static_cast<W*>(vo_)[o] = x;
+}
+
 // The bitmap of used diagonals (bit col - row + nrows - 1) to ascending offsets.
 __global__ void bit_count_kernel(const uint32_t* __restrict__ bits, int64_t words,
                                  int32_t* __restrict__ cnt) {
@@ -1140,6 +1293,17 @@ __global__ __launch_bounds__(kT) void hdc_sizes_kernel(
       hipLaunchKernelGGL(kernel<uint32_t>, grid, dim3(kT), 0, s, __VA_ARGS__);      \
     else                                                                            \
       hipLaunchKernelGGL(kernel<uint16_t>, grid, dim3(kT), 0, s, __VA_ARGS__);      \
+  } while (0)
+
+// kernels of (bool, word)
+#define MPH_LAUNCH_BW(kernel, flag, vsize, grid, s, ...)                                \
+  do {                                                                                  \
+    if ((vsize) == 8)                                                                   \
+      hipLaunchKernelGGL((kernel<flag, uint64_t>), grid, dim3(kT), 0, s, __VA_ARGS__);  \
+    else if ((vsize) == 4)                                                              \
+      hipLaunchKernelGGL((kernel<flag, uint32_t>), grid, dim3(kT), 0, s, __VA_ARGS__);  \
+    else                                                                                \
+      hipLaunchKernelGGL((kernel<flag, uint16_t>), grid, dim3(kT), 0, s, __VA_ARGS__);  \
   } while (0)
 
 // (conversion moves values as raw words: 32-bit integer values too)
@@ -1223,7 +1387,7 @@ int dia_scan(int64_t nrows, int64_t ncols, int64_t nnz, const int32_t* ri, const
   MPH_CHECK_STATUS(t.alloc(&tmp, scan_tmp_elems(D.words)));
   MPH_CHECK_STATUS(fill_zero(D.bits, sizeof(uint32_t) * (size_t)(D.words + 1), s));
   flags = reinterpret_cast<int32_t*>(D.bits + D.words);
-  hipLaunchKernelGGL((coo_scan_kernel<true, false, true>), dim3(scan_blocks(nnz)), dim3(kT), 0, s,
+  hipLaunchKernelGGL((coo_scan_kernel<true, false, kDiagBits>), dim3(scan_blocks(nnz)), dim3(kT), 0, s,
                      ri, ci, nnz, nrows, ncols, (int32_t*)nullptr, D.bits, flags);
   hipLaunchKernelGGL(bit_count_kernel, dim3(blocks_for(D.words)), dim3(kT), 0, s, D.bits, D.words,
                      cnt);
@@ -1254,7 +1418,7 @@ int row_scan(int64_t nrows, int64_t nnz, const int32_t* ri, int64_t K, Tmp& t, R
   MPH_CHECK_STATUS(fill_zero(acc, 3 * sizeof(unsigned long long), s));
   int32_t* flags = reinterpret_cast<int32_t*>(acc + 2);
   if (nnz > 0)
-    hipLaunchKernelGGL((coo_scan_kernel<false, true, false>), dim3(scan_blocks(nnz)), dim3(kT), 0,
+    hipLaunchKernelGGL((coo_scan_kernel<false, true, kNoDiags>), dim3(scan_blocks(nnz)), dim3(kT), 0,
                        s, ri, (const int32_t*)nullptr, nnz, nrows, (int64_t)INT32_MAX, R.ro,
                        (uint32_t*)nullptr, flags);
   else
@@ -1285,6 +1449,41 @@ int row_scan(int64_t nrows, int64_t nnz, const int32_t* ri, int64_t K, Tmp& t, R
     R.longest = *hm;
     R.clipped = (int64_t)*h;
   }
+  return MPH_OK;
+}
+
+// HDC keeps the diagonals with at least a fifth of the rows' entries.
+int32_t hdc_threshold(int64_t nrows) { return (int32_t)((double)nrows * 0.2); }
+
+struct HdcScan {
+  int32_t* cnt = nullptr;  // entries per diagonal
+  int32_t flags = 0;
+  int64_t ndiag = 0, dia_nnz = 0, csr_nnz = 0;
+};
+
+int hdc_scan(int64_t nrows, int64_t ncols, int64_t nnz, const int32_t* ri, const int32_t* ci,
+             Tmp& t, HdcScan& H, hipStream_t s) {
+  const int64_t nb = nrows + ncols - 1;
+  unsigned long long *acc, *h;  // ndiag, dia_nnz, csr_nnz, flags
+  MPH_CHECK_STATUS(t.alloc(&H.cnt, nb));
+  MPH_CHECK_STATUS(t.alloc(&acc, 4));
+  MPH_CHECK_STATUS(fill_zero(H.cnt, sizeof(int32_t) * (size_t)nb, s));
+  MPH_CHECK_STATUS(fill_zero(acc, 4 * sizeof(unsigned long long), s));
+  if (nnz > 0)
+    hipLaunchKernelGGL((coo_scan_kernel<true, false, kDiagCounts>),
+                       dim3((unsigned)std::min<int64_t>(scan_blocks(nnz), kCountBlocks)), dim3(kT),
+                       0, s, ri, ci, nnz, nrows, ncols, (int32_t*)nullptr,
+                       reinterpret_cast<uint32_t*>(H.cnt), reinterpret_cast<int32_t*>(acc + 3));
+  hipLaunchKernelGGL(hdc_sizes_kernel, dim3(reduce_blocks(nb)), dim3(kT), 0, s, H.cnt, nb,
+                     hdc_threshold(nrows), acc);
+  MPH_HIP_CHECK(hipGetLastError());
+  MPH_CHECK_STATUS(t.fetch(acc, &h, 4));
+  MPH_CHECK_STATUS(t.wait());
+  H.flags = (int32_t)h[3];
+  MPH_CHECK_STATUS(scan_status(H.flags));
+  H.ndiag = (int64_t)h[0];
+  H.dia_nnz = (int64_t)h[1];
+  H.csr_nnz = (int64_t)h[2];
   return MPH_OK;
 }
 
@@ -1341,18 +1540,19 @@ int ell_place(int64_t nrows, int64_t nnz, const int32_t* ri, const int32_t* ci, 
 }
 
 // The entries of a DIA part in (row, column) order, shared by DIA -> COO and
-// HDC -> COO; returns their count.
+// HDC -> COO; returns their count (and each row's first entry in rowpos, if
+// given and the part is not empty).
 template <typename W>
 int emit_dia_part_w(int64_t nrows, int64_t ncols, int64_t ndiag, int64_t pitch,
                     const int32_t* off, const void* val, int vt, int64_t cap, int32_t* ri,
-                    int32_t* ci, void* v, int64_t* count, hipStream_t s) {
+                    int32_t* ci, void* v, int32_t* rowpos, int64_t* count, hipStream_t s) {
   *count = 0;
   if (nrows == 0 || ndiag == 0) return MPH_OK;
   Tmp t(s);
-  int32_t *cnt, *rowpos, *htot, *hoff;
+  int32_t *cnt, *htot, *hoff;
   int64_t* tmp;
   MPH_CHECK_STATUS(t.alloc(&cnt, nrows));
-  MPH_CHECK_STATUS(t.alloc(&rowpos, nrows + 1));
+  if (!rowpos) MPH_CHECK_STATUS(t.alloc(&rowpos, nrows + 1));
   MPH_CHECK_STATUS(t.alloc(&tmp, scan_tmp_elems(nrows)));
   DiaSlots<W> src{static_cast<const W*>(val), off, nullptr, pitch, ncols,
                   vt == MPH_I32 ? (W)~(W)0 : RawT<sizeof(W)>::mag};
@@ -1395,10 +1595,10 @@ int emit_dia_part_w(int64_t nrows, int64_t ncols, int64_t ndiag, int64_t pitch,
 
 int emit_dia_part(int64_t nrows, int64_t ncols, int64_t ndiag, int64_t pitch,
                   const int32_t* off, const void* val, int vt, int64_t cap, int32_t* ri,
-                  int32_t* ci, void* v, int64_t* count, hipStream_t s) {
+                  int32_t* ci, void* v, int32_t* rowpos, int64_t* count, hipStream_t s) {
   auto go = [&](auto tag) {
     return emit_dia_part_w<decltype(tag)>(nrows, ncols, ndiag, pitch, off, val, vt, cap, ri, ci, v,
-                                          count, s);
+                                          rowpos, count, s);
   };
   switch (value_size(vt)) {
     case 8: return go(uint64_t{});
@@ -1504,7 +1704,7 @@ int mph_convert_coo_to_csr(int64_t nrows, int64_t nnz, const int32_t* ri, const 
   int32_t h = 0;
   MPH_CHECK_STATUS(t.alloc(&flags, 1));
   MPH_CHECK_STATUS(fill_zero(flags, sizeof(int32_t), s));
-  hipLaunchKernelGGL((coo_scan_kernel<false, true, false>), dim3(scan_blocks(nnz)), dim3(kT), 0, s,
+  hipLaunchKernelGGL((coo_scan_kernel<false, true, kNoDiags>), dim3(scan_blocks(nnz)), dim3(kT), 0, s,
                      ri, ci, nnz, nrows, (int64_t)INT32_MAX, ro_out, (uint32_t*)nullptr, flags);
   MPH_HIP_CHECK(hipGetLastError());
   MPH_CHECK_STATUS(t.read(flags, &h));
@@ -1591,7 +1791,7 @@ int mph_convert_dia_to_coo(int64_t nrows, int64_t ncols, int64_t nnz, int64_t nd
   const int vs = (int)value_size(vt);
   int64_t cnt = 0;
   MPH_CHECK_STATUS(emit_dia_part(nrows, ncols, ndiag, pitch, off, val, vt, nnz, ri_out, ci_out,
-                                 v_out, &cnt, s));
+                                 v_out, nullptr, &cnt, s));
   if (cnt == nnz) return MPH_OK;  // in order
   MPH_CHECK_STATUS(zero_tail(cnt, nnz, ri_out, ci_out, v_out, vs, s));
   return finish_coo(nnz, nrows, ncols, ri_out, ci_out, v_out, vs, s);
@@ -1738,7 +1938,7 @@ int mph_convert_hyb_to_coo(int64_t nrows, int64_t nnz, int64_t width, int64_t pi
   if (P > 0) {
     MPH_CHECK_STATUS(t.alloc(&flags, 1));
     MPH_CHECK_STATUS(fill_zero(flags, sizeof(int32_t), s));
-    hipLaunchKernelGGL((coo_scan_kernel<true, true, false>), dim3(scan_blocks(P)), dim3(kT), 0, s,
+    hipLaunchKernelGGL((coo_scan_kernel<true, true, kNoDiags>), dim3(scan_blocks(P)), dim3(kT), 0, s,
                        cri, cci, P, nrows, (int64_t)INT32_MAX, tro, (uint32_t*)nullptr, flags);
     MPH_HIP_CHECK(hipGetLastError());
     MPH_CHECK_STATUS(t.read(flags, &h));
@@ -1753,7 +1953,7 @@ int mph_convert_hyb_to_coo(int64_t nrows, int64_t nnz, int64_t width, int64_t pi
       MPH_CHECK_STATUS(t.read(d, &first));
       P = first;
       MPH_CHECK_STATUS(fill_zero(flags, sizeof(int32_t), s));
-      hipLaunchKernelGGL((coo_scan_kernel<true, true, false>), dim3(scan_blocks(P)), dim3(kT), 0, s,
+      hipLaunchKernelGGL((coo_scan_kernel<true, true, kNoDiags>), dim3(scan_blocks(P)), dim3(kT), 0, s,
                          cri, cci, P, nrows, (int64_t)INT32_MAX, tro, (uint32_t*)nullptr, flags);
       MPH_HIP_CHECK(hipGetLastError());
       MPH_CHECK_STATUS(t.read(flags, &h));
@@ -1772,26 +1972,14 @@ int mph_convert_coo_to_hdc_size(int64_t nrows, int64_t ncols, int64_t nnz, const
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   if (!ndiag || !dia_nnz || !csr_nnz) return invalid("null size outputs");
   if (nrows <= 0 || ncols <= 0) return invalid("HDC needs a non-empty shape");
-  MPH_CHECK_STATUS(check_coo_in(nrows, ncols, nnz, ri, ci, s));
-  const int32_t thr = (int32_t)((double)nrows * 0.2);
-  const int64_t nb = nrows + ncols - 1;
+  MPH_CHECK_STATUS(check_coo_args(nrows, ncols, nnz, ri, ci, true));
   Tmp t(s);
-  int32_t* cnt;
-  unsigned long long* acc;
-  MPH_CHECK_STATUS(t.alloc(&cnt, nb));
-  MPH_CHECK_STATUS(t.alloc(&acc, 3));
-  MPH_CHECK_STATUS(fill_i32(cnt, nb, 0, s));
-  MPH_CHECK_STATUS(fill_zero(acc, 3 * sizeof(unsigned long long), s));
-  if (nnz > 0)
-    hipLaunchKernelGGL(diag_hist_kernel, dim3(hist_blocks(nnz)), dim3(kT), 0, s, ri, ci, nnz,
-                       nrows, cnt);
-  hipLaunchKernelGGL(hdc_sizes_kernel, dim3(reduce_blocks(nb)), dim3(kT), 0, s, cnt, nb, thr, acc);
-  MPH_HIP_CHECK(hipGetLastError());
-  unsigned long long h[3];
-  MPH_CHECK_STATUS(t.read(acc, h, 3));
-  *ndiag = (int64_t)h[0];
-  *dia_nnz = (int64_t)h[1];
-  *csr_nnz = (int64_t)h[2];
+  HdcScan H;
+  MPH_CHECK_STATUS(hdc_scan(nrows, ncols, nnz, ri, ci, t, H, s));
+  t.idle = true;
+  *ndiag = H.ndiag;
+  *dia_nnz = H.dia_nnz;
+  *csr_nnz = H.csr_nnz;
   if (mph_exceeds_tolerance(nrows, *dia_nnz, *ndiag)) {
     set_error("DiaMatrix fill-in would exceed maximum tolerance");
     return MPH_ERR_FORMAT_CONVERSION;
@@ -1805,31 +1993,33 @@ int mph_convert_coo_to_hdc(int64_t nrows, int64_t ncols, int64_t nnz, const int3
                            int32_t* csr_ci, void* csr_v, mph_stream_t stream) {
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   MPH_CHECK_STATUS(check_vt(vt));
-  int64_t nd, dn, cn;
-  MPH_CHECK_STATUS(mph_convert_coo_to_hdc_size(nrows, ncols, nnz, ri, ci, &nd, &dn, &cn, stream));
-  if (nd != ndiag) return invalid("ndiag does not match the COO entries");
-  if (ndiag > 0 && pitch < nrows) return invalid("pitch must be >= nrows");
-  const int vs = (int)value_size(vt);
-  const int32_t thr = (int32_t)((double)nrows * 0.2);
-  const int64_t nb = nrows + ncols - 1;
+  if (nrows <= 0 || ncols <= 0) return invalid("HDC needs a non-empty shape");
+  MPH_CHECK_STATUS(check_coo_args(nrows, ncols, nnz, ri, ci, true));
   Tmp t(s);
-  int32_t *cnt, *flag, *pos, *win, *rest, *rpos, *rows_rest, *rcnt;
+  HdcScan H;
+  MPH_CHECK_STATUS(hdc_scan(nrows, ncols, nnz, ri, ci, t, H, s));
+  if (mph_exceeds_tolerance(nrows, H.dia_nnz, H.ndiag)) {
+    set_error("DiaMatrix fill-in would exceed maximum tolerance");
+    return MPH_ERR_FORMAT_CONVERSION;
+  }
+  if (H.ndiag != ndiag) return invalid("ndiag does not match the COO entries");
+  if (ndiag > 0 && pitch < nrows) return invalid("pitch must be >= nrows");
+  const int64_t cn = H.csr_nnz, nb = nrows + ncols - 1;
+  const int vs = (int)value_size(vt);
+  const int32_t thr = hdc_threshold(nrows);
+  int32_t *flag, *pos;
   int64_t* tmp;
-  MPH_CHECK_STATUS(t.alloc(&cnt, nb));
-  MPH_CHECK_STATUS(t.alloc(&flag, nb));
-  MPH_CHECK_STATUS(t.alloc(&pos, nb + 1));
   MPH_CHECK_STATUS(t.alloc(&tmp, scan_tmp_elems(std::max(nb, std::max(nnz, nrows)))));
-  MPH_CHECK_STATUS(fill_i32(cnt, nb, 0, s));
-  if (nnz > 0)
-    hipLaunchKernelGGL(diag_hist_kernel, dim3(hist_blocks(nnz)), dim3(kT), 0, s, ri, ci, nnz,
-                       nrows, cnt);
-  hipLaunchKernelGGL(nonzero_flag_kernel, dim3(blocks_for(nb)), dim3(kT), 0, s, cnt, nb, thr,
-                     flag);
-  MPH_CHECK_STATUS(exclusive_scan_i32(flag, pos, nb, tmp, s));
-  if (ndiag > 0)
-    hipLaunchKernelGGL(compact_offsets_kernel, dim3(blocks_for(nb)), dim3(kT), 0, s, flag, pos,
-                       nb, nrows, off_out);
-  MPH_HIP_CHECK(hipGetLastError());
+  if (ndiag > 0) {
+    MPH_CHECK_STATUS(t.alloc(&flag, nb));
+    MPH_CHECK_STATUS(t.alloc(&pos, nb + 1));
+    hipLaunchKernelGGL(nonzero_flag_kernel, dim3(blocks_for(nb)), dim3(kT), 0, s, H.cnt, nb, thr,
+                       flag);
+    MPH_CHECK_STATUS(exclusive_scan_i32(flag, pos, nb, tmp, s));
+    hipLaunchKernelGGL(compact_offsets_kernel, dim3(blocks_for(nb)), dim3(kT), 0, s, flag, pos, nb,
+                       nrows, off_out);
+    MPH_HIP_CHECK(hipGetLastError());
+  }
   // core/src/impl/Hdc/Serial/Morpheus_Convert_Impl.hpp:169-195 records the
   // midpoint bin as offset 0 (its true offset only for square matrices) and
   // then sorts the offsets
@@ -1839,9 +2029,7 @@ int mph_convert_coo_to_hdc(int64_t nrows, int64_t ncols, int64_t nnz, const int3
     MPH_CHECK_STATUS(t.read(flag + mid, &sel));
     if (sel) {
       std::vector<int32_t> h(ndiag);
-      MPH_HIP_CHECK(hipMemcpyAsync(h.data(), off_out, sizeof(int32_t) * ndiag,
-                                   hipMemcpyDeviceToHost, s));
-      MPH_HIP_CHECK(hipStreamSynchronize(s));
+      MPH_CHECK_STATUS(t.read(off_out, h.data(), ndiag));
       const int32_t dmid = (int32_t)(mid - nrows + 1);
       for (auto& o : h)
         if (o == dmid) { o = 0; break; }
@@ -1852,35 +2040,52 @@ int mph_convert_coo_to_hdc(int64_t nrows, int64_t ncols, int64_t nnz, const int3
     }
   }
   // DIA part (later entry wins), the rest in input order to the CSR part
-  MPH_CHECK_STATUS(t.alloc(&win, std::max<int64_t>(pitch * ndiag, 1)));
-  MPH_CHECK_STATUS(t.alloc(&rest, nnz));
-  MPH_CHECK_STATUS(t.alloc(&rpos, nnz + 1));
-  MPH_CHECK_STATUS(fill_i32(win, pitch * ndiag, -1, s));
-  MPH_CHECK_STATUS(fill_i32(rest, nnz, 0, s));
-  MPH_CHECK_STATUS(fill_zero(dv, (size_t)vs * pitch * ndiag, s));
-  if (nnz > 0) {
-    hipLaunchKernelGGL(dia_claim_kernel, dim3(blocks_for(nnz)), dim3(kT), 0, s, ri, ci, nnz,
-                       off_out, ndiag, pitch, win, rest);
-    MPH_LAUNCH_W(dia_place_kernel, vs, dim3(blocks_for(nnz)), s, ri, ci,
-                 v, nnz, off_out, ndiag, pitch, win,
-                 dv);
-  }
-  MPH_CHECK_STATUS(exclusive_scan_i32(rest, rpos, nnz, tmp, s));
-  int32_t nrest = 0;
-  MPH_CHECK_STATUS(t.read(rpos + nnz, &nrest));
-  if (nrest > cn) return invalid("HDC CSR part overflow (non-square midpoint diagonal)");
-  // CSR part: per-row counts of the rest, exclusive scan, row_offsets[n] = cn
+  int32_t *rows_rest, nrest = 0;
   MPH_CHECK_STATUS(t.alloc(&rows_rest, std::max<int64_t>(cn, 1)));
-  MPH_CHECK_STATUS(t.alloc(&rcnt, nrows + 1));
-  MPH_CHECK_STATUS(fill_i32(rcnt, nrows + 1, 0, s));
-  if (nrest > 0) {
-    MPH_LAUNCH_W(tail_place_kernel, vs, dim3(blocks_for(nnz)), s, ri, ci,
-                 v, nnz, rest, rpos, rows_rest,
-                 csr_ci, csr_v);
-    hipLaunchKernelGGL(row_hist_kernel, dim3(hist_blocks(nrest)), dim3(kT), 0, s, rows_rest,
-                       (int64_t)nrest, rcnt);
+  if (nnz > 0 && !(H.flags & kRepeated)) {
+    const unsigned tiles = scan_blocks(nnz);
+    int32_t *tile_n, *tile_pos;
+    MPH_CHECK_STATUS(t.alloc(&tile_n, tiles));
+    MPH_CHECK_STATUS(t.alloc(&tile_pos, (int64_t)tiles + 1));
+    MPH_CHECK_STATUS(fill_zero(dv, (size_t)vs * pitch * ndiag, s));
+    hipLaunchKernelGGL((hdc_split_kernel<false, uint16_t>), dim3(tiles), dim3(kT), 0, s, ri, ci, v,
+                       nnz, off_out, ndiag, pitch, dv, tile_n, (const int32_t*)nullptr,
+                       (int32_t*)nullptr, (int32_t*)nullptr, (void*)nullptr);
+    MPH_CHECK_STATUS(exclusive_scan_i32(tile_n, tile_pos, tiles, tmp, s));
+    MPH_CHECK_STATUS(t.read(tile_pos + tiles, &nrest));
+    if (nrest > cn) return invalid("HDC CSR part overflow (non-square midpoint diagonal)");
+    MPH_LAUNCH_BW(hdc_split_kernel, true, vs, dim3(tiles), s, ri, ci, v, nnz, off_out, ndiag, pitch,
+                  dv, (int32_t*)nullptr, tile_pos, rows_rest, csr_ci, csr_v);
+  } else {
+    int32_t *rest, *rpos;
+    MPH_CHECK_STATUS(t.alloc(&rest, nnz));
+    MPH_CHECK_STATUS(t.alloc(&rpos, nnz + 1));
+    MPH_CHECK_STATUS(fill_i32(rest, nnz, 0, s));
+    MPH_CHECK_STATUS(
+        dia_place(nnz, ri, ci, v, vs, off_out, ndiag, pitch, H.flags, dv, rest, t, s));
+    MPH_CHECK_STATUS(exclusive_scan_i32(rest, rpos, nnz, tmp, s));
+    MPH_CHECK_STATUS(t.read(rpos + nnz, &nrest));
+    if (nrest > cn) return invalid("HDC CSR part overflow (non-square midpoint diagonal)");
+    if (nrest > 0)
+      MPH_LAUNCH_W(tail_place_kernel, vs, dim3(blocks_for(nnz)), s, ri, ci, v, nnz, rest, rpos,
+                   rows_rest, csr_ci, csr_v);
   }
-  MPH_CHECK_STATUS(exclusive_scan_i32(rcnt, csr_ro, nrows, tmp, s));
+  MPH_HIP_CHECK(hipGetLastError());
+  // CSR part: per-row counts of the rest, exclusive scan, row_offsets[n] = cn
+  if (nrest == 0) {
+    MPH_CHECK_STATUS(fill_zero(csr_ro, sizeof(int32_t) * (size_t)(nrows + 1), s));
+  } else if (!(H.flags & kRowsDown)) {
+    int32_t* flags;
+    MPH_CHECK_STATUS(t.alloc(&flags, 1));
+    MPH_CHECK_STATUS(fill_zero(flags, sizeof(int32_t), s));
+    hipLaunchKernelGGL((coo_scan_kernel<false, true, kNoDiags>), dim3(scan_blocks(nrest)), dim3(kT),
+                       0, s, rows_rest, (const int32_t*)nullptr, (int64_t)nrest, nrows,
+                       (int64_t)INT32_MAX, csr_ro, (uint32_t*)nullptr, flags);
+  } else {
+    int32_t* rcnt;
+    MPH_CHECK_STATUS(row_counts(rows_rest, nrest, nrows, t, &rcnt, s));
+    MPH_CHECK_STATUS(exclusive_scan_i32(rcnt, csr_ro, nrows, tmp, s));
+  }
   // the reference writes row_offsets[nrows] = csr_nnz (:225)
   hipLaunchKernelGGL(fill_i32_kernel, dim3(1), dim3(1), 0, s, csr_ro + nrows, (int64_t)1,
                      (int32_t)cn);
@@ -1890,7 +2095,6 @@ int mph_convert_coo_to_hdc(int64_t nrows, int64_t ncols, int64_t nnz, const int3
                                (size_t)vs * (cn - nrest), s));
   }
   MPH_HIP_CHECK(hipGetLastError());
-  MPH_HIP_CHECK(hipStreamSynchronize(s));
   return MPH_OK;
 }
 
@@ -1906,17 +2110,58 @@ int mph_convert_hdc_to_coo(int64_t nrows, int64_t ncols, int64_t nnz, int64_t nd
   MPH_CHECK_STATUS(check_row_offsets(csr_ro, nrows, csr_nnz, s, "HDC CSR row_offsets"));
   const int vs = (int)value_size(vt);
   int64_t nd = 0;
-  MPH_CHECK_STATUS(emit_dia_part(nrows, ncols, ndiag, pitch, doff, dval, vt, nnz, ri_out, ci_out,
-                                 v_out, &nd, s));
-  if (nd + csr_nnz > nnz) return invalid("HDC holds more entries than its nnz");
-  if (csr_nnz > 0) {
-    hipLaunchKernelGGL(expand_rows_kernel, dim3(scan_blocks(csr_nnz)), dim3(kT), 0, s, csr_ro,
-                       nrows, csr_nnz, nd, ri_out);
+  if (csr_nnz == 0) {
+    MPH_CHECK_STATUS(emit_dia_part(nrows, ncols, ndiag, pitch, doff, dval, vt, nnz, ri_out, ci_out,
+                                   v_out, nullptr, &nd, s));
+    if (nd == nnz) return MPH_OK;  // in order
+    MPH_CHECK_STATUS(zero_tail(nd, nnz, ri_out, ci_out, v_out, vs, s));
+    return finish_coo(nnz, nrows, ncols, ri_out, ci_out, v_out, vs, s);
+  }
+  // the CSR part's rows, and whether each row's columns ascend
+  Tmp t(s);
+  int32_t *crow, *rowpos, *flags, h = 0;
+  MPH_CHECK_STATUS(t.alloc(&crow, csr_nnz));
+  MPH_CHECK_STATUS(t.alloc(&flags, 1));
+  MPH_CHECK_STATUS(fill_zero(flags, sizeof(int32_t), s));
+  hipLaunchKernelGGL(expand_rows_kernel, dim3(scan_blocks(csr_nnz)), dim3(kT), 0, s, csr_ro, nrows,
+                     csr_nnz, (int64_t)0, crow);
+  hipLaunchKernelGGL((coo_scan_kernel<true, false, kNoDiags>), dim3(scan_blocks(csr_nnz)), dim3(kT),
+                     0, s, crow, csr_ci, csr_nnz, nrows, ncols, (int32_t*)nullptr,
+                     (uint32_t*)nullptr, flags);
+  MPH_HIP_CHECK(hipGetLastError());
+  MPH_CHECK_STATUS(t.read(flags, &h));
+  const bool sorted = !(h & kUnsorted);
+  if (sorted && ndiag > 0 && nrows > 0) {
+    // both parts in order: the DIA part's entries, then both lists merged (a
+    // DIA entry before the CSR entries of its row and column, as the stable
+    // sort of the DIA entries followed by the CSR entries leaves them)
+    int32_t *dri, *dci;
+    uint8_t* dv;
+    const int64_t cap = std::min(nnz, nrows * ndiag);
+    MPH_CHECK_STATUS(t.alloc(&rowpos, nrows + 1));
+    MPH_CHECK_STATUS(t.alloc(&dri, cap));
+    MPH_CHECK_STATUS(t.alloc(&dci, cap));
+    MPH_CHECK_STATUS(t.alloc(&dv, cap * vs));
+    MPH_CHECK_STATUS(emit_dia_part(nrows, ncols, ndiag, pitch, doff, dval, vt, cap, dri, dci, dv,
+                                   rowpos, &nd, s));
+    if (nd + csr_nnz > nnz) return invalid("HDC holds more entries than its nnz");
+    if (nd > 0)
+      MPH_LAUNCH_BW(merge_rows_kernel, false, vs, dim3(blocks_for(nd)), s, dri, dci, dv, nd, csr_ro,
+                    csr_ci, ri_out, ci_out, v_out);
+    MPH_LAUNCH_BW(merge_rows_kernel, true, vs, dim3(blocks_for(csr_nnz)), s, crow, csr_ci, csr_v,
+                  csr_nnz, rowpos, dci, ri_out, ci_out, v_out);
     MPH_HIP_CHECK(hipGetLastError());
+  } else {
+    // the DIA part's entries, then the CSR part's
+    MPH_CHECK_STATUS(emit_dia_part(nrows, ncols, ndiag, pitch, doff, dval, vt, nnz, ri_out, ci_out,
+                                   v_out, nullptr, &nd, s));
+    if (nd + csr_nnz > nnz) return invalid("HDC holds more entries than its nnz");
+    MPH_CHECK_STATUS(copy_dev(ri_out + nd, crow, sizeof(int32_t) * csr_nnz, s));
     MPH_CHECK_STATUS(copy_dev(ci_out + nd, csr_ci, sizeof(int32_t) * csr_nnz, s));
     MPH_CHECK_STATUS(copy_dev(static_cast<uint8_t*>(v_out) + (size_t)vs * nd, csr_v,
                               (size_t)vs * csr_nnz, s));
   }
+  if (nd + csr_nnz == nnz && sorted && (ndiag == 0 || nrows > 0)) return MPH_OK;
   MPH_CHECK_STATUS(zero_tail(nd + csr_nnz, nnz, ri_out, ci_out, v_out, vs, s));
   return finish_coo(nnz, nrows, ncols, ri_out, ci_out, v_out, vs, s);
 }
