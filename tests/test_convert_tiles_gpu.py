@@ -110,3 +110,48 @@ def test_dia_in_any_order(gpu, offsets, extra):
     nnz = int(np.count_nonzero(v * inside)) + extra
     A = Dia(n, n, nnz, off, v.reshape(-1), pitch)
     assert same_container(gpu_convert(A, COO_FORMAT), oracle.to_coo(A))
+
+
+@pytest.mark.parametrize("nnz", [2, 64, 511, 513, 4095, 4096, 4097, 9000])
+@pytest.mark.parametrize("nrows,ncols", [(1, 1), (2, 300), (257, 255), (70000, 3), (3, 1 << 24),
+                                         (1 << 22, 1 << 23)])
+@pytest.mark.parametrize("dtype", ["f64", "f32", "bf16"])
+def test_sort_tiles_and_key_widths(gpu, nnz, nrows, ncols, dtype):
+    """The COO sort around its tiles of 4096 and over 0 to 45 key bits; equal
+    keys keep their order."""
+    import ctypes as C
+    import torch
+    from morpheus_amd import capi, device
+    rng = np.random.default_rng(nnz + nrows)
+    r = rng.integers(0, nrows, nnz).astype(np.int32)
+    c = rng.integers(0, ncols, nnz).astype(np.int32)
+    v = (np.arange(nnz) % 251).astype(float)
+    ref = oracle.sort_by_row_and_column(Coo(nrows, ncols, r, c, v))
+    tr, tc = torch.from_numpy(r).cuda(), torch.from_numpy(c).cuda()
+    tv = torch.from_numpy(v).cuda().to(device.DTYPES[dtype][0])
+    p = lambda t: C.c_void_p(t.data_ptr())  # noqa: E731
+    capi.call("mph_coo_sort_by_row_and_column", nnz, p(tr), p(tc), p(tv),
+              capi.VALUE_TYPES[dtype], device.stream_handle())
+    assert np.array_equal(tr.cpu().numpy(), ref.row_indices)
+    assert np.array_equal(tc.cpu().numpy(), ref.column_indices)
+    assert np.array_equal(tv.double().cpu().numpy(), ref.values)
+
+
+@pytest.mark.parametrize("nnz", [3, 4096, 5000])
+def test_unsorted_coo_to_csr_in_place(gpu, nnz):
+    """ci_out / v_out may be the input's: rows not in order are sorted in place."""
+    import ctypes as C
+    import torch
+    from morpheus_amd import capi, device
+    rng = np.random.default_rng(nnz)
+    A = Coo(400, 700, rng.integers(0, 400, nnz), rng.integers(0, 700, nnz), 1.0 + np.arange(nnz))
+    ref = oracle.from_coo(A, CSR_FORMAT)
+    i32 = lambda a: torch.from_numpy(np.ascontiguousarray(a, dtype=np.int32)).cuda()  # noqa: E731
+    ri, ci, v = i32(A.row_indices), i32(A.column_indices), torch.from_numpy(A.values).cuda()
+    ro = torch.empty(401, dtype=torch.int32, device="cuda")
+    p = lambda t: C.c_void_p(t.data_ptr())  # noqa: E731
+    capi.call("mph_convert_coo_to_csr", 400, nnz, p(ri), p(ci), p(v), capi.F64, p(ro), p(ci),
+              p(v), device.stream_handle())
+    assert np.array_equal(ro.cpu().numpy(), ref.row_offsets)
+    assert np.array_equal(ci.cpu().numpy(), ref.column_indices)
+    assert np.array_equal(v.cpu().numpy(), ref.values)
