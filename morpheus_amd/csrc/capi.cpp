@@ -125,29 +125,51 @@ int device_cu_count() {
   return g_cu_count;
 }
 
+int plan_alloc(mph_matrix_impl* A, void** p, size_t bytes) {
+  *p = nullptr;
+  if (A->transient) {
+    TmpBlock b;
+    MPH_CHECK_STATUS(tmp_take(&b, bytes, false));
+    A->owned.push_back(b);
+    *p = b.p;
+    return MPH_OK;
+  }
+  MPH_HIP_CHECK(hipMalloc(p, bytes));
+  return MPH_OK;
+}
+
+void plan_free(mph_matrix_impl* A, void* p) {
+  for (const TmpBlock& b : A->owned)
+    if (b.p == p) return;  // given back with the plan
+  dfree(p);
+}
+
+// (a transient handle's stream has been synchronised by then: one_shot)
 void release_plans(mph_matrix_impl* A) {
   RowBlockPlan& p = A->rb;
-  dfree(p.blocks);
-  if (p.partial) dfree(p.partial);
-  if (p.tail_ro) dfree(p.tail_ro);
+  plan_free(A, p.blocks);
+  plan_free(A, p.partial);
+  plan_free(A, p.tail_ro);
   dfree(p.m_ro);
   dfree(p.m_ci);
   dfree(p.m_val);
-  if (p.sblocks) dfree(p.sblocks);
-  dfree(p.krec);
+  dfree(p.sblocks);
+  plan_free(A, p.krec);
   dfree(p.skrec);
-  if (p.smap) dfree(p.smap);
-  if (p.sro) dfree(p.sro);
+  dfree(p.smap);
+  dfree(p.sro);
   dfree(p.ell_cnt);
   xtile_release(p.xt);
   p = RowBlockPlan{};
   CooPlan& c = A->coo;
-  if (c.first_val) dfree(c.first_val);
-  if (c.last_val) dfree(c.last_val);
-  if (c.chunks) dfree(c.chunks);
+  dfree(c.first_val);
+  dfree(c.last_val);
+  dfree(c.chunks);
   xtile_release(c.xt);
   c = CooPlan{};
   A->dia_stage = DiaStage{};
+  for (const TmpBlock& b : A->owned) tmp_give(b);
+  A->owned.clear();
   A->analysed = false;
 }
 
@@ -195,8 +217,7 @@ int check_inputs(mph_matrix_t A, hipStream_t s) {
       return check_index_range(A->coo_ci, A->coo_nnz, m, false, s, "COO column_indices");
     case MPH_CSR:
     case MPH_HDC:
-      MPH_CHECK_STATUS(check_row_offsets(A->csr_ro, n, A->csr_nnz, s, "CSR row_offsets"));
-      return check_index_range(A->csr_ci, A->csr_nnz, m, false, s, "CSR column_indices");
+      return check_csr(A->csr_ro, n, A->csr_nnz, A->csr_ci, m, s);
     case MPH_ELL:
       return check_index_range(A->ell_ci, A->ell_width * A->ell_pitch, m, true, s,
                                "ELL column_indices");
@@ -658,8 +679,13 @@ int mph_multiply_multi(mph_matrix_t A, int32_t k, const void* X, void* Y,
   return multiply_impl(A, k, X, Y, init, reinterpret_cast<hipStream_t>(stream));
 }
 
+// A product that keeps nothing: the plan without the x-tiled pass (whose
+// tile-major copy of the long rows costs more than the one product gains),
+// its arrays temporaries.
 static int one_shot(mph_matrix_t A, const void* x, void* y, int init,
                     mph_stream_t stream) {
+  A->transient = true;
+  A->tuning.xtile = 1;
   int st = mph_multiply(A, x, y, init, stream);
   // the transient analysis is released after the product has run
   hipError_t e = hipStreamSynchronize(reinterpret_cast<hipStream_t>(stream));

@@ -10,6 +10,69 @@
 
 namespace mph {
 
+// Temporaries of one call, from blocks the library keeps per device.  The
+// runtime's stream-ordered pools mapped and unmapped memory at the
+// conversions' synchronisations whatever their release threshold: 25-60 us an
+// allocation and up to 1.1 ms a release, 3 ms of a 5.4 ms CSR -> HYB -> CSR
+// round trip of 16M entries.  A block goes back to the cache only after its
+// stream has been synchronised, so any thread and stream may take it next;
+// the cache holds at most kTmpKeepBytes in kTmpKeepBlocks blocks a device,
+// and mph_finalize, or an allocation that fails, gives them back.
+constexpr size_t kTmpKeepBytes = (size_t)2 << 30;
+constexpr size_t kTmpKeepBlocks = 48;
+struct TmpBlock {
+  void* p = nullptr;
+  size_t bytes = 0;
+  bool host = false;  // pinned host memory
+};
+int tmp_take(TmpBlock* b, size_t bytes, bool host);
+void tmp_give(const TmpBlock& b);
+void tmp_trim();
+
+struct Tmp {
+  hipStream_t s;
+  bool idle = false;  // the stream was synchronised after the last launch
+  std::vector<TmpBlock> blocks;
+  explicit Tmp(hipStream_t st) : s(st) {}
+  Tmp(const Tmp&) = delete;
+  Tmp& operator=(const Tmp&) = delete;
+  ~Tmp() {
+    if (!blocks.empty() && !idle) (void)hipStreamSynchronize(s);
+    for (const TmpBlock& b : blocks) tmp_give(b);
+  }
+  template <typename T>
+  int alloc(T** p, int64_t n, bool host = false) {
+    *p = nullptr;
+    TmpBlock b;
+    const int st = tmp_take(&b, sizeof(T) * (size_t)std::max<int64_t>(n, 1), host);
+    if (st != MPH_OK) return st;
+    blocks.push_back(b);
+    *p = static_cast<T*>(b.p);
+    return MPH_OK;
+  }
+  // enqueues the copy of n words of device memory to pinned memory, there to
+  // be read once the stream has been synchronised
+  template <typename T>
+  int fetch(const T* d, T** pin, int64_t n = 1) {
+    MPH_CHECK_STATUS(alloc(pin, n, true));
+    MPH_HIP_CHECK(hipMemcpyAsync(*pin, d, sizeof(T) * (size_t)n, hipMemcpyDeviceToHost, s));
+    return MPH_OK;
+  }
+  int wait() {
+    MPH_HIP_CHECK(hipStreamSynchronize(s));
+    return MPH_OK;
+  }
+  // n words of device memory to the host, and the stream synchronised
+  template <typename T>
+  int read(const T* d, T* h, int64_t n = 1) {
+    T* pin = nullptr;
+    MPH_CHECK_STATUS(fetch(d, &pin, n));
+    MPH_CHECK_STATUS(wait());
+    std::copy(pin, pin + n, h);
+    return MPH_OK;
+  }
+};
+
 // A row block of the CSR-family kernels.  sub < 0: rows [row, next.row) are
 // reduced from an LDS-staged slice of at most 2*chunk items.  sub >= 0: the
 // sub-th chunk of `chunk` items of the single long row `row`.
@@ -119,7 +182,8 @@ struct RowBlockPlan {
   int32_t* m_ro = nullptr;
   int32_t* m_ci = nullptr;
   void* m_val = nullptr;
-  int32_t nlong = 0;             // rows split into chunks
+  bool nlong = false;            // some rows are split into chunks
+  int32_t longest = 0;           // entries of the longest row
   // the short-block kernel's records, blocks / sblocks order, sentinel
   // included: {row, sub, first item, lanes per row of the block's reduction
   // (picked by the analysis; 0 for chunk and tiled records)}
@@ -220,6 +284,10 @@ struct mph_matrix_impl {
 
   mph_tuning tuning{0, 0, 0, 0};
   int32_t policy = 0;  // MPH_POLICY_* flags
+  // the handle of a one-shot product: its plan's arrays are temporaries
+  // (plan_alloc), given back after the stream has been synchronised
+  bool transient = false;
+  std::vector<TmpBlock> owned;
   bool analysed = false;
   RowBlockPlan rb;
   CooPlan coo;
@@ -244,6 +312,9 @@ int dia_multiply(mph_matrix_impl* A, int k, const void* x, void* y, int init,
 int ell_multiply(mph_matrix_impl* A, int k, const void* x, void* y, int init,
                  hipStream_t s);
 void release_plans(mph_matrix_impl* A);
+// an array of A's plan, and its release
+int plan_alloc(mph_matrix_impl* A, void** p, size_t bytes);
+void plan_free(mph_matrix_impl* A, void* p);
 int rows_sorted(const int32_t* ri, int64_t nnz, int64_t nrows, hipStream_t s,
                 int* sorted);
 int ell_padding_only(const int32_t* ci, int64_t pitch, int64_t nrows, int64_t K,
@@ -259,78 +330,14 @@ int fill_zero(void* p, size_t bytes, hipStream_t s);
 
 int device_cu_count();
 
-// Temporaries of one call, from blocks the library keeps per device.  The
-// runtime's stream-ordered pools mapped and unmapped memory at the
-// conversions' synchronisations whatever their release threshold: 25-60 us an
-// allocation and up to 1.1 ms a release, 3 ms of a 5.4 ms CSR -> HYB -> CSR
-// round trip of 16M entries.  A block goes back to the cache only after its
-// stream has been synchronised, so any thread and stream may take it next;
-// the cache holds at most kTmpKeepBytes in kTmpKeepBlocks blocks a device,
-// and mph_finalize, or an allocation that fails, gives them back.
-constexpr size_t kTmpKeepBytes = (size_t)2 << 30;
-constexpr size_t kTmpKeepBlocks = 48;
-struct TmpBlock {
-  void* p = nullptr;
-  size_t bytes = 0;
-  bool host = false;  // pinned host memory
-};
-int tmp_take(TmpBlock* b, size_t bytes, bool host);
-void tmp_give(const TmpBlock& b);
-void tmp_trim();
-
-struct Tmp {
-  hipStream_t s;
-  bool idle = false;  // the stream was synchronised after the last launch
-  std::vector<TmpBlock> blocks;
-  explicit Tmp(hipStream_t st) : s(st) {}
-  Tmp(const Tmp&) = delete;
-  Tmp& operator=(const Tmp&) = delete;
-  ~Tmp() {
-    if (!blocks.empty() && !idle) (void)hipStreamSynchronize(s);
-    for (const TmpBlock& b : blocks) tmp_give(b);
-  }
-  template <typename T>
-  int alloc(T** p, int64_t n, bool host = false) {
-    *p = nullptr;
-    TmpBlock b;
-    const int st = tmp_take(&b, sizeof(T) * (size_t)std::max<int64_t>(n, 1), host);
-    if (st != MPH_OK) return st;
-    blocks.push_back(b);
-    *p = static_cast<T*>(b.p);
-    return MPH_OK;
-  }
-  // enqueues the copy of n words of device memory to pinned memory, there to
-  // be read once the stream has been synchronised
-  template <typename T>
-  int fetch(const T* d, T** pin, int64_t n = 1) {
-    MPH_CHECK_STATUS(alloc(pin, n, true));
-    MPH_HIP_CHECK(hipMemcpyAsync(*pin, d, sizeof(T) * (size_t)n, hipMemcpyDeviceToHost, s));
-    return MPH_OK;
-  }
-  int wait() {
-    MPH_HIP_CHECK(hipStreamSynchronize(s));
-    return MPH_OK;
-  }
-  // n words of device memory to the host, and the stream synchronised
-  template <typename T>
-  int read(const T* d, T* h, int64_t n = 1) {
-    T* pin = nullptr;
-    MPH_CHECK_STATUS(fetch(d, &pin, n));
-    MPH_CHECK_STATUS(wait());
-    std::copy(pin, pin + n, h);
-    return MPH_OK;
-  }
-};
-
 // validate.hip
 int check_index_range(const int32_t* idx, int64_t n, int64_t hi, bool allow_m1,
                       hipStream_t s, const char* what);
 int check_row_offsets(const int32_t* ro, int64_t nrows, int64_t nnz,
                       hipStream_t s, const char* what);
-int validate_rowblock_plan(const int32_t* d_ro, int64_t nrows, RowBlockPlan& p,
-                           hipStream_t s, std::vector<int32_t>* krec = nullptr);
-// lanes per row for a short block of nr rows of lengths len(0..nr-1)
-uint8_t block_lanes(int nr, const int32_t* ro_begin);
+// row offsets and column indices of a CSR at once
+int check_csr(const int32_t* ro, int64_t nrows, int64_t nnz, const int32_t* ci, int64_t ncols,
+              hipStream_t s);
 
 // x-tiled long rows.  xtile_build plans the candidate rows `lrows` (host row
 // offsets `ro`, device row offsets / columns / values) when the x-tile mode

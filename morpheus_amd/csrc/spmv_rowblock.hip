@@ -1504,15 +1504,31 @@ __device__ __forceinline__ bool rb_is_start(const int32_t* ro, int64_t r,
          plen > long_len;
 }
 
-__global__ void rb_count_kernel(const int32_t* __restrict__ ro, int64_t nrows,
-                                int32_t chunk, int32_t long_len,
-                                int32_t* __restrict__ cnt) {
+// stats: [0] raised by rb_record_kernel when a record breaks the limits, [1]
+// set when some row is split into chunks, [2] entries of the longest row
+constexpr int kRbStats = 3;
+__global__ __launch_bounds__(256) void rb_count_kernel(const int32_t* __restrict__ ro,
+                                                       int64_t nrows, int32_t chunk,
+                                                       int32_t long_len, int32_t* __restrict__ cnt,
+                                                       int32_t* __restrict__ stats) {
+  __shared__ int32_t s_max;
+  if (threadIdx.x == 0) s_max = 0;
+  __syncthreads();
   const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= nrows) return;
-  bool lg;
-  int64_t len;
-  const bool st = rb_is_start(ro, r, chunk, long_len, lg, len);
-  cnt[r] = st ? (lg ? (int32_t)((len + chunk - 1) / chunk) : 1) : 0;
+  int32_t m = 0;
+  if (r < nrows) {
+    bool lg;
+    int64_t len;
+    const bool st = rb_is_start(ro, r, chunk, long_len, lg, len);
+    cnt[r] = st ? (lg ? (int32_t)((len + chunk - 1) / chunk) : 1) : 0;
+    m = (int32_t)len;
+  }
+  for (int d = kWave / 2; d > 0; d >>= 1) m = max(m, shfl_xor(m, d));
+  if (threadIdx.x % kWave == 0) atomicMax(&s_max, m);
+  __syncthreads();
+  if (threadIdx.x == 0 &&
+      __hip_atomic_load(&stats[2], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < s_max)
+    atomicMax(&stats[2], s_max);
 }
 
 __global__ void rb_fill_kernel(const int32_t* __restrict__ ro, int64_t nrows,
@@ -1529,6 +1545,107 @@ __global__ void rb_fill_kernel(const int32_t* __restrict__ ro, int64_t nrows,
   int64_t len;
   rb_is_start(ro, r, chunk, long_len, lg, len);
   for (int32_t q = 0; q < c; q++) blocks[f + q] = RowBlock{(int32_t)r, lg ? q : -1};
+}
+
+// The row-block kernels' records {row, sub, first item, lanes}, one wave per
+// block (the sentinel's included), written after checking the block against
+// the row offsets (check: rows, items and row lengths of short blocks, chunk
+// numbers of long rows).  A record that breaks a limit raises stats[0] and
+// nothing is read beyond the offsets.
+//
+// Lanes per row for the reduction of a short block (rows of lengths
+// ro[r + 1] - ro[r]): the power of two 1..64 with the least modelled time of
+// the block's slowest wave.  Groups of L lanes take rows g, g + 256 / L, ...;
+// each row iteration of a wave costs the longest trip count ceil(len / L)
+// among its groups' rows (an LDS read and an add per trip), 1.5 per shuffle
+// step (log2 L) and 3 of row overhead (offsets, store).  Regular short rows
+// get few lanes (7 entries per row: 1), blocks with a few long rows among
+// short ones more, so that one row does not hold a whole wave.  The rows of
+// one iteration of one wave are 64 / L consecutive rows, so the longest of
+// each such segment comes from the segments half its size; costs are kept
+// doubled, in whole numbers.  On the host, with a copy of the row offsets,
+// the records of a 1M-row power-law matrix took most of the 32 ms of its
+// one-shot product; here 22 us.
+__global__ __launch_bounds__(256) void rb_record_kernel(const RowBlock* __restrict__ blocks,
+                                                        int64_t nb, const int32_t* __restrict__ ro,
+                                                        int64_t nrows, int32_t chunk,
+                                                        int32_t long_len, int check,
+                                                        int32_t* __restrict__ krec,
+                                                        int32_t* __restrict__ stats) {
+  const int lane = threadIdx.x % kWave;
+  const int64_t b = (int64_t)blockIdx.x * (256 / kWave) + threadIdx.x / kWave;
+  if (b > nb) return;
+  const RowBlock k = blocks[b];
+  const bool end = b == nb;
+  bool bad = k.row < 0 || k.row > nrows || (k.row == nrows) != end || (end && k.sub != -1) ||
+             (check && b == 0 && !end && k.row != 0);
+  int lanes = 0;
+  constexpr int kQ = kRowBlockMaxRows / kWave;
+  if (!bad && !end && k.sub == -1) {
+    const int64_t r1 = blocks[b + 1].row;
+    const int nr = (int)(r1 - k.row);
+    bad = r1 <= k.row || r1 > nrows || nr > kRowBlockMaxRows;
+    if (!bad) {
+      bad = (int64_t)ro[r1] - ro[k.row] >= 2 * (int64_t)chunk;
+      int32_t v[kQ];  // longest row of the segment a lane is in, -1 if empty
+#pragma unroll
+      for (int q = 0; q < kQ; q++) {
+        const int i = q * kWave + lane;
+        v[q] = i < nr ? ro[k.row + i + 1] - ro[k.row + i] : -1;
+        bad = bad || v[q] > long_len;
+      }
+      int best = 0;
+#pragma unroll
+      for (int lev = 0; lev <= 6; lev++) {  // segments of 2^lev rows, L = 64 >> lev
+        const int lg = 6 - lev, L = kWave >> lev;
+        int32_t c01 = 0, c23 = 0;  // doubled costs of waves 0 | 1 << 16, 2 | 3 << 16
+#pragma unroll
+        for (int q = 0; q < kQ; q++) {
+          if (lev > 0) v[q] = max(v[q], shfl_xor(v[q], 1 << (lev > 0 ? lev - 1 : 0)));
+          if ((lane & ((1 << lev) - 1)) != 0 || v[q] < 0) continue;
+          const int32_t c = 2 * ((v[q] + L - 1) >> lg) + 3 * lg + 6;
+          const int w = ((q * kWave + lane) >> lev) & 3;
+          const int32_t at = (w & 1) ? c << 16 : c;
+          if (w < 2) c01 += at; else c23 += at;
+        }
+        for (int d = kWave / 2; d > 0; d >>= 1) {
+          c01 += shfl_xor(c01, d);
+          c23 += shfl_xor(c23, d);
+        }
+        const int worst = max(max(c01 & 0xffff, (int)((uint32_t)c01 >> 16)),
+                              max(c23 & 0xffff, (int)((uint32_t)c23 >> 16)));
+        // fewer lanes win a tie
+        if (lev == 0 || worst <= best) {
+          best = worst;
+          lanes = L;
+        }
+      }
+    }
+  } else if (!bad && !end && k.sub >= 0 && check) {
+    const int64_t len = (int64_t)ro[k.row + 1] - ro[k.row];
+    const int64_t nsub = (len + chunk - 1) / chunk;
+    bad = len <= long_len || k.sub >= nsub || b - k.sub < 0;
+    if (!bad) {
+      const RowBlock f = blocks[b - k.sub];
+      bad = f.row != k.row || f.sub != 0 || (k.sub == nsub - 1 && blocks[b + 1].row <= k.row);
+    }
+    if (k.sub == 0 && lane == 0) stats[1] = 1;
+  }
+  const bool any = __ballot(bad) != 0;
+  if (lane != 0) return;
+  if (any) atomicOr(&stats[0], 1);
+  krec[4 * b] = any ? 0 : k.row;
+  krec[4 * b + 1] = any ? -2 : k.sub;
+  krec[4 * b + 2] = any ? 0 : ro[k.row];
+  krec[4 * b + 3] = any ? 0 : lanes;
+}
+
+int rb_records(const RowBlock* blocks, int64_t nb, const int32_t* ro, int64_t nrows, int32_t chunk,
+               int32_t long_len, bool check, int32_t* krec, int32_t* stats, hipStream_t s) {
+  hipLaunchKernelGGL(rb_record_kernel, dim3((unsigned)ceil_div(nb + 1, 256 / kWave)), dim3(256), 0,
+                     s, blocks, nb, ro, nrows, chunk, long_len, check ? 1 : 0, krec, stats);
+  MPH_HIP_CHECK(hipGetLastError());
+  return MPH_OK;
 }
 
 // HYB: row offsets of a row-sorted COO tail.  Entry i is the first of its
@@ -1613,43 +1730,6 @@ __global__ void ell_tail_check_kernel(const int32_t* __restrict__ ci,
 }
 
 // --------------------------------------------------------------- host side
-// Lanes per row for the reduction of one short block (rows of lengths
-// ro[r + 1] - ro[r], r < nr): the power of two 1..64 with the least modelled
-// time of the block's slowest wave.  Groups of L lanes take rows g,
-// g + 256 / L, ...; each row iteration of a wave costs the longest trip
-// count ceil(len / L) among its groups' rows (an LDS read and an add per
-// trip), 1.5 per shuffle step (log2 L) and 3 of row overhead (offsets,
-// store).  Regular short rows get few lanes (S7, 7 per row: 1), blocks with
-// a few long rows among short ones more, so that one row does not hold a
-// whole wave.
-uint8_t block_lanes(int nr, const int32_t* ro) {
-  constexpr int kWaves = kRowBlockThreads / kWave;
-  int best_l = 1;
-  double best = 0;
-  for (int L = 1, lg = 0; L <= kWave; L <<= 1, lg++) {
-    const int groups = kRowBlockThreads / L, per_wave = kWave / L;
-    const int iters = (nr + groups - 1) / groups;
-    double worst = 0;
-    for (int w = 0; w < kWaves; w++) {
-      double c = 0;
-      for (int k = 0; k < iters; k++) {
-        int mx = -1;
-        for (int g = w * per_wave; g < (w + 1) * per_wave; g++) {
-          const int r = k * groups + g;
-          if (r < nr) mx = std::max(mx, (ro[r + 1] - ro[r] + L - 1) / L);
-        }
-        if (mx >= 0) c += mx + 1.5 * lg + 3;
-      }
-      worst = std::max(worst, c);
-    }
-    if (L == 1 || worst < best) {
-      best = worst;
-      best_l = L;
-    }
-  }
-  return (uint8_t)best_l;
-}
-
 int default_chunk(int vt) {
   return vt == MPH_F64 ? kDefaultChunkF64 : kDefaultChunkF32;
 }
@@ -2057,38 +2137,6 @@ namespace {
 // the kernel skips, a row longer than the chunk that the pass does not take
 // keeps its position chunks, and the other rows form short blocks with the
 // usual limits; the records are checked before upload.
-// the longest row of offsets ro (a workgroup maximum, then one atomic)
-__global__ __launch_bounds__(256) void max_row_len_kernel(const int32_t* __restrict__ ro,
-                                                          int64_t nrows, int32_t* __restrict__ out) {
-  __shared__ int32_t s_max;
-  if (threadIdx.x == 0) s_max = 0;
-  __syncthreads();
-  int32_t m = 0;
-  for (int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; r < nrows;
-       r += (int64_t)gridDim.x * blockDim.x)
-    m = max(m, ro[r + 1] - ro[r]);
-  atomicMax(&s_max, m);
-  __syncthreads();
-  if (threadIdx.x == 0) atomicMax(out, s_max);
-}
-
-int max_row_len(const int32_t* d_ro, int64_t nrows, hipStream_t s, int32_t* out) {
-  int32_t* d = nullptr;
-  MPH_HIP_CHECK(hipMalloc(&d, sizeof(int32_t)));
-  const int32_t zero = 0;
-  hipError_t e = hipMemcpyAsync(d, &zero, sizeof(int32_t), hipMemcpyHostToDevice, s);
-  if (e == hipSuccess) {
-    hipLaunchKernelGGL(max_row_len_kernel, dim3((unsigned)std::min<int64_t>(ceil_div(nrows, 256), 2048)),
-                       dim3(256), 0, s, d_ro, nrows, d);
-    e = hipGetLastError();
-  }
-  if (e == hipSuccess) e = hipMemcpyAsync(out, d, sizeof(int32_t), hipMemcpyDeviceToHost, s);
-  if (e == hipSuccess) e = hipStreamSynchronize(s);
-  (void)hipFree(d);
-  MPH_HIP_CHECK(e);
-  return MPH_OK;
-}
-
 // per row, 1 + its last ELL slot holding a column (0 without any)
 __global__ void ell_count_kernel(const int32_t* __restrict__ eci, int64_t pitch, int64_t loop,
                                  int64_t nrows, uint8_t* __restrict__ cnt) {
@@ -2146,13 +2194,9 @@ int split_analyse(mph_matrix_impl* A, const int32_t* d_ro, hipStream_t s) {
                         (A->format == MPH_HDC && A->ndiag > 0);
   const bool split = prefixed && (xt_on || nrows >= kSplitMinRows || p.prefix_apart);
   if ((!xt_on && !split) || nrows == 0 || A->ncols == 0) return MPH_OK;
-  if (xt_on && !split) {
-    // nothing to tile: the plain row-block plan stands (no host pass over
-    // the row offsets)
-    int32_t longest = 0;
-    MPH_CHECK_STATUS(max_row_len(d_ro, nrows, s, &longest));
-    if (longest <= kXTileMinRowLen) return MPH_OK;
-  }
+  // nothing to tile: the plain row-block plan stands (no host pass over the
+  // row offsets)
+  if (xt_on && !split && p.longest <= kXTileMinRowLen) return MPH_OK;
   const int32_t* d_ci = p.ci;
   const void* d_val = p.val;
 
@@ -2239,15 +2283,6 @@ int split_analyse(mph_matrix_impl* A, const int32_t* d_ro, hipStream_t s) {
       return MPH_ERR_RUNTIME;
     }
   }
-  std::vector<int32_t> kr(4 * sb.size());
-  for (size_t b = 0; b < sb.size(); b++) {
-    kr[4 * b] = sb[b].row;
-    kr[4 * b + 1] = sb[b].sub;
-    kr[4 * b + 2] = L[sb[b].row];
-    kr[4 * b + 3] = b + 1 < sb.size() && sb[b].sub == -1
-                        ? block_lanes(sb[b + 1].row - sb[b].row, L.data() + sb[b].row)
-                        : 0;
-  }
   RowBlock* d_sb = nullptr;
   int32_t* d_kr = nullptr;
   void* d_part = nullptr;
@@ -2256,7 +2291,7 @@ int split_analyse(mph_matrix_impl* A, const int32_t* d_ro, hipStream_t s) {
   const int accs = (A->vt == MPH_F64 ? 8 : 4);
   const bool grow = (int64_t)sb.size() > (int64_t)p.nblocks + 1;
   bool fail = hipMalloc(&d_sb, sizeof(RowBlock) * sb.size()) != hipSuccess ||
-              hipMalloc(&d_kr, sizeof(int32_t) * kr.size()) != hipSuccess ||
+              hipMalloc(&d_kr, sizeof(int32_t) * 4 * sb.size()) != hipSuccess ||
               (grow && hipMalloc(&d_part, (size_t)accs * 32 * sb.size()) != hipSuccess);
   if (!fail && split)
     fail = hipMalloc(&d_map, sizeof(int32_t) * (size_t)std::max<int64_t>(m, 1)) != hipSuccess ||
@@ -2272,15 +2307,23 @@ int split_analyse(mph_matrix_impl* A, const int32_t* d_ro, hipStream_t s) {
     return MPH_ERR_OUT_OF_MEMORY;
   }
   fail = hipMemcpyAsync(d_sb, sb.data(), sizeof(RowBlock) * sb.size(), hipMemcpyHostToDevice, s) !=
-             hipSuccess ||
-         hipMemcpyAsync(d_kr, kr.data(), sizeof(int32_t) * kr.size(), hipMemcpyHostToDevice, s) !=
-             hipSuccess;
+         hipSuccess;
   if (!fail && split && m > 0)
     fail = hipMemcpyAsync(d_map, map.data(), sizeof(int32_t) * m, hipMemcpyHostToDevice, s) !=
            hipSuccess;
   if (!fail && split)
     fail = hipMemcpyAsync(d_lro, lro.data(), sizeof(int32_t) * (m + 1), hipMemcpyHostToDevice, s) !=
            hipSuccess;
+  int32_t broken = 0;
+  if (!fail) {
+    Tmp t(s);
+    int32_t* stats = nullptr;
+    fail = t.alloc(&stats, kRbStats) != MPH_OK ||
+           fill_zero(stats, kRbStats * sizeof(int32_t), s) != MPH_OK ||
+           rb_records(d_sb, (int64_t)sb.size() - 1, split ? d_lro : d_ro, m, p.chunk, p.long_len,
+                      false, d_kr, stats, s) != MPH_OK ||
+           t.read(stats, &broken) != MPH_OK || broken != 0;
+  }
   if (fail || hipStreamSynchronize(s) != hipSuccess) {
     dfree(d_sb);
     dfree(d_kr);
@@ -2288,12 +2331,13 @@ int split_analyse(mph_matrix_impl* A, const int32_t* d_ro, hipStream_t s) {
     dfree(d_map);
     dfree(d_lro);
     xtile_release(p.xt);
-    set_error("split SpMV analysis: upload failed");
+    set_error(broken ? "split SpMV analysis check failed: records"
+                     : "split SpMV analysis: upload failed");
     return MPH_ERR_HIP;
   }
   if (grow) {
     // the chunk partials are indexed by the record position in either list
-    dfree(p.partial);
+    plan_free(A, p.partial);
     p.partial = d_part;
   }
   p.sblocks = d_sb;
@@ -2438,7 +2482,8 @@ int rowblock_analyse(mph_matrix_impl* A, hipStream_t s) {
       MPH_CHECK_STATUS(rows_sorted(A->coo_ri, A->coo_nnz, nrows, s, &sorted));
       if (!sorted) return MPH_ERR_NOT_IMPLEMENTED;  // caller falls back
     }
-    MPH_HIP_CHECK(hipMalloc(&p.tail_ro, sizeof(int32_t) * (nrows + 1)));
+    MPH_CHECK_STATUS(plan_alloc(A, reinterpret_cast<void**>(&p.tail_ro),
+                                sizeof(int32_t) * (size_t)(nrows + 1)));
     hipLaunchKernelGGL(tail_offsets_kernel,
                        dim3((unsigned)ceil_div(A->coo_nnz + 1, 256)), dim3(256),
                        0, s, A->coo_ri, A->coo_nnz, nrows, p.tail_ro);
@@ -2470,50 +2515,44 @@ int rowblock_analyse(mph_matrix_impl* A, hipStream_t s) {
     p.nblocks = 0;
     return MPH_OK;
   }
-  int32_t* cnt = nullptr;
-  int32_t* first = nullptr;
-  int64_t* tmp = nullptr;
-  MPH_HIP_CHECK(hipMalloc(&cnt, sizeof(int32_t) * nrows));
-  MPH_HIP_CHECK(hipMalloc(&first, sizeof(int32_t) * (nrows + 1)));
-  MPH_HIP_CHECK(hipMalloc(&tmp, sizeof(int64_t) * scan_tmp_elems(nrows)));
-  const unsigned g = (unsigned)ceil_div(nrows, 256);
-  hipLaunchKernelGGL(rb_count_kernel, dim3(g), dim3(256), 0, s, ro, nrows,
-                     p.chunk, p.long_len, cnt);
-  MPH_HIP_CHECK(hipGetLastError());
-  int st = exclusive_scan_i32(cnt, first, nrows, tmp, s);
-  int32_t nb = 0;
-  if (st == MPH_OK) {
-    MPH_HIP_CHECK(hipMemcpyAsync(&nb, first + nrows, sizeof(int32_t),
-                                 hipMemcpyDeviceToHost, s));
-    MPH_HIP_CHECK(hipStreamSynchronize(s));
-    p.nblocks = nb;
-    const int accs = (A->vt == MPH_F64 ? 8 : 4);
+  {
+    Tmp t(s);
+    int32_t *cnt, *first, *stats, *hb, *hs;
+    int64_t* tmp;
+    MPH_CHECK_STATUS(t.alloc(&cnt, nrows));
+    MPH_CHECK_STATUS(t.alloc(&first, nrows + 1));
+    MPH_CHECK_STATUS(t.alloc(&tmp, scan_tmp_elems(nrows)));
+    MPH_CHECK_STATUS(t.alloc(&stats, kRbStats));
+    MPH_CHECK_STATUS(fill_zero(stats, kRbStats * sizeof(int32_t), s));
+    const unsigned g = (unsigned)ceil_div(nrows, 256);
+    hipLaunchKernelGGL(rb_count_kernel, dim3(g), dim3(256), 0, s, ro, nrows, p.chunk, p.long_len,
+                       cnt, stats);
+    MPH_HIP_CHECK(hipGetLastError());
+    MPH_CHECK_STATUS(exclusive_scan_i32(cnt, first, nrows, tmp, s));
+    MPH_CHECK_STATUS(t.fetch(first + nrows, &hb));
+    MPH_CHECK_STATUS(t.wait());
+    const int64_t nb = *hb;
+    if (nb < 1) return runtime_error("row-block analysis check failed: no blocks");
+    const size_t accs = A->vt == MPH_F64 ? 8 : 4;
     // partials: up to 16 RHS per block (SpMM), as Dot2 pairs in FP32 / BF16
-    MPH_HIP_CHECK(hipMalloc(&p.blocks, sizeof(RowBlock) * (nb + 1)));
-    MPH_HIP_CHECK(hipMalloc(&p.partial, (size_t)accs * 32 * (nb + 1)));
-    {
-      hipLaunchKernelGGL(rb_fill_kernel, dim3(g), dim3(256), 0, s, ro, nrows,
-                         p.chunk, p.long_len, first, p.blocks);
-      MPH_HIP_CHECK(hipGetLastError());
-      MPH_HIP_CHECK(hipStreamSynchronize(s));
-      std::vector<int32_t> krec;
-      st = validate_rowblock_plan(ro, nrows, p, s, &krec);
-      if (st == MPH_OK && nb > 0) {
-        if (hipMalloc(&p.krec, sizeof(int32_t) * krec.size()) != hipSuccess ||
-            hipMemcpyAsync(p.krec, krec.data(), sizeof(int32_t) * krec.size(),
-                           hipMemcpyHostToDevice, s) != hipSuccess ||
-            hipStreamSynchronize(s) != hipSuccess) {
-          set_error("row-block analysis: kernel record upload failed");
-          st = MPH_ERR_HIP;
-        }
-      }
-    }
+    MPH_CHECK_STATUS(plan_alloc(A, reinterpret_cast<void**>(&p.blocks),
+                                sizeof(RowBlock) * (size_t)(nb + 1)));
+    MPH_CHECK_STATUS(plan_alloc(A, &p.partial, accs * 32 * (size_t)(nb + 1)));
+    MPH_CHECK_STATUS(plan_alloc(A, reinterpret_cast<void**>(&p.krec),
+                                sizeof(int32_t) * 4 * (size_t)(nb + 1)));
+    hipLaunchKernelGGL(rb_fill_kernel, dim3(g), dim3(256), 0, s, ro, nrows, p.chunk, p.long_len,
+                       first, p.blocks);
+    MPH_HIP_CHECK(hipGetLastError());
+    MPH_CHECK_STATUS(rb_records(p.blocks, nb, ro, nrows, p.chunk, p.long_len, true, p.krec, stats, s));
+    MPH_CHECK_STATUS(t.fetch(stats, &hs, kRbStats));
+    MPH_CHECK_STATUS(t.wait());
+    t.idle = true;
+    if (hs[0]) return runtime_error("row-block analysis check failed: records");
+    p.nblocks = (int32_t)nb;
+    p.nlong = hs[1] != 0;
+    p.longest = hs[2];
   }
-  dfree(cnt);
-  dfree(first);
-  dfree(tmp);
-  if (st == MPH_OK) st = split_analyse(A, ro, s);
-  return st;
+  return split_analyse(A, ro, s);
 }
 
 namespace {
@@ -2617,7 +2656,7 @@ int launch_spmv(mph_matrix_impl* A, const void* x, void* y, int init,
   hipLaunchKernelGGL((rowblock_spmv_kernel<V, PRE, comp>),
                      dim3((unsigned)A->rb.nblocks), dim3(kRowBlockThreads), lds,
                      s, a);
-  if (A->rb.nlong > 0)
+  if (A->rb.nlong)
     hipLaunchKernelGGL((rowblock_combine_kernel<V, PRE, comp>),
                        dim3((unsigned)ceil_div(A->rb.nblocks, 256)), dim3(256), 0, s, a);
   MPH_HIP_CHECK(hipGetLastError());
@@ -2632,10 +2671,10 @@ int launch_spmm_k(mph_matrix_impl* A, const void* x, void* y, int ld, int init,
                      dim3((unsigned)A->rb.nblocks), dim3(kRowBlockThreads), 0, s,
                      a);
   if constexpr (!std::is_same<V, double>::value)
-    if (A->rb.nlong > 0)
+    if (A->rb.nlong)
       hipLaunchKernelGGL((rowblock_spmm_chunk_kernel<V, KR>), dim3((unsigned)A->rb.nblocks),
                          dim3(kRowBlockThreads), 0, s, a);
-  if (A->rb.nlong > 0)
+  if (A->rb.nlong)
     hipLaunchKernelGGL((rowblock_spmm_combine_kernel<V, PRE, KR>),
                        dim3((unsigned)ceil_div(A->rb.nblocks, 256)), dim3(256), 0, s, a);
   MPH_HIP_CHECK(hipGetLastError());
