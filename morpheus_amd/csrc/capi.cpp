@@ -168,6 +168,7 @@ void release_plans(mph_matrix_impl* A) {
   xtile_release(c.xt);
   c = CooPlan{};
   A->dia_stage = DiaStage{};
+  A->dia_reach = A->dia_runs = 0;
   for (const TmpBlock& b : A->owned) tmp_give(b);
   A->owned.clear();
   A->analysed = false;

@@ -276,6 +276,9 @@ struct mph_matrix_impl {
   const int32_t* dia_off = nullptr;
   const void* dia_v = nullptr;
   DiaStage dia_stage;  // from the analysis
+  // from the analysis: the largest distance of a diagonal, and the runs of
+  // diagonals whose offsets step by one (0: not known)
+  int64_t dia_reach = 0, dia_runs = 0;
   // ELL / HYB-ELL
   int64_t ell_K = 0, ell_width = 0, ell_pitch = 0, ell_nnz = 0;
   int64_t ell_loop = 0;  // slots visited per row (K, or width if needed)

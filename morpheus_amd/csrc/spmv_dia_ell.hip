@@ -43,7 +43,26 @@ struct DiaArgs {
   const int32_t* __restrict__ tro;
   const int32_t* __restrict__ tci;
   const V* __restrict__ tval;
+  // dia_spmm_runs_kernel: workgroups of a plane, and an XCD's share of them
+  // (0: rows in order), see dia_plane_block
+  int32_t plane, plane_xcd;
 };
+
+// The row block of a workgroup, -1 for none.  In order, each XCD walks one
+// contiguous range of rows, and an X row that the outermost diagonals reach
+// comes back a reach of rows later, when its L2 line is gone.  A grid's
+// outermost diagonals lie a plane of nodes away: each XCD then takes an
+// eighth of every plane, plane after plane, so that the rows its neighbours
+// read are still in its L2 (27-point 160^3, 16 FP64 columns: 2.47 GB fetched
+// -> 1.47).
+template <typename V>
+__device__ __forceinline__ int64_t dia_plane_block(const DiaArgs<V>& a, int64_t rows_per_block) {
+  if (a.plane == 0) return xcd_remap(blockIdx.x, gridDim.x);
+  const uint32_t i = blockIdx.x / kNumXcd;
+  const int64_t c = (int64_t)(blockIdx.x % kNumXcd) * a.plane_xcd + i % a.plane_xcd;
+  const int64_t b = (int64_t)(i / a.plane_xcd) * a.plane + c;
+  return c < a.plane && b * rows_per_block < a.nrows ? b : -1;
+}
 
 // t[u][q] += v[u][w] * x[c[u][w]][q] over a batch of 8 diagonals / slots,
 // skipping c < 0.  The x loads are unconditional (c < 0 reads x[0]) and the
@@ -381,14 +400,25 @@ __global__ __launch_bounds__(256) void dia_spmm_kernel(DiaArgs<V> a) {
 
 // DIA SpMM with R consecutive rows per lane group (R = 4): for each run of
 // diagonals whose offsets step by one (o, o + 1, ..., at most kDiaRunMax),
-// the group loads the R + m - 1 X pieces the run covers once and slides
-// over them, instead of one X piece per row and diagonal (the 27-point
-// stencil: 6 X loads for 4 rows x 3 diagonals instead of 12).  Each row
-// still sums its diagonals in storage order, as dia_spmm_kernel does, with
-// the same skips, so the two give identical results.  Loads are
-// unconditional (columns outside x read column 0, a row past the matrix its
-// last row) and the products selected; the workgroup loads the run's values
-// for its rows into LDS together, so no lane group leaves before the end.
+// the workgroup loads the X rows the run covers, and the run's values for its
+// rows, once and coalesced, and hands them over through LDS; each lane reads
+// its R + m - 1 X pieces from there and slides over them.  Each row still
+// sums its diagonals in storage order, as dia_spmm_kernel does, with the same
+// skips, so the two give identical results.  Loads are unconditional (columns
+// outside x read a column inside, a row past the matrix its last row);
+// products are selected only where a workgroup's columns leave x.
+//
+// What bounds it: the L1.  With every lane loading its own X pieces the L1
+// served each X row three times a run and stood still half of the time on
+// rows another lane had requested already (TCP_PENDING_STALL_CYCLES); the
+// fetched bytes, 2.5 or 1.5 GB depending on the order of the workgroups, made
+// no difference.  A workgroup's runs follow one another, so the next run is
+// requested before the current one is summed, and the offsets come 64 at a
+// time into a register, the runs cut from it with scalar code (read from
+// memory, a run's offsets were a chain of round trips).  27-point 160^3,
+// FP64: 16 columns 632 -> 537 us (3.6 TB/s of X, Y and values once each), 8
+// columns 412 -> 324 us; FP32, 16 columns 365 -> 293 us.  VGPRs hold four
+// waves to a SIMD; compiled for five it spills (927 us).
 constexpr int kDiaRunMax = 3;
 
 template <typename V, int KL, int R>
@@ -399,12 +429,16 @@ __global__ __launch_bounds__(256) void dia_spmm_runs_kernel(DiaArgs<V> a) {
   constexpr int Q = P::Q;
   constexpr int W = R + kDiaRunMax - 1;
   constexpr int kRows = 256 / KL * R;  // rows of the workgroup
-  // the run's values for the workgroup's rows, loaded by all its threads in
-  // one coalesced pass per diagonal (each lane then reads its R rows'
-  // values from here instead of R loads of its own)
-  __shared__ V s_val[kDiaRunMax][kRows];
-  const uint32_t b = xcd_remap(blockIdx.x, gridDim.x);
-  const int64_t wr0 = (int64_t)b * kRows;
+  constexpr int kXRows = kRows + kDiaRunMax - 1;
+  constexpr int kX = (kXRows * KL + 255) / 256;            // X pieces a thread loads
+  constexpr int kVals = (kDiaRunMax * kRows + 255) / 256;  // values a thread loads
+  // X rows in LDS, one row left free after every R, so that the lane groups
+  // of a read lie on different banks
+  __shared__ typename P::T s_x[(kXRows + (kXRows - 1) / R) * KL];
+  __shared__ V s_val[kDiaRunMax * kRows];
+  const int64_t wb = dia_plane_block(a, kRows);
+  if (wb < 0) return;  // the whole workgroup
+  const int64_t wr0 = wb * kRows;
   const int gl = threadIdx.x / KL;
   const int64_t row0 = wr0 + (int64_t)gl * R;
   const int l = threadIdx.x % KL;
@@ -414,40 +448,105 @@ __global__ __launch_bounds__(256) void dia_spmm_runs_kernel(DiaArgs<V> a) {
   for (int i = 0; i < R; i++)
 #pragma unroll
     for (int q = 0; q < Q; q++) t[i][q] = 0;
-  for (int d = 0; d < a.ndiag;) {
-    const int64_t o = a.off[d];
-    int m = 1;
-    while (m < kDiaRunMax && d + m < a.ndiag && (int64_t)a.off[d + m] == o + m) m++;
-    // the X rows first: the value stores below wait for every older load
+
+  // the runs: 64 offsets in a register, bit w of `step` set when offset w
+  // continues the one before it
+  const int lane = threadIdx.x % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const uint32_t x_lane = (uint32_t)((gl * a.ld + l * Q) * (int)sizeof(Vec));
+  int32_t offs = 0;
+  uint64_t step = 0;
+  int d = 0, d0 = -kWave;  // next diagonal, first offset held
+  int64_t o = 0;           // the run requested last: first offset, diagonals,
+  int m = 0;
+  bool inner = false;      // and all its columns inside x, all rows inside
+  typename P::T xn[kX];
+  V vn[kVals];
+  auto request = [&]() {
+    if (d - d0 >= kWave) {
+      d0 = d;
+      offs = a.off[min(d + lane, a.ndiag - 1)];
+      const int32_t prev = shfl_up(offs, 1);
+      step = __ballot(lane > 0 && d + lane < a.ndiag && (int64_t)prev + 1 == offs);
+    }
+    const int w = d - d0;
+    o = __builtin_amdgcn_readlane(offs, w);
+    m = 1;
+    while (m < kDiaRunMax && w + m < kWave && ((step >> (w + m)) & 1)) m++;
+    inner = wr0 + kRows <= a.nrows && wr0 + o >= 0 && wr0 + kXRows + o <= a.ncols;
+    if (inner) {
+      // uniform addresses, each lane at a fixed distance
+      const char* xb = reinterpret_cast<const char*>(a.x + (wr0 + o) * a.ld);
+      const int64_t xstep = (int64_t)(256 / KL) * a.ld * sizeof(Vec);
+#pragma unroll
+      for (int k = 0; k < kX; k++)
+        if (k + 1 < kX || gl + k * (256 / KL) < kXRows)
+          xn[k] = *reinterpret_cast<const typename P::T*>(xb + k * xstep + x_lane);
+#pragma unroll
+      for (int k = 0; k < kVals; k++) {
+        const int e = wave * kWave + 256 * k;  // uniform
+        const int j = min(e / kRows, m - 1);
+        vn[k] = ld_stream(a.val + (a.pitch * (d + j) + wr0 + e % kRows) + lane);
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < kX; k++) {
+        const int64_t col = min(max(wr0 + gl + k * (256 / KL) + o, (int64_t)0), a.ncols - 1);
+        xn[k] = *reinterpret_cast<const typename P::T*>(a.x + col * a.ld + l * Q);
+      }
+#pragma unroll
+      for (int k = 0; k < kVals; k++) {
+        const int e = threadIdx.x + 256 * k;
+        const int j = min(e / kRows, m - 1);
+        vn[k] = ld_stream(a.val + a.pitch * (d + j) + min(wr0 + e % kRows, last));
+      }
+    }
+    d += m;
+  };
+
+  if (a.ndiag > 0) request();
+  while (m > 0) {
+    __syncthreads();  // the run before is read
+#pragma unroll
+    for (int k = 0; k < kX; k++) {
+      const int r = gl + k * (256 / KL);
+      if (k + 1 < kX || r < kXRows) s_x[(r + r / R) * KL + l] = xn[k];
+    }
+#pragma unroll
+    for (int k = 0; k < kVals; k++) {
+      const int e = threadIdx.x + 256 * k;
+      if (kVals * 256 == kDiaRunMax * kRows || e < kDiaRunMax * kRows) s_val[e] = vn[k];
+    }
+    __syncthreads();
+    const int64_t co = o;
+    const int cm = m;
+    const bool cin = inner;
+    m = 0;
+    if (d < a.ndiag) request();
     typename P::T xw[W];
 #pragma unroll
-    for (int i = 0; i < W; i++) {
-      const int64_t col = row0 + o + i;
-      const bool in = i < R + m - 1 && col >= 0 && col < a.ncols;
-      xw[i] = *reinterpret_cast<const typename P::T*>(a.x + (in ? col : 0) * a.ld + l * Q);
-    }
-    __syncthreads();  // the previous run's values are read
-    for (int j = 0; j < m; j++)
-      for (int e = threadIdx.x; e < kRows; e += 256)
-        s_val[j][e] = ld_stream(a.val + a.pitch * (d + j) + min(wr0 + e, last));
-    __syncthreads();
+    for (int i = 0; i < W; i++) xw[i] = s_x[(gl * (R + 1) + i + i / R) * KL + l];
 #pragma unroll
     for (int j = 0; j < kDiaRunMax; j++) {
-      if (j < m) {
+      if (j < cm) {
 #pragma unroll
         for (int i = 0; i < R; i++) {
-          const int64_t col = row0 + i + o + j;
-          const bool ok = row0 + i < a.nrows && col >= 0 && col < a.ncols;
-          const Acc vw = vtraits<V>::widen(s_val[j][gl * R + i]);
+          const Acc vw = vtraits<V>::widen(s_val[j * kRows + gl * R + i]);
+          if (cin) {
 #pragma unroll
-          for (int q = 0; q < Q; q++) {
-            const Acc f = t[i][q] + vw * (Acc)xw[i + j][q];
-            t[i][q] = ok ? f : t[i][q];
+            for (int q = 0; q < Q; q++) t[i][q] += vw * (Acc)xw[i + j][q];
+          } else {
+            const int64_t col = row0 + i + co + j;
+            const bool ok = row0 + i < a.nrows && col >= 0 && col < a.ncols;
+#pragma unroll
+            for (int q = 0; q < Q; q++) {
+              const Acc f = t[i][q] + vw * (Acc)xw[i + j][q];
+              t[i][q] = ok ? f : t[i][q];
+            }
           }
         }
       }
     }
-    d += m;
   }
 #pragma unroll
   for (int i = 0; i < R; i++) {
@@ -796,19 +895,34 @@ int launch_spmm_lanes(mph_matrix_impl* A, const void* x, void* y, int ld, int in
     a.ld = ld;
     a.init = init;
     // the run form (4 rows per lane group) where it was measured faster: 4
-    // or more lanes per row (S27 FP64 k = 8 587 -> 423 us, k = 16 1108 ->
-    // 630 us; FP32 k = 16 415 -> 374 us; BF16 k = 16 383 -> 347 us); not with
-    // fewer lanes (FP64 k = 2 213 -> 255 us, k = 4 even; FP32 k = 4 124 ->
-    // 188 us, k = 8 209 -> 258 us; BF16 k = 8 209 -> 254 us);
-    // MPH_DIA_SPMM_RUNS=0 / 1 forces it off / on
+    // or more lanes per row (27-point 160^3 FP64 k = 8 593 -> 324 us, k = 16
+    // 1116 -> 537 us; FP32 k = 16 416 -> 293 us; BF16 k = 16 386 -> 283 us;
+    // 7-point 128^3 FP64 k = 8 even, k = 16 205 -> 182 us), and 2 lanes when
+    // the runs average two diagonals or more (27-point FP64 k = 4 314 ->
+    // 227 us, FP32 k = 8 212 -> 172 us, BF16 204 -> 170 us; the 7-point
+    // stencil's mostly single diagonals: FP64 k = 4 50 -> 72 us); one lane is
+    // even at best (27-point FP64 k = 2 207 -> 194 us, FP32 k = 4 125 ->
+    // 128 us; 7-point FP64 k = 2 31 -> 51 us); MPH_DIA_SPMM_RUNS=0 / 1 forces
+    // it off / on
     const char* env = std::getenv("MPH_DIA_SPMM_RUNS");
     const int mode = env ? std::atoi(env) : -1;
-    constexpr bool wide = KL >= 4;
+    const bool wide = KL >= 4 || (KL == 2 && A->dia_runs > 0 && A->ndiag >= 2 * A->dia_runs);
     const bool runs = A->ncols > 0 && (mode > 0 || (mode < 0 && wide));
     if (runs) {
       constexpr int R = 4;
-      const int64_t nbr = ceil_div(A->nrows, (int64_t)(256 / KL) * R);
-      hipLaunchKernelGGL((dia_spmm_runs_kernel<V, KL, R>), dim3((unsigned)nbr), dim3(256), 0, s, a);
+      // plane order where two reaches of X exceed half an XCD's L2 and a
+      // plane has workgroups to share out (27-point 160^3 FP64 k = 16 551 ->
+      // 537 us, k = 32 1000 -> 950 us, FP32 k = 16 even)
+      constexpr int64_t rows = 256 / KL * R;
+      const int64_t nbr = ceil_div(A->nrows, rows), plane = (A->dia_reach + rows / 2) / rows;
+      int64_t grid = nbr;
+      if (2 * A->dia_reach * ld * (int64_t)sizeof(*a.x) > (2 << 20) && plane >= 4 * kNumXcd &&
+          plane < nbr) {
+        a.plane = (int32_t)plane;
+        a.plane_xcd = (int32_t)ceil_div(plane, kNumXcd);
+        grid = kNumXcd * a.plane_xcd * ceil_div(nbr, plane);
+      }
+      hipLaunchKernelGGL((dia_spmm_runs_kernel<V, KL, R>), dim3((unsigned)grid), dim3(256), 0, s, a);
     } else {
       hipLaunchKernelGGL((dia_spmm_kernel<V, KL>), dim3((unsigned)nb), dim3(256), 0, s, a);
     }
@@ -966,15 +1080,22 @@ int dispatch(mph_matrix_impl* A, int k, const void* x, void* y, int init,
 // the plain kernel (n = 0).
 int dia_analyse(mph_matrix_impl* A, hipStream_t s) {
   A->dia_stage = DiaStage{};
+  A->dia_reach = A->dia_runs = 0;
   const int64_t nd = A->ndiag;
   if (nd < 2 || nd > kDiaStageMaxDiags || A->nrows == 0 || A->ncols == 0) return MPH_OK;
   int mode = 2;  // MPH_DIA_STAGE: 0 off, 1 the one-row kernels only, 2 also the row pairs
   if (const char* env = std::getenv("MPH_DIA_STAGE")) mode = std::atoi(env);
-  if (mode <= 0) return MPH_OK;
   std::vector<int32_t> off((size_t)nd);
   MPH_HIP_CHECK(hipMemcpyAsync(off.data(), A->dia_off, sizeof(int32_t) * nd,
                                hipMemcpyDeviceToHost, s));
   MPH_HIP_CHECK(hipStreamSynchronize(s));
+  // for the SpMM's run form: the farthest diagonal, and the runs
+  for (int64_t i = 0, len = 0; i < nd; i++) {
+    A->dia_reach = std::max<int64_t>(A->dia_reach, std::abs((int64_t)off[i]));
+    len = i > 0 && len < kDiaRunMax && (int64_t)off[i - 1] + 1 == off[i] ? len + 1 : 1;
+    A->dia_runs += len == 1 ? 1 : 0;
+  }
+  if (mode <= 0) return MPH_OK;
   DiaStage st{};
   int32_t used = 0;
   int64_t staged_diags = 0;

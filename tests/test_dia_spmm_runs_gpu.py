@@ -48,11 +48,16 @@ def _cases():
         "past the edge": _dia(2000, 2000, [-3000, -1999, -1, 0, 1, 1999, 2500], 3),
         "rectangular wide": _dia(1500, 4000, [0, 1, 2, 2000, 2001], 4),
         "rectangular tall": _dia(4000, 1500, [-3000, -2999, -1, 0, 1], 5),
+        # more offsets than a wave holds at once
+        "70 diagonals": _dia(2500, 2500, np.arange(-35, 35), 6),
+        # far diagonals: the plane order of the row blocks (k = 16, 32), the
+        # last plane ragged
+        "planes": _dia(66001, 66001, [-20003, -20002, -1, 0, 1, 20001, 20002, 20003], 7),
     }
 
 
 NAMES = ["S27", "5-point", "band 9", "unsorted, repeated", "past the edge",
-         "rectangular wide", "rectangular tall"]
+         "rectangular wide", "rectangular tall", "70 diagonals", "planes"]
 
 
 def _run(monkeypatch, D, dtype, X, Y0, init, runs):
