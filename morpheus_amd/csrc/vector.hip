@@ -15,8 +15,9 @@
 // The CG iteration has no reference counterpart: it is the consumer of the
 // SpMV path.  Each iteration is the matrix handle's product q = A p and three
 // launches that keep every scalar on the device: (p.q partials), (alpha =
-// r.r / p.q; x += alpha p; r -= alpha q; r.r partials) and (beta = r.r' / r.r;
-// p = r + beta p).  Every block sums the partials in the same fixed order, so
+// r.r / p.q; r -= alpha q; r.r partials) and (beta = r.r' / r.r; x += alpha p;
+// p = r + beta p), x moved while p is there: 10 vectors read or written an
+// iteration, with the dot.  Every block sums the partials in the same fixed order, so
 // the scalars are identical across blocks and runs; nothing synchronises
 // with the host and nothing is cleared with a memset, so the loop can be
 // captured in a hipGraph.
@@ -36,19 +37,55 @@ constexpr int kPerThread = 8;
 inline int64_t parts_for(int64_t n) {
   return std::max<int64_t>(1, std::min<int64_t>(kMaxParts, ceil_div(n, (int64_t)kT * kPerThread)));
 }
-inline int64_t chunk_for(int64_t n, int64_t parts) { return ceil_div(std::max<int64_t>(n, 1), parts); }
+// (multiples of 16 bytes, for the wide loads)
+inline int64_t chunk_for(int64_t n, int64_t parts) {
+  return pad_size(ceil_div(std::max<int64_t>(n, 1), parts), 4);
+}
 
-// fixed-order block sum: per-thread values into LDS, then a tree
+inline bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
+
+// 16 bytes of a vector
+template <typename Vec>
+struct Wide;
+template <>
+struct Wide<double> {
+  using T = double __attribute__((ext_vector_type(2)));
+  static constexpr int Q = 2;
+};
+template <>
+struct Wide<float> {
+  using T = float __attribute__((ext_vector_type(4)));
+  static constexpr int Q = 4;
+};
+constexpr int kBatch = 4;  // 16-byte pieces of each vector a thread has in flight
+
+// block sum in a fixed order: a tree over each wave, then the waves
 __device__ double block_sum(double v, double* s) {
-  s[threadIdx.x] = v;
+  for (int m = kWave / 2; m > 0; m >>= 1) v += shfl_xor(v, m);
+  __syncthreads();  // (s may hold the previous sum)
+  if (threadIdx.x % kWave == 0) s[threadIdx.x / kWave] = v;
   __syncthreads();
-  for (int m = kT / 2; m > 0; m >>= 1) {
-    if ((int)threadIdx.x < m) s[threadIdx.x] += s[threadIdx.x + m];
-    __syncthreads();
-  }
-  const double r = s[0];
-  __syncthreads();
+  double r = s[0];
+  for (int w = 1; w < kT / kWave; w++) r += s[w];
   return r;
+}
+
+// The elements [b0, b1) of a block, b0 a multiple of 4: with WIDE (arrays on
+// 16 bytes) batches of kBatch pieces per thread, load(i, u) for all of a
+// batch before use(i, u), then the elements left one by one with one(i).
+template <typename Vec, bool WIDE, typename Load, typename Use, typename One>
+__device__ __forceinline__ void for_chunk(int64_t b0, int64_t b1, Load load, Use use, One one) {
+  constexpr int Q = Wide<Vec>::Q;
+  int64_t i0 = b0;
+  if constexpr (WIDE) {
+    for (; i0 + (int64_t)kT * Q * kBatch <= b1; i0 += (int64_t)kT * Q * kBatch) {
+#pragma unroll
+      for (int u = 0; u < kBatch; u++) load(i0 + (int64_t)(u * kT + threadIdx.x) * Q, u);
+#pragma unroll
+      for (int u = 0; u < kBatch; u++) use(i0 + (int64_t)(u * kT + threadIdx.x) * Q, u);
+    }
+  }
+  for (int64_t i = i0 + threadIdx.x; i < b1; i += kT) one(i);
 }
 
 // sum of parts[0..np) in a fixed order (each thread a strided run, then the
@@ -60,21 +97,46 @@ __device__ double sum_parts(const double* __restrict__ parts, int64_t np, double
 }
 
 // block b: the contiguous chunk [b * chunk, (b + 1) * chunk)
-template <typename Vec>
-__global__ void dot_parts_kernel(const Vec* __restrict__ x, const Vec* __restrict__ y, int64_t n,
-                                 int64_t chunk, double* __restrict__ parts) {
-  __shared__ double s[kT];
+template <typename Vec, bool WIDE>
+__global__ __launch_bounds__(kT) void dot_parts_kernel(const Vec* __restrict__ x,
+                                                       const Vec* __restrict__ y, int64_t n,
+                                                       int64_t chunk, double* __restrict__ parts) {
+  using P = typename Wide<Vec>::T;
+  __shared__ double s[kT / kWave];
   const int64_t b0 = (int64_t)blockIdx.x * chunk, b1 = min(n, b0 + chunk);
   double t = 0;
-  for (int64_t i = b0 + threadIdx.x; i < b1; i += kT) t += (double)x[i] * (double)y[i];
+  P xv[kBatch], yv[kBatch];
+  for_chunk<Vec, WIDE>(
+      b0, b1,
+      [&](int64_t i, int u) {
+        xv[u] = *reinterpret_cast<const P*>(x + i);
+        yv[u] = *reinterpret_cast<const P*>(y + i);
+      },
+      [&](int64_t, int u) {
+#pragma unroll
+        for (int q = 0; q < Wide<Vec>::Q; q++) t += (double)xv[u][q] * (double)yv[u][q];
+      },
+      [&](int64_t i) { t += (double)x[i] * (double)y[i]; });
   t = block_sum(t, s);
   if (threadIdx.x == 0) parts[blockIdx.x] = t;
 }
 
 template <typename Vec>
+void launch_dot_parts(const void* x, const void* y, int64_t n, int64_t np, int64_t chunk,
+                      double* parts, hipStream_t s) {
+  const Vec *xv = static_cast<const Vec*>(x), *yv = static_cast<const Vec*>(y);
+  if (aligned16(x) && aligned16(y))
+    hipLaunchKernelGGL((dot_parts_kernel<Vec, true>), dim3((unsigned)np), dim3(kT), 0, s, xv, yv, n,
+                       chunk, parts);
+  else
+    hipLaunchKernelGGL((dot_parts_kernel<Vec, false>), dim3((unsigned)np), dim3(kT), 0, s, xv, yv,
+                       n, chunk, parts);
+}
+
+template <typename Vec>
 __global__ void reduce_parts_kernel(const Vec* __restrict__ x, int64_t n, int64_t chunk,
                                     double* __restrict__ parts) {
-  __shared__ double s[kT];
+  __shared__ double s[kT / kWave];
   const int64_t b0 = (int64_t)blockIdx.x * chunk, b1 = min(n, b0 + chunk);
   double t = 0, c = 0;
   for (int64_t i = b0 + threadIdx.x; i < b1; i += kT) {
@@ -90,7 +152,7 @@ __global__ void reduce_parts_kernel(const Vec* __restrict__ x, int64_t n, int64_
 
 __global__ void sum_parts_kernel(const double* __restrict__ parts, int64_t np,
                                  double* __restrict__ out) {
-  __shared__ double s[kT];
+  __shared__ double s[kT / kWave];
   const double t = sum_parts(parts, np, s);
   if (threadIdx.x == 0) *out = t;
 }
@@ -109,35 +171,82 @@ __global__ void waxpby_kernel(int64_t n, double alpha, const Vec* __restrict__ x
 }
 
 // ------------------------------------------------------------------ CG
+// The scalars of an iteration: rr of its start (kRr), alpha, rr of its end
+// (kNext, the next one's start) and a place for mph_cg_residual.  Each kernel
+// writes only those that none of its own blocks read.
+enum { kRr, kAlpha, kNext, kResidual, kCgState };
+
+// alpha = rr / p.q, r -= alpha q and the r.r partials.  x is moved with p, in
+// cg_direction_kernel: moved here it read p once more.  On a 128^3 grid, FP64,
+// the two took 18.0 and 14.9 us (100 and 50 MB), one element a load and, for
+// p, one a thread after the sum of the partials; now 9.0 and 14.3 us (50 and
+// 84 MB, 5.7 TB/s).
 template <typename Vec>
-__global__ void cg_update_kernel(Vec* __restrict__ x, Vec* __restrict__ r,
-                                 const Vec* __restrict__ p, const Vec* __restrict__ q, int64_t n,
-                                 int64_t chunk, const double* __restrict__ pq_parts, int64_t np,
-                                 const double* __restrict__ state, double* __restrict__ rr_parts) {
-  __shared__ double s[kT];
-  const double pq = sum_parts(pq_parts, np, s);
-  const Vec alpha = (Vec)(state[0] / pq);
+__global__ __launch_bounds__(kT) void cg_update_kernel(
+    Vec* __restrict__ r, const Vec* __restrict__ q, int64_t n, int64_t chunk,
+    const double* __restrict__ pq_parts, int64_t np, double* __restrict__ state,
+    double* __restrict__ rr_parts) {
+  using P = typename Wide<Vec>::T;
+  __shared__ double s[kT / kWave];
+  const double rr = state[kNext];
+  const double a = rr / sum_parts(pq_parts, np, s);
+  const Vec alpha = (Vec)a;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    state[kRr] = rr;
+    state[kAlpha] = a;
+  }
   const int64_t b0 = (int64_t)blockIdx.x * chunk, b1 = min(n, b0 + chunk);
   double t = 0;
-  for (int64_t i = b0 + threadIdx.x; i < b1; i += kT) {
-    x[i] += alpha * p[i];
-    const Vec ri = r[i] - alpha * q[i];
-    r[i] = ri;
-    t += (double)ri * (double)ri;
-  }
+  P rv[kBatch], qv[kBatch];
+  for_chunk<Vec, true>(
+      b0, b1,
+      [&](int64_t i, int u) {
+        rv[u] = *reinterpret_cast<const P*>(r + i);
+        qv[u] = *reinterpret_cast<const P*>(q + i);
+      },
+      [&](int64_t i, int u) {
+        rv[u] -= alpha * qv[u];
+        *reinterpret_cast<P*>(r + i) = rv[u];
+#pragma unroll
+        for (int k = 0; k < Wide<Vec>::Q; k++) t += (double)rv[u][k] * (double)rv[u][k];
+      },
+      [&](int64_t i) {
+        const Vec ri = r[i] - alpha * q[i];
+        r[i] = ri;
+        t += (double)ri * (double)ri;
+      });
   t = block_sum(t, s);
   if (threadIdx.x == 0) rr_parts[blockIdx.x] = t;
 }
 
-template <typename Vec>
-__global__ void cg_direction_kernel(Vec* __restrict__ p, const Vec* __restrict__ r, int64_t n,
-                                    const double* __restrict__ rr_parts, int64_t np,
-                                    const double* __restrict__ state) {
-  __shared__ double s[kT];
+// beta = r.r / rr, x += alpha p and p = r + beta p
+template <typename Vec, bool WIDE>
+__global__ __launch_bounds__(kT) void cg_direction_kernel(
+    Vec* __restrict__ x, Vec* __restrict__ p, const Vec* __restrict__ r, int64_t n, int64_t chunk,
+    const double* __restrict__ rr_parts, int64_t np, double* __restrict__ state) {
+  using P = typename Wide<Vec>::T;
+  __shared__ double s[kT / kWave];
   const double rr = sum_parts(rr_parts, np, s);
-  const Vec beta = (Vec)(rr / state[0]);
-  for (int64_t i = (int64_t)blockIdx.x * kT + threadIdx.x; i < n; i += (int64_t)gridDim.x * kT)
-    p[i] = r[i] + beta * p[i];
+  const Vec beta = (Vec)(rr / state[kRr]), alpha = (Vec)state[kAlpha];
+  if (blockIdx.x == 0 && threadIdx.x == 0) state[kNext] = rr;
+  const int64_t b0 = (int64_t)blockIdx.x * chunk, b1 = min(n, b0 + chunk);
+  P xv[kBatch], pv[kBatch], rv[kBatch];
+  for_chunk<Vec, WIDE>(
+      b0, b1,
+      [&](int64_t i, int u) {
+        pv[u] = *reinterpret_cast<const P*>(p + i);
+        xv[u] = *reinterpret_cast<const P*>(x + i);
+        rv[u] = *reinterpret_cast<const P*>(r + i);
+      },
+      [&](int64_t i, int u) {
+        *reinterpret_cast<P*>(x + i) = xv[u] + alpha * pv[u];
+        *reinterpret_cast<P*>(p + i) = rv[u] + beta * pv[u];
+      },
+      [&](int64_t i) {
+        const Vec pi = p[i];
+        x[i] += alpha * pi;
+        p[i] = r[i] + beta * pi;
+      });
 }
 
 // r = b - q and p = r, with the r.r partials
@@ -145,7 +254,7 @@ template <typename Vec>
 __global__ void cg_start_kernel(const Vec* __restrict__ b, const Vec* __restrict__ q,
                                 Vec* __restrict__ r, Vec* __restrict__ p, int64_t n, int64_t chunk,
                                 double* __restrict__ rr_parts) {
-  __shared__ double s[kT];
+  __shared__ double s[kT / kWave];
   const int64_t b0 = (int64_t)blockIdx.x * chunk, b1 = min(n, b0 + chunk);
   double t = 0;
   for (int64_t i = b0 + threadIdx.x; i < b1; i += kT) {
@@ -163,8 +272,7 @@ int dot_t(int64_t n, const void* x, const void* y, double* out, hipStream_t s) {
   const int64_t np = parts_for(n), chunk = chunk_for(n, np);
   double* d = nullptr;
   MPH_HIP_CHECK(hipMalloc(&d, sizeof(double) * (np + 1)));
-  hipLaunchKernelGGL((dot_parts_kernel<Vec>), dim3((unsigned)np), dim3(kT), 0, s,
-                     static_cast<const Vec*>(x), static_cast<const Vec*>(y), n, chunk, d);
+  launch_dot_parts<Vec>(x, y, n, np, chunk, d, s);
   hipLaunchKernelGGL(sum_parts_kernel, dim3(1), dim3(kT), 0, s, d, np, d + np);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess) e = hipMemcpyAsync(out, d + np, sizeof(double), hipMemcpyDeviceToHost, s);
@@ -207,7 +315,7 @@ struct mph_cg_s {
   int64_t n = 0;
   int vt = MPH_F64;
   void *r = nullptr, *p = nullptr, *q = nullptr;
-  double* parts = nullptr;  // [np] p.q partials | [np] r.r partials | [2] state
+  double* parts = nullptr;  // [np] p.q partials | [np] r.r partials | [kCgState] state
   int64_t np = 0, chunk = 0;
   bool started = false;
 };
@@ -223,6 +331,8 @@ int cg_start_t(mph_cg_s* c, const void* b, void* x, hipStream_t s) {
   hipLaunchKernelGGL((cg_start_kernel<Vec>), dim3((unsigned)c->np), dim3(kT), 0, s,
                      static_cast<const Vec*>(b), static_cast<const Vec*>(c->q),
                      static_cast<Vec*>(c->r), static_cast<Vec*>(c->p), c->n, c->chunk, rr_parts);
+  hipLaunchKernelGGL(sum_parts_kernel, dim3(1), dim3(kT), 0, s, rr_parts, c->np,
+                     c->parts + 2 * c->np + kNext);
   MPH_HIP_CHECK(hipGetLastError());
   return MPH_OK;
 }
@@ -232,21 +342,19 @@ int cg_iterate_t(mph_cg_s* c, void* x, int32_t iters, hipStream_t s) {
   double* pq_parts = c->parts;
   double* rr_parts = c->parts + c->np;
   double* state = c->parts + 2 * c->np;
-  const unsigned grid_p = (unsigned)std::min<int64_t>(ceil_div(c->n, kT), 8 * 1024);
+  Vec *r = static_cast<Vec*>(c->r), *p = static_cast<Vec*>(c->p);
+  const dim3 g((unsigned)c->np), b(kT);
   for (int32_t k = 0; k < iters; k++) {
-    // state[0] = r.r of the current residual (its partials are rr_parts)
-    hipLaunchKernelGGL(sum_parts_kernel, dim3(1), dim3(kT), 0, s, rr_parts, c->np, state);
     MPH_CHECK_STATUS(mph_multiply(c->A, c->p, c->q, 1, s));
-    hipLaunchKernelGGL((dot_parts_kernel<Vec>), dim3((unsigned)c->np), dim3(kT), 0, s,
-                       static_cast<const Vec*>(c->p), static_cast<const Vec*>(c->q), c->n,
-                       c->chunk, pq_parts);
-    hipLaunchKernelGGL((cg_update_kernel<Vec>), dim3((unsigned)c->np), dim3(kT), 0, s,
-                       static_cast<Vec*>(x), static_cast<Vec*>(c->r),
-                       static_cast<const Vec*>(c->p), static_cast<const Vec*>(c->q), c->n,
+    launch_dot_parts<Vec>(c->p, c->q, c->n, c->np, c->chunk, pq_parts, s);
+    hipLaunchKernelGGL((cg_update_kernel<Vec>), g, b, 0, s, r, static_cast<const Vec*>(c->q), c->n,
                        c->chunk, pq_parts, c->np, state, rr_parts);
-    hipLaunchKernelGGL((cg_direction_kernel<Vec>), dim3(grid_p), dim3(kT), 0, s,
-                       static_cast<Vec*>(c->p), static_cast<const Vec*>(c->r), c->n, rr_parts,
-                       c->np, state);
+    if (aligned16(x))
+      hipLaunchKernelGGL((cg_direction_kernel<Vec, true>), g, b, 0, s, static_cast<Vec*>(x), p, r,
+                         c->n, c->chunk, rr_parts, c->np, state);
+    else
+      hipLaunchKernelGGL((cg_direction_kernel<Vec, false>), g, b, 0, s, static_cast<Vec*>(x), p, r,
+                         c->n, c->chunk, rr_parts, c->np, state);
   }
   MPH_HIP_CHECK(hipGetLastError());
   return MPH_OK;
@@ -318,7 +426,7 @@ int mph_cg_create(mph_cg_t* out, mph_matrix_t A) {
   const size_t vb = vs * (size_t)std::max<int64_t>(c->n, 1);
   if (hipMalloc(&c->r, vb) != hipSuccess || hipMalloc(&c->p, vb) != hipSuccess ||
       hipMalloc(&c->q, vb) != hipSuccess ||
-      hipMalloc(&c->parts, sizeof(double) * (2 * c->np + 2)) != hipSuccess) {
+      hipMalloc(&c->parts, sizeof(double) * (2 * c->np + kCgState)) != hipSuccess) {
     mph_cg_destroy(c);
     set_error("hipMalloc failed in mph_cg_create");
     return MPH_ERR_OUT_OF_MEMORY;
@@ -368,7 +476,7 @@ int mph_cg_residual(mph_cg_t c, double* rr, mph_stream_t stream) {
     return MPH_OK;
   }
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  double* slot = c->parts + 2 * c->np + 1;
+  double* slot = c->parts + 2 * c->np + kResidual;
   hipLaunchKernelGGL(sum_parts_kernel, dim3(1), dim3(kT), 0, s, c->parts + c->np, c->np, slot);
   MPH_HIP_CHECK(hipGetLastError());
   MPH_HIP_CHECK(hipMemcpyAsync(rr, slot, sizeof(double), hipMemcpyDeviceToHost, s));
