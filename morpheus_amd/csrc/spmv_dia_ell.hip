@@ -959,20 +959,24 @@ int launch_fmt(mph_matrix_impl* A, int k, const void* x, void* y, int init,
     Vec* ys = static_cast<Vec*>(y) + done;
     if (pieces && rem >= Q) {
       const int kl = rem >= 16 * Q ? 16 : rem >= 8 * Q ? 8 : rem >= 4 * Q ? 4 : rem >= 2 * Q ? 2 : 1;
-      int st;
-      switch (kl) {
-        case 16: st = launch_spmm_lanes<V, DIA, 16>(A, xs, ys, k, init, s); break;
-        case 8: st = launch_spmm_lanes<V, DIA, 8>(A, xs, ys, k, init, s); break;
-        case 4: st = launch_spmm_lanes<V, DIA, 4>(A, xs, ys, k, init, s); break;
-        case 2: st = launch_spmm_lanes<V, DIA, 2>(A, xs, ys, k, init, s); break;
-        default: st = launch_spmm_lanes<V, DIA, 1>(A, xs, ys, k, init, s); break;
+      // (5 to 7 columns that lane groups would split into passes take one)
+      if (RPT > 1 || rem >= 8 || kl * Q == rem) {
+        int st;
+        switch (kl) {
+          case 16: st = launch_spmm_lanes<V, DIA, 16>(A, xs, ys, k, init, s); break;
+          case 8: st = launch_spmm_lanes<V, DIA, 8>(A, xs, ys, k, init, s); break;
+          case 4: st = launch_spmm_lanes<V, DIA, 4>(A, xs, ys, k, init, s); break;
+          case 2: st = launch_spmm_lanes<V, DIA, 2>(A, xs, ys, k, init, s); break;
+          default: st = launch_spmm_lanes<V, DIA, 1>(A, xs, ys, k, init, s); break;
+        }
+        if (st != MPH_OK) return st;
+        done += kl * Q;
+        continue;
       }
-      if (st != MPH_OK) return st;
-      done += kl * Q;
-      continue;
     }
-    int kr = rem >= 16 ? 16 : rem >= 8 ? 8 : rem >= 4 ? 4 : rem >= 2 ? 2 : 1;
-    if (k == 1) kr = 1;
+    // what is left below 8 columns in one pass over the matrix
+    int kr = rem >= 16 ? 16 : rem >= 8 ? 8 : rem;
+    if (RPT > 1 && kr < 8) kr = rem >= 4 ? 4 : rem >= 2 ? 2 : 1;
     int st;
 #define MPH_LAUNCH(KRV)                                             \
   st = DIA ? launch_dia_k<V, KRV, RPT>(A, xs, ys, k, init, s)       \
@@ -982,7 +986,17 @@ int launch_fmt(mph_matrix_impl* A, int k, const void* x, void* y, int init,
       case 8: MPH_LAUNCH(8); break;
       case 4: MPH_LAUNCH(4); break;
       case 2: MPH_LAUNCH(2); break;
-      default: MPH_LAUNCH(1); break;
+      case 1: MPH_LAUNCH(1); break;
+      default:
+        st = MPH_OK;
+        if constexpr (RPT == 1) {
+          switch (kr) {
+            case 7: MPH_LAUNCH(7); break;
+            case 6: MPH_LAUNCH(6); break;
+            case 5: MPH_LAUNCH(5); break;
+            default: MPH_LAUNCH(3); break;
+          }
+        }
     }
 #undef MPH_LAUNCH
     if (st != MPH_OK) return st;
