@@ -165,6 +165,44 @@ __global__ __launch_bounds__(256) void dia_kernel(DiaArgs<V> a) {
   }
 }
 
+// The x entries a workgroup stages, in two halves: the loads into registers
+// (N a thread, LDS entries first + 256 k), and their stores to LDS, so that a
+// kernel's first values are requested between the two and one round trip to
+// memory serves both (FP64: 27-point 160^3 186 -> 181 us, 7-point 128^3 29.2
+// -> 28.1 us, 4M rows of 9 diagonals 69 -> 64.6 us).  WIN: rows beyond 256 (each cluster's
+// window is that much longer, and starts that much later per cluster).
+template <typename Vec, int N, int WIN>
+__device__ __forceinline__ void stage_load(const DiaStage& cl, const Vec* __restrict__ x,
+                                           int64_t ncols, int64_t r0, int first, Vec (&xr)[N]) {
+  const int total = cl.base[cl.n - 1] + cl.len[cl.n - 1] + WIN * cl.n;
+#pragma unroll
+  for (int k = 0; k < N; k++) {
+    const int e = first + (int)threadIdx.x + 256 * k;
+    int32_t shift = cl.omin[0] - cl.base[0];
+    for (int c = 1; c < cl.n; c++)
+      if (e >= cl.base[c] + WIN * c) shift = cl.omin[c] - cl.base[c] - WIN * c;
+    const int64_t col = r0 + shift + e;
+    xr[k] = (e < total && col >= 0 && col < ncols) ? x[col] : (Vec)0;
+  }
+}
+
+template <typename Vec, int N, int WIN>
+__device__ __forceinline__ void stage_store(const DiaStage& cl, Vec* xs, int first,
+                                            const Vec (&xr)[N]) {
+  const int total = cl.base[cl.n - 1] + cl.len[cl.n - 1] + WIN * cl.n;
+#pragma unroll
+  for (int k = 0; k < N; k++) {
+    const int e = first + (int)threadIdx.x + 256 * k;
+    if (e < total) xs[e] = xr[k];
+  }
+}
+
+// LDS entries a thread requests before the first values; those of a wide
+// stage beyond them follow after (requesting all of the 27-point stencil's
+// windows ahead, 8 a thread, cost its FP64 kernel more in registers than it
+// saved: 180 -> 184 us, and the 7-point stencil's 28.1 -> 31.0 us)
+constexpr int kStageAhead = 4;
+
 // DIA SpMV with x staged in LDS per cluster of nearby diagonals (the
 // clusters come from dia_analyse).  For each cluster of two or more
 // diagonals the workgroup's 256 rows read x[r0 + omin .. r0 + 255 + omax]
@@ -179,12 +217,8 @@ __global__ __launch_bounds__(256) void dia_staged_kernel(DiaArgs<V> a, DiaStage 
   __shared__ Vec xs[kDiaStageMax];
   const int64_t r0 = (int64_t)xcd_remap(blockIdx.x, gridDim.x) * 256;
   const int64_t row = r0 + threadIdx.x;
-  for (int c = 0; c < cl.n; c++)
-    for (int j = threadIdx.x; j < cl.len[c]; j += 256) {
-      const int64_t col = r0 + cl.omin[c] + j;
-      xs[cl.base[c] + j] = (col >= 0 && col < a.ncols) ? a.x[col] : (Vec)0;
-    }
-  __syncthreads();
+  Vec xr[kStageAhead];
+  stage_load<Vec, kStageAhead, 0>(cl, a.x, a.ncols, r0, 0, xr);
   Acc t = 0;
   for (int d0 = 0; d0 < a.ndiag; d0 += 8) {
     V v[8];
@@ -197,6 +231,15 @@ __global__ __launch_bounds__(256) void dia_staged_kernel(DiaArgs<V> a, DiaStage 
       col[w] = row + o;
       ok[w] = d < a.ndiag && row < a.nrows && col[w] >= 0 && col[w] < a.ncols;
       v[w] = ok[w] ? ld_stream(a.val + a.pitch * d + row) : V{};
+    }
+    if (d0 == 0) {
+      stage_store<Vec, kStageAhead, 0>(cl, xs, 0, xr);
+      const int total = cl.base[cl.n - 1] + cl.len[cl.n - 1];
+      for (int first = 256 * kStageAhead; first < total; first += 256 * kStageAhead) {
+        stage_load<Vec, kStageAhead, 0>(cl, a.x, a.ncols, r0, first, xr);
+        stage_store<Vec, kStageAhead, 0>(cl, xs, first, xr);
+      }
+      __syncthreads();
     }
     hold_raw(v);
 #pragma unroll
@@ -706,6 +749,60 @@ __global__ __launch_bounds__(256) void dia_pair_staged_kernel(DiaArgs<V> a, DiaS
   if (row + 1 < a.nrows) a.y[row + 1] = a.init ? t1 : a.y[row + 1] + t1;
 }
 
+// The same for a stage of at most kStageAhead entries a thread (a band, two
+// planes of a small grid): the first batch's value pairs are requested before
+// the stage is stored, raw until their products, 12 diagonals a batch.  A
+// workgroup's rows were three round trips one after another (x, eight
+// diagonals, the rest); 4M rows, 9 diagonals: FP32 40.9 -> 34.3 us, BF16 37.8
+// -> 30.8 us (3.4 TB/s); a wide stage gains nothing (27-point 160^3 FP32 103
+// -> 108 us, BF16 88 -> 99 us) and keeps the kernel above.
+template <typename V>
+__global__ __launch_bounds__(256) void dia_pair_ahead_kernel(DiaArgs<V> a, DiaStage cl) {
+  using P = Pair<V>;
+  constexpr int U = 12;  // diagonals a batch, their pairs raw until the products
+  __shared__ float xs[256 * kStageAhead];
+  const int64_t r0 = (int64_t)xcd_remap(blockIdx.x, gridDim.x) * 512;
+  const int64_t row = r0 + 2 * threadIdx.x;
+  float xr[kStageAhead];
+  stage_load<float, kStageAhead, 256>(cl, a.x, a.ncols, r0, 0, xr);
+  const typename P::T* pv = reinterpret_cast<const typename P::T*>(a.val);
+  float t0 = 0, t1 = 0;
+  for (int d0 = 0; d0 < a.ndiag; d0 += U) {
+    typename P::T pw[U];
+#pragma unroll
+    for (int w = 0; w < U; w++) {
+      const int d = min(d0 + w, a.ndiag - 1);
+      pw[w] = ld_stream(pv + (a.pitch * d + min(row, a.pitch - 2)) / 2);
+    }
+    if (d0 == 0) {
+      stage_store<float, kStageAhead, 256>(cl, xs, 0, xr);
+      __syncthreads();
+    }
+#pragma unroll
+    for (int w = 0; w < U; w++) {
+      const int d = d0 + w;
+      if (d >= a.ndiag) break;
+      const int64_t o = a.off[d];
+      const int32_t lb = cl.lb2[d];  // uniform
+      float v0, v1;
+      P::split(pw[w], v0, v1);
+      const int64_t c0 = row + o, c1 = row + 1 + o;
+      const bool in0 = row < a.nrows && c0 >= 0 && c0 < a.ncols;
+      const bool in1 = row + 1 < a.nrows && c1 >= 0 && c1 < a.ncols;
+      if (lb != kDiaDirect) {
+        // (inside the cluster's window whenever the column is)
+        if (in0) t0 += v0 * xs[lb + (int32_t)(c0 - r0)];
+        if (in1) t1 += v1 * xs[lb + (int32_t)(c1 - r0)];
+      } else {
+        if (in0) t0 += v0 * a.x[c0];
+        if (in1) t1 += v1 * a.x[c1];
+      }
+    }
+  }
+  if (row < a.nrows) a.y[row] = a.init ? t0 : a.y[row] + t0;
+  if (row + 1 < a.nrows) a.y[row + 1] = a.init ? t1 : a.y[row + 1] + t1;
+}
+
 template <typename V>
 __global__ __launch_bounds__(256) void ell_pair_kernel(EllArgs<V> a) {
   using P = Pair<V>;
@@ -1023,7 +1120,11 @@ int launch_pair(mph_matrix_impl* A, const void* x, void* y, int init, hipStream_
     a.y = static_cast<float*>(y);
     a.ld = 1;
     a.init = init;
-    if (A->dia_stage.n > 0 && A->dia_stage.pair)
+    const DiaStage& cl = A->dia_stage;
+    if (cl.n > 0 && cl.pair &&
+        cl.base[cl.n - 1] + cl.len[cl.n - 1] + 256 * cl.n <= 256 * kStageAhead)
+      hipLaunchKernelGGL(dia_pair_ahead_kernel<V>, dim3((unsigned)nb), dim3(256), 0, s, a, cl);
+    else if (cl.n > 0 && cl.pair)
       hipLaunchKernelGGL(dia_pair_staged_kernel<V>, dim3((unsigned)nb), dim3(256), 0, s, a,
                          A->dia_stage);
     else
