@@ -111,7 +111,7 @@ __global__ __launch_bounds__(kT) void row_hist_kernel(const int32_t* __restrict_
 // registers and LDS, and adds its result with one atomic.  An atomic per
 // element on one address was served one at a time: the maxima of 14.6M COO
 // indices took 2.6 ms, now about 15 us (the 58 MB read at the stream rate).
-constexpr int64_t kReduceBlocks = 512;  // (2048 spent 20 us on the atomics)
+constexpr int64_t kReduceBlocks = 256;  // (2048 spent 20 us on the atomics, 512 10)
 inline unsigned reduce_blocks(int64_t n) {
   return (unsigned)std::min<int64_t>(blocks_for(n, 4 * kT), kReduceBlocks);
 }
@@ -919,9 +919,10 @@ __global__ __launch_bounds__(kT) void ell_row_count_kernel(
     const int32_t* __restrict__ eci, int64_t nrows, int64_t width, int64_t pitch,
     const int32_t* __restrict__ tro, const int32_t* __restrict__ tci, int32_t* __restrict__ cnt,
     int32_t* __restrict__ stats) {
-  const int64_t r = (int64_t)blockIdx.x * kT + threadIdx.x;
-  int32_t n = 0, prev = INT32_MIN, bad = 0, top = 0;
-  if (r < nrows) {
+  int32_t bad = 0, top = 0;
+  for (int64_t r = (int64_t)blockIdx.x * kT + threadIdx.x; r < nrows;
+       r += (int64_t)gridDim.x * kT) {
+    int32_t n = 0, prev = INT32_MIN;
     for (int64_t s0 = 0; s0 < width; s0 += kScanPer) {
       int32_t c[kScanPer];
 #pragma unroll
@@ -932,7 +933,7 @@ __global__ __launch_bounds__(kT) void ell_row_count_kernel(
           bad |= c[k] < prev ? 1 : 0;
           prev = c[k];
           n++;
-          top = (int32_t)(s0 + k) + 1;
+          top = max(top, (int32_t)(s0 + k) + 1);
         }
     }
     if (tro) {
@@ -1717,8 +1718,8 @@ int ell_part_to_coo(int64_t nrows, int64_t nnz, int64_t width, int64_t pitch, co
     MPH_CHECK_STATUS(t.alloc(&tmp, scan_tmp_elems(nrows)));
     MPH_CHECK_STATUS(t.alloc(&stats, 2));
     MPH_CHECK_STATUS(fill_zero(stats, 2 * sizeof(int32_t), s));
-    hipLaunchKernelGGL(ell_row_count_kernel, dim3(blocks_for(nrows)), dim3(kT), 0, s, eci, nrows,
-                       width, pitch, tro, tci, cnt, stats);
+    hipLaunchKernelGGL(ell_row_count_kernel, dim3(std::min(blocks_for(nrows), 2048u)), dim3(kT), 0,
+                       s, eci, nrows, width, pitch, tro, tci, cnt, stats);
     MPH_HIP_CHECK(hipGetLastError());
     MPH_CHECK_STATUS(exclusive_scan_i32(cnt, rowpos, nrows, tmp, s));
     MPH_CHECK_STATUS(t.fetch(rowpos + nrows, &ht));

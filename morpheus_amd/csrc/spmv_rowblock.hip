@@ -1514,14 +1514,14 @@ __global__ __launch_bounds__(256) void rb_count_kernel(const int32_t* __restrict
   __shared__ int32_t s_max;
   if (threadIdx.x == 0) s_max = 0;
   __syncthreads();
-  const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   int32_t m = 0;
-  if (r < nrows) {
+  for (int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; r < nrows;
+       r += (int64_t)gridDim.x * blockDim.x) {
     bool lg;
     int64_t len;
     const bool st = rb_is_start(ro, r, chunk, long_len, lg, len);
     cnt[r] = st ? (lg ? (int32_t)((len + chunk - 1) / chunk) : 1) : 0;
-    m = (int32_t)len;
+    m = max(m, (int32_t)len);
   }
   for (int d = kWave / 2; d > 0; d >>= 1) m = max(m, shfl_xor(m, d));
   if (threadIdx.x % kWave == 0) atomicMax(&s_max, m);
@@ -2525,8 +2525,10 @@ int rowblock_analyse(mph_matrix_impl* A, hipStream_t s) {
     MPH_CHECK_STATUS(t.alloc(&stats, kRbStats));
     MPH_CHECK_STATUS(fill_zero(stats, kRbStats * sizeof(int32_t), s));
     const unsigned g = (unsigned)ceil_div(nrows, 256);
-    hipLaunchKernelGGL(rb_count_kernel, dim3(g), dim3(256), 0, s, ro, nrows, p.chunk, p.long_len,
-                       cnt, stats);
+    // (every workgroup reads the one word of the longest row: a workgroup per
+    // 256 of 1M rows took 24 us, 1024 take 13.5)
+    hipLaunchKernelGGL(rb_count_kernel, dim3(std::min(g, 1024u)), dim3(256), 0, s, ro, nrows,
+                       p.chunk, p.long_len, cnt, stats);
     MPH_HIP_CHECK(hipGetLastError());
     MPH_CHECK_STATUS(exclusive_scan_i32(cnt, first, nrows, tmp, s));
     MPH_CHECK_STATUS(t.fetch(first + nrows, &hb));
