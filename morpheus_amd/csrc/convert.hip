@@ -1451,6 +1451,12 @@ int check_coo_args(int64_t nrows, int64_t ncols, int64_t nnz, const int32_t* ri,
   return MPH_OK;
 }
 
+// (diagonals are numbered in 32 bits)
+int check_diagonals(int64_t nrows, int64_t ncols) {
+  if (nrows + ncols - 1 > INT32_MAX) return invalid("more diagonals than the int32 range");
+  return MPH_OK;
+}
+
 // The diagonals a COO list uses, and how its entries are ordered.
 struct DiaScan {
   uint32_t* bits = nullptr;
@@ -1461,6 +1467,7 @@ struct DiaScan {
 
 int dia_scan(int64_t nrows, int64_t ncols, int64_t nnz, const int32_t* ri, const int32_t* ci,
              Tmp& t, DiaScan& D, hipStream_t s) {
+  MPH_CHECK_STATUS(check_diagonals(nrows, ncols));
   D.words = ceil_div(nrows + ncols - 1, 32);
   int32_t *flags, *cnt, *hf, *hn;
   int64_t* tmp;
@@ -1546,6 +1553,7 @@ struct HdcScan {
 
 int hdc_scan(int64_t nrows, int64_t ncols, int64_t nnz, const int32_t* ri, const int32_t* ci,
              Tmp& t, HdcScan& H, hipStream_t s) {
+  MPH_CHECK_STATUS(check_diagonals(nrows, ncols));
   const int64_t nb = nrows + ncols - 1;
   unsigned long long *acc, *h;  // ndiag, dia_nnz, csr_nnz, flags
   MPH_CHECK_STATUS(t.alloc(&H.cnt, nb));
