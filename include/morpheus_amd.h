@@ -181,7 +181,9 @@ int mph_matrix_plan_bytes(mph_matrix_t A, int init, int64_t* bytes);
  *                  The results do not depend on it.  DIA SpMM with 4 or
  *                  more lanes per row (FP64 from 8 columns per pass, FP32 /
  *                  BF16 from 16), or 2 where the runs of diagonals with
- *                  consecutive offsets average two or more, takes 4
+ *                  consecutive offsets average two or more, and rows enough
+ *                  to fill the device (about 384 workgroups in FP64, 768 in
+ *                  FP32 / BF16, of 1024 / lanes rows), takes 4
  *                  consecutive rows per lane group and loads, per run, the X
  *                  rows it covers and its values once, through LDS
  *                  (MPH_DIA_SPMM_RUNS=0 / 1 forces that off / on; the

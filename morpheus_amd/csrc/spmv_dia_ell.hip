@@ -999,11 +999,19 @@ int launch_spmm_lanes(mph_matrix_impl* A, const void* x, void* y, int ld, int in
     // 227 us, FP32 k = 8 212 -> 172 us, BF16 204 -> 170 us; the 7-point
     // stencil's mostly single diagonals: FP64 k = 4 50 -> 72 us); one lane is
     // even at best (27-point FP64 k = 2 207 -> 194 us, FP32 k = 4 125 ->
-    // 128 us; 7-point FP64 k = 2 31 -> 51 us); MPH_DIA_SPMM_RUNS=0 / 1 forces
-    // it off / on
+    // 128 us; 7-point FP64 k = 2 31 -> 51 us).  Its workgroups take four times
+    // the rows and their runs one after another, so it needs 1.5 workgroups a
+    // CU in FP64 and 3 in FP32 / BF16 to win (25-diagonal bands: 65k rows FP64
+    // k = 16, 508 workgroups, 22.1 -> 18.4 us; k = 8, 254, 12.4 -> 16.6; FP32
+    // 260k rows k = 16, 1016, 30.1 -> 24.4, k = 8, 508, 16.9 -> 20.0; 2k rows
+    // 6.3 -> 16 us).  MPH_DIA_SPMM_RUNS=0 / 1 forces it off / on
     const char* env = std::getenv("MPH_DIA_SPMM_RUNS");
     const int mode = env ? std::atoi(env) : -1;
-    const bool wide = KL >= 4 || (KL == 2 && A->dia_runs > 0 && A->ndiag >= 2 * A->dia_runs);
+    const int64_t cus = device_cu_count();
+    const int64_t wgs = ceil_div(A->nrows, (int64_t)(256 / KL) * 4);
+    const bool fills = 2 * wgs >= (A->vt == MPH_F64 ? 3 : 6) * cus;
+    const bool wide =
+        fills && (KL >= 4 || (KL == 2 && A->dia_runs > 0 && A->ndiag >= 2 * A->dia_runs));
     const bool runs = A->ncols > 0 && (mode > 0 || (mode < 0 && wide));
     if (runs) {
       constexpr int R = 4;
