@@ -64,29 +64,29 @@ __device__ __forceinline__ int64_t dia_plane_block(const DiaArgs<V>& a, int64_t 
   return c < a.plane && b * rows_per_block < a.nrows ? b : -1;
 }
 
-// t[u][q] += v[u][w] * x[c[u][w]][q] over a batch of 8 diagonals / slots,
+// t[u][q] += v[u][w] * x[c[u][w]][q] over a batch of B diagonals / slots,
 // skipping c < 0.  The x loads are unconditional (c < 0 reads x[0]) and the
 // sums are selected rather than branched, so the batch's gathers are all in
 // flight before the first product: under a branch each gather was waited on
 // before the next was issued.  Same fused multiply-adds in the same order
 // as t += v * x.  With many right-hand sides (KR * RPT > 2) the gathers of
 // one diagonal / slot are issued together instead, to bound registers.
-template <typename V, int KR, int RPT>
+template <typename V, int KR, int RPT, int B>
 __device__ __forceinline__ void batch_fma(typename vtraits<V>::acc (&t)[RPT][KR],
-                                          const V (&v)[RPT][8], const int64_t (&c)[RPT][8],
+                                          const V (&v)[RPT][B], const int64_t (&c)[RPT][B],
                                           const typename vtraits<V>::vec* __restrict__ x,
                                           int32_t ld) {
   using Acc = typename vtraits<V>::acc;
   if constexpr (KR * RPT <= 2) {
-    Acc xq[RPT][8][KR];
+    Acc xq[RPT][B][KR];
 #pragma unroll
-    for (int w = 0; w < 8; w++)
+    for (int w = 0; w < B; w++)
 #pragma unroll
       for (int u = 0; u < RPT; u++)
 #pragma unroll
         for (int q = 0; q < KR; q++) xq[u][w][q] = (Acc)x[(c[u][w] >= 0 ? c[u][w] : 0) * ld + q];
 #pragma unroll
-    for (int w = 0; w < 8; w++)
+    for (int w = 0; w < B; w++)
 #pragma unroll
       for (int u = 0; u < RPT; u++)
 #pragma unroll
@@ -96,7 +96,7 @@ __device__ __forceinline__ void batch_fma(typename vtraits<V>::acc (&t)[RPT][KR]
         }
   } else {
 #pragma unroll
-    for (int w = 0; w < 8; w++)
+    for (int w = 0; w < B; w++)
 #pragma unroll
       for (int u = 0; u < RPT; u++) {
         const int64_t xc = c[u][w] >= 0 ? c[u][w] : 0;
@@ -312,16 +312,17 @@ __global__ __launch_bounds__(256) void ell_kernel(EllArgs<V> a) {
 #pragma unroll
     for (int u = 0; u < RPT; u++) lim[u] = a.loop;
   }
-  // batches of 8 slots: indices first, then values and x entries
-  for (int n0 = 0; n0 < wl; n0 += 8) {
+  // batches of slots: indices first, then values and x entries
+  auto batch = [&](auto size, int n0) {
+    constexpr int B = decltype(size)::value;
     // index and value loads are unconditional (slots outside the matrix, or
     // beyond the row's count, read slot 0 and are discarded): a load under a
     // branch is waited on where the branch joins, which left one index load
     // in flight at a time
-    int64_t c[RPT][8];
-    int64_t slot[RPT][8];
+    int64_t c[RPT][B];
+    int64_t slot[RPT][B];
 #pragma unroll
-    for (int w = 0; w < 8; w++)
+    for (int w = 0; w < B; w++)
 #pragma unroll
       for (int u = 0; u < RPT; u++) {
         const int64_t row = row0 + u * 256;
@@ -331,16 +332,21 @@ __global__ __launch_bounds__(256) void ell_kernel(EllArgs<V> a) {
         const int32_t ci = ld_stream(a.ci + slot[u][w]);
         c[u][w] = in ? (int64_t)ci : -1;
       }
-    V v[RPT][8];
+    V v[RPT][B];
 #pragma unroll
-    for (int w = 0; w < 8; w++)
+    for (int w = 0; w < B; w++)
 #pragma unroll
       for (int u = 0; u < RPT; u++) v[u][w] = ld_stream(a.val + slot[u][w]);
 #pragma unroll
     for (int u = 0; u < RPT; u++) hold_raw(v[u]);
     // x loads unconditional as well (padding slots read x[0], unused)
     if (a.ncols > 0) batch_fma<V, KR, RPT>(t, v, c, a.x, a.ld);
-  }
+  };
+  // 8 slots a batch, 4 where no more are left: a batch's loads past the last
+  // slot are issued all the same (27 slots are 28 loads of each kind, not 32)
+  int n0 = 0;
+  for (; wl - n0 > 4; n0 += 8) batch(std::integral_constant<int, 8>{}, n0);
+  if (n0 < wl) batch(std::integral_constant<int, 4>{}, n0);
 #pragma unroll
   for (int u = 0; u < RPT; u++) {
     const int64_t row = row0 + u * 256;
