@@ -13,7 +13,7 @@
 // y in a separate launch and then read-modify-writes it per 256-diagonal
 // chunk, and skips the zeroing when ndiag == 0).  ELL visits entries_per_row slots,
 // not the 32-padded width, when the analysis has confirmed that the slots
-// beyond entries_per_row hold only the -1 padding.  FP32 / BF16 SpMV takes
+// beyond entries_per_row hold only the -1 padding.  FP32 / BF16 DIA SpMV takes
 // two adjacent rows per thread (row-pair kernels below); FP32 / BF16 rows of
 // more than kCompensateLen diagonals / slots take a Dot2-compensated kernel.
 // SpMM gives each row a lane group (16 bytes of its columns per lane); with
@@ -342,11 +342,22 @@ __global__ __launch_bounds__(256) void ell_kernel(EllArgs<V> a) {
     // x loads unconditional as well (padding slots read x[0], unused)
     if (a.ncols > 0) batch_fma<V, KR, RPT>(t, v, c, a.x, a.ld);
   };
-  // 8 slots a batch, 4 where no more are left: a batch's loads past the last
-  // slot are issued all the same (27 slots are 28 loads of each kind, not 32)
-  int n0 = 0;
-  for (; wl - n0 > 4; n0 += 8) batch(std::integral_constant<int, 8>{}, n0);
-  if (n0 < wl) batch(std::integral_constant<int, 4>{}, n0);
+  // 8 slots a batch and the rest in one batch of its own size: a batch's loads
+  // past the last slot are issued all the same.  Batches of 8 only, then 8
+  // and a 4, then 8 / 6 / 4 / 2, then this one, FP64: 5-point 1001^2 18.0,
+  // -, 15.8, 14.5 us; band of 9, 4M rows, 117, 104, 98, 95.6 us; 27-point
+  // 127^3 158.5, 148.6, 148.8, 147.7 us; 7-point 127^3 42.1, 42.0, 42.0, 40.0 us
+  for (; wl - n0 >= 8; n0 += 8) batch(std::integral_constant<int, 8>{}, n0);
+  switch (wl - n0) {
+    case 7: batch(std::integral_constant<int, 7>{}, n0); break;
+    case 6: batch(std::integral_constant<int, 6>{}, n0); break;
+    case 5: batch(std::integral_constant<int, 5>{}, n0); break;
+    case 4: batch(std::integral_constant<int, 4>{}, n0); break;
+    case 3: batch(std::integral_constant<int, 3>{}, n0); break;
+    case 2: batch(std::integral_constant<int, 2>{}, n0); break;
+    case 1: batch(std::integral_constant<int, 1>{}, n0); break;
+    default: break;
+  }
 #pragma unroll
   for (int u = 0; u < RPT; u++) {
     const int64_t row = row0 + u * 256;
@@ -666,13 +677,12 @@ __global__ __launch_bounds__(256) void ell_spmm_kernel(EllArgs<V> a) {
 }
 
 // ----------------------------------------------------------- row pairs
-// FP32 / BF16 SpMV: a thread takes the adjacent rows 2t and 2t + 1, so that
-// one load moves the two rows' values of a diagonal / slot (8 B in FP32, 4 B
-// in BF16) and, in ELL, their two column indices (8 B).  With one row per
-// thread a 16-bit value stream moved 128 B per wave load, and BF16 ran
-// slower than FP32.  Used when the pitch is even (a pair never straddles
-// two diagonals / slots; an odd row count then leaves the pair's second
-// element inside the pitch) and the arrays are aligned to the pair.
+// FP32 / BF16 DIA SpMV: a thread takes the adjacent rows 2t and 2t + 1, so
+// that one load moves the two rows' values of a diagonal (8 B in FP32, 4 B in
+// BF16).  With one row per thread a 16-bit value stream moved 128 B per wave
+// load, and BF16 ran slower than FP32.  Used when the pitch is even (a pair
+// never straddles two diagonals; an odd row count then leaves the pair's
+// second element inside the pitch) and the values are aligned to the pair.
 template <typename V>
 __global__ __launch_bounds__(256) void dia_pair_kernel(DiaArgs<V> a) {
   using P = Pair<V>;
@@ -803,43 +813,6 @@ __global__ __launch_bounds__(256) void dia_pair_ahead_kernel(DiaArgs<V> a, DiaSt
         if (in0) t0 += v0 * a.x[c0];
         if (in1) t1 += v1 * a.x[c1];
       }
-    }
-  }
-  if (row < a.nrows) a.y[row] = a.init ? t0 : a.y[row] + t0;
-  if (row + 1 < a.nrows) a.y[row + 1] = a.init ? t1 : a.y[row + 1] + t1;
-}
-
-template <typename V>
-__global__ __launch_bounds__(256) void ell_pair_kernel(EllArgs<V> a) {
-  using P = Pair<V>;
-  const uint32_t b = xcd_remap(blockIdx.x, gridDim.x);
-  const int64_t row = ((int64_t)b * 256 + threadIdx.x) * 2;
-  const typename P::T* pv = reinterpret_cast<const typename P::T*>(a.val);
-  const uint64_t* pc = reinterpret_cast<const uint64_t*>(a.ci);
-  float t0 = 0, t1 = 0;
-  const bool in = row < a.nrows;
-  for (int n0 = 0; n0 < a.loop; n0 += 8) {
-    int32_t c0[8], c1[8];
-#pragma unroll
-    for (int w = 0; w < 8; w++) {
-      const int n = n0 + w;
-      const uint64_t cw = in && n < a.loop ? ld_stream(pc + (a.pitch * n + row) / 2) : ~0ull;
-      c0[w] = (int32_t)(uint32_t)cw;
-      // the pair's second row may lie past nrows, inside the pitch
-      c1[w] = row + 1 < a.nrows ? (int32_t)(uint32_t)(cw >> 32) : -1;
-    }
-    float v0[8], v1[8];
-#pragma unroll
-    for (int w = 0; w < 8; w++) {
-      const int n = n0 + w;
-      const typename P::T pw =
-          (c0[w] >= 0 || c1[w] >= 0) ? ld_stream(pv + (a.pitch * n + row) / 2) : (typename P::T)0;
-      P::split(pw, v0[w], v1[w]);
-    }
-#pragma unroll
-    for (int w = 0; w < 8; w++) {
-      if (c0[w] >= 0) t0 += v0[w] * a.x[c0[w]];
-      if (c1[w] >= 0) t1 += v1[w] * a.x[c1[w]];
     }
   }
   if (row < a.nrows) a.y[row] = a.init ? t0 : a.y[row] + t0;
@@ -1116,60 +1089,44 @@ int launch_fmt(mph_matrix_impl* A, int k, const void* x, void* y, int init,
   return MPH_OK;
 }
 
-// the row-pair kernels: FP32 / BF16 SpMV with the default launch shape, an
-// even pitch and arrays aligned to the pair loads
-template <typename V, bool DIA>
-int launch_pair(mph_matrix_impl* A, const void* x, void* y, int init, hipStream_t s) {
+// the DIA row-pair kernels: FP32 / BF16 SpMV with the default launch shape, an
+// even pitch and values aligned to the pair loads.  ELL keeps one row per
+// thread at every pitch: pairs, with their loads under branches, took 96-98 us
+// in FP32 and 78.5 in BF16 on the 27-point 128^3 grid where ell_kernel takes
+// 76.7 and 55.6 (7-point 128^3: 25.8 and 21.8, now 21.6 and 18.7; 5-point
+// 1000^2, the closest: 9.7 and 7.6, now 9.1 and 7.5); pairs without branches
+// took 102 and 82 (28 and 23).
+template <typename V>
+int launch_dia_pair(mph_matrix_impl* A, const void* x, void* y, int init, hipStream_t s) {
   const int64_t nb = ceil_div(A->nrows, 512);
   if (nb == 0) return MPH_OK;
-  if constexpr (DIA) {
-    DiaArgs<V> a{};
-    a.nrows = A->nrows;
-    a.ncols = A->ncols;
-    a.ndiag = (int32_t)A->ndiag;
-    a.pitch = A->dia_pitch;
-    a.off = A->dia_off;
-    a.val = static_cast<const V*>(A->dia_v);
-    a.x = static_cast<const float*>(x);
-    a.y = static_cast<float*>(y);
-    a.ld = 1;
-    a.init = init;
-    const DiaStage& cl = A->dia_stage;
-    if (cl.n > 0 && cl.pair &&
-        cl.base[cl.n - 1] + cl.len[cl.n - 1] + 256 * cl.n <= 256 * kStageAhead)
-      hipLaunchKernelGGL(dia_pair_ahead_kernel<V>, dim3((unsigned)nb), dim3(256), 0, s, a, cl);
-    else if (cl.n > 0 && cl.pair)
-      hipLaunchKernelGGL(dia_pair_staged_kernel<V>, dim3((unsigned)nb), dim3(256), 0, s, a,
-                         A->dia_stage);
-    else
-      hipLaunchKernelGGL(dia_pair_kernel<V>, dim3((unsigned)nb), dim3(256), 0, s, a);
-  } else {
-    EllArgs<V> a{};
-    a.nrows = A->nrows;
-    a.loop = (int32_t)A->ell_loop;
-    a.pitch = A->ell_pitch;
-    a.ci = A->ell_ci;
-    a.val = static_cast<const V*>(A->ell_v);
-    a.x = static_cast<const float*>(x);
-    a.y = static_cast<float*>(y);
-    a.ld = 1;
-    a.init = init;
-    hipLaunchKernelGGL(ell_pair_kernel<V>, dim3((unsigned)nb), dim3(256), 0, s, a);
-  }
+  DiaArgs<V> a{};
+  a.nrows = A->nrows;
+  a.ncols = A->ncols;
+  a.ndiag = (int32_t)A->ndiag;
+  a.pitch = A->dia_pitch;
+  a.off = A->dia_off;
+  a.val = static_cast<const V*>(A->dia_v);
+  a.x = static_cast<const float*>(x);
+  a.y = static_cast<float*>(y);
+  a.ld = 1;
+  a.init = init;
+  const DiaStage& cl = A->dia_stage;
+  if (cl.n > 0 && cl.pair && cl.base[cl.n - 1] + cl.len[cl.n - 1] + 256 * cl.n <= 256 * kStageAhead)
+    hipLaunchKernelGGL(dia_pair_ahead_kernel<V>, dim3((unsigned)nb), dim3(256), 0, s, a, cl);
+  else if (cl.n > 0 && cl.pair)
+    hipLaunchKernelGGL(dia_pair_staged_kernel<V>, dim3((unsigned)nb), dim3(256), 0, s, a, cl);
+  else
+    hipLaunchKernelGGL(dia_pair_kernel<V>, dim3((unsigned)nb), dim3(256), 0, s, a);
   MPH_HIP_CHECK(hipGetLastError());
   return MPH_OK;
 }
 
-template <bool DIA>
-bool pair_ok(const mph_matrix_impl* A, int k) {
+bool dia_pair_ok(const mph_matrix_impl* A, int k) {
   if (k != 1 || A->tuning.rows_per_thread != 0) return false;
   if (A->vt != MPH_F32 && A->vt != MPH_BF16) return false;
-  if (!DIA && A->rb.ell_cnt) return false;  // the counted one-row kernel
-  const int64_t pitch = DIA ? A->dia_pitch : A->ell_pitch;
-  const uintptr_t v = reinterpret_cast<uintptr_t>(DIA ? A->dia_v : A->ell_v);
-  const size_t pair_bytes = 2 * value_size(A->vt);
-  if (pitch % 2 != 0 || v % pair_bytes != 0) return false;
-  return DIA || reinterpret_cast<uintptr_t>(A->ell_ci) % 8 == 0;
+  return A->dia_pitch % 2 == 0 &&
+         reinterpret_cast<uintptr_t>(A->dia_v) % (2 * value_size(A->vt)) == 0;
 }
 
 template <bool DIA>
@@ -1178,9 +1135,9 @@ int dispatch(mph_matrix_impl* A, int k, const void* x, void* y, int init,
   if (A->vt != MPH_F64 && (DIA ? A->ndiag : A->ell_loop) > kCompensateLen)
     return A->vt == MPH_F32 ? launch_comp<float, DIA>(A, k, x, y, init, s)
                             : launch_comp<bf16, DIA>(A, k, x, y, init, s);
-  if (pair_ok<DIA>(A, k))
-    return A->vt == MPH_F32 ? launch_pair<float, DIA>(A, x, y, init, s)
-                            : launch_pair<bf16, DIA>(A, x, y, init, s);
+  if (DIA && dia_pair_ok(A, k))
+    return A->vt == MPH_F32 ? launch_dia_pair<float>(A, x, y, init, s)
+                            : launch_dia_pair<bf16>(A, x, y, init, s);
   if (DIA && k == 1 && A->dia_stage.n > 0 && A->tuning.rows_per_thread == 0)
     return A->vt == MPH_F64   ? launch_dia_staged<double>(A, x, y, init, s)
            : A->vt == MPH_F32 ? launch_dia_staged<float>(A, x, y, init, s)
