@@ -347,6 +347,7 @@ __global__ __launch_bounds__(256) void ell_kernel(EllArgs<V> a) {
   // and a 4, then 8 / 6 / 4 / 2, then this one, FP64: 5-point 1001^2 18.0,
   // -, 15.8, 14.5 us; band of 9, 4M rows, 117, 104, 98, 95.6 us; 27-point
   // 127^3 158.5, 148.6, 148.8, 147.7 us; 7-point 127^3 42.1, 42.0, 42.0, 40.0 us
+  int n0 = 0;
   for (; wl - n0 >= 8; n0 += 8) batch(std::integral_constant<int, 8>{}, n0);
   switch (wl - n0) {
     case 7: batch(std::integral_constant<int, 7>{}, n0); break;
