@@ -300,8 +300,8 @@ __device__ __forceinline__ void count_keys(int32_t* __restrict__ cnt, int32_t* h
 }
 
 // What coo_scan_kernel also gathers: the bitmap of the diagonals used, a
-// count per diagonal, or the bits that any row / any column has (flags[1] /
-// flags[2]: as wide as the largest index, without a maximum pass).
+// count per diagonal, or the bits that any row / any column from 0 has
+// (flags[1] / flags[2]: as wide as the largest index, without a maximum pass).
 enum DiagMode { kNoDiags, kDiagBits, kDiagCounts, kWidths };
 
 template <bool COLS, bool OFFSETS, DiagMode DIAGS>
@@ -344,7 +344,7 @@ __global__ __launch_bounds__(kT) void coo_scan_kernel(
       const bool col_ok = !COLS || (c[k] >= 0 && c[k] < ncols);
       if (in) {
         wide_r |= r[k];
-        wide_c |= c[k];
+        wide_c |= max(c[k], 0);
         if (!row_ok) bad |= kBadRow;
         if (!col_ok) bad |= kBadCol;
         if (i > 0) {
@@ -477,14 +477,14 @@ constexpr int kSortWaves = kSortThreads / kWave;
 struct SortKeys {
   const int32_t *ri, *ci;    // first pass: the key is (ri << cb) | ci
   const uint64_t* key;       // later passes
-  int cb, shift;
+  int cb, shift, mask;       // the pass's digit: mask of the key shifted
   template <bool FIRST>
   __device__ __forceinline__ uint64_t get(int64_t i) const {
     if (!FIRST) return key[i];
     return ((uint64_t)(uint32_t)ri[i] << cb) | (uint32_t)ci[i];
   }
   __device__ __forceinline__ int digit(uint64_t k) const {
-    return (int)(k >> shift) & (kSortBins - 1);
+    return (int)(k >> shift) & mask;
   }
 };
 
@@ -640,18 +640,39 @@ int copy_dev(void* dst, const void* src, size_t bytes, hipStream_t s) {
 }
 
 // Stable sort of COO entries by (row, col), rows below 2^rb and columns below
-// 2^cb; by_col false: by row only, the columns carried along.  The outputs
-// may be the inputs.
+// 2^cb; kByRow: by row only, the columns carried along.  kLowBits: the columns
+// carried whole too, and sorted by their low cb bits, rounded up to a multiple
+// of 4 (a column below 0 has no other order).  The outputs may be the inputs.
+enum SortBy { kByRowCol, kByRow, kLowBits };
+
 template <typename W>
-int radix_sort(int64_t n, int rb, int cb, bool by_col, const int32_t* ri, const int32_t* ci,
+int radix_sort(int64_t n, int rb, int cb, SortBy by, const int32_t* ri, const int32_t* ci,
                const void* v, int32_t* ri_out, int32_t* ci_out, void* v_out, hipStream_t s) {
   if (n <= 0) return MPH_OK;
   Tmp t(s);
   const int64_t nb = ceil_div(n, kSortTile);
-  if (!by_col) cb = 32;
-  const int from = by_col ? 0 : cb;
+  // the digits: shift and mask of each pass
+  constexpr int kMaxPasses = 8;
+  int shift[kMaxPasses], mask[kMaxPasses], passes = 0;
+  auto digits = [&](int from, int to) {
+    for (int b = from; b < to; b += kSortBits) {
+      shift[passes] = b;
+      mask[passes++] = (1 << std::min(kSortBits, to - b)) - 1;
+    }
+  };
+  if (by == kByRowCol) {
+    digits(0, rb + cb);
+  } else {
+    if (by == kLowBits) digits(0, (int)ceil_div(cb, 4) * 4);
+    cb = 32;
+    digits(cb, cb + rb);
+  }
   // at least two passes: the last one's input is never the arrays it writes
-  const int passes = std::max(2, (int)ceil_div(rb + cb - from, kSortBits));
+  // (a pass that sees digits 0 only moves)
+  while (passes < 2) {
+    shift[passes] = 0;
+    mask[passes++] = 0;
+  }
   uint64_t* key[2];
   W* val[2];
   int32_t *hist, *offs;
@@ -665,9 +686,7 @@ int radix_sort(int64_t n, int rb, int cb, bool by_col, const int32_t* ri, const 
   MPH_CHECK_STATUS(t.alloc(&tmp, scan_tmp_elems(kSortBins * nb)));
   const dim3 g((unsigned)nb), b(kSortThreads);
   for (int q = 0; q < passes; q++) {
-    // (a pass beyond the keys' bits sees digits 0 and only moves)
-    const SortKeys K{ri, ci, q > 0 ? key[(q - 1) & 1] : nullptr, cb,
-                     std::min(from + q * kSortBits, 56)};
+    const SortKeys K{ri, ci, q > 0 ? key[(q - 1) & 1] : nullptr, cb, shift[q], mask[q]};
     const W* vin = q > 0 ? val[(q - 1) & 1] : static_cast<const W*>(v);
     if (q == 0)
       hipLaunchKernelGGL(sort_count_kernel<true>, g, b, 0, s, K, n, hist, nb);
@@ -691,14 +710,14 @@ int radix_sort(int64_t n, int rb, int cb, bool by_col, const int32_t* ri, const 
   return MPH_OK;  // (t waits for the stream)
 }
 
-int radix_sort(int64_t n, int rb, int cb, bool by_col, const int32_t* ri, const int32_t* ci,
+int radix_sort(int64_t n, int rb, int cb, SortBy by, const int32_t* ri, const int32_t* ci,
                const void* v, int vsize, int32_t* ri_out, int32_t* ci_out, void* v_out,
                hipStream_t s) {
   if (vsize == 8)
-    return radix_sort<uint64_t>(n, rb, cb, by_col, ri, ci, v, ri_out, ci_out, v_out, s);
+    return radix_sort<uint64_t>(n, rb, cb, by, ri, ci, v, ri_out, ci_out, v_out, s);
   if (vsize == 4)
-    return radix_sort<uint32_t>(n, rb, cb, by_col, ri, ci, v, ri_out, ci_out, v_out, s);
-  return radix_sort<uint16_t>(n, rb, cb, by_col, ri, ci, v, ri_out, ci_out, v_out, s);
+    return radix_sort<uint32_t>(n, rb, cb, by, ri, ci, v, ri_out, ci_out, v_out, s);
+  return radix_sort<uint16_t>(n, rb, cb, by, ri, ci, v, ri_out, ci_out, v_out, s);
 }
 
 // What coo_scan_kernel finds, as an error.
@@ -734,7 +753,7 @@ int is_sorted_dev(const int32_t* ri, const int32_t* ci, int64_t nnz, hipStream_t
 }
 
 // in-place stable (row, col) sort of COO arrays, if they are not in order;
-// check: with indices below 0 refused
+// check: with indices below 0 refused (the conversions carry such columns)
 int sort_coo(int64_t nnz, int32_t* ri, int32_t* ci, void* v, int vsize, bool check,
              hipStream_t s) {
   if (nnz <= 1) return MPH_OK;
@@ -742,8 +761,8 @@ int sort_coo(int64_t nnz, int32_t* ri, int32_t* ci, void* v, int vsize, bool che
   MPH_CHECK_STATUS(scan_order(ri, ci, nnz, s, flags));
   if (check) MPH_CHECK_STATUS(scan_status(flags[0]));
   if (!(flags[0] & kUnsorted)) return MPH_OK;
-  return radix_sort(nnz, bits_for(flags[1]), bits_for(flags[2]), true, ri, ci, v, vsize, ri, ci, v,
-                    s);
+  return radix_sort(nnz, bits_for(flags[1]), bits_for(flags[2]),
+                    (flags[0] & kBadCol) ? kLowBits : kByRowCol, ri, ci, v, vsize, ri, ci, v, s);
 }
 
 // ------------------------------------------------------------- emitters
@@ -1809,7 +1828,7 @@ int mph_convert_coo_to_csr(int64_t nrows, int64_t nnz, const int32_t* ri, const 
   // stable scatter by row in input order == stable sort by row
   int32_t* rows;
   MPH_CHECK_STATUS(t.alloc(&rows, nnz));
-  MPH_CHECK_STATUS(radix_sort(nnz, bits_for(nrows - 1), 0, false, ri, ci, v, vs, rows, ci_out,
+  MPH_CHECK_STATUS(radix_sort(nnz, bits_for(nrows - 1), 0, kByRow, ri, ci, v, vs, rows, ci_out,
                               v_out, s));
   hipLaunchKernelGGL((coo_scan_kernel<false, true, kNoDiags>), dim3(scan_blocks(nnz)), dim3(kT), 0,
                      s, rows, (const int32_t*)nullptr, nnz, nrows, (int64_t)INT32_MAX, ro_out,
@@ -2212,7 +2231,8 @@ int mph_convert_hdc_to_coo(int64_t nrows, int64_t ncols, int64_t nnz, int64_t nd
   MPH_HIP_CHECK(hipGetLastError());
   MPH_CHECK_STATUS(t.read(flags, &h));
   const bool sorted = !(h & kUnsorted);
-  if (sorted && ndiag > 0 && nrows > 0) {
+  bool in_order;
+  if (sorted && !(h & kBadCol) && ndiag > 0 && nrows > 0) {
     // both parts in order: the DIA part's entries, then both lists merged (a
     // DIA entry before the CSR entries of its row and column, as the stable
     // sort of the DIA entries followed by the CSR entries leaves them)
@@ -2232,6 +2252,7 @@ int mph_convert_hdc_to_coo(int64_t nrows, int64_t ncols, int64_t nnz, int64_t nd
     MPH_LAUNCH_BW(merge_rows_kernel, true, vs, dim3(blocks_for(csr_nnz)), s, crow, csr_ci, csr_v,
                   csr_nnz, rowpos, dci, ri_out, ci_out, v_out);
     MPH_HIP_CHECK(hipGetLastError());
+    in_order = true;
   } else {
     // the DIA part's entries, then the CSR part's
     MPH_CHECK_STATUS(emit_dia_part(nrows, ncols, ndiag, pitch, doff, dval, vt, nnz, ri_out, ci_out,
@@ -2241,8 +2262,9 @@ int mph_convert_hdc_to_coo(int64_t nrows, int64_t ncols, int64_t nnz, int64_t nd
     MPH_CHECK_STATUS(copy_dev(ci_out + nd, csr_ci, sizeof(int32_t) * csr_nnz, s));
     MPH_CHECK_STATUS(copy_dev(static_cast<uint8_t*>(v_out) + (size_t)vs * nd, csr_v,
                               (size_t)vs * csr_nnz, s));
+    in_order = sorted && nd == 0;
   }
-  if (nd + csr_nnz == nnz && sorted && (ndiag == 0 || nrows > 0)) return MPH_OK;
+  if (nd + csr_nnz == nnz && in_order) return MPH_OK;
   MPH_CHECK_STATUS(zero_tail(nd + csr_nnz, nnz, ri_out, ci_out, v_out, vs, s));
   return sort_coo(nnz, ri_out, ci_out, v_out, vs, false, s);
 }
