@@ -17,12 +17,15 @@ namespace mph {
 namespace {
 
 // Bad entries raise `bit` in flag[0]: eight indices a thread, loaded
-// together (one a thread took 22 us for 16M indices, 2.9 TB/s).
+// together (one a thread took 22 us for 16M indices, 2.9 TB/s).  Nothing is
+// read when a launch before this one raised a bit of `unless`: n is then not
+// known to be the array's length.
 constexpr int kCheckPer = 8;
 __global__ __launch_bounds__(256) void index_range_kernel(const int32_t* __restrict__ idx,
                                                           int64_t n, int64_t hi, int allow_m1,
-                                                          int32_t bit,
+                                                          int32_t bit, int32_t unless,
                                                           int32_t* __restrict__ flag) {
+  if (__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & unless) return;
   const int64_t base = (int64_t)blockIdx.x * 256 * kCheckPer + threadIdx.x;
   int32_t v[kCheckPer];
   bool ok = true;
@@ -47,9 +50,9 @@ __global__ __launch_bounds__(256) void row_offsets_kernel(const int32_t* __restr
 }
 
 void launch_index_range(const int32_t* idx, int64_t n, int64_t hi, bool allow_m1, int32_t bit,
-                        int32_t* flag, hipStream_t s) {
+                        int32_t unless, int32_t* flag, hipStream_t s) {
   hipLaunchKernelGGL(index_range_kernel, dim3((unsigned)ceil_div(n, 256 * kCheckPer)), dim3(256), 0,
-                     s, idx, n, hi, allow_m1 ? 1 : 0, bit, flag);
+                     s, idx, n, hi, allow_m1 ? 1 : 0, bit, unless, flag);
 }
 
 void launch_row_offsets(const int32_t* ro, int64_t nrows, int64_t nnz, int32_t bit, int32_t* flag,
@@ -78,7 +81,7 @@ int check_index_range(const int32_t* idx, int64_t n, int64_t hi, bool allow_m1,
   if (n <= 0) return MPH_OK;
   int bad = 0;
   MPH_CHECK_STATUS(run_flag_check(s, &bad, [&](int32_t* flag) {
-    launch_index_range(idx, n, hi, allow_m1, 1, flag, s);
+    launch_index_range(idx, n, hi, allow_m1, 1, 0, flag, s);
   }));
   if (bad) return invalid(std::string(what) + ": index out of range");
   return MPH_OK;
@@ -101,7 +104,8 @@ int check_csr(const int32_t* ro, int64_t nrows, int64_t nnz, const int32_t* ci, 
   int bad = 0;
   MPH_CHECK_STATUS(run_flag_check(s, &bad, [&](int32_t* flag) {
     launch_row_offsets(ro, nrows, nnz, 1, flag, s);
-    if (nnz > 0) launch_index_range(ci, nnz, ncols, false, 2, flag, s);
+    // (nnz columns only if the offsets end there)
+    if (nnz > 0) launch_index_range(ci, nnz, ncols, false, 2, 1, flag, s);
   }));
   if (bad & 1)
     return invalid("CSR row_offsets: row offsets must start at 0, not decrease and end at nnz");

@@ -89,3 +89,18 @@ def test_malformed_csr_is_refused(gpu, fault):
     with pytest.raises(capi.InvalidInputException):
         capi.call("mph_csr_multiply", 2000, 3000, A.nnz, _p(t[0]), _p(t[1]), _p(t[2]), capi.F64,
                   _p(x), _p(y), 1, device.stream_handle())
+
+
+@pytest.mark.parametrize("nnz", [8001, 2 ** 30])
+def test_columns_are_not_read_past_the_offsets(gpu, nnz):
+    """An nnz that the row offsets do not end at is refused by them, before a
+    column is read: the arrays hold 8000."""
+    import torch
+    A = _matrix([4] * 2000, 3000, 2)
+    ro, ci, v = (torch.from_numpy(a).cuda() for a in (
+        A.row_offsets.astype(np.int32), A.column_indices.astype(np.int32), A.values))
+    x = torch.zeros(3000, dtype=torch.float64, device="cuda")
+    y = torch.zeros(2000, dtype=torch.float64, device="cuda")
+    with pytest.raises(capi.InvalidInputException, match="row_offsets"):
+        capi.call("mph_csr_multiply", 2000, 3000, nnz, _p(ro), _p(ci), _p(v), capi.F64, _p(x),
+                  _p(y), 1, device.stream_handle())
