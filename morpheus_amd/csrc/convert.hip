@@ -746,6 +746,8 @@ int scan_order(const int32_t* ri, const int32_t* ci, int64_t nnz, hipStream_t s,
 
 int is_sorted_dev(const int32_t* ri, const int32_t* ci, int64_t nnz, hipStream_t s,
                   int* sorted) {
+  *sorted = 1;
+  if (nnz <= 1) return MPH_OK;  // (the arrays are not looked at)
   int32_t flags[3];
   MPH_CHECK_STATUS(scan_order(ri, ci, nnz, s, flags));
   *sorted = !(flags[0] & kUnsorted);

@@ -2,10 +2,13 @@
 entries, 32 slots a batch), bit-exact against the CPU oracle: entry counts and
 row counts around the tiles, long runs of empty rows, repeated and unsorted
 entries, diagonals in any order and repeated, sizes that leave phantom slots."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 import oracle
+from morpheus_amd import capi, device
 from morpheus_amd.formats import (COO_FORMAT, CSR_FORMAT, DIA_FORMAT, ELL_FORMAT, HDC_FORMAT,
                                   HYB_FORMAT, Coo, Dia)
 from tests.helpers import same_container
@@ -155,3 +158,11 @@ def test_unsorted_coo_to_csr_in_place(gpu, nnz):
     assert np.array_equal(ro.cpu().numpy(), ref.row_offsets)
     assert np.array_equal(ci.cpu().numpy(), ref.column_indices)
     assert np.array_equal(v.cpu().numpy(), ref.values)
+
+
+@pytest.mark.parametrize("nnz", [0, 1])
+def test_is_sorted_reads_no_pair(gpu, nnz):
+    """One entry is sorted; its arrays are not looked at."""
+    out = C.c_int(-1)
+    capi.call("mph_coo_is_sorted", nnz, None, None, C.byref(out), device.stream_handle())
+    assert out.value == 1
