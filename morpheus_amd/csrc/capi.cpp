@@ -18,23 +18,18 @@ std::mutex g_dev_mutex;
 int g_cu_count = 0;
 int g_cu_device = -1;
 
-// free blocks of temporaries, per device (-1: pinned host memory)
-struct TmpCache {
-  std::mutex m;
-  std::vector<std::pair<int, TmpBlock>> blocks;
-  size_t bytes = 0;
-};
 TmpCache& tmp_cache() {
   static TmpCache* c = new TmpCache;  // lives as long as the process
   return *c;
 }
 int tmp_device(bool host) {
+  if (host) return kTmpHost;
   int dev = 0;
-  if (host || hipGetDevice(&dev) != hipSuccess) return -1;
+  (void)hipGetDevice(&dev);
   return dev;
 }
 void tmp_release(const TmpBlock& b) {
-  if (b.host)
+  if (b.device == kTmpHost)
     (void)hipHostFree(b.p);
   else
     (void)hipFree(b.p);
@@ -44,41 +39,17 @@ void tmp_release(const TmpBlock& b) {
 void set_error(const std::string& msg) { g_last_error = msg; }
 
 int tmp_take(TmpBlock* b, size_t bytes, bool host) {
-  // sizes in steps of an eighth of their power of two, at least 4 KiB, so
-  // that calls of like size share blocks
-  size_t step = 4096;
-  while (step * 16 <= bytes) step <<= 1;
-  bytes = (bytes + step - 1) / step * step;
+  bytes = TmpCache::rounded(bytes);
   const int dev = tmp_device(host);
-  TmpCache& c = tmp_cache();
-  {
-    std::lock_guard<std::mutex> lk(c.m);
-    size_t best = c.blocks.size();
-    for (size_t i = 0; i < c.blocks.size(); i++) {
-      const TmpBlock& f = c.blocks[i].second;
-      if (c.blocks[i].first == dev && f.host == host && f.bytes >= bytes &&
-          f.bytes <= std::max<size_t>(4 * bytes, 1 << 16) &&
-          (best == c.blocks.size() || f.bytes < c.blocks[best].second.bytes))
-        best = i;
-    }
-    if (best < c.blocks.size()) {
-      *b = c.blocks[best].second;
-      c.bytes -= b->bytes;
-      c.blocks.erase(c.blocks.begin() + best);
-      return MPH_OK;
-    }
-  }
-  b->bytes = bytes;
-  b->host = host;
+  if (tmp_cache().take(dev, bytes, b)) return MPH_OK;
+  *b = TmpBlock{nullptr, bytes, dev};
+  hipError_t e = hipSuccess;
   auto get = [&]() {
-    return host ? hipHostMalloc(&b->p, bytes, hipHostMallocDefault) : hipMalloc(&b->p, bytes);
+    e = host ? hipHostMalloc(&b->p, bytes, hipHostMallocDefault) : hipMalloc(&b->p, bytes);
+    if (e == hipErrorOutOfMemory) (void)hipGetLastError();
+    return e != hipErrorOutOfMemory;
   };
-  hipError_t e = get();
-  if (e == hipErrorOutOfMemory) {
-    (void)hipGetLastError();
-    tmp_trim();
-    e = get();
-  }
+  (void)tmp_cache().get_or_trim(dev, get, tmp_release);
   if (e != hipSuccess) {
     b->p = nullptr;
     set_error(std::string("temporary: ") + hipGetErrorString(e));
@@ -87,30 +58,9 @@ int tmp_take(TmpBlock* b, size_t bytes, bool host) {
   return MPH_OK;
 }
 
-void tmp_give(const TmpBlock& b) {
-  const int dev = tmp_device(b.host);
-  TmpCache& c = tmp_cache();
-  {
-    std::lock_guard<std::mutex> lk(c.m);
-    if (c.bytes + b.bytes <= kTmpKeepBytes && c.blocks.size() < kTmpKeepBlocks) {
-      c.blocks.emplace_back(dev, b);
-      c.bytes += b.bytes;
-      return;
-    }
-  }
-  tmp_release(b);
-}
+void tmp_give(const TmpBlock& b) { tmp_cache().give(b, tmp_release); }
 
-void tmp_trim() {
-  TmpCache& c = tmp_cache();
-  std::vector<std::pair<int, TmpBlock>> out;
-  {
-    std::lock_guard<std::mutex> lk(c.m);
-    out.swap(c.blocks);
-    c.bytes = 0;
-  }
-  for (auto& f : out) tmp_release(f.second);
-}
+void tmp_trim() { tmp_cache().trim_all(tmp_release); }
 
 int device_cu_count() {
   int dev = 0;

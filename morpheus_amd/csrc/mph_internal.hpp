@@ -7,6 +7,7 @@
 #include <vector>
 
 #include "mph_common.hpp"
+#include "tmp_cache.hpp"
 
 namespace mph {
 
@@ -16,15 +17,8 @@ namespace mph {
 // allocation and up to 1.1 ms a release, 3 ms of a 5.4 ms CSR -> HYB -> CSR
 // round trip of 16M entries.  A block goes back to the cache only after its
 // stream has been synchronised, so any thread and stream may take it next;
-// the cache holds at most kTmpKeepBytes in kTmpKeepBlocks blocks a device,
-// and mph_finalize, or an allocation that fails, gives them back.
-constexpr size_t kTmpKeepBytes = (size_t)2 << 30;
-constexpr size_t kTmpKeepBlocks = 48;
-struct TmpBlock {
-  void* p = nullptr;
-  size_t bytes = 0;
-  bool host = false;  // pinned host memory
-};
+// the cache is bounded (tmp_cache.hpp), and mph_finalize, or an allocation of
+// a temporary that fails, gives its blocks back.
 int tmp_take(TmpBlock* b, size_t bytes, bool host);
 void tmp_give(const TmpBlock& b);
 void tmp_trim();
