@@ -376,7 +376,7 @@ int mph_i32_stats(const int32_t* v, int64_t n, double mean, int32_t threshold,
   const int64_t chunk = std::max<int64_t>(kT * 16, ceil_div(n, (int64_t)1024));
   const int64_t nparts = ceil_div(n, chunk);
   I32Part* d = nullptr;
-  MPH_HIP_CHECK(hipMalloc(&d, sizeof(I32Part) * (nparts + 1)));
+  MPH_HIP_CHECK(dmalloc(&d, sizeof(I32Part) * (nparts + 1)));
   hipLaunchKernelGGL(i32_stats_kernel, dim3((unsigned)nparts), dim3(kT), 0, s, v, n, chunk, mean,
                      threshold, d);
   hipLaunchKernelGGL(i32_stats_final_kernel, dim3(1), dim3(kT), 0, s, d, nparts, d + nparts);

@@ -49,7 +49,7 @@ struct DevBuf {
   void* p = nullptr;
   ~DevBuf() { dfree(p); }
   int alloc(size_t bytes) {
-    MPH_HIP_CHECK(hipMalloc(&p, std::max<size_t>(bytes, 16)));
+    MPH_HIP_CHECK(dmalloc(&p, std::max<size_t>(bytes, 16)));
     return MPH_OK;
   }
 };

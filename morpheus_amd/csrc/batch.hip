@@ -951,7 +951,7 @@ int mph_batch_create(mph_batch_t* out, int32_t nmat, const mph_matrix_t* mats, i
       MPH_CHECK_STATUS(rows_sorted(A->coo_ri, A->coo_nnz, A->nrows, s, &sorted));
       if (!sorted) return invalid("a COO matrix with unsorted rows cannot be batched");
       int32_t* d_ro = nullptr;
-      MPH_HIP_CHECK(hipMalloc(&d_ro, sizeof(int32_t) * (A->nrows + 1)));
+      MPH_HIP_CHECK(dmalloc(&d_ro, sizeof(int32_t) * (A->nrows + 1)));
       owned.push_back(d_ro);
       MPH_CHECK_STATUS(coo_row_offsets(A->coo_ri, A->coo_nnz, A->nrows, d_ro, s));
       m.ro = d_ro;
@@ -1025,15 +1025,15 @@ int mph_batch_create(mph_batch_t* out, int32_t nmat, const mph_matrix_t* mats, i
   b->ntiles = (int32_t)ts.tiles.size();
   b->ncomp = (int32_t)ts.comp.size();
   hipError_t e = hipSuccess;
-  if (b->ntiles > 0) e = hipMalloc(&b->d_tiles, sizeof(BatchTile) * b->ntiles);
+  if (b->ntiles > 0) e = dmalloc(&b->d_tiles, sizeof(BatchTile) * b->ntiles);
   if (e == hipSuccess && b->ntiles > 0)
     e = hipMemcpyAsync(b->d_tiles, ts.tiles.data(), sizeof(BatchTile) * b->ntiles,
                        hipMemcpyHostToDevice, s);
-  if (e == hipSuccess && !ts.rows.empty()) e = hipMalloc(&b->d_rows, sizeof(int32_t) * ts.rows.size());
+  if (e == hipSuccess && !ts.rows.empty()) e = dmalloc(&b->d_rows, sizeof(int32_t) * ts.rows.size());
   if (e == hipSuccess && !ts.rows.empty())
     e = hipMemcpyAsync(b->d_rows, ts.rows.data(), sizeof(int32_t) * ts.rows.size(),
                        hipMemcpyHostToDevice, s);
-  if (e == hipSuccess && b->ncomp > 0) e = hipMalloc(&b->d_comp, sizeof(BatchTile) * b->ncomp);
+  if (e == hipSuccess && b->ncomp > 0) e = dmalloc(&b->d_comp, sizeof(BatchTile) * b->ncomp);
   if (e == hipSuccess && b->ncomp > 0)
     e = hipMemcpyAsync(b->d_comp, ts.comp.data(), sizeof(BatchTile) * b->ncomp,
                        hipMemcpyHostToDevice, s);

@@ -38,18 +38,35 @@ void tmp_release(const TmpBlock& b) {
 
 void set_error(const std::string& msg) { g_last_error = msg; }
 
+namespace {
+// an allocation that, where memory runs out, gets the temporaries held
+template <typename Alloc>
+hipError_t alloc_or_trim(int dev, Alloc alloc) {
+  hipError_t e = hipSuccess;
+  (void)tmp_cache().get_or_trim(
+      dev,
+      [&]() {
+        e = alloc();
+        if (e == hipErrorOutOfMemory) (void)hipGetLastError();
+        return e != hipErrorOutOfMemory;
+      },
+      tmp_release);
+  return e;
+}
+}  // namespace
+
+hipError_t dmalloc_bytes(void** p, size_t bytes) {
+  return alloc_or_trim(tmp_device(false), [&]() { return hipMalloc(p, bytes); });
+}
+
 int tmp_take(TmpBlock* b, size_t bytes, bool host) {
   bytes = TmpCache::rounded(bytes);
   const int dev = tmp_device(host);
   if (tmp_cache().take(dev, bytes, b)) return MPH_OK;
   *b = TmpBlock{nullptr, bytes, dev};
-  hipError_t e = hipSuccess;
-  auto get = [&]() {
-    e = host ? hipHostMalloc(&b->p, bytes, hipHostMallocDefault) : hipMalloc(&b->p, bytes);
-    if (e == hipErrorOutOfMemory) (void)hipGetLastError();
-    return e != hipErrorOutOfMemory;
-  };
-  (void)tmp_cache().get_or_trim(dev, get, tmp_release);
+  const hipError_t e = alloc_or_trim(dev, [&]() {
+    return host ? hipHostMalloc(&b->p, bytes, hipHostMallocDefault) : hipMalloc(&b->p, bytes);
+  });
   if (e != hipSuccess) {
     b->p = nullptr;
     set_error(std::string("temporary: ") + hipGetErrorString(e));
@@ -84,7 +101,7 @@ int plan_alloc(mph_matrix_impl* A, void** p, size_t bytes) {
     *p = b.p;
     return MPH_OK;
   }
-  MPH_HIP_CHECK(hipMalloc(p, bytes));
+  MPH_HIP_CHECK(dmalloc(p, bytes));
   return MPH_OK;
 }
 

@@ -65,7 +65,7 @@ int mph_index_narrow(const int64_t* src, int64_t n, int32_t* dst, mph_stream_t s
   if (n < 0 || (n > 0 && (!src || !dst))) return invalid("mph_index_narrow: bad arguments");
   if (n == 0) return MPH_OK;
   int32_t* bad = nullptr;
-  MPH_HIP_CHECK(hipMalloc(&bad, sizeof(int32_t)));
+  MPH_HIP_CHECK(dmalloc(&bad, sizeof(int32_t)));
   int32_t flag = 0;
   hipLaunchKernelGGL(clear_flag_kernel, dim3(1), dim3(1), 0, s, bad);
   hipError_t e = hipGetLastError();

@@ -271,6 +271,14 @@ inline int runtime_error(const std::string& msg) {
   return MPH_ERR_RUNTIME;
 }
 
+// hipMalloc on the current device; when memory has run out, the temporaries
+// that the library holds there (tmp_cache.hpp) are given back first
+hipError_t dmalloc_bytes(void** p, size_t bytes);
+template <typename T>
+inline hipError_t dmalloc(T** p, size_t bytes) {
+  return dmalloc_bytes(reinterpret_cast<void**>(p), bytes);
+}
+
 // device free whose status is deliberately ignored (release paths)
 inline void dfree(void* p) {
   if (p) (void)hipFree(p);

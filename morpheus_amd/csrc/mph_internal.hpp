@@ -17,8 +17,8 @@ namespace mph {
 // allocation and up to 1.1 ms a release, 3 ms of a 5.4 ms CSR -> HYB -> CSR
 // round trip of 16M entries.  A block goes back to the cache only after its
 // stream has been synchronised, so any thread and stream may take it next;
-// the cache is bounded (tmp_cache.hpp), and mph_finalize, or an allocation of
-// a temporary that fails, gives its blocks back.
+// the cache is bounded (tmp_cache.hpp), and mph_finalize, or any allocation of
+// the library that finds no memory, gives its blocks back.
 int tmp_take(TmpBlock* b, size_t bytes, bool host);
 void tmp_give(const TmpBlock& b);
 void tmp_trim();

@@ -337,7 +337,7 @@ int coo_xtile_analyse(mph_matrix_impl* A, hipStream_t s) {
   const bool on = mode == 2 || (mode == 0 && (int64_t)A->ncols * (int64_t)vec_bytes >= kXTileMinXBytes);
   if (!on || nnz == 0 || nrows == 0 || A->ncols == 0) return MPH_OK;
   int32_t* d_ro = nullptr;
-  MPH_HIP_CHECK(hipMalloc(&d_ro, sizeof(int32_t) * (nrows + 1)));
+  MPH_HIP_CHECK(dmalloc(&d_ro, sizeof(int32_t) * (nrows + 1)));
   std::vector<int32_t> ro(nrows + 1);
   int st = coo_row_offsets(A->coo_ri, nnz, nrows, d_ro, s);
   if (st == MPH_OK &&
@@ -386,7 +386,7 @@ int coo_xtile_analyse(mph_matrix_impl* A, hipStream_t s) {
   p.nblocks = (int32_t)ceil_div(p.nchunks, (int64_t)(256 / kWave));
   p.prezero = true;
   if (!ch.empty()) {
-    MPH_HIP_CHECK(hipMalloc(&p.chunks, sizeof(CooChunk) * ch.size()));
+    MPH_HIP_CHECK(dmalloc(&p.chunks, sizeof(CooChunk) * ch.size()));
     MPH_HIP_CHECK(hipMemcpyAsync(p.chunks, ch.data(), sizeof(CooChunk) * ch.size(),
                                  hipMemcpyHostToDevice, s));
     MPH_HIP_CHECK(hipStreamSynchronize(s));
@@ -413,7 +413,7 @@ int coo_analyse(mph_matrix_impl* A, hipStream_t s) {
   p.prezero = false;
   if (A->nnz > 0 && sorted) {
     int32_t* g = nullptr;
-    MPH_HIP_CHECK(hipMalloc(&g, sizeof(int32_t)));
+    MPH_HIP_CHECK(dmalloc(&g, sizeof(int32_t)));
     int st = fill_zero(g, sizeof(int32_t), s);
     if (st == MPH_OK) {
       hipLaunchKernelGGL(coo_gap_kernel, dim3((unsigned)ceil_div(A->nnz + 1, 256)),
@@ -430,8 +430,8 @@ int coo_analyse(mph_matrix_impl* A, hipStream_t s) {
   const size_t acc = A->vt == MPH_F64 ? 8 : 4;
   const size_t pair = A->vt == MPH_F64 ? 1 : 2;  // compensated pairs in FP32
   const size_t n = (size_t)std::max<int64_t>(p.nchunks, 1);
-  MPH_HIP_CHECK(hipMalloc(&p.first_val, acc * pair * n));
-  MPH_HIP_CHECK(hipMalloc(&p.last_val, acc * pair * n));
+  MPH_HIP_CHECK(dmalloc(&p.first_val, acc * pair * n));
+  MPH_HIP_CHECK(dmalloc(&p.last_val, acc * pair * n));
   MPH_HIP_CHECK(hipStreamSynchronize(s));
   return MPH_OK;
 }

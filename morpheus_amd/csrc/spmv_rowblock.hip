@@ -1819,9 +1819,9 @@ int xtile_build(mph_matrix_impl* A, const std::vector<int32_t>& ro, const int32_
     bnd.assign((size_t)nl * (ntiles + 1), 0);
     int32_t *d_rows = nullptr, *d_bnd = nullptr, *d_uns = nullptr;
     int st = MPH_OK;
-    if (hipMalloc(&d_rows, sizeof(int32_t) * nl) != hipSuccess ||
-        hipMalloc(&d_bnd, sizeof(int32_t) * bnd.size()) != hipSuccess ||
-        hipMalloc(&d_uns, sizeof(int32_t) * nl) != hipSuccess) {
+    if (dmalloc(&d_rows, sizeof(int32_t) * nl) != hipSuccess ||
+        dmalloc(&d_bnd, sizeof(int32_t) * bnd.size()) != hipSuccess ||
+        dmalloc(&d_uns, sizeof(int32_t) * nl) != hipSuccess) {
       set_error("hipMalloc failed in the x-tile analysis");
       st = MPH_ERR_OUT_OF_MEMORY;
     }
@@ -2023,17 +2023,17 @@ int xtile_build(mph_matrix_impl* A, const std::vector<int32_t>& ro, const int32_
     dfree(d_part);
     dfree(d_rpos);
   };
-  if (hipMalloc(&d_row, sizeof(int32_t) * nt) != hipSuccess ||
-      hipMalloc(&d_lro, sizeof(int32_t) * lro.size()) != hipSuccess ||
-      hipMalloc(&d_ss, sizeof(int32_t) * sub_start.size()) != hipSuccess ||
-      hipMalloc(&d_tb, sizeof(int32_t) * tb.size()) != hipSuccess ||
-      hipMalloc(&d_rs, sizeof(int32_t) * run_sub.size()) != hipSuccess ||
-      hipMalloc(&d_sub, sizeof(XTSub) * subs.size()) != hipSuccess ||
-      hipMalloc(&d_head, head.size()) != hipSuccess ||
-      hipMalloc(&d_col, sizeof(uint16_t) * std::max<int64_t>(slots, 1)) != hipSuccess ||
-      (!direct && hipMalloc(&d_cv, vsz * std::max<int64_t>(slots, 1)) != hipSuccess) ||
-      (direct && hipMalloc(&d_rpos, sizeof(int32_t) * rpos.size()) != hipSuccess) ||
-      hipMalloc(&d_part, acc * pair * (size_t)ntiles * nt) != hipSuccess) {
+  if (dmalloc(&d_row, sizeof(int32_t) * nt) != hipSuccess ||
+      dmalloc(&d_lro, sizeof(int32_t) * lro.size()) != hipSuccess ||
+      dmalloc(&d_ss, sizeof(int32_t) * sub_start.size()) != hipSuccess ||
+      dmalloc(&d_tb, sizeof(int32_t) * tb.size()) != hipSuccess ||
+      dmalloc(&d_rs, sizeof(int32_t) * run_sub.size()) != hipSuccess ||
+      dmalloc(&d_sub, sizeof(XTSub) * subs.size()) != hipSuccess ||
+      dmalloc(&d_head, head.size()) != hipSuccess ||
+      dmalloc(&d_col, sizeof(uint16_t) * std::max<int64_t>(slots, 1)) != hipSuccess ||
+      (!direct && dmalloc(&d_cv, vsz * std::max<int64_t>(slots, 1)) != hipSuccess) ||
+      (direct && dmalloc(&d_rpos, sizeof(int32_t) * rpos.size()) != hipSuccess) ||
+      dmalloc(&d_part, acc * pair * (size_t)ntiles * nt) != hipSuccess) {
     release();
     set_error("hipMalloc failed in the x-tile analysis");
     return MPH_ERR_OUT_OF_MEMORY;
@@ -2156,7 +2156,7 @@ int ell_counts(mph_matrix_impl* A, hipStream_t s) {
   const int64_t nrows = A->nrows, loop = A->ell_loop;
   if (loop <= 0 || loop > 255 || nrows == 0) return MPH_OK;
   uint8_t* d = nullptr;
-  MPH_HIP_CHECK(hipMalloc(&d, (size_t)nrows));
+  MPH_HIP_CHECK(dmalloc(&d, (size_t)nrows));
   hipLaunchKernelGGL(ell_count_kernel, dim3((unsigned)ceil_div(nrows, 256)), dim3(256), 0, s,
                      A->ell_ci, A->ell_pitch, loop, nrows, d);
   std::vector<uint8_t> h(nrows);
@@ -2290,12 +2290,12 @@ int split_analyse(mph_matrix_impl* A, const int32_t* d_ro, hipStream_t s) {
   int32_t* d_lro = nullptr;
   const int accs = (A->vt == MPH_F64 ? 8 : 4);
   const bool grow = (int64_t)sb.size() > (int64_t)p.nblocks + 1;
-  bool fail = hipMalloc(&d_sb, sizeof(RowBlock) * sb.size()) != hipSuccess ||
-              hipMalloc(&d_kr, sizeof(int32_t) * 4 * sb.size()) != hipSuccess ||
-              (grow && hipMalloc(&d_part, (size_t)accs * 32 * sb.size()) != hipSuccess);
+  bool fail = dmalloc(&d_sb, sizeof(RowBlock) * sb.size()) != hipSuccess ||
+              dmalloc(&d_kr, sizeof(int32_t) * 4 * sb.size()) != hipSuccess ||
+              (grow && dmalloc(&d_part, (size_t)accs * 32 * sb.size()) != hipSuccess);
   if (!fail && split)
-    fail = hipMalloc(&d_map, sizeof(int32_t) * (size_t)std::max<int64_t>(m, 1)) != hipSuccess ||
-           hipMalloc(&d_lro, sizeof(int32_t) * (size_t)(m + 1)) != hipSuccess;
+    fail = dmalloc(&d_map, sizeof(int32_t) * (size_t)std::max<int64_t>(m, 1)) != hipSuccess ||
+           dmalloc(&d_lro, sizeof(int32_t) * (size_t)(m + 1)) != hipSuccess;
   if (fail) {
     dfree(d_sb);
     dfree(d_kr);
@@ -2389,9 +2389,9 @@ int hyb_merge(mph_matrix_impl* A, hipStream_t s) {
     dfree(tmp);
     return st;
   };
-  if (hipMalloc(&cnt, sizeof(int32_t) * nrows) != hipSuccess ||
-      hipMalloc(&mro, sizeof(int32_t) * (nrows + 1)) != hipSuccess ||
-      hipMalloc(&tmp, sizeof(int64_t) * scan_tmp_elems(nrows)) != hipSuccess) {
+  if (dmalloc(&cnt, sizeof(int32_t) * nrows) != hipSuccess ||
+      dmalloc(&mro, sizeof(int32_t) * (nrows + 1)) != hipSuccess ||
+      dmalloc(&tmp, sizeof(int64_t) * scan_tmp_elems(nrows)) != hipSuccess) {
     set_error("hipMalloc failed in the HYB merge analysis");
     return fail(MPH_ERR_OUT_OF_MEMORY);
   }
@@ -2430,8 +2430,8 @@ int hyb_merge(mph_matrix_impl* A, hipStream_t s) {
     if (tail_rows * kHybMergeTailRows <= nrows) return fail(MPH_OK);
   }
   const size_t vs = value_size(A->vt);
-  if (hipMalloc(&p.m_ci, sizeof(int32_t) * std::max<int64_t>(total, 1)) != hipSuccess ||
-      hipMalloc(&p.m_val, vs * std::max<int64_t>(total, 1)) != hipSuccess) {
+  if (dmalloc(&p.m_ci, sizeof(int32_t) * std::max<int64_t>(total, 1)) != hipSuccess ||
+      dmalloc(&p.m_val, vs * std::max<int64_t>(total, 1)) != hipSuccess) {
     dfree(p.m_ci);
     dfree(p.m_val);
     p.m_ci = nullptr;
@@ -2872,7 +2872,7 @@ int xtile_multiply_k_t(mph_matrix_impl* A, XTilePlan& xp, const void* x, void* y
   if (xp.partial_k_cols < KR) {
     void* d = nullptr;
     const size_t bytes = sizeof(Acc) * (comp ? 2 : 1) * (size_t)xp.ntiles * (size_t)xp.rows * KR;
-    MPH_HIP_CHECK(hipMalloc(&d, bytes));
+    MPH_HIP_CHECK(dmalloc(&d, bytes));
     const hipError_t e = hipFuncSetAttribute(
         reinterpret_cast<const void*>(&xtile_kernel_k<V, comp, KR, kXTileKThreads>),
         hipFuncAttributeMaxDynamicSharedMemorySize, (int)xlds);

@@ -271,7 +271,7 @@ template <typename Vec>
 int dot_t(int64_t n, const void* x, const void* y, double* out, hipStream_t s) {
   const int64_t np = parts_for(n), chunk = chunk_for(n, np);
   double* d = nullptr;
-  MPH_HIP_CHECK(hipMalloc(&d, sizeof(double) * (np + 1)));
+  MPH_HIP_CHECK(dmalloc(&d, sizeof(double) * (np + 1)));
   launch_dot_parts<Vec>(x, y, n, np, chunk, d, s);
   hipLaunchKernelGGL(sum_parts_kernel, dim3(1), dim3(kT), 0, s, d, np, d + np);
   hipError_t e = hipGetLastError();
@@ -286,7 +286,7 @@ template <typename Vec>
 int reduce_t(int64_t n, const void* x, double* out, hipStream_t s) {
   const int64_t np = parts_for(n), chunk = chunk_for(n, np);
   double* d = nullptr;
-  MPH_HIP_CHECK(hipMalloc(&d, sizeof(double) * (np + 1)));
+  MPH_HIP_CHECK(dmalloc(&d, sizeof(double) * (np + 1)));
   hipLaunchKernelGGL((reduce_parts_kernel<Vec>), dim3((unsigned)np), dim3(kT), 0, s,
                      static_cast<const Vec*>(x), n, chunk, d);
   hipLaunchKernelGGL(sum_parts_kernel, dim3(1), dim3(kT), 0, s, d, np, d + np);
@@ -424,9 +424,9 @@ int mph_cg_create(mph_cg_t* out, mph_matrix_t A) {
   c->chunk = chunk_for(c->n, c->np);
   const size_t vs = c->vt == MPH_F64 ? 8 : 4;
   const size_t vb = vs * (size_t)std::max<int64_t>(c->n, 1);
-  if (hipMalloc(&c->r, vb) != hipSuccess || hipMalloc(&c->p, vb) != hipSuccess ||
-      hipMalloc(&c->q, vb) != hipSuccess ||
-      hipMalloc(&c->parts, sizeof(double) * (2 * c->np + kCgState)) != hipSuccess) {
+  if (dmalloc(&c->r, vb) != hipSuccess || dmalloc(&c->p, vb) != hipSuccess ||
+      dmalloc(&c->q, vb) != hipSuccess ||
+      dmalloc(&c->parts, sizeof(double) * (2 * c->np + kCgState)) != hipSuccess) {
     mph_cg_destroy(c);
     set_error("hipMalloc failed in mph_cg_create");
     return MPH_ERR_OUT_OF_MEMORY;

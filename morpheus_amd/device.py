@@ -258,12 +258,21 @@ def multiply(A: DeviceMatrix, x, y, init: bool = True, stream=None) -> None:
 _VSIZE = {"f64": 8, "f32": 4, "bf16": 2}
 
 
+def _empty(n, dtype):
+    n = max(int(n), 0)
+    try:
+        return torch.empty(n, dtype=dtype, device="cuda")
+    except torch.OutOfMemoryError:
+        capi.call("mph_finalize")  # the temporaries that the library holds
+        return torch.empty(n, dtype=dtype, device="cuda")
+
+
 def _empty_i(n):
-    return torch.empty(max(int(n), 0), dtype=torch.int32, device="cuda")
+    return _empty(n, torch.int32)
 
 
 def _empty_v(n, dtype):
-    return torch.empty(max(int(n), 0), dtype=DTYPES[dtype][0], device="cuda")
+    return _empty(n, DTYPES[dtype][0])
 
 
 def to_coo(A: DeviceMatrix, stream=None, share: bool = False) -> DeviceMatrix:

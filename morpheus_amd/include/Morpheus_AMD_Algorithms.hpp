@@ -123,7 +123,7 @@ inline void copy_sparse(const S& src, D& dst) {
 struct DevBuf {
   void* p = nullptr;
   explicit DevBuf(size_t bytes) {
-    if (bytes) hip_check(hipMalloc(&p, bytes), "Morpheus: device scratch");
+    if (bytes) hip_check(device_malloc(&p, bytes), "Morpheus: device scratch");
   }
   ~DevBuf() {
     if (p) (void)hipFree(p);

@@ -59,6 +59,17 @@ inline void hip_check(hipError_t e, const char* what) {
     throw RuntimeException(std::string(what) + ": " + hipGetErrorString(e));
 }
 
+// hipMalloc; when memory has run out, the temporaries that the library holds
+// are given back first
+inline hipError_t device_malloc(void** p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e == hipErrorOutOfMemory && mph_finalize() == MPH_OK) {
+    (void)hipGetLastError();
+    e = hipMalloc(p, bytes);
+  }
+  return e;
+}
+
 // core/src/impl/Dia/Morpheus_Utils_Impl.hpp:33-36
 template <typename T>
 inline T get_pad_size(T len, T alignment) {
@@ -225,7 +236,7 @@ class Array {
     }
     if constexpr (Mem::is_device) {
       void* p = nullptr;
-      hip_check(hipMalloc(&p, n * sizeof(T)), "hipMalloc");
+      hip_check(device_malloc(&p, n * sizeof(T)), "hipMalloc");
       hip_check(hipMemset(p, 0, n * sizeof(T)), "hipMemset");
       ptr_ = std::shared_ptr<T>(static_cast<T*>(p), [](T* q) { (void)hipFree(q); });
     } else {
