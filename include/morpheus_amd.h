@@ -178,16 +178,15 @@ int mph_matrix_plan_bytes(mph_matrix_t A, int init, int64_t* bytes);
  *                  the clusters average 8 diagonals or more.  The
  *                  environment variable MPH_DIA_STAGE, read at analysis,
  *                  sets 0 = no staging, 1 = the one-row kernels only.
- *                  The results do not depend on it.  DIA SpMM with 4 or
- *                  more lanes per row (FP64 from 8 columns per pass, FP32 /
- *                  BF16 from 16), or 2 where the runs of diagonals with
- *                  consecutive offsets average two or more, and rows enough
- *                  to fill the device (about 384 workgroups in FP64, 768 in
- *                  FP32 / BF16, of 1024 / lanes rows), takes 4
- *                  consecutive rows per lane group and loads, per run, the X
- *                  rows it covers and its values once, through LDS
- *                  (MPH_DIA_SPMM_RUNS=0 / 1 forces that off / on; the
- *                  results are the same bits).
+ *                  The results do not depend on it.  DIA SpMM with 2 or
+ *                  more lanes per row (FP64 from 4 columns per pass, FP32 /
+ *                  BF16 from 8) may take 4 consecutive rows per lane group,
+ *                  which share the X rows of each run of diagonals with
+ *                  consecutive offsets, loaded by each lane or staged in LDS
+ *                  by the workgroup, by the size of the matrix and the
+ *                  length of its runs (MPH_DIA_SPMM_RUNS=0 forces one row
+ *                  per group, 1 the staged form, 2 the other; the results
+ *                  are the same bits).
  *   xtile        : x-tiled long rows of CSR / COO / HYB / HDC SpMV (1 = off,
  *                  2 = on; 0 = on when x exceeds 2 MiB).  Rows longer than
  *                  512 entries with sorted columns are summed per 32 KiB tile

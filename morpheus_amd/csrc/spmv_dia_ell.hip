@@ -16,9 +16,9 @@
 // beyond entries_per_row hold only the -1 padding.  FP32 / BF16 DIA SpMV takes
 // two adjacent rows per thread (row-pair kernels below); FP32 / BF16 rows of
 // more than kCompensateLen diagonals / slots take a Dot2-compensated kernel.
-// SpMM gives each row a lane group (16 bytes of its columns per lane); with
-// 4 or more lanes per row DIA gives each group 4 consecutive rows and loads
-// the X rows of each run of consecutive diagonals once.  A split FP64 HDC
+// SpMM gives each row a lane group (16 bytes of its columns per lane); DIA may
+// give each group 4 consecutive rows, which share the X rows of each run of
+// consecutive diagonals (dia_spmm_form).  A split FP64 HDC
 // whose CSR rows are short adds them in the staged DIA pass.
 #include <algorithm>
 #include <cstdlib>
@@ -459,15 +459,104 @@ __global__ __launch_bounds__(256) void dia_spmm_kernel(DiaArgs<V> a) {
   *yp = out;
 }
 
-// DIA SpMM with R consecutive rows per lane group (R = 4): for each run of
-// diagonals whose offsets step by one (o, o + 1, ..., at most kDiaRunMax),
-// the workgroup loads the X rows the run covers, and the run's values for its
-// rows, once and coalesced, and hands them over through LDS; each lane reads
-// its R + m - 1 X pieces from there and slides over them.  Each row still
-// sums its diagonals in storage order, as dia_spmm_kernel does, with the same
-// skips, so the two give identical results.  Loads are unconditional (columns
-// outside x read a column inside, a row past the matrix its last row);
-// products are selected only where a workgroup's columns leave x.
+// DIA SpMM with R consecutive rows per lane group (R = 4), in two forms.  For
+// each run of diagonals whose offsets step by one (o, o + 1, ..., at most
+// kDiaRunMax), a group loads the R + m - 1 X pieces that the run covers once
+// and slides over them, instead of one X piece per row and diagonal (the
+// 27-point stencil: 6 X loads for 4 rows x 3 diagonals instead of 12).  Each
+// row still sums its diagonals in storage order, as dia_spmm_kernel does, with
+// the same skips, so all give identical results.  Loads are unconditional
+// (columns outside x read a column inside, a row past the matrix its last
+// row).  Which form runs where: dia_spmm_form.
+constexpr int kDiaRunMax = 3;
+constexpr int kDiaSpmmRows = 4;  // R
+
+// The slide form: each lane loads its X pieces itself, the run's values come
+// through LDS (loaded by the whole workgroup, so no lane group leaves before
+// the end).  Nothing is requested ahead: a run costs two round trips, but many
+// workgroups fit a CU, so it wins where the staged form's few would not fill
+// the device.
+template <typename V, int KL, int R>
+__global__ __launch_bounds__(256) void dia_spmm_slide_kernel(DiaArgs<V> a) {
+  using Acc = typename vtraits<V>::acc;
+  using Vec = typename vtraits<V>::vec;
+  using P = Piece<Vec>;
+  constexpr int Q = P::Q;
+  constexpr int W = R + kDiaRunMax - 1;
+  constexpr int kRows = 256 / KL * R;  // rows of the workgroup
+  // the run's values for the workgroup's rows, loaded by all its threads in
+  // one coalesced pass per diagonal (each lane then reads its R rows'
+  // values from here instead of R loads of its own)
+  __shared__ V s_val[kDiaRunMax][kRows];
+  const uint32_t b = xcd_remap(blockIdx.x, gridDim.x);
+  const int64_t wr0 = (int64_t)b * kRows;
+  const int gl = threadIdx.x / KL;
+  const int64_t row0 = wr0 + (int64_t)gl * R;
+  const int l = threadIdx.x % KL;
+  const int64_t last = a.nrows - 1;
+  Acc t[R][Q];
+#pragma unroll
+  for (int i = 0; i < R; i++)
+#pragma unroll
+    for (int q = 0; q < Q; q++) t[i][q] = 0;
+  for (int d = 0; d < a.ndiag;) {
+    const int64_t o = a.off[d];
+    int m = 1;
+    while (m < kDiaRunMax && d + m < a.ndiag && (int64_t)a.off[d + m] == o + m) m++;
+    // the X rows first: the value stores below wait for every older load
+    typename P::T xw[W];
+#pragma unroll
+    for (int i = 0; i < W; i++) {
+      const int64_t col = row0 + o + i;
+      const bool in = i < R + m - 1 && col >= 0 && col < a.ncols;
+      xw[i] = *reinterpret_cast<const typename P::T*>(a.x + (in ? col : 0) * a.ld + l * Q);
+    }
+    __syncthreads();  // the previous run's values are read
+    for (int j = 0; j < m; j++)
+      for (int e = threadIdx.x; e < kRows; e += 256)
+        s_val[j][e] = ld_stream(a.val + a.pitch * (d + j) + min(wr0 + e, last));
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kDiaRunMax; j++) {
+      if (j < m) {
+#pragma unroll
+        for (int i = 0; i < R; i++) {
+          const int64_t col = row0 + i + o + j;
+          const bool ok = row0 + i < a.nrows && col >= 0 && col < a.ncols;
+          const Acc vw = vtraits<V>::widen(s_val[j][gl * R + i]);
+#pragma unroll
+          for (int q = 0; q < Q; q++) {
+            const Acc f = t[i][q] + vw * (Acc)xw[i + j][q];
+            t[i][q] = ok ? f : t[i][q];
+          }
+        }
+      }
+    }
+    d += m;
+  }
+#pragma unroll
+  for (int i = 0; i < R; i++) {
+    const int64_t row = row0 + i;
+    if (row < a.nrows) {
+      typename P::T* yp = reinterpret_cast<typename P::T*>(a.y + row * a.ld + l * Q);
+      typename P::T out;
+      if (a.init) {
+#pragma unroll
+        for (int q = 0; q < Q; q++) out[q] = (Vec)t[i][q];
+      } else {
+        const typename P::T old = *yp;
+#pragma unroll
+        for (int q = 0; q < Q; q++) out[q] = (Vec)((Acc)old[q] + t[i][q]);
+      }
+      *yp = out;
+    }
+  }
+}
+
+// The staged form: the workgroup loads the X rows of the run too, once and
+// coalesced, and hands them over through LDS; each lane reads its R + m - 1 X
+// pieces from there.  Products are selected only where a workgroup's columns
+// leave x.
 //
 // What bounds it: the L1.  With every lane loading its own X pieces the L1
 // served each X row three times a run and stood still half of the time on
@@ -480,8 +569,6 @@ __global__ __launch_bounds__(256) void dia_spmm_kernel(DiaArgs<V> a) {
 // FP64: 16 columns 632 -> 537 us (3.6 TB/s of X, Y and values once each), 8
 // columns 412 -> 324 us; FP32, 16 columns 365 -> 293 us.  VGPRs hold four
 // waves to a SIMD; compiled for five it spills (927 us).
-constexpr int kDiaRunMax = 3;
-
 template <typename V, int KL, int R>
 __global__ __launch_bounds__(256) void dia_spmm_runs_kernel(DiaArgs<V> a) {
   using Acc = typename vtraits<V>::acc;
@@ -954,6 +1041,75 @@ int launch_ell_k(mph_matrix_impl* A, const void* x, void* y, int ld, int init,
   return MPH_OK;
 }
 
+// Which kernel takes a DIA SpMM pass of `lanes` lanes a row: one row per lane
+// group (dia_spmm_kernel), or kDiaSpmmRows in the slide or the staged form.
+// The lines lie where the three were measured: FP64 k = 4, 8, 16, FP32 / BF16
+// k = 8, 16, 32, bands of 3 to 25 diagonals of 10k to 2M rows, 5-, 7- and
+// 27-point grids of 30 to 1000 a side; no point is more than 3% slower than
+// the slide form from 4 lanes and the one-row kernel below, which ran there
+// before the staged form.  `full`: workgroups of the forms (1024 / lanes
+// rows) a CU.
+//  * 2 lanes: the staged form on runs of nearly three diagonals once it fills
+//    the device (27-point 128^3 FP64 157 -> 117 us, FP32 107 -> 86; below,
+//    9-diagonal band of 131k rows FP64 6.4 -> 7.1), BF16 four times as late
+//    (27-point 100^3 43.1 -> 45.0, 128^3 85.5 -> 79.2); shorter runs lose
+//    (5-point 1000^2 FP64 21.0 -> 24.8).
+//  * The staged form requests a run ahead, and four of its workgroups fit a
+//    CU: it wins from 3 a CU in FP64 (slide against staged: 27-point 160^3
+//    k = 16 632 -> 537 us; 500k rows, 9 diagonals, k = 8 28.0 -> 21.3) or 2
+//    with 9 diagonals or more (131k rows, k = 8 9.8 -> 8.0), and in FP32 where
+//    its last round is full (9 diagonals, k = 32, 1024 workgroups 12.2 -> 10.4;
+//    1563: 17.2 -> 17.8; 3907: 37.6 -> 34.8), with 16 lanes later (27-point
+//    64^3 k = 64 71.6 -> 75.6).  One or two runs and a second round barely
+//    begun lose in FP64 too (1563, 3 diagonals, k = 16 10.7 -> 12.2).  BF16
+//    moves half the values for the same X: the staged form gains once X leaves
+//    the last cache (27-point 128^3 k = 16 186 -> 158 us; 100^3 67.2 -> 73.3),
+//    or, where the diagonals reach no farther than a workgroup's rows, from
+//    10.5 a CU (420k rows, 9 diagonals, k = 32 28.1 -> 26.0) and in one full
+//    round (131k rows, 17 diagonals, k = 32 16.1 -> 15.2).
+//  * The slide form beats the one-row kernel where its workgroups fill the
+//    device (300k rows, 9 diagonals, BF16 k = 16 15.4 -> 12.3), with fewer
+//    only where the one-row kernel's batches of 8 diagonals run part empty
+//    (131k rows FP32 k = 16: 3 diagonals 5.7 -> 4.7 us, 9 8.4 -> 7.2, 7 6.0 ->
+//    6.6), and loses on runs of mostly one diagonal (7-point 64^3 BF16 k = 16
+//    9.5 -> 11.3).
+// MPH_DIA_SPMM_RUNS=0 / 1 / 2 forces the one-row kernel / the staged form /
+// the slide form.
+enum class DiaSpmm { kRow, kSlide, kStage };
+
+DiaSpmm dia_spmm_form(const mph_matrix_impl* A, int lanes) {
+  if (A->ncols == 0) return DiaSpmm::kRow;
+  if (const char* env = std::getenv("MPH_DIA_SPMM_RUNS")) {
+    const int mode = std::atoi(env);
+    return mode <= 0 ? DiaSpmm::kRow : mode == 1 ? DiaSpmm::kStage : DiaSpmm::kSlide;
+  }
+  const int64_t nd = A->ndiag, runs = A->dia_runs, rows = 256 / lanes * kDiaSpmmRows;
+  if (lanes < 2 || runs == 0) return DiaSpmm::kRow;
+  const double full = (double)ceil_div(A->nrows, rows) / device_cu_count();
+  const bool f64 = A->vt == MPH_F64, f32 = A->vt == MPH_F32;
+  // one or two runs, and a second round of workgroups barely begun
+  const bool brief = runs <= 2 && full > 5 && full < 6.4;
+  if (lanes == 2)
+    return 10 * nd >= 27 * runs && full >= (f64 ? 2 : f32 ? 3.5 : 15) && !brief ? DiaSpmm::kStage
+                                                                               : DiaSpmm::kRow;
+  const bool singles = 2 * nd < 3 * runs;  // runs of mostly one diagonal
+  const bool near = A->dia_reach <= rows;
+  const bool one_round = full >= 3.5 && full <= 4;
+  bool stage;
+  if (f64)
+    stage = (full >= 3 || (full >= 1.9 && nd >= 9 && !singles)) && !brief;
+  else if (f32)
+    stage = one_round || (full >= 3 && full <= 4 && nd >= 9) ||
+            full >= (lanes < 16 ? 6.4 : near ? 10 : 24);
+  else
+    stage = !singles && (near ? one_round || full >= 10.5 : full >= 24);
+  if (stage) return DiaSpmm::kStage;
+  if (singles && full < 24) return DiaSpmm::kRow;
+  const double used = (double)nd / (double)(8 * ceil_div(nd, 8));  // of the one-row kernel's batches
+  const bool slide = full >= 3 || (full >= 1.9 && used <= 0.71) || (full >= 1 && used <= (f64 ? 0.6 : 0.4));
+  return slide ? DiaSpmm::kSlide : DiaSpmm::kRow;
+}
+
 template <typename V, bool DIA, int KL>
 int launch_spmm_lanes(mph_matrix_impl* A, const void* x, void* y, int ld, int init,
                       hipStream_t s) {
@@ -971,30 +1127,9 @@ int launch_spmm_lanes(mph_matrix_impl* A, const void* x, void* y, int ld, int in
     a.y = static_cast<typename vtraits<V>::vec*>(y);
     a.ld = ld;
     a.init = init;
-    // the run form (4 rows per lane group) where it was measured faster: 4
-    // or more lanes per row (27-point 160^3 FP64 k = 8 593 -> 324 us, k = 16
-    // 1116 -> 537 us; FP32 k = 16 416 -> 293 us; BF16 k = 16 386 -> 283 us;
-    // 7-point 128^3 FP64 k = 8 even, k = 16 205 -> 182 us), and 2 lanes when
-    // the runs average two diagonals or more (27-point FP64 k = 4 314 ->
-    // 227 us, FP32 k = 8 212 -> 172 us, BF16 204 -> 170 us; the 7-point
-    // stencil's mostly single diagonals: FP64 k = 4 50 -> 72 us); one lane is
-    // even at best (27-point FP64 k = 2 207 -> 194 us, FP32 k = 4 125 ->
-    // 128 us; 7-point FP64 k = 2 31 -> 51 us).  Its workgroups take four times
-    // the rows and their runs one after another, so it needs 1.5 workgroups a
-    // CU in FP64 and 3 in FP32 / BF16 to win (25-diagonal bands: 65k rows FP64
-    // k = 16, 508 workgroups, 22.1 -> 18.4 us; k = 8, 254, 12.4 -> 16.6; FP32
-    // 260k rows k = 16, 1016, 30.1 -> 24.4, k = 8, 508, 16.9 -> 20.0; 2k rows
-    // 6.3 -> 16 us).  MPH_DIA_SPMM_RUNS=0 / 1 forces it off / on
-    const char* env = std::getenv("MPH_DIA_SPMM_RUNS");
-    const int mode = env ? std::atoi(env) : -1;
-    const int64_t cus = device_cu_count();
-    const int64_t wgs = ceil_div(A->nrows, (int64_t)(256 / KL) * 4);
-    const bool fills = 2 * wgs >= (A->vt == MPH_F64 ? 3 : 6) * cus;
-    const bool wide =
-        fills && (KL >= 4 || (KL == 2 && A->dia_runs > 0 && A->ndiag >= 2 * A->dia_runs));
-    const bool runs = A->ncols > 0 && (mode > 0 || (mode < 0 && wide));
-    if (runs) {
-      constexpr int R = 4;
+    const DiaSpmm form = dia_spmm_form(A, KL);
+    constexpr int R = kDiaSpmmRows;
+    if (form == DiaSpmm::kStage) {
       // plane order where two reaches of X exceed half an XCD's L2 and a
       // plane has workgroups to share out (27-point 160^3 FP64 k = 16 551 ->
       // 537 us, k = 32 1000 -> 950 us, FP32 k = 16 even)
@@ -1008,6 +1143,10 @@ int launch_spmm_lanes(mph_matrix_impl* A, const void* x, void* y, int ld, int in
         grid = kNumXcd * a.plane_xcd * ceil_div(nbr, plane);
       }
       hipLaunchKernelGGL((dia_spmm_runs_kernel<V, KL, R>), dim3((unsigned)grid), dim3(256), 0, s, a);
+    } else if (form == DiaSpmm::kSlide) {
+      hipLaunchKernelGGL((dia_spmm_slide_kernel<V, KL, R>),
+                         dim3((unsigned)ceil_div(A->nrows, (int64_t)(256 / KL) * R)), dim3(256), 0, s,
+                         a);
     } else {
       hipLaunchKernelGGL((dia_spmm_kernel<V, KL>), dim3((unsigned)nb), dim3(256), 0, s, a);
     }
@@ -1169,20 +1308,20 @@ int dia_analyse(mph_matrix_impl* A, hipStream_t s) {
   A->dia_stage = DiaStage{};
   A->dia_reach = A->dia_runs = 0;
   const int64_t nd = A->ndiag;
-  if (nd < 2 || nd > kDiaStageMaxDiags || A->nrows == 0 || A->ncols == 0) return MPH_OK;
+  if (nd < 1 || A->nrows == 0 || A->ncols == 0) return MPH_OK;
   int mode = 2;  // MPH_DIA_STAGE: 0 off, 1 the one-row kernels only, 2 also the row pairs
   if (const char* env = std::getenv("MPH_DIA_STAGE")) mode = std::atoi(env);
   std::vector<int32_t> off((size_t)nd);
   MPH_HIP_CHECK(hipMemcpyAsync(off.data(), A->dia_off, sizeof(int32_t) * nd,
                                hipMemcpyDeviceToHost, s));
   MPH_HIP_CHECK(hipStreamSynchronize(s));
-  // for the SpMM's run form: the farthest diagonal, and the runs
+  // for the SpMM's run forms: the farthest diagonal, and the runs
   for (int64_t i = 0, len = 0; i < nd; i++) {
     A->dia_reach = std::max<int64_t>(A->dia_reach, std::abs((int64_t)off[i]));
     len = i > 0 && len < kDiaRunMax && (int64_t)off[i - 1] + 1 == off[i] ? len + 1 : 1;
     A->dia_runs += len == 1 ? 1 : 0;
   }
-  if (mode <= 0) return MPH_OK;
+  if (mode <= 0 || nd < 2 || nd > kDiaStageMaxDiags) return MPH_OK;
   DiaStage st{};
   int32_t used = 0;
   int64_t staged_diags = 0;

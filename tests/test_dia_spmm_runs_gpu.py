@@ -63,7 +63,7 @@ NAMES = ["S27", "5-point", "band 9", "unsorted, repeated", "past the edge",
 def _run(monkeypatch, D, dtype, X, Y0, init, runs):
     import torch
     from morpheus_amd import device
-    monkeypatch.setenv("MPH_DIA_SPMM_RUNS", "1" if runs else "0")
+    monkeypatch.setenv("MPH_DIA_SPMM_RUNS", str(int(runs)))
     M = device.to_device(D, dtype)
     vdt = device.vector_dtype(dtype)
     xt = torch.from_numpy(np.ascontiguousarray(X)).cuda().to(vdt)
@@ -106,3 +106,35 @@ def test_runs_equal_groups_widths(gpu, monkeypatch, name, dtype, k):
     yr = _run(monkeypatch, D, dtype, X, Y0, True, True)
     yg = _run(monkeypatch, D, dtype, X, Y0, True, False)
     assert np.array_equal(yr, yg)
+
+
+@pytest.mark.parametrize("name", NAMES)
+@pytest.mark.parametrize("dtype,k", [("f64", 4), ("f64", 16), ("f32", 16), ("bf16", 32)])
+@pytest.mark.parametrize("init", [True, False])
+def test_slide_form_equals_groups(gpu, monkeypatch, name, dtype, k, init):
+    """MPH_DIA_SPMM_RUNS=2: the X pieces loaded by each lane itself."""
+    D = _cases()[name]
+    rng = np.random.default_rng(73)
+    X = rng.uniform(-1, 1, (D.ncols, k))
+    Y0 = rng.uniform(-1, 1, (D.nrows, k))
+    ys = _run(monkeypatch, D, dtype, X, Y0, init, 2)
+    yg = _run(monkeypatch, D, dtype, X, Y0, init, False)
+    assert np.array_equal(ys, yg)
+
+
+@pytest.mark.parametrize("nrows", [200_000, 262_144])
+@pytest.mark.parametrize("half", [1, 4])
+@pytest.mark.parametrize("dtype,k", [("f64", 16), ("f32", 16), ("f32", 32), ("bf16", 16)])
+def test_default_form_equals_groups(gpu, monkeypatch, nrows, half, dtype, k):
+    """Sizes about the lines between the forms."""
+    from morpheus_amd import device
+    D = _dia(nrows, nrows, np.arange(-half, half + 1), 8)
+    X = np.random.default_rng(74).uniform(-1, 1, (nrows, k))
+    Y0 = np.zeros((nrows, k))
+    yg = _run(monkeypatch, D, dtype, X, Y0, True, False)
+    import torch
+    M = device.to_device(D, dtype)
+    vdt = device.vector_dtype(dtype)
+    y = torch.zeros((nrows, k), dtype=vdt, device="cuda")
+    M.multiply_multi(torch.from_numpy(X).cuda().to(vdt), y)
+    assert np.array_equal(y.cpu().numpy().astype(np.float64), yg)
