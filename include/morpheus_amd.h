@@ -168,9 +168,10 @@ int mph_matrix_plan_bytes(mph_matrix_t A, int init, int64_t* bytes);
  *                  over row offsets derived from its row indices (rows_chunk
  *                  and lanes apply), an unsorted one the atomic pass
  *   rows_per_thread : DIA / ELL rows per thread (1 or 2, strided by 256 rows);
- *                  0 = one row, and in FP32 / BF16 DIA SpMV two adjacent
- *                  rows whose values are loaded as pairs, when the pitch
- *                  is even; with 0, DIA SpMV (and
+ *                  0 = one row, and in FP32 / BF16 SpMV of DIA, or of ELL
+ *                  with few slots and many rows, two adjacent rows whose
+ *                  values (and ELL column indices) are loaded as pairs, when
+ *                  the pitch is even; with 0, DIA SpMV (and
  *                  HDC's DIA pass) stages the x entries of each cluster of
  *                  nearby diagonals (offsets within 512, two or more
  *                  diagonals; at most 64 diagonals and 8 such clusters) in

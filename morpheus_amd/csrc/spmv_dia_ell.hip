@@ -13,8 +13,9 @@
 // y in a separate launch and then read-modify-writes it per 256-diagonal
 // chunk, and skips the zeroing when ndiag == 0).  ELL visits entries_per_row slots,
 // not the 32-padded width, when the analysis has confirmed that the slots
-// beyond entries_per_row hold only the -1 padding.  FP32 / BF16 DIA SpMV takes
-// two adjacent rows per thread (row-pair kernels below); FP32 / BF16 rows of
+// beyond entries_per_row hold only the -1 padding.  FP32 / BF16 SpMV of DIA, and
+// of ELL with few slots and many rows, takes two adjacent rows per thread
+// (row-pair kernels below); FP32 / BF16 rows of
 // more than kCompensateLen diagonals / slots take a Dot2-compensated kernel.
 // SpMM gives each row a lane group (16 bytes of its columns per lane); DIA may
 // give each group 4 consecutive rows, which share the X rows of each run of
@@ -864,6 +865,45 @@ __global__ __launch_bounds__(256) void dia_pair_staged_kernel(DiaArgs<V> a, DiaS
   if (row + 1 < a.nrows) a.y[row + 1] = a.init ? t1 : a.y[row + 1] + t1;
 }
 
+// ELL: the pair's two column indices are one load too (8 B).  Which sizes it
+// takes: ell_pair_ok.
+template <typename V>
+__global__ __launch_bounds__(256) void ell_pair_kernel(EllArgs<V> a) {
+  using P = Pair<V>;
+  const uint32_t b = xcd_remap(blockIdx.x, gridDim.x);
+  const int64_t row = ((int64_t)b * 256 + threadIdx.x) * 2;
+  const typename P::T* pv = reinterpret_cast<const typename P::T*>(a.val);
+  const uint64_t* pc = reinterpret_cast<const uint64_t*>(a.ci);
+  float t0 = 0, t1 = 0;
+  const bool in = row < a.nrows;
+  for (int n0 = 0; n0 < a.loop; n0 += 8) {
+    int32_t c0[8], c1[8];
+#pragma unroll
+    for (int w = 0; w < 8; w++) {
+      const int n = n0 + w;
+      const uint64_t cw = in && n < a.loop ? ld_stream(pc + (a.pitch * n + row) / 2) : ~0ull;
+      c0[w] = (int32_t)(uint32_t)cw;
+      // the pair's second row may lie past nrows, inside the pitch
+      c1[w] = row + 1 < a.nrows ? (int32_t)(uint32_t)(cw >> 32) : -1;
+    }
+    float v0[8], v1[8];
+#pragma unroll
+    for (int w = 0; w < 8; w++) {
+      const int n = n0 + w;
+      const typename P::T pw =
+          (c0[w] >= 0 || c1[w] >= 0) ? ld_stream(pv + (a.pitch * n + row) / 2) : (typename P::T)0;
+      P::split(pw, v0[w], v1[w]);
+    }
+#pragma unroll
+    for (int w = 0; w < 8; w++) {
+      if (c0[w] >= 0) t0 += v0[w] * a.x[c0[w]];
+      if (c1[w] >= 0) t1 += v1[w] * a.x[c1[w]];
+    }
+  }
+  if (row < a.nrows) a.y[row] = a.init ? t0 : a.y[row] + t0;
+  if (row + 1 < a.nrows) a.y[row + 1] = a.init ? t1 : a.y[row + 1] + t1;
+}
+
 // The same for a stage of at most kStageAhead entries a thread (a band, two
 // planes of a small grid): the first batch's value pairs are requested before
 // the stage is stored, raw until their products, 12 diagonals a batch.  A
@@ -1241,12 +1281,7 @@ int launch_fmt(mph_matrix_impl* A, int k, const void* x, void* y, int init,
 }
 
 // the DIA row-pair kernels: FP32 / BF16 SpMV with the default launch shape, an
-// even pitch and values aligned to the pair loads.  ELL keeps one row per
-// thread at every pitch: pairs, with their loads under branches, took 96-98 us
-// in FP32 and 78.5 in BF16 on the 27-point 128^3 grid where ell_kernel takes
-// 76.7 and 55.6 (7-point 128^3: 25.8 and 21.8, now 21.6 and 18.7; 5-point
-// 1000^2, the closest: 9.7 and 7.6, now 9.1 and 7.5); pairs without branches
-// took 102 and 82 (28 and 23).
+// even pitch and values aligned to the pair loads
 template <typename V>
 int launch_dia_pair(mph_matrix_impl* A, const void* x, void* y, int init, hipStream_t s) {
   const int64_t nb = ceil_div(A->nrows, 512);
@@ -1273,11 +1308,43 @@ int launch_dia_pair(mph_matrix_impl* A, const void* x, void* y, int init, hipStr
   return MPH_OK;
 }
 
-bool dia_pair_ok(const mph_matrix_impl* A, int k) {
-  if (k != 1 || A->tuning.rows_per_thread != 0) return false;
-  if (A->vt != MPH_F32 && A->vt != MPH_BF16) return false;
-  return A->dia_pitch % 2 == 0 &&
-         reinterpret_cast<uintptr_t>(A->dia_v) % (2 * value_size(A->vt)) == 0;
+template <typename V>
+int launch_ell_pair(mph_matrix_impl* A, const void* x, void* y, int init, hipStream_t s) {
+  EllArgs<V> a{};
+  a.nrows = A->nrows;
+  a.loop = (int32_t)A->ell_loop;
+  a.pitch = A->ell_pitch;
+  a.ci = A->ell_ci;
+  a.val = static_cast<const V*>(A->ell_v);
+  a.x = static_cast<const float*>(x);
+  a.y = static_cast<float*>(y);
+  a.ld = 1;
+  a.init = init;
+  hipLaunchKernelGGL(ell_pair_kernel<V>, dim3((unsigned)ceil_div(A->nrows, 512)), dim3(256), 0, s,
+                     a);
+  MPH_HIP_CHECK(hipGetLastError());
+  return MPH_OK;
+}
+
+bool pair_ok(const mph_matrix_impl* A, int k, int64_t pitch, const void* v) {
+  return k == 1 && A->tuning.rows_per_thread == 0 && (A->vt == MPH_F32 || A->vt == MPH_BF16) &&
+         pitch % 2 == 0 && reinterpret_cast<uintptr_t>(v) % (2 * value_size(A->vt)) == 0;
+}
+
+bool dia_pair_ok(const mph_matrix_impl* A, int k) { return pair_ok(A, k, A->dia_pitch, A->dia_v); }
+
+// ELL takes row pairs where the one-row kernel's workgroups, 8 a CU at once,
+// do not fit and have little to do: up to 3 slots (FP32, 1M rows: 2 slots one
+// row 5.5 us, pairs 4.7; 3 slots 6.8, 6.0; 3M 19.0, 18.6; even at 500k), up to
+// 5 while the second round of them is short (850k rows: 4 slots 7.2, 6.4; 1.5M
+// 10.9, 12.9).  Elsewhere one row per thread wins: its loads are not under
+// branches (27-point 128^3 FP32 pairs 96-98 us, one row 76.7; pairs without
+// branches 102).
+bool ell_pair_ok(const mph_matrix_impl* A, int k) {
+  const int64_t wgs = ceil_div(A->nrows, 256), cus = device_cu_count();
+  return pair_ok(A, k, A->ell_pitch, A->ell_v) && !A->rb.ell_cnt &&
+         reinterpret_cast<uintptr_t>(A->ell_ci) % 8 == 0 && wgs > 8 * cus &&
+         (A->ell_loop <= 3 || (A->ell_loop <= 5 && wgs <= 14 * cus));
 }
 
 template <bool DIA>
@@ -1289,6 +1356,9 @@ int dispatch(mph_matrix_impl* A, int k, const void* x, void* y, int init,
   if (DIA && dia_pair_ok(A, k))
     return A->vt == MPH_F32 ? launch_dia_pair<float>(A, x, y, init, s)
                             : launch_dia_pair<bf16>(A, x, y, init, s);
+  if (!DIA && ell_pair_ok(A, k))
+    return A->vt == MPH_F32 ? launch_ell_pair<float>(A, x, y, init, s)
+                            : launch_ell_pair<bf16>(A, x, y, init, s);
   if (DIA && k == 1 && A->dia_stage.n > 0 && A->tuning.rows_per_thread == 0)
     return A->vt == MPH_F64   ? launch_dia_staged<double>(A, x, y, init, s)
            : A->vt == MPH_F32 ? launch_dia_staged<float>(A, x, y, init, s)

@@ -59,3 +59,34 @@ def test_batches(gpu, n, width, dtype):
             assert np.all(np.abs(Yh[:, j] - ref) <= bound(nrow, scale))
             assert np.all(np.abs(Yah[:, j] - (Y0h[:, j] + ref))
                           <= bound(nrow + 1, scale + np.abs(Y0h[:, j])))
+
+
+@pytest.mark.parametrize("n,pitch", [(524_288, 524_288), (524_289, 524_290), (600_001, 600_001),
+                                     (917_503, 917_504), (917_505, 917_506)])
+@pytest.mark.parametrize("width", [1, 3, 4, 5])
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_row_pairs_of_few_slots(gpu, n, pitch, width, dtype):
+    """Row counts about the line to the row pairs (2048 workgroups of 256
+    rows; 3584 with 4 or 5 slots), even and odd, against two rows per thread."""
+    import torch
+    rng = torch.Generator(device="cuda").manual_seed(n + width)
+    ci = torch.randint(-1, n, (width, pitch), dtype=torch.int32, device="cuda", generator=rng)
+    ci[-1, n - 1] = n - 1  # the last row's last slot is filled
+    v = torch.rand((width, pitch), device="cuda", generator=rng).to(device.DTYPES[dtype][0])
+    D = device.DeviceMatrix(ELL_FORMAT, n, n, width * n, dtype,
+                            dict(ci=ci.reshape(-1), v=v.reshape(-1)),
+                            dict(K=width, width=width, pitch=pitch))
+    x = torch.rand(n, device="cuda", generator=rng)
+    y0 = torch.rand(n, device="cuda", generator=rng)
+    out = []
+    for rows in (0, 2):
+        D.set_tuning(rows_per_thread=rows)
+        y, ya = torch.full_like(y0, float("nan")), y0.clone()
+        D.multiply(x, y)
+        D.multiply(x, ya, init=False)
+        out.append((y, ya))
+    assert all(torch.equal(p, q) for p, q in zip(*out))
+    at = ci[:, :n].long()
+    ref = torch.where(at >= 0, v[:, :n].double() * x.double()[at.clamp_min(0)], 0.0).sum(0)
+    # at most 5 products, rounded once each in FP32
+    assert torch.all((out[0][0].double() - ref).abs() <= 2 * 5 * 2.0 ** -24 * ref.abs() + 1e-30)
