@@ -1298,7 +1298,15 @@ int launch_dia_pair(mph_matrix_impl* A, const void* x, void* y, int init, hipStr
   a.ld = 1;
   a.init = init;
   const DiaStage& cl = A->dia_stage;
-  if (cl.n > 0 && cl.pair && cl.base[cl.n - 1] + cl.len[cl.n - 1] + 256 * cl.n <= 256 * kStageAhead)
+  // the kernel that requests ahead takes 12 diagonals a batch, the other 8,
+  // and both load a batch past its last diagonal all the same: the first where
+  // it pads no more, up to 20 diagonals (4M rows FP32: 9 diagonals 39.1 ->
+  // 32.8 us, 17 61.2 -> 59.1; 13 46.0 -> 49.8, 15 51.0 -> 54.5, BF16 23
+  // 57.5 -> 59.7, 31 73.2 -> 79.1)
+  const int64_t nd = A->ndiag;
+  const bool ahead = nd <= 20 && 12 * ceil_div(nd, 12) <= 8 * ceil_div(nd, 8) && cl.n > 0 &&
+                     cl.base[cl.n - 1] + cl.len[cl.n - 1] + 256 * cl.n <= 256 * kStageAhead;
+  if (cl.n > 0 && cl.pair && ahead)
     hipLaunchKernelGGL(dia_pair_ahead_kernel<V>, dim3((unsigned)nb), dim3(256), 0, s, a, cl);
   else if (cl.n > 0 && cl.pair)
     hipLaunchKernelGGL(dia_pair_staged_kernel<V>, dim3((unsigned)nb), dim3(256), 0, s, a, cl);

@@ -22,3 +22,15 @@ def test_ahead_equals_plain(gpu, nrows, ndiag, span, dtype):
     for init in (True, False):
         ys = _product(D, x, y0, init, plain=False, dtype=dtype)
         assert np.array_equal(ys, _product(D, x, y0, init, plain=True, dtype=dtype))
+
+
+@pytest.mark.parametrize("nrows", [1, 511, 513, 5001])
+@pytest.mark.parametrize("ndiag", [16, 17, 20, 21])
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_ahead_in_two_batches(gpu, nrows, ndiag, dtype):
+    """Diagonals about those that take two batches of 12."""
+    D = _dia(nrows, nrows + 40, np.arange(-(ndiag // 2), ndiag - ndiag // 2), nrows + ndiag)
+    x, y0 = gen.random_vector(D.ncols, 1), gen.random_vector(D.nrows, 2)
+    for init in (True, False):
+        ys = _product(D, x, y0, init, plain=False, dtype=dtype)
+        assert np.array_equal(ys, _product(D, x, y0, init, plain=True, dtype=dtype))
