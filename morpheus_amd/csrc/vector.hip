@@ -42,19 +42,19 @@ inline int64_t chunk_for(int64_t n, int64_t parts) {
   return pad_size(ceil_div(std::max<int64_t>(n, 1), parts), 4);
 }
 
-inline bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
-
-// 16 bytes of a vector
+// 16 bytes of a vector, loaded and stored as such wherever the array starts
+// (global memory takes 16-byte accesses on any element's address), so that the
+// order of the sums, and with it their bits, does not depend on that
 template <typename Vec>
 struct Wide;
 template <>
 struct Wide<double> {
-  using T = double __attribute__((ext_vector_type(2)));
+  using T = double __attribute__((ext_vector_type(2), aligned(8)));
   static constexpr int Q = 2;
 };
 template <>
 struct Wide<float> {
-  using T = float __attribute__((ext_vector_type(4)));
+  using T = float __attribute__((ext_vector_type(4), aligned(4)));
   static constexpr int Q = 4;
 };
 constexpr int kBatch = 4;  // 16-byte pieces of each vector a thread has in flight
@@ -70,20 +70,18 @@ __device__ double block_sum(double v, double* s) {
   return r;
 }
 
-// The elements [b0, b1) of a block, b0 a multiple of 4: with WIDE (arrays on
-// 16 bytes) batches of kBatch pieces per thread, load(i, u) for all of a
-// batch before use(i, u), then the elements left one by one with one(i).
-template <typename Vec, bool WIDE, typename Load, typename Use, typename One>
+// The elements [b0, b1) of a block: batches of kBatch pieces per thread,
+// load(i, u) for all of a batch before use(i, u), then the elements left (all
+// of them in a block shorter than a batch) one by one with one(i).
+template <typename Vec, typename Load, typename Use, typename One>
 __device__ __forceinline__ void for_chunk(int64_t b0, int64_t b1, Load load, Use use, One one) {
   constexpr int Q = Wide<Vec>::Q;
   int64_t i0 = b0;
-  if constexpr (WIDE) {
-    for (; i0 + (int64_t)kT * Q * kBatch <= b1; i0 += (int64_t)kT * Q * kBatch) {
+  for (; i0 + (int64_t)kT * Q * kBatch <= b1; i0 += (int64_t)kT * Q * kBatch) {
 #pragma unroll
-      for (int u = 0; u < kBatch; u++) load(i0 + (int64_t)(u * kT + threadIdx.x) * Q, u);
+    for (int u = 0; u < kBatch; u++) load(i0 + (int64_t)(u * kT + threadIdx.x) * Q, u);
 #pragma unroll
-      for (int u = 0; u < kBatch; u++) use(i0 + (int64_t)(u * kT + threadIdx.x) * Q, u);
-    }
+    for (int u = 0; u < kBatch; u++) use(i0 + (int64_t)(u * kT + threadIdx.x) * Q, u);
   }
   for (int64_t i = i0 + threadIdx.x; i < b1; i += kT) one(i);
 }
@@ -97,7 +95,7 @@ __device__ double sum_parts(const double* __restrict__ parts, int64_t np, double
 }
 
 // block b: the contiguous chunk [b * chunk, (b + 1) * chunk)
-template <typename Vec, bool WIDE>
+template <typename Vec>
 __global__ __launch_bounds__(kT) void dot_parts_kernel(const Vec* __restrict__ x,
                                                        const Vec* __restrict__ y, int64_t n,
                                                        int64_t chunk, double* __restrict__ parts) {
@@ -106,7 +104,7 @@ __global__ __launch_bounds__(kT) void dot_parts_kernel(const Vec* __restrict__ x
   const int64_t b0 = (int64_t)blockIdx.x * chunk, b1 = min(n, b0 + chunk);
   double t = 0;
   P xv[kBatch], yv[kBatch];
-  for_chunk<Vec, WIDE>(
+  for_chunk<Vec>(
       b0, b1,
       [&](int64_t i, int u) {
         xv[u] = *reinterpret_cast<const P*>(x + i);
@@ -125,12 +123,8 @@ template <typename Vec>
 void launch_dot_parts(const void* x, const void* y, int64_t n, int64_t np, int64_t chunk,
                       double* parts, hipStream_t s) {
   const Vec *xv = static_cast<const Vec*>(x), *yv = static_cast<const Vec*>(y);
-  if (aligned16(x) && aligned16(y))
-    hipLaunchKernelGGL((dot_parts_kernel<Vec, true>), dim3((unsigned)np), dim3(kT), 0, s, xv, yv, n,
-                       chunk, parts);
-  else
-    hipLaunchKernelGGL((dot_parts_kernel<Vec, false>), dim3((unsigned)np), dim3(kT), 0, s, xv, yv,
-                       n, chunk, parts);
+  hipLaunchKernelGGL((dot_parts_kernel<Vec>), dim3((unsigned)np), dim3(kT), 0, s, xv, yv, n, chunk,
+                     parts);
 }
 
 template <typename Vec>
@@ -198,7 +192,7 @@ __global__ __launch_bounds__(kT) void cg_update_kernel(
   const int64_t b0 = (int64_t)blockIdx.x * chunk, b1 = min(n, b0 + chunk);
   double t = 0;
   P rv[kBatch], qv[kBatch];
-  for_chunk<Vec, true>(
+  for_chunk<Vec>(
       b0, b1,
       [&](int64_t i, int u) {
         rv[u] = *reinterpret_cast<const P*>(r + i);
@@ -220,7 +214,7 @@ __global__ __launch_bounds__(kT) void cg_update_kernel(
 }
 
 // beta = r.r / rr, x += alpha p and p = r + beta p
-template <typename Vec, bool WIDE>
+template <typename Vec>
 __global__ __launch_bounds__(kT) void cg_direction_kernel(
     Vec* __restrict__ x, Vec* __restrict__ p, const Vec* __restrict__ r, int64_t n, int64_t chunk,
     const double* __restrict__ rr_parts, int64_t np, double* __restrict__ state) {
@@ -231,7 +225,7 @@ __global__ __launch_bounds__(kT) void cg_direction_kernel(
   if (blockIdx.x == 0 && threadIdx.x == 0) state[kNext] = rr;
   const int64_t b0 = (int64_t)blockIdx.x * chunk, b1 = min(n, b0 + chunk);
   P xv[kBatch], pv[kBatch], rv[kBatch];
-  for_chunk<Vec, WIDE>(
+  for_chunk<Vec>(
       b0, b1,
       [&](int64_t i, int u) {
         pv[u] = *reinterpret_cast<const P*>(p + i);
@@ -349,12 +343,8 @@ int cg_iterate_t(mph_cg_s* c, void* x, int32_t iters, hipStream_t s) {
     launch_dot_parts<Vec>(c->p, c->q, c->n, c->np, c->chunk, pq_parts, s);
     hipLaunchKernelGGL((cg_update_kernel<Vec>), g, b, 0, s, r, static_cast<const Vec*>(c->q), c->n,
                        c->chunk, pq_parts, c->np, state, rr_parts);
-    if (aligned16(x))
-      hipLaunchKernelGGL((cg_direction_kernel<Vec, true>), g, b, 0, s, static_cast<Vec*>(x), p, r,
-                         c->n, c->chunk, rr_parts, c->np, state);
-    else
-      hipLaunchKernelGGL((cg_direction_kernel<Vec, false>), g, b, 0, s, static_cast<Vec*>(x), p, r,
-                         c->n, c->chunk, rr_parts, c->np, state);
+    hipLaunchKernelGGL((cg_direction_kernel<Vec>), g, b, 0, s, static_cast<Vec*>(x), p, r, c->n,
+                       c->chunk, rr_parts, c->np, state);
   }
   MPH_HIP_CHECK(hipGetLastError());
   return MPH_OK;
