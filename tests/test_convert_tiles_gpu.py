@@ -166,3 +166,21 @@ def test_is_sorted_reads_no_pair(gpu, nnz):
     out = C.c_int(-1)
     capi.call("mph_coo_is_sorted", nnz, None, None, C.byref(out), device.stream_handle())
     assert out.value == 1
+
+
+@pytest.mark.parametrize("nrows", [4096 * 2048 - 1, 4096 * 2048, 4096 * 2048 + 1,
+                                   3 * 4096 * 2048 + 7])
+def test_long_scans(gpu, nrows):
+    """Row positions about the longest prefix sum that takes two launches
+    (4096 tiles of 2048 counts), and well past it."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(nrows)
+    ci = torch.randint(-1, 3, (nrows,), dtype=torch.int32, device="cuda", generator=g)
+    ci[-1] = 1
+    v = torch.rand(nrows, device="cuda", generator=g)
+    rows = torch.nonzero(ci >= 0).reshape(-1)
+    ri, co = (torch.empty(rows.numel(), dtype=torch.int32, device="cuda") for _ in range(2))
+    vo = torch.empty(rows.numel(), device="cuda")
+    capi.call("mph_convert_ell_to_coo", nrows, rows.numel(), 1, nrows, ci.data_ptr(), v.data_ptr(),
+              capi.F32, ri.data_ptr(), co.data_ptr(), vo.data_ptr(), device.stream_handle())
+    assert torch.equal(ri, rows.int()) and torch.equal(co, ci[rows]) and torch.equal(vo, v[rows])
