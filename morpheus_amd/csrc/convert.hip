@@ -163,27 +163,23 @@ __global__ void first_descent_kernel(const int32_t* __restrict__ ri, int64_t n,
 // 8 B an entry once, where the range checks, the sortedness test and a row
 // histogram (an LDS hash table: 6 ps an entry) each were a pass.  With
 // indices out of range, or rows that decrease, ro is incomplete; every write
-// stays inside it.
-constexpr int32_t kBadRow = 1, kBadCol = 2, kRowsDown = 4, kUnsorted = 8, kRepeated = 16;
+// stays inside it.  More than kLongGap rows without an entry are left out and
+// raise kGaps, for gap_offsets_kernel: filled here, each by the lane or wave
+// that met it, the gaps of rows in no order came to a third of the rows an
+// entry (2M shuffled entries on 1M rows 127 ms), and one gap of 4M rows took
+// 1.8 ms.
+constexpr int32_t kBadRow = 1, kBadCol = 2, kRowsDown = 4, kUnsorted = 8, kRepeated = 16,
+                  kGaps = 32;
 constexpr int kScanPer = 8;  // entries per thread
 constexpr int kScanTile = kT * kScanPer;
+constexpr int64_t kLongGap = 32;
 
-// rows (lo, hi] start at entry i; long gaps are filled by the whole wave
-__device__ __forceinline__ void fill_offsets(int32_t* __restrict__ ro, int64_t lo, int64_t hi,
-                                             int32_t i) {
-  constexpr int64_t kLongGap = 32;
-  const int lane = threadIdx.x % kWave;
-  const bool lng = hi - lo > kLongGap;
-  if (!lng)
-    for (int64_t r = lo + 1; r <= hi; r++) ro[r] = i;
-  uint64_t m = __ballot(lng);
-  while (m) {
-    const int src = __ffsll((unsigned long long)m) - 1;
-    m &= m - 1;
-    const int64_t l = shfl((int32_t)lo, src), h = shfl((int32_t)hi, src);
-    const int32_t at = shfl(i, src);
-    for (int64_t r = l + 1 + lane; r <= h; r += kWave) ro[r] = at;
-  }
+// rows (lo, hi] start at entry i
+__device__ __forceinline__ int32_t fill_offsets(int32_t* __restrict__ ro, int64_t lo, int64_t hi,
+                                                int32_t i) {
+  if (hi - lo > kLongGap) return kGaps;
+  for (int64_t r = lo + 1; r <= hi; r++) ro[r] = i;
+  return 0;
 }
 
 // Sets the bits of `bad` that any thread of the workgroup has; a word that
@@ -354,9 +350,12 @@ __global__ __launch_bounds__(kT) void coo_scan_kernel(
         }
       }
       if (OFFSETS) {
-        const int64_t hi = in && row_ok ? r[k] : 0;
-        const int64_t lo = in && row_ok ? (i == 0 ? -1 : min((int64_t)max(pr, -1), hi)) : 0;
-        fill_offsets(ro, lo, hi, (int32_t)i);
+        // (a wave that sees rows decrease leaves them: ro is not used then)
+        if (__ballot(in && i > 0 && pr > r[k]) == 0) {
+          const int64_t hi = in && row_ok ? r[k] : 0;
+          const int64_t lo = in && row_ok ? (i == 0 ? -1 : min((int64_t)max(pr, -1), hi)) : 0;
+          bad |= fill_offsets(ro, lo, hi, (int32_t)i);
+        }
         if (in && i == nnz - 1 && row_ok) last = r[k];
       }
       const int32_t key = (int32_t)((int64_t)c[k] - r[k] + nrows - 1);
@@ -366,7 +365,7 @@ __global__ __launch_bounds__(kT) void coo_scan_kernel(
     }
   }
   if (OFFSETS)  // the rows after the last entry's
-    fill_offsets(ro, last >= -1 ? last : 0, last >= -1 ? nrows : 0, (int32_t)nnz);
+    bad |= fill_offsets(ro, last >= -1 ? last : 0, last >= -1 ? nrows : 0, (int32_t)nnz);
   raise_flags(flags, bad);
   if (DIAGS == kWidths) {
     raise_flags(flags + 1, wide_r);
@@ -377,6 +376,50 @@ __global__ __launch_bounds__(kT) void coo_scan_kernel(
     __syncthreads();
     for (int q = threadIdx.x; q < kSeen; q += kT)
       if (seen_n[q] > 0) atomicAdd(reinterpret_cast<int32_t*>(diags) + seen[q], seen_n[q]);
+  }
+}
+
+// The first entry from row r on of n entries in row order, by one wave, 64
+// probes a round.
+__device__ __forceinline__ int64_t wave_first_entry(const int32_t* __restrict__ ri, int64_t n,
+                                                    int64_t r) {
+  const int lane = threadIdx.x % kWave;
+  int64_t lo = -1, hi = n;  // ri[lo] < r <= ri[hi]
+  while (hi - lo > 1) {
+    const int64_t step = (hi - lo - 1 + kWave - 1) / kWave;
+    const int64_t at = lo + 1 + step * lane;
+    const uint64_t lt = __ballot(at < hi && ri[at] < r);
+    const int below = __popcll(lt);  // probes 0 .. below - 1
+    const int64_t next = below < kWave ? min(hi, lo + 1 + step * below) : hi;
+    if (below > 0) lo = lo + 1 + step * (below - 1);
+    hi = next;
+  }
+  return hi;
+}
+
+// The row offsets of entries in row order that coo_scan_kernel left out rows
+// of (flags, if given: its word; without kGaps, or with decreasing rows, there
+// is nothing to do).  A workgroup takes kScanTile rows: the entries of all of
+// them by two wave searches, and each row's first by a search among those.
+__global__ __launch_bounds__(kT) void gap_offsets_kernel(const int32_t* __restrict__ ri, int64_t nnz,
+                                                         int64_t nrows, int32_t* __restrict__ ro,
+                                                         const int32_t* __restrict__ flags) {
+  if (flags && (*flags & (kGaps | kRowsDown | kBadRow)) != kGaps) return;
+  __shared__ int64_t ends[2];
+  const int64_t base = (int64_t)blockIdx.x * kScanTile;
+  const int64_t top = min(base + kScanTile, nrows + 1);  // rows [base, top)
+  if (threadIdx.x < 2 * kWave) {
+    const int64_t e = wave_first_entry(ri, nnz, threadIdx.x < kWave ? base : top - 1);
+    if (threadIdx.x % kWave == 0) ends[threadIdx.x / kWave] = e;
+  }
+  __syncthreads();
+  for (int64_t r = base + threadIdx.x; r < top; r += kT) {
+    int64_t lo = ends[0], hi = ends[1];
+    while (lo < hi) {
+      const int64_t mid = (lo + hi) >> 1;
+      if (ri[mid] < r) lo = mid + 1; else hi = mid;
+    }
+    ro[r] = (int32_t)lo;
   }
 }
 
@@ -1512,6 +1555,16 @@ int dia_scan(int64_t nrows, int64_t ncols, int64_t nnz, const int32_t* ri, const
   return scan_status(D.flags);
 }
 
+// what coo_scan_kernel left of the row offsets (flags as it raised them; null:
+// known to be kGaps)
+int fill_gaps(const int32_t* ri, int64_t nnz, int64_t nrows, int32_t* ro, const int32_t* flags,
+              hipStream_t s) {
+  hipLaunchKernelGGL(gap_offsets_kernel, dim3(scan_blocks(nrows + 1)), dim3(kT), 0, s, ri, nnz, nrows,
+                     ro, flags);
+  MPH_HIP_CHECK(hipGetLastError());
+  return MPH_OK;
+}
+
 // The rows of a COO list: the longest, the sum of min(length, K), the order
 // of the entries and, rows not decreasing, their offsets.
 struct RowScan {
@@ -1534,14 +1587,22 @@ int row_scan(int64_t nrows, int64_t nnz, const int32_t* ri, int64_t K, Tmp& t, R
                        (uint32_t*)nullptr, flags);
   else
     MPH_CHECK_STATUS(fill_zero(R.ro, sizeof(int32_t) * (size_t)(nrows + 1), s));
-  // (offsets left incomplete by decreasing rows give numbers not used)
-  hipLaunchKernelGGL(row_lengths_kernel, dim3(reduce_blocks(nrows)), dim3(kT), 0, s, R.ro, nrows, k,
-                     acc);
-  MPH_HIP_CHECK(hipGetLastError());
-  MPH_CHECK_STATUS(t.fetch(acc, &h, 3));
-  MPH_CHECK_STATUS(t.wait());
+  // (incomplete offsets give numbers not used)
+  auto lengths = [&]() -> int {
+    hipLaunchKernelGGL(row_lengths_kernel, dim3(reduce_blocks(nrows)), dim3(kT), 0, s, R.ro, nrows, k,
+                       acc);
+    MPH_HIP_CHECK(hipGetLastError());
+    MPH_CHECK_STATUS(t.fetch(acc, &h, 3));
+    return t.wait();
+  };
+  MPH_CHECK_STATUS(lengths());
   R.flags = (int32_t)h[2];
   MPH_CHECK_STATUS(scan_status(R.flags));
+  if ((R.flags & (kGaps | kRowsDown)) == kGaps) {
+    MPH_CHECK_STATUS(fill_gaps(ri, nnz, nrows, R.ro, nullptr, s));
+    MPH_CHECK_STATUS(fill_zero(acc, 2 * sizeof(unsigned long long), s));
+    MPH_CHECK_STATUS(lengths());
+  }
   R.longest = (int64_t)h[0];
   R.clipped = (int64_t)h[1];
   if (R.flags & kRowsDown) {  // count the entries of each row
@@ -1823,6 +1884,7 @@ int mph_convert_coo_to_csr(int64_t nrows, int64_t nnz, const int32_t* ri, const 
   MPH_CHECK_STATUS(scan_status(h));
   if (!(h & kRowsDown)) {
     t.idle = true;
+    if (h & kGaps) MPH_CHECK_STATUS(fill_gaps(ri, nnz, nrows, ro_out, nullptr, s));
     if (ci_out != ci) MPH_CHECK_STATUS(copy_dev(ci_out, ci, sizeof(int32_t) * nnz, s));
     if (v_out != v) MPH_CHECK_STATUS(copy_dev(v_out, v, (size_t)vs * nnz, s));
     return MPH_OK;
@@ -1832,11 +1894,12 @@ int mph_convert_coo_to_csr(int64_t nrows, int64_t nnz, const int32_t* ri, const 
   MPH_CHECK_STATUS(t.alloc(&rows, nnz));
   MPH_CHECK_STATUS(radix_sort(nnz, bits_for(nrows - 1), 0, kByRow, ri, ci, v, vs, rows, ci_out,
                               v_out, s));
+  MPH_CHECK_STATUS(fill_zero(flags, sizeof(int32_t), s));
   hipLaunchKernelGGL((coo_scan_kernel<false, true, kNoDiags>), dim3(scan_blocks(nnz)), dim3(kT), 0,
                      s, rows, (const int32_t*)nullptr, nnz, nrows, (int64_t)INT32_MAX, ro_out,
                      (uint32_t*)nullptr, flags);
   MPH_HIP_CHECK(hipGetLastError());
-  return MPH_OK;
+  return fill_gaps(rows, nnz, nrows, ro_out, flags, s);
 }
 
 int mph_convert_coo_to_dia_size(int64_t nrows, int64_t ncols, int64_t nnz, const int32_t* ri,
@@ -2060,6 +2123,7 @@ int mph_convert_hyb_to_coo(int64_t nrows, int64_t nnz, int64_t width, int64_t pi
       MPH_HIP_CHECK(hipGetLastError());
       MPH_CHECK_STATUS(t.read(flags, &h));
     }
+    if (h & kGaps) MPH_CHECK_STATUS(fill_gaps(cri, P, nrows, tro, nullptr, s));
   } else {
     MPH_CHECK_STATUS(fill_zero(tro, sizeof(int32_t) * (size_t)(std::max<int64_t>(nrows, 0) + 1), s));
   }
@@ -2183,6 +2247,8 @@ int mph_convert_coo_to_hdc(int64_t nrows, int64_t ncols, int64_t nnz, const int3
     hipLaunchKernelGGL((coo_scan_kernel<false, true, kNoDiags>), dim3(scan_blocks(nrest)), dim3(kT),
                        0, s, rows_rest, (const int32_t*)nullptr, (int64_t)nrest, nrows,
                        (int64_t)INT32_MAX, csr_ro, (uint32_t*)nullptr, flags);
+    MPH_HIP_CHECK(hipGetLastError());
+    MPH_CHECK_STATUS(fill_gaps(rows_rest, nrest, nrows, csr_ro, flags, s));
   } else {
     int32_t* rcnt;
     MPH_CHECK_STATUS(row_counts(rows_rest, nrest, nrows, t, &rcnt, s));

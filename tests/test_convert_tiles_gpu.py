@@ -184,3 +184,55 @@ def test_long_scans(gpu, nrows):
     capi.call("mph_convert_ell_to_coo", nrows, rows.numel(), 1, nrows, ci.data_ptr(), v.data_ptr(),
               capi.F32, ri.data_ptr(), co.data_ptr(), vo.data_ptr(), device.stream_handle())
     assert torch.equal(ri, rows.int()) and torch.equal(co, ci[rows]) and torch.equal(vo, v[rows])
+
+
+@pytest.mark.parametrize("gap", [31, 32, 33, 34, 2047, 2048, 2049, 7000])
+@pytest.mark.parametrize("where", ["first", "middle", "last", "all"])
+@pytest.mark.parametrize("fmt", [CSR_FORMAT, HYB_FORMAT, HDC_FORMAT])
+def test_gaps_between_rows(gpu, gap, where, fmt):
+    """Rows without entries about the lengths where a scan of the entries no
+    longer fills their offsets (32 rows) and of the tiles that do (2048)."""
+    lead, mid, tail = (gap if where in (w, "all") else 0 for w in ("first", "middle", "last"))
+    a = lead + np.arange(300)
+    rows = np.r_[a, a[-1] + 1 + mid + np.arange(40)]
+    n = rows[-1] + 1 + tail
+    rows = np.repeat(rows, 1 + np.arange(rows.size) % 4 // 3)
+    cols = (np.arange(rows.size) * 37) % n
+    A = Coo(n, n, rows, cols, 1.0 + np.arange(rows.size))
+    at = np.lexsort((A.column_indices, A.row_indices))
+    A = Coo(n, n, rows[at], cols[at], A.values[at])
+    _check(A, fmt)
+    perm = np.random.default_rng(gap).permutation(rows.size)
+    _check(Coo(n, n, A.row_indices[perm], A.column_indices[perm], A.values[perm]), fmt)
+
+
+@pytest.mark.parametrize("order", ["shuffled", "runs", "ends"])
+def test_offsets_take_time_by_entries_and_rows(gpu, order):
+    """Rows in no order, in many ascending runs, and at both ends of a long
+    matrix: a scan that fills the rows between an entry and the one before it
+    took 8 to 240 ms."""
+    import torch
+    n, nnz = 4_000_000, 2_000_000
+    g = torch.Generator(device="cuda").manual_seed(1)
+    ri = torch.randint(0, n, (nnz,), dtype=torch.int32, device="cuda", generator=g).sort().values
+    if order == "shuffled":
+        ri = ri[torch.randperm(nnz, device="cuda", generator=g)]
+    elif order == "runs":
+        ri = ri.reshape(-1, 64).t().reshape(-1).contiguous()
+    else:
+        ri = torch.cat([ri[:500] % 500, n - 1 - ri[:500] % 500]).sort().values
+    A = device.DeviceMatrix(COO_FORMAT, n, n, ri.numel(), "f64",
+                            dict(ri=ri, ci=ri.clone(), v=ri.double()), {})
+    ms = []
+    for _ in range(4):
+        t = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        t[0].record()
+        B = device.from_coo(A, CSR_FORMAT)
+        t[1].record()
+        t[1].synchronize()
+        ms.append(t[0].elapsed_time(t[1]))
+    ro = torch.zeros(n + 1, dtype=torch.int64, device="cuda")
+    ro[1:] = torch.cumsum(torch.bincount(ri.long(), minlength=n), 0)
+    assert torch.equal(B.arrays["ro"], ro.int())
+    assert torch.equal(B.arrays["v"], ri.sort(stable=True).values.double())
+    assert min(ms) < (1.2 if order == "ends" else 4)
