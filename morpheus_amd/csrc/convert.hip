@@ -1107,16 +1107,17 @@ __global__ void tail_place_kernel(const int32_t* __restrict__ ri, const int32_t*
 
 // COO -> ELL / HYB when the rows do not decrease: row r's entries are
 // [ro[r], ro[r + 1]), its n-th in slot n, so every slot is written once, in
-// row order per slot (coalesced), padding (-1, 0) included.  64 rows a
-// workgroup, each wave every fourth slot; the rows' entries are read
+// row order per slot (coalesced), padding (-1, 0) included.  64 rows and `per`
+// slots a workgroup, each wave every fourth slot; the rows' entries are read
 // coalesced into LDS when they fit, or directly.  (With rows that decrease,
 // a row may have several runs, and the latest entry claims each slot first,
 // above.)
 constexpr int kEllStage = 2048;
+constexpr int64_t kFillBlocks = 2048;  // workgroups enough to fill the device
 template <typename W>
 __global__ __launch_bounds__(kT) void ell_fill_rows_kernel(
     const int32_t* __restrict__ ro, const int32_t* __restrict__ ci, const void* __restrict__ v_,
-    int64_t nrows, int64_t K, int64_t width, int64_t pitch, int32_t* __restrict__ eci,
+    int64_t nrows, int64_t K, int64_t width, int64_t per, int64_t pitch, int32_t* __restrict__ eci,
     void* __restrict__ ev_) {
   __shared__ int32_t sc[kEllStage];
   __shared__ W sv[kEllStage];
@@ -1135,7 +1136,8 @@ __global__ __launch_bounds__(kT) void ell_fill_rows_kernel(
   }
   if (r >= pitch) return;
   const int64_t b = r < nrows ? ro[r] : 0, len = r < nrows ? min((int64_t)ro[r + 1] - b, K) : 0;
-  for (int64_t n = wave; n < width; n += kT / kWave) {
+  const int64_t n0 = per * blockIdx.y, n1 = min(width, n0 + per);
+  for (int64_t n = n0 + wave; n < n1; n += kT / kWave) {
     int32_t c = -1;
     W x = 0;
     if (n < len) {
@@ -1145,6 +1147,22 @@ __global__ __launch_bounds__(kT) void ell_fill_rows_kernel(
     eci[r + pitch * n] = c;
     ev[r + pitch * n] = x;
   }
+}
+
+// The same for fewer rows than a wave has lanes: a thread per slot, the rows
+// of one slot next to each other.
+template <typename W>
+__global__ __launch_bounds__(kT) void ell_fill_slots_kernel(
+    const int32_t* __restrict__ ro, const int32_t* __restrict__ ci, const void* __restrict__ v_,
+    int64_t nrows, int64_t K, int64_t slots, int64_t pitch, int32_t* __restrict__ eci,
+    void* __restrict__ ev_) {
+  const int64_t i = (int64_t)blockIdx.x * kT + threadIdx.x;
+  if (i >= slots) return;
+  const int64_t n = i / pitch, r = i - n * pitch;
+  const int64_t b = r < nrows ? ro[r] : 0;
+  const bool in = r < nrows && n < min((int64_t)ro[r + 1] - b, K);
+  eci[i] = in ? ci[b + n] : -1;
+  static_cast<W*>(ev_)[i] = in ? static_cast<const W*>(v_)[b + n] : 0;
 }
 
 // entries past a row's first K, per row
@@ -1692,8 +1710,19 @@ int ell_place(int64_t nrows, int64_t nnz, const int32_t* ri, const int32_t* ci, 
               void* ev, int32_t* over, Tmp& t, hipStream_t s) {
   if (width * pitch == 0) return MPH_OK;
   if (!(S.flags & kRowsDown)) {
-    MPH_LAUNCH_W(ell_fill_rows_kernel, vs, dim3(blocks_for(pitch, kWave)), s, S.ro, ci, v, nrows, K,
-                 width, pitch, eci, ev);
+    if (pitch < kWave) {
+      MPH_LAUNCH_W(ell_fill_slots_kernel, vs, dim3(blocks_for(width * pitch)), s, S.ro, ci, v, nrows,
+                   K, width * pitch, pitch, eci, ev);
+    } else {
+      // few rows and many slots: the slots shared out too, 32 or more a
+      // workgroup (one workgroup per 64 rows took 1.2 ms for 100 rows of 20k
+      // entries, 24 ms for 4 of 500k)
+      const int64_t gx = ceil_div(pitch, kWave);
+      const int64_t gy = std::max<int64_t>(1, std::min(ceil_div(width, 32), kFillBlocks / gx));
+      const int64_t per = ceil_div(width, gy);
+      MPH_LAUNCH_W(ell_fill_rows_kernel, vs, dim3((unsigned)gx, (unsigned)ceil_div(width, per)), s,
+                   S.ro, ci, v, nrows, K, width, per, pitch, eci, ev);
+    }
     MPH_HIP_CHECK(hipGetLastError());
     return MPH_OK;
   }
