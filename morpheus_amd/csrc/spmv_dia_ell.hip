@@ -1135,9 +1135,13 @@ DiaSpmm dia_spmm_form(const mph_matrix_impl* A, int lanes) {
     return mode <= 0 ? DiaSpmm::kRow : mode == 1 ? DiaSpmm::kStage : DiaSpmm::kSlide;
   }
   const int64_t nd = A->ndiag, runs = A->dia_runs, rows = 256 / lanes * kDiaSpmmRows;
-  if (lanes < 2 || runs == 0) return DiaSpmm::kRow;
+  if (lanes < 2) return DiaSpmm::kRow;
   const double full = (double)ceil_div(A->nrows, rows) / device_cu_count();
   const bool f64 = A->vt == MPH_F64, f32 = A->vt == MPH_F32;
+  // one diagonal, or more than kDiaStageMaxDiags: the analysis does not look
+  // at the runs (its copy of the offsets would cost it 19 us)
+  if (runs == 0)
+    return lanes < 4 || full < 3 ? DiaSpmm::kRow : f64 ? DiaSpmm::kStage : DiaSpmm::kSlide;
   // one or two runs, and a second round of workgroups barely begun
   const bool brief = runs <= 2 && full > 5 && full < 6.4;
   if (lanes == 2)
@@ -1397,7 +1401,7 @@ int dia_analyse(mph_matrix_impl* A, hipStream_t s) {
   A->dia_stage = DiaStage{};
   A->dia_reach = A->dia_runs = 0;
   const int64_t nd = A->ndiag;
-  if (nd < 1 || A->nrows == 0 || A->ncols == 0) return MPH_OK;
+  if (nd < 2 || nd > kDiaStageMaxDiags || A->nrows == 0 || A->ncols == 0) return MPH_OK;
   int mode = 2;  // MPH_DIA_STAGE: 0 off, 1 the one-row kernels only, 2 also the row pairs
   if (const char* env = std::getenv("MPH_DIA_STAGE")) mode = std::atoi(env);
   std::vector<int32_t> off((size_t)nd);
@@ -1410,7 +1414,7 @@ int dia_analyse(mph_matrix_impl* A, hipStream_t s) {
     len = i > 0 && len < kDiaRunMax && (int64_t)off[i - 1] + 1 == off[i] ? len + 1 : 1;
     A->dia_runs += len == 1 ? 1 : 0;
   }
-  if (mode <= 0 || nd < 2 || nd > kDiaStageMaxDiags) return MPH_OK;
+  if (mode <= 0) return MPH_OK;
   DiaStage st{};
   int32_t used = 0;
   int64_t staged_diags = 0;
