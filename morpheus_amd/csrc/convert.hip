@@ -853,44 +853,76 @@ struct EllSlots {
   }
 };
 
+// The slots of a row in segments of `len`, counted and emitted as if they were
+// rows of their own, in the order (row, segment): one where rows are short,
+// more where a few rows hold many slots (a thread or lane per row took 500 ms
+// for one row of 2M diagonals, 254 ms for as many ELL slots).
+struct Segs {
+  int32_t len, n;
+};
+constexpr int kSegSlots = 256;
+
+Segs segments(int64_t nrows, int64_t slots) {
+  if (slots <= kSegSlots) return {kSegSlots, 1};
+  int64_t len = kSegSlots;
+  // shorter, down to a batch of the emission, where they would not fill the
+  // device (one row of 2M diagonals 376 -> 144 us)
+  while (len > 32 && nrows * ceil_div(slots, len) < 65536) len /= 2;
+  while (ceil_div(slots, len) > 32768 && nrows >= kWave) len *= 2;  // (a grid's second dimension)
+  return {(int32_t)len, (int32_t)ceil_div(slots, len)};
+}
+
+// the row and segment of thread t: rows next to each other
+__device__ __forceinline__ void row_segment(int64_t t, int64_t nrows, const Segs& g, int64_t& r,
+                                            int32_t& y) {
+  y = g.n > 1 ? (int32_t)(t / nrows) : 0;
+  r = t - (int64_t)y * nrows;
+}
+
 template <typename W>
 __global__ __launch_bounds__(kT) void dia_row_count_kernel(DiaSlots<W> src, int64_t nrows,
-                                                           int32_t ns,
+                                                           int32_t ns, Segs g,
                                                            int32_t* __restrict__ cnt) {
-  const int64_t r = (int64_t)blockIdx.x * kT + threadIdx.x;
-  if (r >= nrows) return;
+  const int64_t t = (int64_t)blockIdx.x * kT + threadIdx.x;
+  if (t >= nrows * g.n) return;
+  int64_t r;
+  int32_t y;
+  row_segment(t, nrows, g, r, y);
   int32_t n = 0;
-  for (int s0 = 0; s0 < ns; s0 += kScanPer) {
+  const int64_t end = min((int64_t)ns, ((int64_t)y + 1) * g.len);
+  for (int64_t s0 = (int64_t)y * g.len; s0 < end; s0 += kScanPer) {
     W v[kScanPer];
     bool ok[kScanPer];
     int32_t c;
 #pragma unroll
     for (int k = 0; k < kScanPer; k++) {
       ok[k] = false;
-      if (s0 + k < ns) src.load(r, s0 + k, c, v[k], ok[k]);
+      if (s0 + k < end) src.load(r, (int)(s0 + k), c, v[k], ok[k]);
     }
 #pragma unroll
     for (int k = 0; k < kScanPer; k++) {
-      if (ok[k]) src.finish(r, s0 + k, c, v[k], ok[k]);
+      if (ok[k]) src.finish(r, (int)(s0 + k), c, v[k], ok[k]);
       n += ok[k] ? 1 : 0;
     }
   }
-  cnt[r] = n;
+  cnt[r * g.n + y] = n;
 }
 
-// The entries of 64 rows a workgroup: lane = row, each wave a quarter of the
-// slots, batches of 32 slots.  The entries are staged in LDS in output order
-// and written coalesced (written from the row walk, each store of a wave
-// spreads over 64 rows' entries); row r's go to rowpos[r], rowpos[r] + 1, ...
-// (a row's range may be longer: HYB's COO entries follow).  Reads the slots
-// once, coalesced, writes 8 + W bytes an entry once.
+// The entries of 64 rows' segments a workgroup: lane = row, of the segment
+// blockIdx.y, or, with fewer rows than lanes (NARROW), lane = one of 64
+// consecutive (row, segment); each wave a quarter of the slots, batches of 32
+// slots.  The entries are staged in LDS in output order and written coalesced
+// (written from the row walk, each store of a wave spreads over 64 rows'
+// entries); those of segment q = (row, segment) go to rowpos[q], rowpos[q] + 1,
+// ... (a row's range may be longer: HYB's COO entries follow).  Reads the
+// slots once, coalesced, writes 8 + W bytes an entry once.
 constexpr int kEmitRows = kWave;
 constexpr int kEmitWaves = kT / kWave;
 constexpr int kEmitPer = 8;  // slots per lane and batch
 constexpr int kEmitBatch = kEmitWaves * kEmitPer;
 
-template <typename W, typename Src>
-__global__ __launch_bounds__(kT) void emit_rows_kernel(Src src, int64_t nrows, int32_t ns,
+template <typename W, typename Src, bool NARROW>
+__global__ __launch_bounds__(kT) void emit_rows_kernel(Src src, int64_t nrows, int32_t ns, Segs g,
                                                        const int32_t* __restrict__ rowpos,
                                                        int32_t* __restrict__ ri,
                                                        int32_t* __restrict__ ci,
@@ -902,24 +934,36 @@ __global__ __launch_bounds__(kT) void emit_rows_kernel(Src src, int64_t nrows, i
   __shared__ int32_t dst[kEmitRows];  // output position of the row's first entry, less its LDS place
   __shared__ int32_t total;
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-  const int64_t r0 = (int64_t)blockIdx.x * kEmitRows, r = r0 + lane;
-  int32_t pos = r < nrows ? rowpos[r] : 0;
-  for (int s0 = 0; s0 < ns; s0 += kEmitBatch) {
+  __shared__ int32_t srow[NARROW ? kEmitRows : 1];
+  const int64_t r0 = (int64_t)blockIdx.x * kEmitRows;
+  int64_t r = r0 + lane;
+  int32_t first_slot = (int32_t)blockIdx.y * g.len, seg = (int32_t)blockIdx.y;
+  if (NARROW) {
+    const int64_t q = r;
+    r = q / g.n;
+    seg = (int32_t)(q - r * g.n);
+    first_slot = seg * g.len;
+    if (wave == 0) srow[lane] = (int32_t)r;  // (read after the barriers below)
+  }
+  int32_t pos = r < nrows ? rowpos[r * g.n + seg] : 0;
+  const int32_t len = NARROW ? g.len : min(g.len, ns - first_slot);
+  for (int s0 = 0; s0 < len; s0 += kEmitBatch) {
     // the batch's slots in order over the waves
-    const int per = (min(kEmitBatch, ns - s0) + kEmitWaves - 1) / kEmitWaves;
-    const int sb = s0 + wave * per, se = min(min(sb + per, s0 + kEmitBatch), (int)ns);
+    const int per = (min(kEmitBatch, len - s0) + kEmitWaves - 1) / kEmitWaves;
+    const int64_t sl = (int64_t)first_slot + s0, sb = sl + wave * per;
+    const int64_t se = min(min(sb + per, sl + kEmitBatch), min((int64_t)ns, (int64_t)first_slot + len));
     W v[kEmitPer];
     int32_t c[kEmitPer];
     bool ok[kEmitPer];
 #pragma unroll
     for (int k = 0; k < kEmitPer; k++) {
       ok[k] = false;
-      if (sb + k < se && r < nrows) src.load(r, sb + k, c[k], v[k], ok[k]);
+      if (sb + k < se && r < nrows) src.load(r, (int)(sb + k), c[k], v[k], ok[k]);
     }
     int32_t n = 0;
 #pragma unroll
     for (int k = 0; k < kEmitPer; k++) {
-      if (ok[k]) src.finish(r, sb + k, c[k], v[k], ok[k]);
+      if (ok[k]) src.finish(r, (int)(sb + k), c[k], v[k], ok[k]);
       n += ok[k] ? 1 : 0;
     }
     cnt[wave][lane] = n;
@@ -953,13 +997,25 @@ __global__ __launch_bounds__(kT) void emit_rows_kernel(Src src, int64_t nrows, i
     for (int j = threadIdx.x; j < total; j += kT) {
       const int q = sr[j];
       const int64_t o = (int64_t)dst[q] + j;
-      ri[o] = (int32_t)(r0 + q);
+      ri[o] = NARROW ? srow[q] : (int32_t)(r0 + q);
       ci[o] = sc[j];
       vo[o] = sv[j];
     }
     pos += row_n;
     __syncthreads();
   }
+}
+
+template <typename W, typename Src>
+void emit_rows(const Src& src, int64_t nrows, int32_t ns, const Segs& g, const int32_t* rowpos,
+               int32_t* ri, int32_t* ci, void* v, hipStream_t s) {
+  if (g.n > 1 && nrows < kEmitRows)
+    hipLaunchKernelGGL((emit_rows_kernel<W, Src, true>), dim3(blocks_for(nrows * g.n, kEmitRows)),
+                       dim3(kT), 0, s, src, nrows, ns, g, rowpos, ri, ci, static_cast<W*>(v));
+  else
+    hipLaunchKernelGGL((emit_rows_kernel<W, Src, false>),
+                       dim3(blocks_for(nrows, kEmitRows), (unsigned)ceil_div(ns, g.len)), dim3(kT),
+                       0, s, src, nrows, ns, g, rowpos, ri, ci, static_cast<W*>(v));
 }
 
 // zero the COO slots [from, nnz) left unfilled
@@ -974,38 +1030,52 @@ __global__ void zero_tail_kernel(int64_t from, int64_t nnz, int32_t* ri, int32_t
   }
 }
 
-// Per row, the ELL slots that hold a column plus the row's entries of the
-// row-sorted COO part (tro null: none); stats: [0] raised when some row's
-// columns are not in ascending order (its COO entries after its slots; the
-// order among the COO entries is checked by coo_scan_kernel), [1] 1 + the
-// last slot any row uses.
+// Per row and segment, the ELL slots that hold a column, plus with the row's
+// last segment its entries of the row-sorted COO part (tro null: none); stats:
+// [0] raised when some row's columns are not in ascending order (its COO
+// entries after its slots; the order among the COO entries is checked by
+// coo_scan_kernel), [1] 1 + the last slot any row uses.  A segment looks up to
+// kSegBack slots back for the column before its first; not finding one counts
+// as out of order (the list is then sorted, whatever its order).
+constexpr int kSegBack = 64;
 __global__ __launch_bounds__(kT) void ell_row_count_kernel(
-    const int32_t* __restrict__ eci, int64_t nrows, int64_t width, int64_t pitch,
+    const int32_t* __restrict__ eci, int64_t nrows, int64_t width, int64_t pitch, Segs g,
     const int32_t* __restrict__ tro, const int32_t* __restrict__ tci, int32_t* __restrict__ cnt,
     int32_t* __restrict__ stats) {
   int32_t bad = 0, top = 0;
-  for (int64_t r = (int64_t)blockIdx.x * kT + threadIdx.x; r < nrows;
-       r += (int64_t)gridDim.x * kT) {
+  for (int64_t t = (int64_t)blockIdx.x * kT + threadIdx.x; t < nrows * g.n;
+       t += (int64_t)gridDim.x * kT) {
+    int64_t r;
+    int32_t y;
+    row_segment(t, nrows, g, r, y);
     int32_t n = 0, prev = INT32_MIN;
-    for (int64_t s0 = 0; s0 < width; s0 += kScanPer) {
+    const int64_t begin = (int64_t)y * g.len, end = min(width, begin + g.len);
+    bool known = y == 0;
+    for (int64_t b = begin - 1; !known && b >= max(begin - kSegBack, (int64_t)0); b--) {
+      const int32_t c = eci[r + pitch * b];
+      known = c != -1;
+      if (known) prev = c;
+    }
+    for (int64_t s0 = begin; s0 < end; s0 += kScanPer) {
       int32_t c[kScanPer];
 #pragma unroll
-      for (int k = 0; k < kScanPer; k++) c[k] = s0 + k < width ? eci[r + pitch * (s0 + k)] : -1;
+      for (int k = 0; k < kScanPer; k++) c[k] = s0 + k < end ? eci[r + pitch * (s0 + k)] : -1;
 #pragma unroll
       for (int k = 0; k < kScanPer; k++)
         if (c[k] != -1) {
-          bad |= c[k] < prev ? 1 : 0;
+          bad |= c[k] < prev || !known ? 1 : 0;
+          known = true;
           prev = c[k];
           n++;
           top = max(top, (int32_t)(s0 + k) + 1);
         }
     }
-    if (tro) {
+    if (tro && y == g.n - 1) {
       const int32_t ts = tro[r], te = tro[r + 1];
-      if (te > ts && n > 0 && tci[ts] < prev) bad = 1;
+      if (te > ts && ((y > 0 && !known) || (prev != INT32_MIN && tci[ts] < prev))) bad = 1;
       n += te - ts;
     }
-    cnt[r] = n;
+    cnt[r * g.n + y] = n;
   }
   raise_flags(&stats[0], bad);
   top = block_reduce(top, [](int32_t u, int32_t v) { return max(u, v); });
@@ -1020,14 +1090,15 @@ __global__ void hyb_tail_emit_kernel(const int32_t* __restrict__ tri,
                                      const int32_t* __restrict__ tci,
                                      const void* __restrict__ tv_, int64_t n,
                                      const int32_t* __restrict__ tro,
-                                     const int32_t* __restrict__ rowpos, int32_t* __restrict__ ri,
-                                     int32_t* __restrict__ ci, void* __restrict__ vo_) {
+                                     const int32_t* __restrict__ rowpos, int32_t segs,
+                                     int32_t* __restrict__ ri, int32_t* __restrict__ ci,
+                                     void* __restrict__ vo_) {
   const W* tv = static_cast<const W*>(tv_);
   W* vo = static_cast<W*>(vo_);
   const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= n) return;
   const int32_t r = tri[j];
-  const int64_t o = (int64_t)rowpos[r + 1] - tro[r + 1] + j;
+  const int64_t o = (int64_t)rowpos[((int64_t)r + 1) * segs] - tro[r + 1] + j;
   ri[o] = r;
   ci[o] = tci[j];
   vo[o] = tv[j];
@@ -1373,17 +1444,18 @@ __global__ __launch_bounds__(kT) void hdc_split_kernel(
 }
 
 // Two lists in (row, column) order merged: entry e of list A lands after the
-// B entries before it.  LATER: A's entries follow equal ones of B.
+// B entries before it (row r's from bro[r * step] on).  LATER: A's entries
+// follow equal ones of B.
 template <bool LATER, typename W>
 __global__ __launch_bounds__(kT) void merge_rows_kernel(
     const int32_t* __restrict__ ri, const int32_t* __restrict__ ci, const void* __restrict__ v_,
-    int64_t n, const int32_t* __restrict__ bro, const int32_t* __restrict__ bci,
+    int64_t n, const int32_t* __restrict__ bro, int32_t step, const int32_t* __restrict__ bci,
     int32_t* __restrict__ ri_out, int32_t* __restrict__ ci_out, void* __restrict__ vo_) {
   const int64_t e = (int64_t)blockIdx.x * kT + threadIdx.x;
   if (e >= n) return;
   const int32_t r = ri[e], c = ci[e];
   const W x = static_cast<const W*>(v_)[e];
-  int64_t lo = bro[r], hi = bro[r + 1];  // B entries of the row before (r, c)
+  int64_t lo = bro[(int64_t)r * step], hi = bro[((int64_t)r + 1) * step];  // B entries of the row before (r, c)
   while (lo < hi) {
     const int64_t mid = (lo + hi) >> 1;
     if (LATER ? bci[mid] <= c : bci[mid] < c) lo = mid + 1; else hi = mid;
@@ -1742,8 +1814,8 @@ int ell_place(int64_t nrows, int64_t nnz, const int32_t* ri, const int32_t* ci, 
 }
 
 // The entries of a DIA part in (row, column) order, shared by DIA -> COO and
-// HDC -> COO; returns their count (and each row's first entry in rowpos, if
-// given and the part is not empty).
+// HDC -> COO; returns their count (and the first entry of each row and segment
+// (segments(nrows, ndiag)) in rowpos, if given and the part is not empty).
 template <typename W>
 int emit_dia_part_w(int64_t nrows, int64_t ncols, int64_t ndiag, int64_t pitch,
                     const int32_t* off, const void* val, int vt, int64_t cap, int32_t* ri,
@@ -1753,21 +1825,39 @@ int emit_dia_part_w(int64_t nrows, int64_t ncols, int64_t ndiag, int64_t pitch,
   Tmp t(s);
   int32_t *cnt, *htot, *hoff;
   int64_t* tmp;
-  MPH_CHECK_STATUS(t.alloc(&cnt, nrows));
-  if (!rowpos) MPH_CHECK_STATUS(t.alloc(&rowpos, nrows + 1));
-  MPH_CHECK_STATUS(t.alloc(&tmp, scan_tmp_elems(nrows)));
+  const Segs g = segments(nrows, ndiag);
+  const int64_t parts = nrows * g.n;
+  MPH_CHECK_STATUS(t.alloc(&cnt, parts));
+  if (!rowpos) MPH_CHECK_STATUS(t.alloc(&rowpos, parts + 1));
+  MPH_CHECK_STATUS(t.alloc(&tmp, scan_tmp_elems(parts)));
   DiaSlots<W> src{static_cast<const W*>(val), off, nullptr, pitch, ncols,
                   vt == MPH_I32 ? (W)~(W)0 : RawT<sizeof(W)>::mag};
-  hipLaunchKernelGGL(dia_row_count_kernel<W>, dim3(blocks_for(nrows)), dim3(kT), 0, s, src, nrows,
-                     (int32_t)ndiag, cnt);
+  hipLaunchKernelGGL(dia_row_count_kernel<W>, dim3(blocks_for(parts)), dim3(kT), 0, s, src, nrows,
+                     (int32_t)ndiag, g, cnt);
   MPH_HIP_CHECK(hipGetLastError());
-  MPH_CHECK_STATUS(exclusive_scan_i32(cnt, rowpos, nrows, tmp, s));
-  MPH_CHECK_STATUS(t.fetch(rowpos + nrows, &htot));
-  MPH_CHECK_STATUS(t.fetch(off, &hoff, ndiag));
+  MPH_CHECK_STATUS(exclusive_scan_i32(cnt, rowpos, parts, tmp, s));
+  MPH_CHECK_STATUS(t.fetch(rowpos + parts, &htot));
+  // whether the offsets ascend: on the host, which then orders the slots, or,
+  // where rows have several segments (counted in storage order) and the copy
+  // may take long, on the device, the order left to the sort
+  const bool few = g.n == 1;
+  if (few) {
+    MPH_CHECK_STATUS(t.fetch(off, &hoff, ndiag));
+  } else {
+    int32_t* d;
+    MPH_CHECK_STATUS(t.alloc(&d, 1));
+    MPH_CHECK_STATUS(fill_zero(d, sizeof(int32_t), s));
+    hipLaunchKernelGGL((coo_scan_kernel<false, false, kNoDiags>), dim3(scan_blocks(ndiag)), dim3(kT),
+                       0, s, off, (const int32_t*)nullptr, ndiag, (int64_t)INT32_MAX,
+                       (int64_t)INT32_MAX, (int32_t*)nullptr, (uint32_t*)nullptr, d);
+    MPH_HIP_CHECK(hipGetLastError());
+    MPH_CHECK_STATUS(t.fetch(d, &hoff));
+  }
   MPH_CHECK_STATUS(t.wait());
   const int64_t tot = *htot;
   if (tot > cap) return invalid("DIA holds more non-zeros than its nnz");
-  if (!std::is_sorted(hoff, hoff + ndiag)) {
+  const bool ascend = few ? std::is_sorted(hoff, hoff + ndiag) : !(*hoff & kRowsDown);
+  if (few && !ascend) {
     // slots in ascending order of the offsets, equal ones in storage order
     std::vector<int32_t> ord(ndiag);
     for (int64_t d = 0; d < ndiag; d++) ord[d] = (int32_t)d;
@@ -1786,10 +1876,9 @@ int emit_dia_part_w(int64_t nrows, int64_t ncols, int64_t ndiag, int64_t pitch,
     src.off = d_off;
   }
   if (tot > 0) {
-    hipLaunchKernelGGL((emit_rows_kernel<W, DiaSlots<W>>), dim3(blocks_for(nrows, kEmitRows)),
-                       dim3(kT), 0, s, src, nrows, (int32_t)ndiag, rowpos, ri, ci,
-                       static_cast<W*>(v));
+    emit_rows<W>(src, nrows, (int32_t)ndiag, g, rowpos, ri, ci, v, s);
     MPH_HIP_CHECK(hipGetLastError());
+    if (!few && !ascend) MPH_CHECK_STATUS(sort_coo(tot, ri, ci, v, sizeof(W), false, s));
   }
   *count = tot;
   return MPH_OK;  // (t waits for the stream)
@@ -1832,16 +1921,18 @@ int ell_part_to_coo(int64_t nrows, int64_t nnz, int64_t width, int64_t pitch, co
     Tmp t(s);
     int32_t *cnt, *rowpos, *stats, *ht, *hs;
     int64_t* tmp;
-    MPH_CHECK_STATUS(t.alloc(&cnt, nrows));
-    MPH_CHECK_STATUS(t.alloc(&rowpos, nrows + 1));
-    MPH_CHECK_STATUS(t.alloc(&tmp, scan_tmp_elems(nrows)));
+    const Segs g = segments(nrows, width);
+    const int64_t parts = nrows * g.n;
+    MPH_CHECK_STATUS(t.alloc(&cnt, parts));
+    MPH_CHECK_STATUS(t.alloc(&rowpos, parts + 1));
+    MPH_CHECK_STATUS(t.alloc(&tmp, scan_tmp_elems(parts)));
     MPH_CHECK_STATUS(t.alloc(&stats, 2));
     MPH_CHECK_STATUS(fill_zero(stats, 2 * sizeof(int32_t), s));
-    hipLaunchKernelGGL(ell_row_count_kernel, dim3(std::min(blocks_for(nrows), 2048u)), dim3(kT), 0,
-                       s, eci, nrows, width, pitch, tro, tci, cnt, stats);
+    hipLaunchKernelGGL(ell_row_count_kernel, dim3(std::min(blocks_for(parts), 2048u)), dim3(kT), 0,
+                       s, eci, nrows, width, pitch, g, tro, tci, cnt, stats);
     MPH_HIP_CHECK(hipGetLastError());
-    MPH_CHECK_STATUS(exclusive_scan_i32(cnt, rowpos, nrows, tmp, s));
-    MPH_CHECK_STATUS(t.fetch(rowpos + nrows, &ht));
+    MPH_CHECK_STATUS(exclusive_scan_i32(cnt, rowpos, parts, tmp, s));
+    MPH_CHECK_STATUS(t.fetch(rowpos + parts, &ht));
     MPH_CHECK_STATUS(t.fetch(stats, &hs, 2));
     MPH_CHECK_STATUS(t.wait());
     tot = *ht;
@@ -1851,9 +1942,8 @@ int ell_part_to_coo(int64_t nrows, int64_t nnz, int64_t width, int64_t pitch, co
     if (slots > 0) {
       auto emit = [&](auto tag) {
         using W = decltype(tag);
-        hipLaunchKernelGGL((emit_rows_kernel<W, EllSlots<W>>), dim3(blocks_for(nrows, kEmitRows)),
-                           dim3(kT), 0, s, EllSlots<W>{eci, static_cast<const W*>(ev), pitch},
-                           nrows, slots, rowpos, ri_out, ci_out, static_cast<W*>(v_out));
+        emit_rows<W>(EllSlots<W>{eci, static_cast<const W*>(ev), pitch}, nrows, slots, g, rowpos,
+                     ri_out, ci_out, v_out, s);
       };
       if (vs == 8) emit(uint64_t{});
       else if (vs == 4) emit(uint32_t{});
@@ -1861,7 +1951,7 @@ int ell_part_to_coo(int64_t nrows, int64_t nnz, int64_t width, int64_t pitch, co
     }
     if (tnnz > 0)
       MPH_LAUNCH_W(hyb_tail_emit_kernel, vs, dim3(blocks_for(tnnz)), s, tri, tci, tv, tnnz, tro,
-                   rowpos, ri_out, ci_out, v_out);
+                   rowpos, g.n, ri_out, ci_out, v_out);
     MPH_HIP_CHECK(hipGetLastError());
   }
   if (tot == nnz && sorted) return MPH_OK;
@@ -2336,7 +2426,8 @@ int mph_convert_hdc_to_coo(int64_t nrows, int64_t ncols, int64_t nnz, int64_t nd
     int32_t *dri, *dci;
     uint8_t* dv;
     const int64_t cap = std::min(nnz, nrows * ndiag);
-    MPH_CHECK_STATUS(t.alloc(&rowpos, nrows + 1));
+    const Segs dia_segs = segments(nrows, ndiag);
+    MPH_CHECK_STATUS(t.alloc(&rowpos, nrows * dia_segs.n + 1));
     MPH_CHECK_STATUS(t.alloc(&dri, cap));
     MPH_CHECK_STATUS(t.alloc(&dci, cap));
     MPH_CHECK_STATUS(t.alloc(&dv, cap * vs));
@@ -2344,10 +2435,10 @@ int mph_convert_hdc_to_coo(int64_t nrows, int64_t ncols, int64_t nnz, int64_t nd
                                    rowpos, &nd, s));
     if (nd + csr_nnz > nnz) return invalid("HDC holds more entries than its nnz");
     if (nd > 0)
-      MPH_LAUNCH_BW(merge_rows_kernel, false, vs, dim3(blocks_for(nd)), s, dri, dci, dv, nd, csr_ro,
+      MPH_LAUNCH_BW(merge_rows_kernel, false, vs, dim3(blocks_for(nd)), s, dri, dci, dv, nd, csr_ro, 1,
                     csr_ci, ri_out, ci_out, v_out);
     MPH_LAUNCH_BW(merge_rows_kernel, true, vs, dim3(blocks_for(csr_nnz)), s, crow, csr_ci, csr_v,
-                  csr_nnz, rowpos, dci, ri_out, ci_out, v_out);
+                  csr_nnz, rowpos, dia_segs.n, dci, ri_out, ci_out, v_out);
     MPH_HIP_CHECK(hipGetLastError());
     in_order = true;
   } else {

@@ -236,3 +236,104 @@ def test_offsets_take_time_by_entries_and_rows(gpu, order):
     assert torch.equal(B.arrays["ro"], ro.int())
     assert torch.equal(B.arrays["v"], ri.sort(stable=True).values.double())
     assert min(ms) < (1.2 if order == "ends" else 4)
+
+
+def _wide(nrows, per, ncols, seed):
+    """`per` distinct columns a row (fewer in every third row), in order."""
+    rng = np.random.default_rng(seed)
+    lens = [per - (per // 2 if r % 3 == 1 else 0) for r in range(nrows)]
+    cols = [np.sort(rng.choice(ncols, n, replace=False)) for n in lens]
+    rows = np.repeat(np.arange(nrows), lens)
+    return Coo(nrows, ncols, rows, np.concatenate(cols), 1.0 + np.arange(rows.size) % 200)
+
+
+@pytest.mark.parametrize("nrows", [1, 2, 7, 63, 64, 65, 130])
+@pytest.mark.parametrize("per", [224, 256, 257, 480, 513, 1100])
+@pytest.mark.parametrize("dtype", ["f64", "bf16"])
+def test_long_rows(gpu, nrows, per, dtype):
+    """Few rows of many slots and diagonals: segments of 256, their ends, rows
+    fewer than a wave's lanes and more."""
+    A = _wide(nrows, per, 1300, nrows + per)
+    for fmt in COO_TARGETS:
+        try:
+            B = oracle.from_coo(round_values(A, dtype), fmt)
+        except oracle.OracleError:  # (HDC's midpoint on some shapes that are not square)
+            continue
+        _check(A, fmt, dtype)
+        _check(B, COO_FORMAT, dtype)
+
+
+@pytest.mark.parametrize("nrows", [3, 70])
+def test_long_rows_with_holes(gpu, nrows):
+    """ELL slots left empty before, inside and after a segment's start, and
+    columns that step back where the empty slots hide the one before."""
+    import torch
+    rng = np.random.default_rng(nrows)
+    width = 900
+    ci = np.sort(rng.choice(5000, (nrows, width)), axis=1).astype(np.int32)
+    ci[0, 100:400] = -1
+    ci[1, 250:260] = -1
+    ci[2, 256:] = -1
+    ci[nrows - 1, 300] = 4999
+    v = 1.0 + np.arange(nrows * width).reshape(nrows, width)
+    keep = ci.ravel() >= 0
+    rows = np.repeat(np.arange(nrows), width)[keep]
+    cols, vals = ci.ravel()[keep], v.ravel()[keep]
+    at = np.lexsort((cols, rows))  # stable
+    e = [torch.from_numpy(np.ascontiguousarray(a.T.ravel())).cuda() for a in (ci, v)]
+    out = [torch.empty(rows.size, dtype=t, device="cuda")
+           for t in (torch.int32, torch.int32, torch.float64)]
+    capi.call("mph_convert_ell_to_coo", nrows, rows.size, width, nrows, e[0].data_ptr(),
+              e[1].data_ptr(), capi.F64, *(t.data_ptr() for t in out), device.stream_handle())
+    for got, want in zip(out, (rows[at], cols[at], vals[at])):
+        assert np.array_equal(got.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("order", ["ascending", "descending", "repeated"])
+@pytest.mark.parametrize("ndiag", [255, 256, 257, 512, 513, 9000])
+def test_many_diagonals(gpu, ndiag, order):
+    """Offsets whose order is looked at on the host and on the device."""
+    n = 20
+    off = np.arange(ndiag) - 10
+    if order == "descending":
+        off = off[::-1]
+    elif order == "repeated":
+        off = np.sort(off // 2)
+        off[[5, 9]] = off[[9, 5]]
+    pitch = 32
+    val = np.zeros(pitch * ndiag)
+    for r in range(n):
+        d = np.arange(r, ndiag, 3)
+        d = d[(r + off[d] >= 0) & (r + off[d] < ndiag)]
+        val[d * pitch + r] = 1.0 + (d * 7 + r) % 250
+    D = Dia(n, ndiag, int(np.count_nonzero(val)), off.astype(np.int32), val, pitch)
+    _check(D, COO_FORMAT)
+
+
+@pytest.mark.parametrize("nrows,ncols", [(1, 2_000_000), (4, 500_000), (100, 20_000)])
+def test_long_rows_take_time_by_entries(gpu, nrows, ncols):
+    """A full matrix of a few long rows: a lane, thread or workgroup for each
+    took 1.5 to 500 ms a conversion."""
+    import torch
+    nnz = nrows * ncols
+    at = torch.arange(nnz, device="cuda")
+    A = device.DeviceMatrix(COO_FORMAT, nrows, ncols, nnz, "f64",
+                            dict(ri=(at // ncols).int(), ci=(at % ncols).int(),
+                                 v=1.0 + (at % 1000).double()), {})
+    for fmt in (DIA_FORMAT, ELL_FORMAT, HYB_FORMAT):
+        try:
+            B = device.from_coo(A, fmt)
+        except capi.FormatConversionException:
+            continue
+        for f in (lambda: device.from_coo(A, fmt), lambda: device.to_coo(B)):
+            ms = []
+            for _ in range(4):
+                t = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+                t[0].record()
+                C2 = f()
+                t[1].record()
+                t[1].synchronize()
+                ms.append(t[0].elapsed_time(t[1]))
+            limit = 6 if fmt == DIA_FORMAT else 1.2
+            assert min(ms) < limit, (fmt, ms)
+        assert all(torch.equal(C2.arrays[k], A.arrays[k]) for k in ("ri", "ci", "v"))
