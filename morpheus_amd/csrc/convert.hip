@@ -163,23 +163,39 @@ __global__ void first_descent_kernel(const int32_t* __restrict__ ri, int64_t n,
 // 8 B an entry once, where the range checks, the sortedness test and a row
 // histogram (an LDS hash table: 6 ps an entry) each were a pass.  With
 // indices out of range, or rows that decrease, ro is incomplete; every write
-// stays inside it.  More than kLongGap rows without an entry are left out and
+// stays inside it.  More than kFarGap rows without an entry are left out and
 // raise kGaps, for gap_offsets_kernel: filled here, each by the lane or wave
 // that met it, the gaps of rows in no order came to a third of the rows an
 // entry (2M shuffled entries on 1M rows 127 ms), and one gap of 4M rows took
-// 1.8 ms.
+// 1.8 ms.  (The COO part of a power-law HYB has gaps of more than 32 rows, none
+// that far: left out too, they cost the other kernel 40 us on 1M rows.)
 constexpr int32_t kBadRow = 1, kBadCol = 2, kRowsDown = 4, kUnsorted = 8, kRepeated = 16,
                   kGaps = 32;
 constexpr int kScanPer = 8;  // entries per thread
 constexpr int kScanTile = kT * kScanPer;
-constexpr int64_t kLongGap = 32;
+constexpr uint32_t kLongGap = 32, kFarGap = 1024;
 
-// rows (lo, hi] start at entry i
-__device__ __forceinline__ int32_t fill_offsets(int32_t* __restrict__ ro, int64_t lo, int64_t hi,
-                                                int32_t i) {
-  if (hi - lo > kLongGap) return kGaps;
-  for (int64_t r = lo + 1; r <= hi; r++) ro[r] = i;
-  return 0;
+// The `gap` rows up to `row` start at entry i: by the lane, long gaps by the
+// whole wave, unless one of its lanes saw rows decrease (ro is not used then).
+__device__ __forceinline__ void fill_offsets(int32_t* __restrict__ ro, int32_t row, uint32_t gap,
+                                             int32_t i, bool down, int32_t& bad) {
+  const bool lng = gap > kLongGap;
+  if (!lng) {
+    int32_t* p = ro + row - gap;
+    for (uint32_t k = 1; k <= gap; k++) p[k] = i;
+  }
+  uint64_t m = __ballot(lng && gap <= kFarGap);
+  if (lng && gap > kFarGap) bad |= kGaps;
+  if (m == 0 || __ballot(down) != 0) return;
+  const int lane = threadIdx.x % kWave;
+  while (m) {
+    const int src = __ffsll((unsigned long long)m) - 1;
+    m &= m - 1;
+    int32_t* p = ro + (int64_t)shfl(row, src) - shfl(gap, src);
+    const uint32_t n = shfl(gap, src);
+    const int32_t at = shfl(i, src);
+    for (uint32_t k = 1 + lane; k <= n; k += kWave) p[k] = at;
+  }
 }
 
 // Sets the bits of `bad` that any thread of the workgroup has; a word that
@@ -350,12 +366,10 @@ __global__ __launch_bounds__(kT) void coo_scan_kernel(
         }
       }
       if (OFFSETS) {
-        // (a wave that sees rows decrease leaves them: ro is not used then)
-        if (__ballot(in && i > 0 && pr > r[k]) == 0) {
-          const int64_t hi = in && row_ok ? r[k] : 0;
-          const int64_t lo = in && row_ok ? (i == 0 ? -1 : min((int64_t)max(pr, -1), hi)) : 0;
-          bad |= fill_offsets(ro, lo, hi, (int32_t)i);
-        }
+        const int32_t before = i == 0 ? -1 : max(pr, -1);
+        const bool up = in && row_ok && before < r[k];
+        fill_offsets(ro, r[k], up ? (uint32_t)r[k] - (uint32_t)before : 0u, (int32_t)i,
+                     in && i > 0 && pr > r[k], bad);
         if (in && i == nnz - 1 && row_ok) last = r[k];
       }
       const int32_t key = (int32_t)((int64_t)c[k] - r[k] + nrows - 1);
@@ -364,8 +378,12 @@ __global__ __launch_bounds__(kT) void coo_scan_kernel(
         count_keys(reinterpret_cast<int32_t*>(diags), seen, seen_n, key, in && row_ok && col_ok);
     }
   }
-  if (OFFSETS)  // the rows after the last entry's
-    bad |= fill_offsets(ro, last >= -1 ? last : 0, last >= -1 ? nrows : 0, (int32_t)nnz);
+  if (OFFSETS && last >= -1) {  // the rows after the last entry's, by its lane
+    if (nrows - last > kFarGap)
+      bad |= kGaps;
+    else
+      for (int64_t q = last + 1; q <= nrows; q++) ro[q] = (int32_t)nnz;
+  }
   raise_flags(flags, bad);
   if (DIAGS == kWidths) {
     raise_flags(flags + 1, wide_r);
@@ -872,25 +890,28 @@ Segs segments(int64_t nrows, int64_t slots) {
   return {(int32_t)len, (int32_t)ceil_div(slots, len)};
 }
 
-// the row and segment of thread t: rows next to each other
-__device__ __forceinline__ void row_segment(int64_t t, int64_t nrows, const Segs& g, int64_t& r,
-                                            int32_t& y) {
-  y = g.n > 1 ? (int32_t)(t / nrows) : 0;
+// The row and segment of thread t: rows next to each other.  (The kernels over
+// rows of one segment are instances of their own, SEGS false: the segments
+// took them registers and 3 to 5% of their time.)
+template <bool SEGS>
+__device__ __forceinline__ void row_segment(int64_t t, int64_t nrows, int64_t& r, int32_t& y) {
+  y = SEGS ? (int32_t)(t / nrows) : 0;
   r = t - (int64_t)y * nrows;
 }
 
-template <typename W>
+template <bool SEGS, typename W>
 __global__ __launch_bounds__(kT) void dia_row_count_kernel(DiaSlots<W> src, int64_t nrows,
                                                            int32_t ns, Segs g,
                                                            int32_t* __restrict__ cnt) {
+  using I = std::conditional_t<SEGS, int64_t, int32_t>;
   const int64_t t = (int64_t)blockIdx.x * kT + threadIdx.x;
-  if (t >= nrows * g.n) return;
+  if (t >= (SEGS ? nrows * g.n : nrows)) return;
   int64_t r;
   int32_t y;
-  row_segment(t, nrows, g, r, y);
+  row_segment<SEGS>(t, nrows, r, y);
   int32_t n = 0;
-  const int64_t end = min((int64_t)ns, ((int64_t)y + 1) * g.len);
-  for (int64_t s0 = (int64_t)y * g.len; s0 < end; s0 += kScanPer) {
+  const I end = SEGS ? (I)min((int64_t)ns, ((int64_t)y + 1) * g.len) : (I)ns;
+  for (I s0 = SEGS ? (I)y * g.len : 0; s0 < end; s0 += kScanPer) {
     W v[kScanPer];
     bool ok[kScanPer];
     int32_t c;
@@ -905,12 +926,12 @@ __global__ __launch_bounds__(kT) void dia_row_count_kernel(DiaSlots<W> src, int6
       n += ok[k] ? 1 : 0;
     }
   }
-  cnt[r * g.n + y] = n;
+  cnt[SEGS ? r * g.n + y : r] = n;
 }
 
-// The entries of 64 rows' segments a workgroup: lane = row, of the segment
-// blockIdx.y, or, with fewer rows than lanes (NARROW), lane = one of 64
-// consecutive (row, segment); each wave a quarter of the slots, batches of 32
+// The entries of 64 rows' segments a workgroup: lane = row (kWhole: of one
+// segment), of the segment blockIdx.y (kSegment), or, with fewer rows than
+// lanes, lane = one of 64 consecutive (row, segment) (kNarrow); each wave a quarter of the slots, batches of 32
 // slots.  The entries are staged in LDS in output order and written coalesced
 // (written from the row walk, each store of a wave spreads over 64 rows'
 // entries); those of segment q = (row, segment) go to rowpos[q], rowpos[q] + 1,
@@ -921,7 +942,9 @@ constexpr int kEmitWaves = kT / kWave;
 constexpr int kEmitPer = 8;  // slots per lane and batch
 constexpr int kEmitBatch = kEmitWaves * kEmitPer;
 
-template <typename W, typename Src, bool NARROW>
+enum EmitBy { kWhole, kSegment, kNarrow };
+
+template <EmitBy BY, typename W, typename Src>
 __global__ __launch_bounds__(kT) void emit_rows_kernel(Src src, int64_t nrows, int32_t ns, Segs g,
                                                        const int32_t* __restrict__ rowpos,
                                                        int32_t* __restrict__ ri,
@@ -934,24 +957,26 @@ __global__ __launch_bounds__(kT) void emit_rows_kernel(Src src, int64_t nrows, i
   __shared__ int32_t dst[kEmitRows];  // output position of the row's first entry, less its LDS place
   __shared__ int32_t total;
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+  constexpr bool NARROW = BY == kNarrow;
+  using I = std::conditional_t<NARROW, int64_t, int32_t>;  // (a segment may end past the slots)
   __shared__ int32_t srow[NARROW ? kEmitRows : 1];
   const int64_t r0 = (int64_t)blockIdx.x * kEmitRows;
   int64_t r = r0 + lane;
-  int32_t first_slot = (int32_t)blockIdx.y * g.len, seg = (int32_t)blockIdx.y;
+  int32_t seg = BY == kSegment ? (int32_t)blockIdx.y : 0;
   if (NARROW) {
     const int64_t q = r;
     r = q / g.n;
     seg = (int32_t)(q - r * g.n);
-    first_slot = seg * g.len;
     if (wave == 0) srow[lane] = (int32_t)r;  // (read after the barriers below)
   }
-  int32_t pos = r < nrows ? rowpos[r * g.n + seg] : 0;
-  const int32_t len = NARROW ? g.len : min(g.len, ns - first_slot);
+  const int32_t first_slot = BY == kWhole ? 0 : seg * g.len;
+  const int32_t len = NARROW ? g.len : BY == kSegment ? min(g.len, ns - first_slot) : ns;
+  int32_t pos = r < nrows ? rowpos[BY == kWhole ? r : r * g.n + seg] : 0;
   for (int s0 = 0; s0 < len; s0 += kEmitBatch) {
     // the batch's slots in order over the waves
     const int per = (min(kEmitBatch, len - s0) + kEmitWaves - 1) / kEmitWaves;
-    const int64_t sl = (int64_t)first_slot + s0, sb = sl + wave * per;
-    const int64_t se = min(min(sb + per, sl + kEmitBatch), min((int64_t)ns, (int64_t)first_slot + len));
+    const I sl = (I)first_slot + s0, sb = sl + wave * per;
+    const I se = min(min((I)(sb + per), (I)(sl + kEmitBatch)), min((I)ns, (I)((I)first_slot + len)));
     W v[kEmitPer];
     int32_t c[kEmitPer];
     bool ok[kEmitPer];
@@ -1008,14 +1033,20 @@ __global__ __launch_bounds__(kT) void emit_rows_kernel(Src src, int64_t nrows, i
 
 template <typename W, typename Src>
 void emit_rows(const Src& src, int64_t nrows, int32_t ns, const Segs& g, const int32_t* rowpos,
-               int32_t* ri, int32_t* ci, void* v, hipStream_t s) {
-  if (g.n > 1 && nrows < kEmitRows)
-    hipLaunchKernelGGL((emit_rows_kernel<W, Src, true>), dim3(blocks_for(nrows * g.n, kEmitRows)),
-                       dim3(kT), 0, s, src, nrows, ns, g, rowpos, ri, ci, static_cast<W*>(v));
+               int32_t* ri, int32_t* ci, void* v_, hipStream_t s) {
+  W* v = static_cast<W*>(v_);
+  const unsigned gx = blocks_for(nrows, kEmitRows);
+  if (g.n == 1)
+    hipLaunchKernelGGL((emit_rows_kernel<kWhole, W, Src>), dim3(gx), dim3(kT), 0, s, src, nrows, ns,
+                       g, rowpos, ri, ci, v);
+  else if (nrows < kEmitRows)
+    hipLaunchKernelGGL((emit_rows_kernel<kNarrow, W, Src>),
+                       dim3(blocks_for(nrows * g.n, kEmitRows)), dim3(kT), 0, s, src, nrows, ns, g,
+                       rowpos, ri, ci, v);
   else
-    hipLaunchKernelGGL((emit_rows_kernel<W, Src, false>),
-                       dim3(blocks_for(nrows, kEmitRows), (unsigned)ceil_div(ns, g.len)), dim3(kT),
-                       0, s, src, nrows, ns, g, rowpos, ri, ci, static_cast<W*>(v));
+    hipLaunchKernelGGL((emit_rows_kernel<kSegment, W, Src>),
+                       dim3(gx, (unsigned)ceil_div(ns, g.len)), dim3(kT), 0, s, src, nrows, ns, g,
+                       rowpos, ri, ci, v);
 }
 
 // zero the COO slots [from, nnz) left unfilled
@@ -1038,19 +1069,21 @@ __global__ void zero_tail_kernel(int64_t from, int64_t nnz, int32_t* ri, int32_t
 // kSegBack slots back for the column before its first; not finding one counts
 // as out of order (the list is then sorted, whatever its order).
 constexpr int kSegBack = 64;
+template <bool SEGS>
 __global__ __launch_bounds__(kT) void ell_row_count_kernel(
     const int32_t* __restrict__ eci, int64_t nrows, int64_t width, int64_t pitch, Segs g,
     const int32_t* __restrict__ tro, const int32_t* __restrict__ tci, int32_t* __restrict__ cnt,
     int32_t* __restrict__ stats) {
   int32_t bad = 0, top = 0;
-  for (int64_t t = (int64_t)blockIdx.x * kT + threadIdx.x; t < nrows * g.n;
+  for (int64_t t = (int64_t)blockIdx.x * kT + threadIdx.x; t < (SEGS ? nrows * g.n : nrows);
        t += (int64_t)gridDim.x * kT) {
     int64_t r;
     int32_t y;
-    row_segment(t, nrows, g, r, y);
+    row_segment<SEGS>(t, nrows, r, y);
     int32_t n = 0, prev = INT32_MIN;
-    const int64_t begin = (int64_t)y * g.len, end = min(width, begin + g.len);
-    bool known = y == 0;
+    const int64_t begin = SEGS ? (int64_t)y * g.len : 0;
+    const int64_t end = SEGS ? min(width, begin + g.len) : width;
+    bool known = !SEGS || y == 0;
     for (int64_t b = begin - 1; !known && b >= max(begin - kSegBack, (int64_t)0); b--) {
       const int32_t c = eci[r + pitch * b];
       known = c != -1;
@@ -1064,18 +1097,18 @@ __global__ __launch_bounds__(kT) void ell_row_count_kernel(
       for (int k = 0; k < kScanPer; k++)
         if (c[k] != -1) {
           bad |= c[k] < prev || !known ? 1 : 0;
-          known = true;
+          if (SEGS) known = true;
           prev = c[k];
           n++;
           top = max(top, (int32_t)(s0 + k) + 1);
         }
     }
-    if (tro && y == g.n - 1) {
+    if (tro && (!SEGS || y == g.n - 1)) {
       const int32_t ts = tro[r], te = tro[r + 1];
-      if (te > ts && ((y > 0 && !known) || (prev != INT32_MIN && tci[ts] < prev))) bad = 1;
+      if (te > ts && (!known || (prev != INT32_MIN && tci[ts] < prev))) bad = 1;
       n += te - ts;
     }
-    cnt[r * g.n + y] = n;
+    cnt[SEGS ? r * g.n + y : r] = n;
   }
   raise_flags(&stats[0], bad);
   top = block_reduce(top, [](int32_t u, int32_t v) { return max(u, v); });
@@ -1832,8 +1865,9 @@ int emit_dia_part_w(int64_t nrows, int64_t ncols, int64_t ndiag, int64_t pitch,
   MPH_CHECK_STATUS(t.alloc(&tmp, scan_tmp_elems(parts)));
   DiaSlots<W> src{static_cast<const W*>(val), off, nullptr, pitch, ncols,
                   vt == MPH_I32 ? (W)~(W)0 : RawT<sizeof(W)>::mag};
-  hipLaunchKernelGGL(dia_row_count_kernel<W>, dim3(blocks_for(parts)), dim3(kT), 0, s, src, nrows,
-                     (int32_t)ndiag, g, cnt);
+  auto row_count = g.n > 1 ? dia_row_count_kernel<true, W> : dia_row_count_kernel<false, W>;
+  hipLaunchKernelGGL(row_count, dim3(blocks_for(parts)), dim3(kT), 0, s, src, nrows, (int32_t)ndiag, g,
+                     cnt);
   MPH_HIP_CHECK(hipGetLastError());
   MPH_CHECK_STATUS(exclusive_scan_i32(cnt, rowpos, parts, tmp, s));
   MPH_CHECK_STATUS(t.fetch(rowpos + parts, &htot));
@@ -1928,8 +1962,9 @@ int ell_part_to_coo(int64_t nrows, int64_t nnz, int64_t width, int64_t pitch, co
     MPH_CHECK_STATUS(t.alloc(&tmp, scan_tmp_elems(parts)));
     MPH_CHECK_STATUS(t.alloc(&stats, 2));
     MPH_CHECK_STATUS(fill_zero(stats, 2 * sizeof(int32_t), s));
-    hipLaunchKernelGGL(ell_row_count_kernel, dim3(std::min(blocks_for(parts), 2048u)), dim3(kT), 0,
-                       s, eci, nrows, width, pitch, g, tro, tci, cnt, stats);
+    auto count = g.n > 1 ? ell_row_count_kernel<true> : ell_row_count_kernel<false>;
+    hipLaunchKernelGGL(count, dim3(std::min(blocks_for(parts), 2048u)), dim3(kT), 0, s, eci, nrows,
+                       width, pitch, g, tro, tci, cnt, stats);
     MPH_HIP_CHECK(hipGetLastError());
     MPH_CHECK_STATUS(exclusive_scan_i32(cnt, rowpos, parts, tmp, s));
     MPH_CHECK_STATUS(t.fetch(rowpos + parts, &ht));

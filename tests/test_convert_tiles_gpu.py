@@ -186,12 +186,13 @@ def test_long_scans(gpu, nrows):
     assert torch.equal(ri, rows.int()) and torch.equal(co, ci[rows]) and torch.equal(vo, v[rows])
 
 
-@pytest.mark.parametrize("gap", [31, 32, 33, 34, 2047, 2048, 2049, 7000])
+@pytest.mark.parametrize("gap", [31, 32, 33, 95, 1023, 1024, 1025, 2048, 7000])
 @pytest.mark.parametrize("where", ["first", "middle", "last", "all"])
 @pytest.mark.parametrize("fmt", [CSR_FORMAT, HYB_FORMAT, HDC_FORMAT])
 def test_gaps_between_rows(gpu, gap, where, fmt):
-    """Rows without entries about the lengths where a scan of the entries no
-    longer fills their offsets (32 rows) and of the tiles that do (2048)."""
+    """Rows without entries about the lengths up to which the scan of the
+    entries fills their offsets by lanes (32) and by waves (1024 rows), and of
+    the tiles that are filled afterwards (2048)."""
     lead, mid, tail = (gap if where in (w, "all") else 0 for w in ("first", "middle", "last"))
     a = lead + np.arange(300)
     rows = np.r_[a, a[-1] + 1 + mid + np.arange(40)]
