@@ -291,10 +291,11 @@ int mph_ell_multiply(int64_t nrows, int64_t ncols, int64_t nnz,
  * HIP converters throw NotImplementedException
  * (core/src/impl/Csr/HIP/Morpheus_Convert_Impl.hpp:39-76); these succeed.
  * Size queries synchronise `stream`; fills may be asynchronous, and use
- * temporary arrays of the library's own, which keeps up to 2 GiB of them
- * until mph_finalize; a call whose temporaries the device still reads waits
- * for `stream` before it returns.  Output arrays are caller-owned and sized
- * from the size queries; every entry is written.
+ * temporary arrays of the library's own, which keeps up to 2 GiB of them a
+ * device (those unused longest make room) until mph_finalize, or until one of
+ * its allocations finds no memory; a call whose temporaries the device still
+ * reads waits for `stream` before it returns.  Output arrays are caller-owned
+ * and sized from the size queries; every entry is written.
  * Between CSR and COO, ci_out and v_out may be the input's ci and v: the
  * entries then stay where they are (or, COO rows not sorted, are sorted in
  * place). */

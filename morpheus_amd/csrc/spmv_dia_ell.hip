@@ -578,9 +578,10 @@ __global__ __launch_bounds__(256) void dia_spmm_slide_kernel(DiaArgs<V> a) {
 // requested before the current one is summed, and the offsets come 64 at a
 // time into a register, the runs cut from it with scalar code (read from
 // memory, a run's offsets were a chain of round trips).  27-point 160^3,
-// FP64: 16 columns 632 -> 537 us (3.6 TB/s of X, Y and values once each), 8
-// columns 412 -> 324 us; FP32, 16 columns 365 -> 293 us.  VGPRs hold four
-// waves to a SIMD; compiled for five it spills (927 us).
+// FP64: 16 columns 632 -> 531 us (3.6 TB/s of X, Y and values once each; the
+// L1's return path is still busy 92% of the time), 8 columns 412 -> 324 us;
+// FP32, 16 columns 365 -> 293 us.  VGPRs hold four waves to a SIMD; compiled
+// for five it spills (927 us).
 template <typename V, int KL, int R>
 __global__ __launch_bounds__(256) void dia_spmm_runs_kernel(DiaArgs<V> a) {
   using Acc = typename vtraits<V>::acc;
@@ -1107,7 +1108,7 @@ int launch_ell_k(mph_matrix_impl* A, const void* x, void* y, int ld, int init,
 //    (5-point 1000^2 FP64 21.0 -> 24.8).
 //  * The staged form requests a run ahead, and four of its workgroups fit a
 //    CU: it wins from 3 a CU in FP64 (slide against staged: 27-point 160^3
-//    k = 16 632 -> 537 us; 500k rows, 9 diagonals, k = 8 28.0 -> 21.3) or 2
+//    k = 16 632 -> 531 us; 500k rows, 9 diagonals, k = 8 28.0 -> 21.3) or 2
 //    with 9 diagonals or more (131k rows, k = 8 9.8 -> 8.0), and in FP32 where
 //    its last round is full (9 diagonals, k = 32, 1024 workgroups 12.2 -> 10.4;
 //    1563: 17.2 -> 17.8; 3907: 37.6 -> 34.8), with 16 lanes later (27-point

@@ -2125,18 +2125,6 @@ void xtile_release(XTilePlan& xp) {
 
 namespace {
 
-// The split SpMV plan of CSR / HYB / HDC, built on the host around the
-// x-tiled rows:
-// * x-tiling on: rows longer than kXTileMinRowLen go to the x-tiled pass;
-// * HYB / HDC with x-tiling on or at least kSplitMinRows rows: the ELL / DIA
-//   part of every row is computed first by its own coalesced pass, and the
-//   rows whose tail / CSR part is non-empty form a compacted row list (list
-//   row i is matrix row map[i]; its items start at offset lro[i], and
-//   lro[i + 1] ends them, since the rows left out hold no items).
-// Over the list (all rows for CSR), a tiled row becomes a {row, -2} record
-// the kernel skips, a row longer than the chunk that the pass does not take
-// keeps its position chunks, and the other rows form short blocks with the
-// usual limits; the records are checked before upload.
 // per row, 1 + its last ELL slot holding a column (0 without any)
 __global__ void ell_count_kernel(const int32_t* __restrict__ eci, int64_t pitch, int64_t loop,
                                  int64_t nrows, uint8_t* __restrict__ cnt) {
@@ -2179,6 +2167,18 @@ int ell_counts(mph_matrix_impl* A, hipStream_t s) {
   return MPH_OK;
 }
 
+// The split SpMV plan of CSR / HYB / HDC, built on the host around the
+// x-tiled rows:
+// * x-tiling on: rows longer than kXTileMinRowLen go to the x-tiled pass;
+// * HYB / HDC with x-tiling on or at least kSplitMinRows rows: the ELL / DIA
+//   part of every row is computed first by its own coalesced pass, and the
+//   rows whose tail / CSR part is non-empty form a compacted row list (list
+//   row i is matrix row map[i]; its items start at offset lro[i], and
+//   lro[i + 1] ends them, since the rows left out hold no items).
+// Over the list (all rows for CSR), a tiled row becomes a {row, -2} record
+// the kernel skips, a row longer than the chunk that the pass does not take
+// keeps its position chunks, and the other rows form short blocks with the
+// usual limits; the records are checked before upload.
 int split_analyse(mph_matrix_impl* A, const int32_t* d_ro, hipStream_t s) {
   RowBlockPlan& p = A->rb;
   const int64_t nrows = A->nrows;
@@ -2738,7 +2738,8 @@ int launch_spmm(mph_matrix_impl* A, int k, const void* x, void* y, int init,
   // split k into column groups of 16, 8 and what is left (1..7), sharing the
   // leading dim k: the rest in one pass, since a pass reads the whole matrix
   // and gathers the same lines of X again (k = 5 as 4 + 1 on a 2M-row
-  // power-law(1.2) matrix, FP32: the short rows 148 + 140 us, as 5 144 us)
+  // power-law(1.2) matrix, FP32: the short rows 148 + 140 us, as 5 144 us).
+  // The x-tiled rows have their own groups, of 4, 2 and single columns, below.
   int done = 0;
   while (done < k) {
     const int rem = k - done;
