@@ -34,6 +34,20 @@ def log(*a):
     print(*a, file=sys.stderr, flush=True)
 
 
+# the long tables of the result
+TABLES = ("precision_sweep", "large_configs")
+
+
+def emit(line):
+    """The result: one JSON line on stdout.  The long tables, 13 of its 20 kB
+    and more than a reader of the line may keep, go to stderr as a JSON line
+    of their own before it."""
+    tables = {k: line[k] for k in TABLES if line.get(k) is not None}
+    if tables:
+        log(json.dumps(tables))
+    print(json.dumps({k: v for k, v in line.items() if k not in tables}), flush=True)
+
+
 def parse():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -1192,7 +1206,7 @@ def main():
     }
     if large is not None:
         line["large_configs"] = large
-    print(json.dumps(line), flush=True)
+    emit(line)
 
 
 if __name__ == "__main__":
